@@ -9,7 +9,7 @@
 // decompressor: a code emits its symbol, an escape (255) emits the next byte
 // literally, a trailing escape is dropped (fsst.cu:273-281).
 //
-// One 256-thread workgroup decodes one chunk of up to FSST_CHUNK_ROWS rows.
+// One 512-thread workgroup decodes one chunk of up to FSST_CHUNK_ROWS rows.
 // Chunks are numbered in column row order and claimed in that order (an
 // atomic ticket or the position in a claimed work queue), so a chunk only
 // ever waits on chunks already running: each chunk publishes its
@@ -17,16 +17,17 @@
 // exclusive prefix (a decoupled look-back), writes its rows' int32 offsets
 // and then its chars.
 //
-// The chunk's compressed bytes are staged in LDS once and walked twice, in
-// storage order, by spans: thread t takes the t-th 16-byte-aligned slice of
-// the staged bytes whatever rows it cuts, so every lane of a wave does the
-// same number of byte steps however the row lengths vary.  The first walk
-// sums decoded lengths and records, at every 16-byte grid point, the walk
-// state (decoded prefix, escape flag, row); the second walk restarts from
-// those states and ORs each symbol into a zeroed LDS copy of the chunk's
-// output, which leaves in 16-byte stores.  Chunks whose compressed bytes do
-// not fit the stage, malformed ones and rows longer than the output window
-// take a row-per-thread path that reads global memory.
+// A chunk's compressed bytes are one contiguous range (rows are stored back
+// to front), cut on a 16-byte grid into groups that are spread over the
+// threads whatever rows they cut, and held in registers between two walks.
+// The first walk looks up the decoded length of every byte and leaves, per
+// group, their prefix sums (packed bytes) and, per row, the prefix at the
+// row's first byte; the second ORs every symbol into a zeroed LDS copy of the
+// chunk's output, which leaves in 16-byte stores.  Neither walk follows rows
+// byte by byte: a bitmap holds the row starts, and a byte's row is the
+// population count of the bits up to it.  Chunks whose compressed bytes do
+// not fit the registers and malformed ones take a row-per-thread path that
+// reads global memory.
 #pragma once
 
 #include "sdr_device.hpp"
@@ -34,9 +35,11 @@
 
 namespace sdr {
 
-constexpr uint32_t FSST_THREADS   = 256;
+constexpr uint32_t FSST_THREADS   = 512;  // a chunk's workgroup
 constexpr uint32_t FSST_WAVES     = FSST_THREADS / WAVE;
 constexpr uint32_t ROWS_PER_THR   = FSST_CHUNK_ROWS / FSST_THREADS;
+constexpr uint32_t PREP_THREADS   = 256;  // the segment pre-passes' workgroups: one symbol code per thread
+constexpr uint32_t PREP_WAVES     = PREP_THREADS / WAVE;
 constexpr uint32_t FSST_PIECE     = 8192;  // LDS output piece of the row-wise path
 constexpr uint32_t FSST_ESC       = 255;
 constexpr uint32_t FSST_NSYM      = 255;
@@ -107,22 +110,6 @@ struct BitCursor {
   }
 };
 
-// Sum of the w-bit fields [i0, i1) of the stream at `base`; the fields must
-// lie inside [base, end) or the slow bounded reader is used.
-__device__ __forceinline__ uint32_t sum_fields(const uint8_t* base, const uint8_t* end, uint32_t i0, uint32_t i1,
-                                               uint32_t w)
-{
-  if (i0 >= i1 || w == 0) return 0;
-  uint32_t s = 0;
-  if (base + ((uint64_t{i1} * w + 7u) >> 3) <= end) {
-    BitCursor bc(base, uint64_t{i0} * w);
-    for (uint32_t i = i0; i < i1; ++i) s += bc.next(w);
-  } else {
-    for (uint32_t i = i0; i < i1; ++i) s += stream_bits32(base, end, uint64_t{i} * w, w);
-  }
-  return s;
-}
-
 // Sequential byte reader over global bytes [p, p + n) using aligned 4-byte loads.
 struct ByteReader {
   gptr<const uint32_t> w;
@@ -150,83 +137,101 @@ struct ByteReader {
 // tell apart from register loads.)
 __device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// Block-wide exclusive scan of one value per thread; returns the exclusive
-// prefix and writes the block total to *total.  LdsOnly: its barriers leave
-// global loads in flight.
-template <bool LdsOnly = false>
+// Block-wide exclusive scan of one value per thread (NW wavefronts); returns
+// the exclusive prefix and writes the block total to *total.
+template <uint32_t NW = FSST_WAVES>
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* s_wave, uint32_t* total)
 {
   const uint32_t incl = wave_incl_sum_u32(v);
   const uint32_t w    = threadIdx.x >> 6;
   if (lane_id() == 63) s_wave[w] = incl;
-  if constexpr (LdsOnly) lds_barrier();
-  else __syncthreads();
+  __syncthreads();
   uint32_t before = 0, tot = 0;
 #pragma unroll
-  for (uint32_t k = 0; k < FSST_WAVES; ++k) {
+  for (uint32_t k = 0; k < NW; ++k) {
     const uint32_t x = s_wave[k];
     before += k < w ? x : 0u;
     tot += x;
   }
-  if constexpr (LdsOnly) lds_barrier();
-  else __syncthreads();
+  __syncthreads();
   *total = tot;
   return before + incl - v;
 }
 
-// Shared memory of one chunk decode.
+// Exclusive scans of two values per thread with one barrier, for LDS alone
+// (global loads stay in flight); s_wave[2 * FSST_WAVES] must not be written
+// again before the caller's next barrier.
+__device__ __forceinline__ void block_excl_scan2(uint32_t a, uint32_t b, uint32_t* s_wave, uint32_t& pre_a,
+                                                 uint32_t& pre_b, uint32_t& tot_a, uint32_t& tot_b)
+{
+  static_assert(FSST_WAVES == 8, "both values' wave sums fill one 16-lane DPP row");
+  const uint32_t ia = wave_incl_sum_u32(a), ib = wave_incl_sum_u32(b);
+  const uint32_t w  = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)));
+  if (lane_id() == WAVE - 1u) {
+    s_wave[w]              = ia;
+    s_wave[FSST_WAVES + w] = ib;
+  }
+  lds_barrier();
+  // every wave scans the wave sums, the second value's on top of the first's
+  const uint32_t ws = s_wave[lane_id() & (2u * FSST_WAVES - 1u)];
+  const uint32_t wi = row_incl_sum_u32(ws);
+  tot_a             = __builtin_amdgcn_readlane(wi, FSST_WAVES - 1u);
+  tot_b             = __builtin_amdgcn_readlane(wi, 2u * FSST_WAVES - 1u) - tot_a;
+  pre_a = __builtin_amdgcn_readlane(wi, w) - __builtin_amdgcn_readlane(ws, w) + ia - a;
+  pre_b = __builtin_amdgcn_readlane(wi, FSST_WAVES + w) - __builtin_amdgcn_readlane(ws, FSST_WAVES + w) - tot_a + ib - b;
+}
+
+// Shape of a chunk decode, and why.  The decode is bound by the instructions
+// that every compressed byte costs (VALU, at one wave instruction per cycle and
+// CU, and LDS: 4-7 cycles for each lookup or OR of 64 lanes at random
+// addresses), not by HBM.  The form before this one walked rows byte by byte
+// in 256-thread workgroups with an 11 KiB window: 70 VALU and 52 LDS cycles
+// per 64 bytes, 560 us for 16 Mi rows of 27 chars (12.9 compressed).  Row
+// starts as a bitmap, packed prefix sums and two lookups and two to three ORs
+// per byte take it to 39 VALU and 32 LDS cycles and 318 us.  512 threads with
+// two groups each keep a 16 KiB run in registers, so nothing is read twice;
+// three such workgroups share a CU (51 KB of LDS, 80 VGPRs), whose 38 KiB
+// window builds most chunks in one piece.  Rows of 70 and 200 chars, whose
+// chunks take several runs, went from 945 to 305 and from 2956 to 440 us (137
+// and 197 MB of chars); the row-wise path is left to malformed chunks and to
+// rows that no run holds.
 constexpr uint32_t FSST_SYMSTAGE = 17u + 8u * FSST_NSYM;  // the largest symbol table (2057 bytes)
-constexpr uint32_t FSST_CSTAGE   = 16384;                  // chunk compressed bytes staged in LDS
-constexpr uint32_t FSST_NGRID    = (FSST_CSTAGE + 16u) / 16u + 2u;
-// Output windows.  An 11 KiB window keeps a chunk kernel's LDS at 27.0 KB,
-// and with at most 80 VGPRs it runs six workgroups per CU (1.6-3% faster
-// than five with 16 KiB).  Both kernels decode one chunk per block: a
-// persistent loop around the chunk took the batch kernel to 96 VGPRs.
-constexpr uint32_t FSST_OUT_COLUMN = 11264;  // output window of the per-column kernel (6 blocks per CU)
-constexpr uint32_t FSST_OUT_BATCH  = 11264;  // ... of the batch kernel (6 blocks per CU)
-// 16-byte groups of a thread's first-walk span of a chunk's compressed bytes
-// (at most FSST_CSTAGE of them after a head of up to 15 bytes), loaded into
-// registers at the chunk's start
-constexpr uint32_t SPAN_GROUPS = (FSST_CSTAGE + 15u + 16u * FSST_THREADS - 1u) / (16u * FSST_THREADS);
-static_assert(SPAN_GROUPS == 5, "first-walk span registers");
-// s_waitcnt vmcnt(SPAN_GROUPS), expcnt and lgkmcnt left at their maxima
-// (gfx9 encoding: vmcnt bits 3:0, expcnt 6:4, lgkmcnt 11:8)
-constexpr int WAITCNT_VMEM_SPANS = 0x0F70 | static_cast<int>(SPAN_GROUPS);
-// What a chunk without compressed bytes loads as its span (never used).
+// Compressed bytes that the staged path takes at a time, the head of up to
+// 15 bytes before them included: GROUPS_PER_THR 16-byte groups per thread.
+constexpr uint32_t FSST_CSTAGE    = 16384;
+constexpr uint32_t GROUPS_PER_THR = FSST_CSTAGE / (16u * FSST_THREADS);
+static_assert(GROUPS_PER_THR == 2, "the staged path's registers and its packed scans");
+// Output window: at most this many chars are built in LDS at a time.
+constexpr uint32_t FSST_WINDOW = 38u << 10;
+// What a chunk without compressed bytes loads as its groups (never used).
 static __device__ __attribute__((aligned(16))) const uint32_t fsst_zero_group[4] = {0u, 0u, 0u, 0u};
 
-// Walk state at a grid point: decoded prefix (bits 0-19), escape flag (bit
-// 20), row (bits 21-31).  A staged chunk decodes to at most 8 * FSST_CSTAGE
-// bytes and holds at most 1024 rows, so the fields never overflow.
-constexpr uint32_t GS_ESC   = 1u << 20;
-constexpr uint32_t GS_ROW   = 21;
-constexpr uint32_t GS_S     = GS_ESC - 1u;
 constexpr uint32_t ROW_HUGE = 1u << 20;  // a staged row is shorter than this
+// The first walk's packed prefixes: decoded bytes (at most 8 * FSST_CSTAGE,
+// bits 0-17) with a count of at most 1024 rows above.
+constexpr uint32_t PK_LEN = 18;
+// len[] of the escape code in a staged chunk's table, so that the lengths a
+// group looks up tell whether it holds an escape.
+constexpr uint32_t LEN_ESC = 0x80;
 
-template <uint32_t OUT_CAP>
-struct FsstSmemT {
+struct FsstSmem {
   // the segment's FsstSymTab, staged whole
   __attribute__((aligned(16))) uint64_t sym[256];  // symbol bytes, zero above its length
   uint8_t len[256];
-  uint32_t comp[FSST_CHUNK_ROWS + 1];  // segment-relative inclusive compressed prefix
-  uint32_t dec[FSST_CHUNK_ROWS + 1];   // chunk-relative exclusive decoded offset
-  uint32_t gst[FSST_NGRID];            // walk state at each 16-byte grid point of the stage
-  uint32_t part[FSST_THREADS];         // decoded bytes before each thread's span
-  // output window; before that, pieces of the compressed-length stream
-  __attribute__((aligned(16))) uint8_t out[(OUT_CAP > FSST_PIECE ? OUT_CAP : FSST_PIECE) + 48];
-  uint32_t wave[FSST_WAVES];
+  // row-wise path: comp[] is the segment-relative inclusive compressed prefix,
+  // dec[] the chunk-relative exclusive decoded offset.  Staged path, rows with
+  // compressed bytes in storage order (rank): comp[k] is the decoded prefix at
+  // row k's first byte, dec[k + 1] what takes a decoded prefix inside row k to
+  // its output position.
+  uint32_t comp[FSST_CHUNK_ROWS + 1];
+  uint32_t dec[FSST_CHUNK_ROWS + 4];
+  uint32_t bits[FSST_CSTAGE / 32];  // bit y: a row's first byte is stage position y
+  // output window (and the slack its last symbol's words reach); before that,
+  // the compressed-length fields
+  __attribute__((aligned(16))) uint8_t out[FSST_WINDOW + 48];
+  uint32_t wave[2 * FSST_WAVES];
+  uint32_t part[2 * FSST_WAVES];
   uint64_t base;
-
-  // The second walk's output window.  The chunk's compressed bytes are not
-  // staged in LDS: the first walk holds each thread's span in registers and
-  // the second reads the same 16-byte blocks again from L2.
-  static constexpr uint32_t WINDOW = OUT_CAP > FSST_PIECE ? OUT_CAP : FSST_PIECE;
-  __device__ __forceinline__ uint8_t* window()
-  {
-    // a window of nout <= WINDOW + 15 bytes (16-byte head) is cleared in 4-byte words below nout + 32
-    static_assert((WINDOW + 15u + 31u) / 4u * 4u + 4u <= sizeof(out), "a window's clear stays inside out[]");
-    return out;
-  }
 };
 
 // Walk the n compressed bytes of one row with DuckDB's serial semantics:
@@ -352,385 +357,328 @@ __device__ __attribute__((noinline)) void fsst_emit_rows(SM& sm, const uint8_t* 
   }
 }
 
-// ---- span path (staged chunks) ----
+// ---- staged path ----
 //
-// Stage coordinates: the chunk's compressed bytes sit at stage positions [c_h, c_h + C);
-// row r occupies [top - comp[r + 1], top - comp[r]) with top = c_h + c_hi
-// (rows are stored back to front, so row indices fall as the position
-// rises).  A walk's row variable r is the row holding the byte it is about
-// to read; `rend` is that row's end, and at rend the walk steps to the next
-// lower row (several, over empty rows).
+// A chunk's rows are taken whole, as many at a time as their compressed bytes
+// fit FSST_CSTAGE (a run of rows; nearly always the whole chunk).  Stage
+// coordinates: the run's bytes are stage positions [c_h, y_hi), position 0
+// being the 16-byte-aligned address at or below the first of them.  Rows are
+// stored back to front, so row indices fall as the position rises; the rows
+// that have bytes are ranked in that order.
 
-// Span of thread t over [lo, hi), cut on a 16-byte grid starting at g0.
-__device__ __forceinline__ uint32_t span_bytes(uint32_t g0, uint32_t hi)
-{
-  return ((hi - g0 + 16u * FSST_THREADS - 1u) / (16u * FSST_THREADS)) * 16u;
-}
+// One thread's 16-byte group between the two walks.
+struct FsstGroup {
+  uint32_t q[4];  // the bytes
+  uint32_t p[4];      // decoded bytes of the group before each byte, packed like q
+  uint32_t m;     // bit j: a row starts at byte j
+  uint32_t lit;   // bit j: byte j is a literal (it follows an escape)
+  uint32_t d;     // decoded bytes of the run before the group
+  uint32_t r;     // rows that start before the group
+};
 
 // Byte j (0..15) of a 16-byte group.
-__device__ __forceinline__ uint32_t group_byte(const u32x4& q, uint32_t j)
+__device__ __forceinline__ uint32_t group_byte(const uint32_t (&q)[4], uint32_t j)
 {
   return (q[j >> 2] >> (8u * (j & 3u))) & 0xFFu;
 }
 
-// First walk: decoded lengths.  Records the walk state at each grid point
-// and, per row, the decoded prefix at its start; returns the chunk's decoded
-// total and leaves dec[] as the chunk-relative exclusive decoded offsets.
-// Thread t's first-walk span: the 16-byte groups [t * span, t * span + span)
-// of stage positions below y_hi, stage position 0 being the 16-byte-aligned
-// address `stage` (the blocks an LDS stage of the chunk would hold).
-//
-// Every thread issues exactly SPAN_GROUPS loads (y_hi > 0), with no branch
-// around them: a group outside its span rereads the stage's last group and
-// is never used.  The caller can then wait for the loads issued before these
-// with vmcnt(SPAN_GROUPS).
-__device__ __forceinline__ void fsst_span_load(u32x4 (&qv)[SPAN_GROUPS], const uint8_t* stage, uint32_t y_hi)
-{
-  const uint32_t span = span_bytes(0, y_hi);
-  const uint32_t s0   = threadIdx.x * span;
-  const uint32_t last = (y_hi - 1u) >> 4;
-  const gptr<const u32x4> cg = gbl(reinterpret_cast<const u32x4*>(stage));
-#pragma unroll
-  for (uint32_t k = 0; k < SPAN_GROUPS; ++k)
-    qv[k] = cg[16u * k < span && s0 + 16u * k < y_hi ? (s0 >> 4) + k : last];
-}
+// 0x01 in byte i for each bit i (0..3) of x.
+__device__ __forceinline__ uint32_t spread4(uint32_t x) { return ((x & 15u) * 0x00204081u) & 0x01010101u; }
 
-// The last word of thread t's span (the four bytes before thread t + 1's
-// first byte), for the escape parity of the thread after it.
-__device__ __forceinline__ uint32_t fsst_span_tail(const u32x4 (&qv)[SPAN_GROUPS], uint32_t y_hi)
+// The literals of a group: a byte follows an escape of its own row.  e: the
+// bytes equal to 255, m: the row starts, esc: an escape ends just before the
+// group.
+__device__ __forceinline__ uint32_t literal_mask(uint32_t e, uint32_t m, bool esc)
 {
-  const uint32_t last = span_bytes(0, y_hi) / 16u - 1u;
-  uint32_t w          = 0;
-#pragma unroll
-  for (uint32_t k = 0; k < SPAN_GROUPS; ++k) w = k == last ? qv[k][3] : w;
-  return w;
-}
-
-template <class SM>
-__device__ __forceinline__ uint32_t fsst_lengths_staged(SM& sm, uint32_t rows, uint32_t c_h, uint32_t c_hi,
-                                                        uint32_t C, const u32x4 (&qv)[SPAN_GROUPS],
-                                                        const uint8_t* stage)
-{
-  const uint32_t tid  = threadIdx.x;
-  const uint32_t y_hi = c_h + C;
-  const uint32_t top  = c_h + c_hi;
-  const uint32_t span = span_bytes(0, y_hi);
-  const uint32_t ya   = tid * span > c_h ? tid * span : c_h;
-  const uint32_t yb   = tid * span + span < y_hi ? tid * span + span : y_hi;
-  uint32_t acc        = 0;
-  if (ya < yb) {
-    // the row holding byte ya: the largest r <= rows with comp[r] <= top - ya
-    // (r == rows, a row above the first, when ya is the first byte)
-    const uint32_t u0 = top - ya;
-    uint32_t r        = 0;
-#pragma unroll
-    for (uint32_t s = 1024; s; s >>= 1)
-      if (r + s <= rows && sm.comp[r + s] <= u0) r += s;
-    uint32_t rend  = top - sm.comp[r];
-    uint32_t rnext = r ? top - sm.comp[r - 1] : rend;  // end of row r - 1
-    bool esc       = false;
-    if (r < rows) {  // ya inside row r: an odd run of 255s before it escapes it
-      // the four bytes before ya come from the previous thread's span (sm.part,
-      // written before the barrier that ends the compressed-prefix scan),
-      // earlier ones from L2
-      const uint32_t rs = top - sm.comp[r + 1];
-      const uint32_t pw = tid ? sm.part[tid - 1] : 0u;
-      for (uint32_t y = ya; y > rs; --y) {
-        const uint32_t d = ya - y;
-        const uint32_t b = d < 4u ? (pw >> (24u - 8u * d)) & 0xFFu : ld_u8(stage + y - 1u);
-        if (b != FSST_ESC) break;
-        esc = !esc;
-      }
-    }
-    u32x4 qr[SPAN_GROUPS];
-#pragma unroll
-    for (uint32_t k = 0; k < SPAN_GROUPS; ++k) qr[k] = qv[k];
+  uint32_t lit = 0;
 #pragma unroll 1
-    for (uint32_t g = ya & ~15u; g < yb; g += 16) {
-      const u32x4 q = qr[0];
-#pragma unroll
-      for (uint32_t k = 0; k + 1 < SPAN_GROUPS; ++k) qr[k] = qr[k + 1];
-      uint32_t L[16];
-#pragma unroll
-      for (uint32_t j = 0; j < 16; ++j) L[j] = sm.len[group_byte(q, j)];
-      const uint32_t lo = ya > g ? ya - g : 0u;  // the group's bytes of this span: [lo, hi)
-      const uint32_t hi = yb - g < 16u ? yb - g : 16u;
-#pragma unroll
-      for (uint32_t j = 0; j < 16; ++j) {
-        const uint32_t y = g + j;
-        if (y == rend && r) {  // rows starting at y
-          do {
-            --r;
-            sm.dec[r + 1] = acc;  // the prefix at row r's start
-            rend          = rnext;
-            rnext         = r ? top - sm.comp[r - 1] : rend;
-          } while (y == rend && r);
-          esc = false;
-        }
-        if (j == 0 && lo == 0) sm.gst[g >> 4] = acc | (esc ? GS_ESC : 0u) | (r << GS_ROW);
-        const uint32_t b  = group_byte(q, j);
-        const bool valid  = j >= lo && j < hi;
-        acc += valid ? (esc ? 1u : L[j]) : 0u;
-        esc = valid ? (!esc && b == FSST_ESC) : esc;
-      }
-    }
-    // rows starting at the last byte's end (empty rows below the others)
-    if (yb == y_hi)
-      while (rend == y_hi && r) {
-        --r;
-        sm.dec[r + 1] = acc;
-        rend          = rnext;
-        rnext         = r ? top - sm.comp[r - 1] : rend;
-      }
+  for (uint32_t j = 0; j < 16; ++j) {
+    const uint32_t b = 1u << j;
+    esc              = esc && !(m & b);
+    lit |= esc ? b : 0u;
+    esc = !esc && (e & b);
   }
-  uint32_t T         = 0;
-  const uint32_t pre = block_excl_scan(acc, sm.wave, &T);
-  sm.part[tid]       = pre;
-  if (ya < yb)
-    for (uint32_t g = (ya + 15u) & ~15u; g < yb; g += 16) sm.gst[g >> 4] += pre;
-  __syncthreads();
-  // dec[r + 1] = T - (decoded prefix at row r's start); the prefix was
-  // recorded at dec[r + 1], span-relative, by the thread whose span holds
-  // that start, so each slot is read and rewritten by one thread here
-#pragma unroll
-  for (uint32_t k = 0; k < ROWS_PER_THR; ++k) {
-    const uint32_t r = k * FSST_THREADS + tid;
-    if (r < rows) {
-      const uint32_t p = top - sm.comp[r + 1];
-      sm.dec[r + 1]    = T - (sm.dec[r + 1] + sm.part[(p < y_hi ? p : y_hi - 1u) / span]);
-    }
-  }
-  if (tid == 0) sm.dec[0] = 0;
-  __syncthreads();
-  return T;
+  return lit;
 }
 
-// One byte of the second walk for a lane whose next row start is in
-// registers or LDS (the per-byte form, used when a 16-byte group holds more
-// row starts than the prefetch covers).  `y` is the byte's stage position.
-template <class SM>
-__device__ __forceinline__ void emit_byte_slow(SM& sm, uint32_t y, uint32_t b, bool valid, uint32_t top,
-                                               uint32_t wofs, uint32_t& r, uint32_t& rend, uint32_t& o, bool& esc)
+// The groups of a run whose last byte is stage position y_hi - 1, and the
+// word before each wave's first one: 2 * GROUPS_PER_THR loads per thread, with
+// no branch around them (a group past the run's bytes rereads the last one).
+__device__ __forceinline__ void fsst_load_groups(FsstGroup (&gr)[GROUPS_PER_THR], uint32_t (&prev)[GROUPS_PER_THR],
+                                                 const uint8_t* stage, uint32_t y_hi)
 {
-  if (valid && y == rend) {  // rows starting at y
-    do {
-      --r;
-      rend = top - sm.comp[r];
-    } while (y == rend);
-    o   = sm.dec[r] - wofs;
-    esc = false;
+  const gptr<const u32x4> cg    = gbl(reinterpret_cast<const u32x4*>(stage));
+  const gptr<const uint32_t> cw = gbl(reinterpret_cast<const uint32_t*>(stage));
+  const uint32_t last           = y_hi ? (y_hi - 1u) >> 4 : 0u;
+#pragma unroll
+  for (uint32_t k = 0; k < GROUPS_PER_THR; ++k) {
+    const uint32_t g  = k * FSST_THREADS + threadIdx.x;
+    const uint32_t wg = k * FSST_THREADS + (threadIdx.x & ~(WAVE - 1u));
+    const u32x4 q     = cg[g < last ? g : last];
+#pragma unroll
+    for (uint32_t d = 0; d < 4; ++d) gr[k].q[d] = q[d];
+    prev[k] = cw[wg && wg <= last ? 4u * wg - 1u : 0u];
   }
-  const bool lit   = esc;
-  const uint32_t l = lit ? 1u : sm.len[b];
-  const uint64_t v = lit ? uint64_t{b} : sm.sym[b];
-  esc              = !lit && b == FSST_ESC;
-  if (valid) {
-    const uint32_t sh = 8u * (o & 3u);
-    const uint64_t w  = v << sh;
-    uint32_t* d       = reinterpret_cast<uint32_t*>(&sm.window()[o & ~3u]);
-    __hip_atomic_fetch_or(d, static_cast<uint32_t>(w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __hip_atomic_fetch_or(d + 1, static_cast<uint32_t>(w >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __hip_atomic_fetch_or(d + 2, static_cast<uint32_t>((uint64_t{static_cast<uint32_t>(v >> 32)} << sh) >> 32),
-                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  }
-  o += l;
 }
 
-constexpr uint32_t EMIT_AHEAD = 4;  // row starts a lane prefetches per 16-byte group
-
-// Second walk: chars.  Rows are emitted in windows of whole rows whose
-// output fits OUT_CAP bytes; each window's output is built in LDS (zeroed,
-// then every symbol ORed in at its byte position, so neighbouring spans
-// may share words) and leaves in 16-byte stores.  Returns false, having
-// written nothing more, when a single row's output exceeds OUT_CAP.
-//
-// A lane walks its span 16 bytes at a time.  At each group it loads, with
-// the group's symbols, the ends and output starts of the next EMIT_AHEAD
-// rows, so the bytes themselves only compare and select: a row starting at
-// byte j moves the output position to its start and clears the escape
-// flag (empty rows start where the next row starts; the last match wins).
-// A lane whose group holds more row starts than that takes the group byte
-// by byte.
-//
-// The window is SM::WINDOW bytes of LDS; byte i of a window is chunk output
-// position wlo + i, whatever the chunk's place in the column, so a window can
-// be built before the chunk's base is known.  `get_base()` returns the base;
-// every thread calls it after each window's ORs, and it synchronises the
-// workgroup (after the first window's ORs the look-back completes there).
-// The stores shift the window to the destination's 16-byte alignment.  The
-// compressed bytes come from global memory at `stage`, the address of stage
-// position 0 (16-byte blocks read again from L2).  A lane loads its first
-// group while the window is cleared, and each next group while it emits the
-// current one.
-template <class SM, class GetBase>
-__device__ __forceinline__ bool fsst_emit_staged(SM& sm, uint32_t rows, uint32_t c_h, uint32_t c_hi, uint32_t T,
-                                                 GetBase&& get_base, uint8_t* chars, uint64_t chars_cap,
-                                                 const uint8_t* stage)
+// First walk of group g: every byte's decoded length, summed.  `prev` is the
+// word before the group.  Bytes that are not the run's become escapes, whose
+// symbol is empty.  Returns the group's decoded bytes; *lits is wave-uniform:
+// some group of the wave holds a literal.
+__device__ __forceinline__ uint32_t fsst_group_lengths(FsstGroup& gr, const FsstSmem& sm, uint32_t g, uint32_t prev,
+                                                       uint32_t c_h, uint32_t y_hi, const uint8_t* stage, bool* lits)
 {
-  constexpr uint32_t OUT_CAP = SM::WINDOW;
-  uint8_t* const wb         = sm.window();
-  const gptr<const u32x4> cg = gbl(reinterpret_cast<const u32x4*>(stage));
+  const bool live = 16u * g < y_hi;
+  uint32_t L[4];
+#pragma unroll
+  for (uint32_t d = 0; d < 4; ++d) {
+    const uint32_t w = gr.q[d];
+    L[d] = sm.len[w & 0xFFu] | static_cast<uint32_t>(sm.len[(w >> 8) & 0xFFu]) << 8 |
+           static_cast<uint32_t>(sm.len[(w >> 16) & 0xFFu]) << 16 | static_cast<uint32_t>(sm.len[w >> 24]) << 24;
+  }
+  gr.m               = live ? (sm.bits[g >> 1] >> (16u * (g & 1u))) & 0xFFFFu : 0u;
+  gr.lit             = 0;
+  const bool has_esc = ((L[0] | L[1] | L[2] | L[3]) & 0x80808080u) != 0;
+  const bool edge    = 16u * g < c_h || 16u * g + 16u > y_hi;
+  const bool after   = (prev >> 24) == FSST_ESC && 16u * g > c_h;
+  *lits              = false;
+  if (ballot(live && (has_esc || edge || after)) != 0) {
+    const uint32_t y     = 16u * g;
+    const uint32_t lo    = c_h > y ? c_h - y : 0u;  // c_h < 16
+    const uint32_t hi    = live ? (y_hi - y < 16u ? y_hi - y : 16u) : lo;
+    const uint32_t valid = ((1u << hi) - 1u) & ~((1u << lo) - 1u);
+    uint32_t e           = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < 16; ++j) e |= group_byte(gr.q, j) == FSST_ESC ? 1u << j : 0u;
+    e &= valid;
+    bool esc = false;  // an odd run of 255s of the row ends just before the group
+    if (live && after && !(gr.m & 1u)) {
+      for (uint32_t x = y; x > c_h; --x) {
+        if (ld_u8(stage + x - 1u) != FSST_ESC) break;
+        esc = !esc;
+        if ((sm.bits[(x - 1u) >> 5] >> ((x - 1u) & 31u)) & 1u) break;  // the row's first byte
+      }
+    }
+    gr.lit = literal_mask(e, gr.m, esc) & valid;
+#pragma unroll
+    for (uint32_t d = 0; d < 4; ++d) {
+      const uint32_t one = spread4(gr.lit >> (4u * d)), in = spread4(valid >> (4u * d)) * 0xFFu;
+      L[d]               = (L[d] & 0x7F7F7F7Fu & in & ~(one * 0xFFu)) | one;
+      gr.q[d] |= ~in;
+    }
+    *lits = ballot(gr.lit != 0) != 0;
+  }
+  // exclusive prefixes of the 16 lengths, four to a word (at most 128 in all)
+  uint32_t t = 0;  // the running total in every byte
+#pragma unroll
+  for (uint32_t d = 0; d < 4; ++d) {
+    const uint32_t s2 = (L[d] << 8) + L[d], s = (s2 << 16) + s2;  // inclusive within the word
+    gr.p[d]           = (s << 8) + t;
+    t                 = __builtin_amdgcn_perm(0u, s + t, 0x03030303u);
+  }
+  return live ? t & 0xFFu : 0u;
+}
+
+// Both groups' first walk, the run's decoded total *T, and sm.comp[] (the
+// decoded prefix at every first byte of a row, and after the last byte).  The caller's next barrier makes sm.comp[] visible.
+__device__ __forceinline__ void fsst_walk_lengths(FsstGroup (&gr)[GROUPS_PER_THR], FsstSmem& sm,
+                                                  const uint32_t (&prev)[GROUPS_PER_THR], uint32_t c_h, uint32_t y_hi,
+                                                  const uint8_t* stage, bool (&lits)[GROUPS_PER_THR], uint32_t* T)
+{
   const uint32_t tid  = threadIdx.x;
   const uint32_t lane = lane_id();
-  const uint32_t top  = c_h + c_hi;
-  const uintptr_t cb  = reinterpret_cast<uintptr_t>(chars);
-  uint32_t r_hi       = rows - 1;  // highest row of the next window
-  // The lowest row of the window whose highest row is hi: the lowest r_lo
-  // with dec[hi + 1] - dec[r_lo] <= OUT_CAP (~0u: row hi alone is larger).
-  // Every wave searches for itself (the same answer from the same dec[]),
-  // so no barrier hands it out.
-  auto find_window = [&](uint32_t hi) -> uint32_t {
-    const uint32_t d_top = sm.dec[hi + 1];
-    if (d_top <= OUT_CAP) return 0u;
-    if (d_top - sm.dec[hi] > OUT_CAP) return ~0u;
-    // 64-way search rounds over (a, b] (fails at a, holds at b)
-    uint32_t a = 0, b = hi;
-    while (b - a > 1u) {
-      const uint32_t step = (b - a + WAVE - 1u) / WAVE;
-      const uint32_t m    = a + (lane + 1u) * step < b ? a + (lane + 1u) * step : b;
-      const uint64_t hold = ballot(d_top - sm.dec[m] <= OUT_CAP);
-      const uint32_t f    = static_cast<uint32_t>(__builtin_ctzll(hold));  // lane 63 tests b, which holds
-      const uint32_t nb   = a + (f + 1u) * step < b ? a + (f + 1u) * step : b;
-      a                   = a + f * step;
-      b                   = nb;
+  const uint32_t w    = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(tid >> 6)));
+  uint32_t v[GROUPS_PER_THR], incl[GROUPS_PER_THR];
+#pragma unroll
+  for (uint32_t k = 0; k < GROUPS_PER_THR; ++k) {
+    // the word before the group: the lane below holds it, lane 0 loaded it
+    uint32_t pw = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+      static_cast<int>(prev[k]), static_cast<int>(gr[k].q[3]), 0x138, 0xF, 0xF, false));  // wave_shr:1
+    v[k] = fsst_group_lengths(gr[k], sm, k * FSST_THREADS + tid, pw, c_h, y_hi, stage, &lits[k]);
+    v[k] |= static_cast<uint32_t>(__builtin_popcount(gr[k].m)) << PK_LEN;
+    incl[k] = wave_incl_sum_u32(v[k]);
+    if (lane == WAVE - 1) sm.part[k * FSST_WAVES + w] = incl[k];
+  }
+  lds_barrier();
+  // every wave scans the 2 x FSST_WAVES wave sums in one 16-lane row
+  static_assert(GROUPS_PER_THR * FSST_WAVES == 16, "one DPP row of wave sums");
+  const uint32_t ws  = sm.part[lane & 15u];
+  const uint32_t wi  = row_incl_sum_u32(ws);
+  const uint32_t tot = __builtin_amdgcn_readlane(wi, 15);
+  *T = tot & ((1u << PK_LEN) - 1u);
+#pragma unroll
+  for (uint32_t k = 0; k < GROUPS_PER_THR; ++k) {
+    const uint32_t i  = k * FSST_WAVES + w;
+    const uint32_t ex = __builtin_amdgcn_readlane(wi, i) - __builtin_amdgcn_readlane(ws, i) + incl[k] - v[k];
+    gr[k].d           = ex & ((1u << PK_LEN) - 1u);
+    gr[k].r           = ex >> PK_LEN;
+    const uint64_t lo = gr[k].p[0] | uint64_t{gr[k].p[1]} << 32, hi = gr[k].p[2] | uint64_t{gr[k].p[3]} << 32;
+    uint32_t m = gr[k].m, rank = gr[k].r;
+    while (m) {
+      const uint32_t j = static_cast<uint32_t>(__builtin_ctz(m));
+      m &= m - 1u;
+      sm.comp[rank++] = gr[k].d + (static_cast<uint32_t>((j & 8u ? hi : lo) >> (8u * (j & 7u))) & 0xFFu);
     }
-    return b;
-  };
-  uint32_t r_lo = find_window(r_hi);
-  for (;;) {
-    if (r_lo == ~0u) return false;
-    const uint32_t wlo  = sm.dec[r_lo];
-    const uint32_t whi  = sm.dec[r_hi + 1];
-    {
-      const uint32_t nout = whi - wlo;
-      const uint32_t wofs = wlo;  // chunk output position of window byte 0
-      const uint32_t ya   = top - sm.comp[r_hi + 1];
-      const uint32_t yb   = top - sm.comp[r_lo];
-      const uint32_t g0   = ya & ~15u;
-      const uint32_t span = span_bytes(g0, yb);
-      const uint32_t s0   = g0 + tid * span;
-      const uint32_t ys   = tid ? s0 : ya;
-      const uint32_t ye   = s0 + span < yb ? s0 + span : yb;
-      u32x4 qn            = u32x4{0u, 0u, 0u, 0u};
-      if (ys < ye) qn = cg[ys >> 4];
-      // Cleared with 4-byte stores.  Measured on gfx950: clearing with
-      // 16-byte stores (ds_write_b128) and then ORing from other waves
-      // after a barrier lost about 0.2% of the ORed bytes once five or more
-      // workgroups shared a CU; 4-byte stores never did.
-      for (uint32_t i = tid * 4u; i < nout + 32u; i += FSST_THREADS * 4u)
-        *reinterpret_cast<uint32_t*>(&wb[i]) = 0u;
-      __syncthreads();
-      // bytes outside [ys, ye) OR into this word, which is never flushed
-      const uint32_t trash = (nout + 19u) & ~3u;
-      if (ys < ye) {
-        // thread 0 starts above the window's highest row and steps into it
-        // at ya; the others resume a grid-point state of the first walk
-        uint32_t r = r_hi + 1, o = 0;
-        bool esc   = false;
-        if (tid) {
-          const uint32_t gs = sm.gst[ys >> 4];
-          r                 = gs >> GS_ROW;
-          esc               = (gs & GS_ESC) != 0;
-          o = sm.dec[r] + (gs & GS_S) - (T - sm.dec[r + 1]) - wofs;
-        }
-        uint32_t rend = top - sm.comp[r];
-#pragma unroll 1
-        for (uint32_t g = ys & ~15u; g < ye; g += 16) {
-          const u32x4 q = qn;
-          if (g + 16u < ye) qn = cg[(g >> 4) + 1u];
-          // the next EMIT_AHEAD rows below r: ends e[k] and output starts
-          // d[k]; row r - k - 1 starts at e[k - 1] (e[-1] = rend)
-          uint32_t e[EMIT_AHEAD], d[EMIT_AHEAD];
+  }
+  if (tid == 0) sm.comp[tot >> PK_LEN] = tot & ((1u << PK_LEN) - 1u);
+}
+
+// OR symbol bytes v at window position o.
+__device__ __forceinline__ void window_or(uint8_t* out, uint32_t o, uint64_t v)
+{
+  const uint32_t s  = (o << 3) & 24u;
+  const uint64_t x  = v << s;
+  const uint32_t x2 = (static_cast<uint32_t>(v >> 32) >> 1) >> (31u - s);
+  uint32_t* d       = reinterpret_cast<uint32_t*>(out + (o & 0xFFFCu));
+  __hip_atomic_fetch_or(d, static_cast<uint32_t>(x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  __hip_atomic_fetch_or(d + 1, static_cast<uint32_t>(x >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  if (x2) __hip_atomic_fetch_or(d + 2, x2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Second walk of one group into the window over output bytes [w0, w0 +
+// FSST_WINDOW) of the run's T.  MULTI: the run's output takes several windows;
+// a wave skips a window that none of its groups reaches, and words outside
+// the window go to a word past it.
+template <bool MULTI>
+__device__ __forceinline__ void fsst_group_emit(const FsstGroup& gr, FsstSmem& sm, uint32_t g, uint32_t y_hi, bool lits,
+                                                uint32_t T, uint32_t w0)
+{
+  bool live         = 16u * g < y_hi;
+  const uint32_t pc = static_cast<uint32_t>(__builtin_popcount(gr.m));
+  if constexpr (MULTI) {
+    // the rows that the group touches are output bytes [lo, hi)
+    const uint32_t lo = live ? T - sm.comp[gr.r + pc] : 0u;
+    const uint32_t hi = live && gr.r ? T - sm.comp[gr.r - 1u] : T;
+    live              = live && lo < w0 + FSST_WINDOW && hi > w0;
+  } else if (!lits && !ballot(live && pc > 3u)) {
+    if (!live) return;
+    // at most four rows cross a group: what takes a prefix to its output
+    // position, 16 bits for each, in two registers; a byte's row (0..3)
+    // selects one with a byte permutation
+    const uint32_t* b  = &sm.dec[gr.r];
+    const uint32_t b01 = __builtin_amdgcn_perm(b[1] + gr.d, b[0] + gr.d, 0x05040100u);
+    const uint32_t b23 = __builtin_amdgcn_perm(b[3] + gr.d, b[2] + gr.d, 0x05040100u);
 #pragma unroll
-          for (uint32_t k = 0; k < EMIT_AHEAD; ++k) {
-            const bool in    = r > k;
-            const uint32_t i = in ? r - k - 1u : 0u;
-            e[k]             = in ? top - sm.comp[i] : ~0u;
-            d[k]             = sm.dec[i] - wofs;
-          }
-          const uint32_t lim = ye - g < 16u ? ye - g : 16u;  // bytes of the group in the span: [lo, lim)
-          const uint32_t lo  = ys > g ? ys - g : 0u;
-          const bool more    = e[EMIT_AHEAD - 1] - g < lim;  // another row starts inside the group
-          if (!more) {
-            uint32_t st[EMIT_AHEAD];  // start offsets in the group (>= 16 when none)
+    for (uint32_t h = 0; h < 16; h += 8) {
+      uint64_t v[8];
 #pragma unroll
-            for (uint32_t k = 0; k < EMIT_AHEAD; ++k) st[k] = (k ? e[k - 1] : rend) - g;
-            // symbols and lengths in two halves of eight bytes (fewer live registers)
+      for (uint32_t i = 0; i < 8; ++i) v[i] = sm.sym[group_byte(gr.q, h + i)];
 #pragma unroll
-            for (uint32_t h = 0; h < 16; h += 8) {
-            uint32_t L[8];
-            uint64_t V[8];
-#pragma unroll
-            for (uint32_t i = 0; i < 8; ++i) {
-              const uint32_t bj = group_byte(q, h + i);
-              L[i]              = sm.len[bj];
-              V[i]              = sm.sym[bj];
-            }
-#pragma unroll
-            for (uint32_t i = 0; i < 8; ++i) {
-              const uint32_t j = h + i;
-              bool start = false;
-#pragma unroll
-              for (uint32_t k = 0; k < EMIT_AHEAD; ++k) {
-                const bool s = st[k] == j;
-                o            = s ? d[k] : o;
-                start |= s;
-              }
-              const uint32_t bj = group_byte(q, j);
-              const bool lit    = esc && !start;
-              const uint32_t l  = lit ? 1u : L[i];
-              const uint64_t v  = lit ? uint64_t{bj} : V[i];
-              esc               = !lit && bj == FSST_ESC;
-              const bool valid  = j >= lo && j < lim;
-              const uint32_t sh = 8u * (o & 3u);
-              const uint64_t w  = v << sh;
-              const uint32_t w2 = static_cast<uint32_t>((uint64_t{static_cast<uint32_t>(v >> 32)} << sh) >> 32);
-              uint32_t* dw      = reinterpret_cast<uint32_t*>(&wb[valid ? (o & ~3u) : trash]);
-              __hip_atomic_fetch_or(dw, static_cast<uint32_t>(w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-              __hip_atomic_fetch_or(dw + 1, static_cast<uint32_t>(w >> 32), __ATOMIC_RELAXED,
-                                    __HIP_MEMORY_SCOPE_WORKGROUP);
-              __hip_atomic_fetch_or(dw + 2, w2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-              o += l;
-            }
-            }
-            // rows started in the group
-#pragma unroll
-            for (uint32_t k = 0; k < EMIT_AHEAD; ++k)
-              if (st[k] < lim) {
-                r    = r - 1u;
-                rend = e[k];
-              }
-          } else {
-#pragma unroll 1
-            for (uint32_t j = 0; j < 16; ++j)
-              emit_byte_slow(sm, g + j, group_byte(q, j), j >= lo && j < lim, top, wofs, r, rend, o, esc);
-          }
-        }
-      }
-      const uint64_t base  = get_base();  // synchronises the workgroup
-      const uintptr_t g_lo = cb + base + wlo;
-      const uintptr_t g_hi = cb + (base + whi < chars_cap ? base + whi : chars_cap);
-      const uint32_t* ww   = reinterpret_cast<const uint32_t*>(wb);
-      for (uintptr_t blk = (g_lo & ~uintptr_t{15}) + uintptr_t{tid} * 16u; blk < g_hi;
-           blk += uintptr_t{FSST_THREADS} * 16u) {
-        if (blk >= g_lo && blk + 16u <= g_hi) {
-          // window bytes [i, i + 16), i = blk - g_lo, from five aligned words
-          const uint32_t i  = static_cast<uint32_t>(blk - g_lo);
-          const uint32_t w  = i >> 2, sh = i & 3u;
-          const uint32_t x0 = ww[w], x1 = ww[w + 1], x2 = ww[w + 2], x3 = ww[w + 3], x4 = ww[w + 4];
-          const u32x4 v     = u32x4{__builtin_amdgcn_alignbyte(x1, x0, sh), __builtin_amdgcn_alignbyte(x2, x1, sh),
-                                __builtin_amdgcn_alignbyte(x3, x2, sh), __builtin_amdgcn_alignbyte(x4, x3, sh)};
-          __builtin_nontemporal_store(v, gbl(reinterpret_cast<u32x4*>(blk)));
-        } else {
-          for (uintptr_t x = blk; x < blk + 16u; ++x)
-            if (x >= g_lo && x < g_hi) *gbl(reinterpret_cast<uint8_t*>(x)) = wb[x - g_lo];
-        }
+      for (uint32_t i = 0; i < 8; ++i) {
+        const uint32_t j   = h + i;
+        const uint32_t row = static_cast<uint32_t>(__builtin_popcount(gr.m & ((2u << j) - 1u)));
+        const uint32_t bo  = __builtin_amdgcn_perm(b23, b01, 0x0C0C0100u + row * 0x0202u);
+        window_or(sm.out, bo + group_byte(gr.p, j), v[i]);
       }
     }
-    __syncthreads();
-    if (r_lo == 0) return true;
-    r_hi = r_lo - 1;
-    r_lo = find_window(r_hi);
+    return;
+  }
+  if (!live) return;
+  // any number of rows and partial windows: four bytes at a time, the row's
+  // entry read for each
+  uint32_t q[4], p[4];
+#pragma unroll
+  for (uint32_t d = 0; d < 4; ++d) {
+    q[d] = gr.q[d];
+    p[d] = gr.p[d];
+  }
+  uint32_t m = gr.m, lit = gr.lit, row = gr.r;
+#pragma unroll 1
+  for (uint32_t d = 0; d < 4; ++d) {
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+      const uint32_t c = (q[0] >> (8u * j)) & 0xFFu;
+      row += (m >> j) & 1u;
+      const uint64_t v = (lit >> j) & 1u ? uint64_t{c} : sm.sym[c];
+      const uint32_t o = sm.dec[row] + gr.d + ((p[0] >> (8u * j)) & 0xFFu) - w0;
+      if constexpr (!MULTI) {
+        window_or(sm.out, o, v);
+      } else {
+        const uint32_t s  = (o << 3) & 24u;
+        const uint64_t x  = v << s;
+        const uint32_t x2 = (static_cast<uint32_t>(v >> 32) >> 1) >> (31u - s);
+        const int32_t w   = static_cast<int32_t>(o) >> 2;
+        auto put          = [&](int32_t i, uint32_t b) {
+          const uint32_t at = static_cast<uint32_t>(i) < FSST_WINDOW / 4u ? static_cast<uint32_t>(i) : FSST_WINDOW / 4u + 4u;
+          __hip_atomic_fetch_or(reinterpret_cast<uint32_t*>(sm.out) + at, b, __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_WORKGROUP);
+        };
+        put(w, static_cast<uint32_t>(x));
+        put(w + 1, static_cast<uint32_t>(x >> 32));
+        put(w + 2, x2);
+      }
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 3; ++i) {
+      q[i] = q[i + 1];
+      p[i] = p[i + 1];
+    }
+    m >>= 4;
+    lit >>= 4;
+  }
+}
+
+// Clear the window's bytes [0, n) and the words a last symbol may reach.
+__device__ __forceinline__ void window_clear(FsstSmem& sm, uint32_t n)
+{
+  for (uint32_t i = threadIdx.x * 8u; i < n + 12u; i += FSST_THREADS * 8u)
+    *reinterpret_cast<uint64_t*>(&sm.out[i]) = 0u;
+}
+
+// 16 bytes at byte 16 - D (D = 1..16) of the pair of blocks a, b.
+template <uint32_t WORD>
+__device__ __forceinline__ u32x4 funnel16(const u32x4& a, const u32x4& b, uint32_t byte)
+{
+  const uint32_t c[9] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3], 0u};
+  return u32x4{__builtin_amdgcn_alignbyte(c[WORD + 1], c[WORD], byte),
+               __builtin_amdgcn_alignbyte(c[WORD + 2], c[WORD + 1], byte),
+               __builtin_amdgcn_alignbyte(c[WORD + 3], c[WORD + 2], byte),
+               __builtin_amdgcn_alignbyte(c[WORD + 4], c[WORD + 3], byte)};
+}
+
+// Whole 16-byte blocks of the window's store: block i of the destination
+// (16-byte aligned) starts at window byte 16 i - skew, so its bytes come from
+// the aligned window blocks i - 1 and i at an offset that is the same for the
+// whole chunk.
+template <uint32_t WORD>
+__device__ __forceinline__ void window_store_blocks(const FsstSmem& sm, uintptr_t dst, uint32_t i0, uint32_t i1,
+                                                    uint32_t byte)
+{
+  const u32x4* w = reinterpret_cast<const u32x4*>(sm.out);
+  for (uint32_t i = i0 + threadIdx.x; i < i1; i += FSST_THREADS) {
+    u32x4 v;
+    if constexpr (WORD == 4) v = w[i];
+    else v = funnel16<WORD>(w[i - 1u], w[i], byte);
+    __builtin_nontemporal_store(v, gbl(reinterpret_cast<u32x4*>(dst + 16u * uintptr_t{i})));
+  }
+}
+
+// The window's n bytes to global address g: 16-byte stores, single bytes
+// where the first and last 16-byte blocks are shared with other chunks.
+__device__ __forceinline__ void window_store(const FsstSmem& sm, uintptr_t g, uint32_t n)
+{
+  const uint32_t skew = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(g & 15u)));
+  const uintptr_t dst = g - skew;
+  const uint32_t i0   = skew ? 1u : 0u;       // first whole block
+  const uint32_t i1   = (skew + n) / 16u;     // past the last whole block
+  const uint32_t at   = 16u - skew;           // the first byte's place in a pair of window blocks
+  if (i1 > i0) {
+    switch (at >> 2) {
+      case 0: window_store_blocks<0>(sm, dst, i0, i1, at & 3u); break;
+      case 1: window_store_blocks<1>(sm, dst, i0, i1, at & 3u); break;
+      case 2: window_store_blocks<2>(sm, dst, i0, i1, at & 3u); break;
+      case 3: window_store_blocks<3>(sm, dst, i0, i1, at & 3u); break;
+      default: window_store_blocks<4>(sm, dst, i0, i1, 0u); break;
+    }
+  }
+  // bytes before the first whole block and after the last one
+  const uint32_t head = skew ? (16u - skew < n ? 16u - skew : n) : 0u;
+  const uint32_t tail = i1 >= i0 && i1 * 16u > skew ? i1 * 16u - skew : head;
+  if (threadIdx.x < 16u) {
+    if (threadIdx.x < head) *gbl(reinterpret_cast<uint8_t*>(g + threadIdx.x)) = sm.out[threadIdx.x];
+  } else if (threadIdx.x < 32u) {
+    const uint32_t x = (tail > head ? tail : head) + threadIdx.x - 16u;
+    if (x < n) *gbl(reinterpret_cast<uint8_t*>(g + x)) = sm.out[x];
   }
 }
 
@@ -828,9 +776,9 @@ __device__ __forceinline__ void fsst_offsets(const FsstChunk& ch, uint32_t c, ui
 struct FsstPrepSmem {
   __attribute__((aligned(16))) uint8_t st[FSST_SYMSTAGE + 48];
   uint8_t len[256];  // code lengths of a DICT_FSST dictionary's table
-  uint32_t sum[FSST_THREADS];
-  uint32_t huge[FSST_THREADS];
-  uint32_t wave[FSST_WAVES];
+  uint32_t sum[PREP_THREADS];
+  uint32_t huge[PREP_THREADS];
+  uint32_t wave[PREP_WAVES];
 };
 
 // Sum of the w-bit fields [f0, f1) of the length stream at `base`, and
@@ -900,7 +848,7 @@ __device__ __forceinline__ void plain_prep_segment(const FsstSeg& sg, FsstChunkI
     ok       = dict_end <= sg.bytes_size;
   }
   const uint32_t flags = (dict ? FI_DICT | (width & FI_WIDTH) : FI_UNC) | (ok ? FI_OK : 0u);
-  for (uint32_t k = threadIdx.x; k * FSST_CHUNK_ROWS < sg.row_count; k += FSST_THREADS) {
+  for (uint32_t k = threadIdx.x; k * FSST_CHUNK_ROWS < sg.row_count; k += PREP_THREADS) {
     FsstChunkInfo ci;
     ci.bytes      = seg;
     ci.c_lo       = ibo;
@@ -1118,7 +1066,7 @@ __device__ __forceinline__ uint32_t import_symtab(const uint8_t* seg, uint32_t b
   if (ok) {
     sym_n = bytes_size - symoff;
     if (sym_n > FSST_SYMSTAGE) sym_n = FSST_SYMSTAGE;
-    sym_h = block_stage<FSST_THREADS>(reinterpret_cast<uint32_t*>(sm.st), seg + symoff, sym_n);
+    sym_h = block_stage<PREP_THREADS>(reinterpret_cast<uint32_t*>(sm.st), seg + symoff, sym_n);
   }
   __syncthreads();
   uint32_t len = 0;
@@ -1185,7 +1133,7 @@ __device__ __forceinline__ void dfsst_prep_segment(const DictFsstSeg& d, uint32_
   const uint8_t* slens = seg + d.off_slens;
   const uint8_t* dict  = seg + d.off_dict;
   uint32_t carry_b = 0, carry_d = 0, first_len = 0;
-  for (uint32_t k0 = 0; k0 < d.dict_count; k0 += 4u * FSST_THREADS) {
+  for (uint32_t k0 = 0; k0 < d.dict_count; k0 += 4u * PREP_THREADS) {
     uint32_t v[4], dl[4], sb = 0, sd = 0;
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {
@@ -1194,7 +1142,7 @@ __device__ __forceinline__ void dfsst_prep_segment(const DictFsstSeg& d, uint32_
       sb += v[i];
     }
     uint32_t tb = 0;
-    uint32_t run = carry_b + block_excl_scan(sb, sm.wave, &tb);
+    uint32_t run = carry_b + block_excl_scan<PREP_WAVES>(sb, sm.wave, &tb);
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {
       const uint32_t k = k0 + 4u * tid + i;
@@ -1205,7 +1153,7 @@ __device__ __forceinline__ void dfsst_prep_segment(const DictFsstSeg& d, uint32_
       sd += dl[i];
     }
     uint32_t td = 0;
-    uint32_t rd = carry_d + block_excl_scan(sd, sm.wave, &td);
+    uint32_t rd = carry_d + block_excl_scan<PREP_WAVES>(sd, sm.wave, &td);
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {
       const uint32_t k = k0 + 4u * tid + i;
@@ -1257,7 +1205,7 @@ __device__ __forceinline__ void dfsst_predecode(const DictFsstSeg& d, const uint
   }
 }
 
-// Range `si` with the calling 256-thread workgroup: its chunk descriptors
+// Range `si` with the calling PREP_THREADS-thread workgroup: its chunk descriptors
 // into chunks[first_chunk + k]; for a segment, header checks
 // (fsst.cu:79-87), the symbol table import, one code per thread
 // (detail/fsst.cuh:50-96), into `tab`, and for each chunk k its
@@ -1272,7 +1220,7 @@ __device__ __forceinline__ void fsst_prep_segment(const FsstSeg sg, uint32_t si,
   const uint8_t* seg = sg.bytes;
   const uint8_t* end = seg + sg.bytes_size;
   const bool gap     = seg == nullptr;
-  for (uint32_t k = tid; k * FSST_CHUNK_ROWS < sg.row_count; k += FSST_THREADS) {
+  for (uint32_t k = tid; k * FSST_CHUNK_ROWS < sg.row_count; k += PREP_THREADS) {
     const uint32_t r0 = k * FSST_CHUNK_ROWS;
     const uint32_t n  = sg.row_count - r0 < FSST_CHUNK_ROWS ? sg.row_count - r0 : FSST_CHUNK_ROWS;
     const FsstChunk fc{gap ? FSST_GAP : si, gap ? 0u : r0, n, sg.col_row + r0};
@@ -1284,7 +1232,7 @@ __device__ __forceinline__ void fsst_prep_segment(const FsstSeg sg, uint32_t si,
     return;  // uniform per segment
   }
   if (sg.codec == SDR_CODEC_DICT_FSST) {  // bytes: the range's DictFsstSeg; pad: 1 if valid
-    for (uint32_t k = tid; k * FSST_CHUNK_ROWS < sg.row_count; k += FSST_THREADS) {
+    for (uint32_t k = tid; k * FSST_CHUNK_ROWS < sg.row_count; k += PREP_THREADS) {
       FsstChunkInfo ci{sg.bytes, 0u, 0u, 0u, FI_DFSST | (sg.pad ? FI_OK : 0u), 0u, 0u};
       const gptr<u32x4> dst = gbl(reinterpret_cast<u32x4*>(info + sg.first_chunk + k));
       const u32x8 cv        = __builtin_bit_cast(u32x8, ci);
@@ -1309,10 +1257,10 @@ __device__ __forceinline__ void fsst_prep_segment(const FsstSeg sg, uint32_t si,
   const uint32_t wv   = tid / WAVE;
   const uint32_t lane = lane_id();
   uint32_t carry      = 0;
-  for (uint32_t k0 = 0; k0 < nch; k0 += FSST_THREADS) {
-    const uint32_t cnt = nch - k0 < FSST_THREADS ? nch - k0 : FSST_THREADS;
+  for (uint32_t k0 = 0; k0 < nch; k0 += PREP_THREADS) {
+    const uint32_t cnt = nch - k0 < PREP_THREADS ? nch - k0 : PREP_THREADS;
     if (ok)
-      for (uint32_t k = k0 + wv; k < k0 + cnt; k += FSST_WAVES) {
+      for (uint32_t k = k0 + wv; k < k0 + cnt; k += PREP_WAVES) {
         const uint32_t r0 = k * FSST_CHUNK_ROWS;
         const uint32_t r1 = rows - r0 < FSST_CHUNK_ROWS ? rows : r0 + FSST_CHUNK_ROWS;
         const uint32_t f0 = r0 + 16u * lane < r1 ? r0 + 16u * lane : r1;
@@ -1329,7 +1277,7 @@ __device__ __forceinline__ void fsst_prep_segment(const FsstSeg sg, uint32_t si,
     __syncthreads();
     const uint32_t v  = (ok && tid < cnt) ? sm.sum[tid] : 0u;
     uint32_t T        = 0;
-    const uint32_t ex = block_excl_scan(v, sm.wave, &T);
+    const uint32_t ex = block_excl_scan<PREP_WAVES>(v, sm.wave, &T);
     if (tid < cnt) {
       const uint32_t k  = k0 + tid;
       const uint32_t r1 = rows - k * FSST_CHUNK_ROWS < FSST_CHUNK_ROWS ? rows : (k + 1u) * FSST_CHUNK_ROWS;
@@ -1359,139 +1307,313 @@ __device__ __forceinline__ void fsst_prep_segment(const FsstSeg sg, uint32_t si,
 
 // ---- chunk decode ----
 
+// Row r's compressed-length field (0 past the chunk's rows); lw: the fields
+// staged in LDS from bit bit0 when they all lie inside the segment (lfast).
+__device__ __forceinline__ uint32_t fsst_field(const uint32_t* lw, uint32_t bit0, bool lfast, const uint8_t* seg,
+                                               const uint8_t* end, uint32_t row_begin, uint32_t width, uint32_t r,
+                                               uint32_t rows)
+{
+  if (!width || r >= rows) return 0u;
+  return lfast ? lds_bits32(lw, bit0 + r * width, width)
+               : stream_bits32(seg + 16, end, uint64_t{row_begin + r} * width, width);
+}
+
+// The segment's symbol table and the chunk's length fields on their way to
+// LDS (LDS-direct loads); returns bit0 of fsst_field.
+__device__ __forceinline__ uint32_t fsst_issue_front(FsstSmem& sm, bool ok, const FsstSymTab* tab, bool lfast,
+                                                     const uint8_t* seg, uint32_t row_begin, uint32_t rows,
+                                                     uint32_t width)
+{
+  if (ok) block_issue<FSST_THREADS>(reinterpret_cast<uint32_t*>(sm.sym), reinterpret_cast<const uint8_t*>(tab),
+                                    sizeof(FsstSymTab));
+  if (!lfast) return 0;
+  const uint64_t b0 = (uint64_t{row_begin} * width) >> 3;
+  const uint64_t b1 = (uint64_t{row_begin + rows} * width + 7u) >> 3;
+  const uint32_t h  = block_issue<FSST_THREADS>(reinterpret_cast<uint32_t*>(sm.out), seg + 16 + b0,
+                                               static_cast<uint32_t>(b1 - b0));
+  return h * 8u + static_cast<uint32_t>((uint64_t{row_begin} * width) & 7u);
+}
+
+// The offsets of thread t's rows 2t and 2t + 1, and the column's closing one.
+__device__ __forceinline__ void fsst_row_offsets(uint32_t c, uint32_t n_chunks, uint32_t col_row, uint32_t rows,
+                                                 uint64_t T, uint64_t base, uint32_t o0, uint32_t o1, int32_t* offsets,
+                                                 uint32_t total_rows)
+{
+  const uint32_t r        = 2u * threadIdx.x;
+  const gptr<int32_t> off = gbl(offsets) + col_row;
+  if (r < rows) off[r] = static_cast<int32_t>(static_cast<uint32_t>(base) + o0);
+  if (r + 1u < rows) off[r + 1u] = static_cast<int32_t>(static_cast<uint32_t>(base) + o1);
+  if (c == n_chunks - 1u && threadIdx.x == 0)
+    gbl(offsets)[total_rows] = static_cast<int32_t>(static_cast<uint32_t>(base + T));
+}
+
+// The row starts of a run: thread t's rows end at run positions e0, e1 in
+// row order (compressed bytes of the run up to and including the row).
+__device__ __forceinline__ void fsst_mark_row(FsstSmem& sm, uint32_t y)
+{
+  __hip_atomic_fetch_or(&sm.bits[y >> 5], 1u << (y & 31u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// A run's chars from its walked groups: window by window when they pass
+// FSST_WINDOW.  The window is cleared for the first one, and sm.comp[] and
+// sm.dec[] are complete.  `get_base()` gives the chars offset of the run (it
+// is called once, after the first window's ORs, and synchronises the
+// workgroup).
+template <class GetBase>
+__device__ __forceinline__ void fsst_emit_run(FsstGroup (&gr)[GROUPS_PER_THR], FsstSmem& sm, uint32_t y_hi,
+                                              const bool (&lits)[GROUPS_PER_THR], uint32_t T, uint8_t* chars,
+                                              uint64_t chars_cap, GetBase&& get_base)
+{
+  const uint32_t tid = threadIdx.x;
+  // the groups' bytes are taken apart again, not kept from the first walk in
+  // a register each
+#pragma unroll
+  for (uint32_t k = 0; k < GROUPS_PER_THR; ++k)
+#pragma unroll
+    for (uint32_t d = 0; d < 4; ++d) __asm__ volatile("" : "+v"(gr[k].q[d]), "+v"(gr[k].p[d]));
+  if (T <= FSST_WINDOW) {
+#pragma unroll
+    for (uint32_t k = 0; k < GROUPS_PER_THR; ++k)
+      fsst_group_emit<false>(gr[k], sm, k * FSST_THREADS + tid, y_hi, lits[k], T, 0u);
+    const uint64_t at = get_base();
+    if (at < chars_cap)
+      window_store(sm, reinterpret_cast<uintptr_t>(chars) + at,
+                   at + T <= chars_cap ? T : static_cast<uint32_t>(chars_cap - at));
+    return;
+  }
+  uint64_t base = 0;
+#pragma unroll 1
+  for (uint32_t w0 = 0; w0 < T; w0 += FSST_WINDOW) {
+    const uint32_t nw = T - w0 < FSST_WINDOW ? T - w0 : FSST_WINDOW;
+    if (w0) {
+      __syncthreads();  // the stores have read the window
+      window_clear(sm, nw);
+      __syncthreads();
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < GROUPS_PER_THR; ++k)
+      fsst_group_emit<true>(gr[k], sm, k * FSST_THREADS + tid, y_hi, lits[k], T, w0);
+    if (w0) __syncthreads();
+    else base = get_base();
+    const uint64_t at = base + w0;
+    if (at >= chars_cap) return;
+    window_store(sm, reinterpret_cast<uintptr_t>(chars) + at,
+                 at + nw <= chars_cap ? nw : static_cast<uint32_t>(chars_cap - at));
+  }
+}
+
+// A chunk that is not one run: several runs, all walked for their decoded
+// lengths first and again, each before it is emitted; or (malformed, or a row
+// that no run holds) the row-wise path.  A call with scalar arguments, as
+// plain_chunk.
+__device__ __attribute__((noinline)) void fsst_chunk_runs(const uint8_t* seg, uint32_t bytes_size, uint32_t dict_end,
+                                                          uint32_t flags, uint32_t c_lo, uint32_t c_hi,
+                                                          uint32_t row_begin, uint32_t rows, uint32_t col_row,
+                                                          const FsstSymTab* __restrict__ tab, uint32_t c,
+                                                          uint32_t n_chunks, FsstState* __restrict__ st,
+                                                          int32_t* __restrict__ offsets, uint8_t* __restrict__ chars,
+                                                          uint64_t chars_cap, uint32_t total_rows, uint32_t spin_limit,
+                                                          LdsPtr<FsstSmem> smp)
+{
+  FsstSmem& sm         = *(FsstSmem*)smp;
+  const uint32_t tid   = threadIdx.x;
+  const bool ok        = flags & FI_OK;
+  const uint8_t* end   = seg + bytes_size;
+  const uint32_t width = flags & FI_WIDTH;
+  const bool lfast     = ok && width && (flags & FI_LFAST);
+  const uint32_t bit0  = fsst_issue_front(sm, ok, tab, lfast, seg, row_begin, rows, width);
+  __builtin_amdgcn_s_waitcnt(WAITCNT_VMEM_DONE);
+  __syncthreads();
+  const uint32_t* lw = reinterpret_cast<const uint32_t*>(sm.out);
+  const uint32_t r0 = 2u * tid, r1 = r0 + 1u;
+  const uint32_t cl0 = fsst_field(lw, bit0, lfast, seg, end, row_begin, width, r0, rows);
+  const uint32_t cl1 = fsst_field(lw, bit0, lfast, seg, end, row_begin, width, r1, rows);
+  const uint32_t ne0 = cl0 ? 1u : 0u, ne1 = cl1 ? 1u : 0u;  // rows with bytes
+  constexpr uint32_t RUN_MAX = FSST_CSTAGE - 15u;            // whatever the run's alignment
+  const uint32_t wide        = cl0 > RUN_MAX || cl1 > RUN_MAX ? 1u << 16 : 0u;
+  uint32_t x0, n0, x_all, n_all;
+  block_excl_scan2(cl0 + cl1, ne0 + ne1 + wide, sm.wave, x0, n0, x_all, n_all);
+  const uint32_t x1 = x0 + cl0, x2 = x1 + cl1;
+  // Rows shorter than 1 MiB keep the prefix sums from wrapping, so they rise
+  // from c_lo to c_hi.
+  if (!ok || (flags & FI_HUGE) || c_hi < c_lo || c_hi > dict_end || n_all >> 16) {
+    if (tid == 0) sm.comp[0] = c_lo;
+    if (r0 < rows) sm.comp[r0 + 1u] = c_lo + x1;
+    if (r1 < rows) sm.comp[r1 + 1u] = c_lo + x2;
+    __syncthreads();
+    const uint32_t T    = fsst_lengths_rows(sm, ok, seg, dict_end, rows);
+    const uint64_t base = fsst_lookback(c, n_chunks, T, st, spin_limit, sm);
+    fsst_offsets(FsstChunk{0u, row_begin, rows, col_row}, c, n_chunks, rows, T, base, offsets, total_rows, sm);
+    if (T == 0 || base >= chars_cap) return;
+    fsst_emit_rows(sm, seg, dict_end, rows, T, base, chars, chars_cap);
+    return;
+  }
+  n0 &= 0xFFFFu;
+  const uint32_t n1 = n0 + ne0;
+  if (tid == 0) sm.len[FSST_ESC] = LEN_ESC;
+  // the run: rows [ra, rb), compressed bytes [xa, xb) of the chunk, nb rows
+  // with bytes below rb; t_before decoded bytes of the chunk precede it
+  uint32_t ra = 0, rb = 0, xa = 0, xb = 0, nb = 0, o0 = 0, o1 = 0;
+  uint64_t t_before = 0, base = 0;
+  bool measured     = false;
+#pragma unroll 1
+  for (;;) {
+    // as many rows as fit; the last of them tells where the run ends
+    __syncthreads();  // the previous run's users of LDS are done
+    const bool f0       = r0 >= ra && r0 < rows && x1 - xa <= RUN_MAX;
+    const bool f1       = r1 >= ra && r1 < rows && x2 - xa <= RUN_MAX;
+    const uint32_t fits = static_cast<uint32_t>(__builtin_popcountll(ballot(f0)) + __builtin_popcountll(ballot(f1)));
+    if (lane_id() == 0) sm.part[tid >> 6] = fits;
+    for (uint32_t i = tid; i < FSST_CSTAGE / 32u; i += FSST_THREADS) sm.bits[i] = 0u;
+    __syncthreads();
+    rb = ra + __builtin_amdgcn_readlane(row_incl_sum_u32(sm.part[lane_id() & (FSST_WAVES - 1u)]), FSST_WAVES - 1u);
+    if (r0 == rb - 1u || r1 == rb - 1u) {
+      sm.wave[0] = r0 == rb - 1u ? x1 : x2;
+      sm.wave[1] = r0 == rb - 1u ? n1 : n1 + ne1;
+    }
+    __syncthreads();
+    xb = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(sm.wave[0])));
+    nb = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(sm.wave[1])));
+    const bool some      = xb != xa;
+    const uintptr_t sa   = reinterpret_cast<uintptr_t>(seg + dict_end - c_lo - xb);
+    const uint32_t c_h   = some ? static_cast<uint32_t>(sa & 15u) : 0u;
+    const uint32_t y_hi  = some ? c_h + (xb - xa) : 0u;
+    const uint8_t* stage = some ? reinterpret_cast<const uint8_t*>(sa - c_h)
+                                : reinterpret_cast<const uint8_t*>(fsst_zero_group);
+    FsstGroup gr[GROUPS_PER_THR];
+    uint32_t prev[GROUPS_PER_THR];
+    fsst_load_groups(gr, prev, stage, y_hi);
+    const bool in0 = r0 >= ra && r0 < rb, in1 = r1 >= ra && r1 < rb;
+    if (in0 && ne0) fsst_mark_row(sm, y_hi - (x1 - xa));
+    if (in1 && ne1) fsst_mark_row(sm, y_hi - (x2 - xa));
+    __syncthreads();
+    bool lits[GROUPS_PER_THR];
+    uint32_t T = 0;
+    fsst_walk_lengths(gr, sm, prev, c_h, y_hi, stage, lits, &T);
+    window_clear(sm, T < FSST_WINDOW ? T : FSST_WINDOW);
+    __syncthreads();
+    if (in0 || in1) {  // as in fsst_chunk
+      const uint32_t k0 = nb - (in0 ? n0 : n1), k1 = nb - n1;
+      const uint32_t e0 = sm.comp[k0], e1 = sm.comp[k1];
+      if (in0) o0 = static_cast<uint32_t>(t_before) + T - e0;
+      if (in1) o1 = static_cast<uint32_t>(t_before) + T - e1;
+      if (in0 && ne0) sm.dec[k0] = T - e0 - e1;
+      if (in1 && ne1) sm.dec[k1] = T - e1 - sm.comp[k1 - 1u];
+    }
+    if (tid == 0) sm.dec[0] = T;
+    __syncthreads();
+    if (measured) {
+      fsst_emit_run(gr, sm, y_hi, lits, T, chars, chars_cap, [&]() -> uint64_t {
+        __syncthreads();
+        return base + t_before;
+      });
+      if (rb >= rows) return;
+    }
+    t_before += T;
+    ra = rb;
+    xa = xb;
+    if (rb < rows) continue;
+    measured = true;
+    fsst_lookback_publish(c, t_before, st, spin_limit);
+    base = fsst_lookback_wait(c, n_chunks, t_before, st, spin_limit, sm);
+    fsst_row_offsets(c, n_chunks, col_row, rows, t_before, base, o0, o1, offsets, total_rows);
+    ra = xa  = 0;
+    t_before = 0;
+  }
+}
+
 // Decode chunk `c` (its position in the column's chunk order) with the
-// calling 256-thread workgroup.  Every thread must call it, after a
-// workgroup barrier that follows any earlier use of `sm` (the callers' claim
-// of the chunk ends with one), so the first loads issue without waiting.
-// `ci` and `tab` are the segment pre-pass's output for the chunk and its
-// segment (unused for a chunk of uncovered rows).
+// calling workgroup.  Every thread must call it, after a workgroup barrier
+// that follows any earlier use of `sm` (the callers' claim of the chunk ends
+// with one), so the first loads issue without waiting.  `ci` and `tab` are the
+// segment pre-pass's output for the chunk and its segment (unused for a chunk
+// of uncovered rows).
 //
-// One memory round trip stages, with LDS-direct loads, the symbol table,
-// the chunk's compressed-length fields and its compressed bytes; a second
-// is the look-back for the column-wide chars offset.
-template <uint32_t OUT_CAP>
+// One memory round trip brings the symbol table and the chunk's
+// compressed-length fields to LDS (LDS-direct loads) and its compressed bytes
+// to registers; a second is the look-back for the column-wide chars offset.
 __device__ __forceinline__ void fsst_chunk(const FsstChunk ch, const FsstChunkInfo ci, const FsstSymTab* tab,
                                            uint32_t c, uint32_t n_chunks, FsstState* __restrict__ st,
                                            int32_t* __restrict__ offsets, uint8_t* __restrict__ chars,
-                                           uint64_t chars_cap, uint32_t total_rows, uint32_t spin_limit,
-                                           FsstSmemT<OUT_CAP>& sm)
+                                           uint64_t chars_cap, uint32_t total_rows, uint32_t spin_limit, FsstSmem& sm)
 {
-  const uint32_t tid      = threadIdx.x;
-  const bool ok           = ch.seg != FSST_GAP && (ci.flags & FI_OK);
+  const uint32_t tid  = threadIdx.x;
+  const bool ok       = ch.seg != FSST_GAP && (ci.flags & FI_OK);
+  const uint32_t rows = ch.rows;
   if (ok && (ci.flags & (FI_DICT | FI_UNC | FI_DFSST))) {  // uniform per chunk
-    plain_chunk(ci.bytes, ci.bytes_size, ci.dict_end, ci.flags, ci.c_lo, ci.c_hi, ch.row_begin, ch.rows, ch.col_row,
-                c, n_chunks, st, offsets, chars, chars_cap, total_rows, spin_limit, sm);
+    plain_chunk(ci.bytes, ci.bytes_size, ci.dict_end, ci.flags, ci.c_lo, ci.c_hi, ch.row_begin, rows, ch.col_row, c,
+                n_chunks, st, offsets, chars, chars_cap, total_rows, spin_limit, sm);
     return;
   }
-  const uint8_t* seg      = ok ? ci.bytes : nullptr;
-  const uint8_t* end      = ok ? ci.bytes + ci.bytes_size : nullptr;
-  const uint32_t dict_end = ok ? ci.dict_end : 0u;
-  const uint32_t width    = ok ? (ci.flags & FI_WIDTH) : 0u;
-  const uint32_t rows     = ch.rows;
-  const uint32_t c_lo     = ok ? ci.c_lo : 0u;
-  const uint32_t c_hi     = ok ? ci.c_hi : 0u;
-  const bool lfast        = ok && width && (ci.flags & FI_LFAST);
-  // Rows shorter than 1 MiB keep the prefix sums from wrapping, so comp[]
-  // rises from c_lo to c_hi.
-  const bool staged = ok && rows && !(ci.flags & FI_HUGE) && c_hi >= c_lo && c_hi <= dict_end &&
-                      c_hi - c_lo <= FSST_CSTAGE;
+  // Rows are stored back to front ending at dict_end: the chunk's bytes are
+  // [dict_end - c_hi, dict_end - c_lo).  One run holds them nearly always.
+  const uint8_t* seg = ci.bytes;
+  const uint32_t C   = ci.c_hi - ci.c_lo;
+  const uintptr_t ca = reinterpret_cast<uintptr_t>(seg + ci.dict_end - ci.c_hi);
+  const uint32_t c_h = static_cast<uint32_t>(ca & 15u);
+  if (!ok || !rows || (ci.flags & FI_HUGE) || ci.c_hi <= ci.c_lo || ci.c_hi > ci.dict_end || C > FSST_CSTAGE - c_h) {
+    fsst_chunk_runs(ok ? seg : nullptr, ok ? ci.bytes_size : 0u, ok ? ci.dict_end : 0u, ok ? ci.flags : 0u,
+                    ok ? ci.c_lo : 0u, ok ? ci.c_hi : 0u, ch.row_begin, rows, ch.col_row, tab, c, n_chunks, st,
+                    offsets, chars, chars_cap, total_rows, spin_limit, (LdsPtr<FsstSmem>)(&sm));
+    return;
+  }
+  const uint8_t* end   = seg + ci.bytes_size;
+  const uint32_t width = ci.flags & FI_WIDTH;
+  const bool lfast     = width && (ci.flags & FI_LFAST);
+  const uint32_t y_hi  = c_h + C;
+  const uint8_t* stage = reinterpret_cast<const uint8_t*>(ca - c_h);
+  const uint32_t bit0  = fsst_issue_front(sm, true, tab, lfast, seg, ch.row_begin, rows, width);
+  // The groups' loads go out last and unconditionally, so the wait below
+  // leaves exactly these 2 * GROUPS_PER_THR loads in flight: the compressed
+  // prefix runs while they arrive.
+  __builtin_amdgcn_sched_barrier(0);
+  FsstGroup gr[GROUPS_PER_THR];
+  uint32_t prev[GROUPS_PER_THR];
+  fsst_load_groups(gr, prev, stage, y_hi);
+  for (uint32_t i = tid; i < FSST_CSTAGE / 32u; i += FSST_THREADS) sm.bits[i] = 0u;
+  static_assert(GROUPS_PER_THR == 2, "the wait below leaves the groups' four loads in flight");
+  __asm__ volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
-  if (ok) block_issue<FSST_THREADS>(reinterpret_cast<uint32_t*>(sm.sym), reinterpret_cast<const uint8_t*>(tab),
-                                    sizeof(FsstSymTab));
-  uint32_t bit0 = 0;
-  if (lfast) {
-    const uint64_t b0 = (uint64_t{ch.row_begin} * width) >> 3;
-    const uint64_t b1 = (uint64_t{ch.row_begin + rows} * width + 7u) >> 3;
-    const uint32_t h  = block_issue<FSST_THREADS>(reinterpret_cast<uint32_t*>(sm.out), seg + 16 + b0,
-                                                 static_cast<uint32_t>(b1 - b0));
-    bit0 = h * 8u + static_cast<uint32_t>((uint64_t{ch.row_begin} * width) & 7u);
-  }
-  // Rows are stored back to front ending at dict_end: row r is
-  // [dict_end - comp[r+1], dict_end - comp[r]).  Stage position 0 is the
-  // 16-byte-aligned address at or below the chunk's first compressed byte;
-  // each thread loads its first-walk span into registers.
-  uint32_t c_h         = 0;
-  const uint8_t* stage = nullptr;
-  if (staged) {
-    const uintptr_t a = reinterpret_cast<uintptr_t>(seg + dict_end - c_hi);
-    c_h               = static_cast<uint32_t>(a & 15u);
-    stage             = reinterpret_cast<const uint8_t*>(a - c_h);
-  }
-  // The span loads go out last and unconditionally (a chunk with no
-  // compressed bytes reads a zero group), so the wait below covers the
-  // symbol table and length fields only: the compressed prefix runs while
-  // the spans still arrive.
-  const bool spans = staged && c_h + (c_hi - c_lo) != 0;
-  u32x4 qv[SPAN_GROUPS];
-  fsst_span_load(qv, spans ? stage : reinterpret_cast<const uint8_t*>(fsst_zero_group),
-                 spans ? c_h + (c_hi - c_lo) : 16u);
-  static_assert(SPAN_GROUPS == 5, "the wait below leaves the five span loads in flight");
-  __asm__ volatile("s_waitcnt vmcnt(5) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  // ---- rows: compressed lengths (fsst.cu:132-188) and starts; thread t owns
+  // rows 2t, 2t + 1 ----
+  static_assert(ROWS_PER_THR == 2, "the staged path's row arithmetic");
+  const uint32_t* lw = reinterpret_cast<const uint32_t*>(sm.out);
+  const uint32_t cl0 = fsst_field(lw, bit0, lfast, seg, end, ch.row_begin, width, 2u * tid, rows);
+  const uint32_t cl1 = fsst_field(lw, bit0, lfast, seg, end, ch.row_begin, width, 2u * tid + 1u, rows);
+  const uint32_t ne0 = cl0 ? 1u : 0u, ne1 = cl1 ? 1u : 0u;  // rows with bytes
+  uint32_t x0, n0, x_all, n_all;
+  block_excl_scan2(cl0 + cl1, ne0 + ne1, sm.wave, x0, n0, x_all, n_all);
+  if (ne0) fsst_mark_row(sm, y_hi - (x0 + cl0));
+  if (ne1) fsst_mark_row(sm, y_hi - (x0 + cl0 + cl1));
+  if (tid == 0) sm.len[FSST_ESC] = LEN_ESC;
+  lds_barrier();
 
-  // ---- compressed prefix comp[] (fsst.cu:132-188); thread t owns rows
-  // 4t .. 4t + 3 here ----
-  {
-    const uint32_t* lw = reinterpret_cast<const uint32_t*>(sm.out);
-    uint32_t cl[ROWS_PER_THR];
-    uint32_t sum = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < ROWS_PER_THR; ++i) {
-      const uint32_t r = ROWS_PER_THR * tid + i;
-      uint32_t v       = 0;
-      if (width && r < rows)
-        v = lfast ? lds_bits32(lw, bit0 + r * width, width)
-                  : stream_bits32(seg + 16, end, uint64_t{ch.row_begin + r} * width, width);
-      cl[i] = v;
-      sum += v;
-    }
-    uint32_t tot     = 0;
-    uint32_t run     = c_lo + block_excl_scan<true>(sum, sm.wave, &tot);  // the spans still arrive
-    if (tid == 0) sm.comp[0] = c_lo;
-#pragma unroll
-    for (uint32_t i = 0; i < ROWS_PER_THR; ++i) {
-      const uint32_t r = ROWS_PER_THR * tid + i;
-      run += cl[i];
-      if (r < rows) sm.comp[r + 1] = run;
-    }
-  }
-  if (staged) sm.part[tid] = fsst_span_tail(qv, c_h + (c_hi - c_lo));
-  __syncthreads();
+  // ---- first walk ----
+  bool lits[GROUPS_PER_THR];
+  uint32_t T = 0;
+  fsst_walk_lengths(gr, sm, prev, c_h, y_hi, stage, lits, &T);
+  // The aggregate is published now; the look-back's wait, and the offsets,
+  // come once the first window's chars are in LDS.
+  fsst_lookback_publish(c, T, st, spin_limit);
+  window_clear(sm, T < FSST_WINDOW ? T : FSST_WINDOW);
+  lds_barrier();
 
-  if (staged) {
-    const uint32_t C = c_hi - c_lo;
-    uint32_t T       = 0;
-    if (C) {
-      T = fsst_lengths_staged(sm, rows, c_h, c_hi, C, qv, stage);
-    } else {
-      for (uint32_t i = tid; i <= rows; i += FSST_THREADS) sm.dec[i] = 0;
-      __syncthreads();
-    }
-    // The aggregate is published now; the look-back's wait, and the offsets,
-    // come once the first window's chars are in LDS.
-    fsst_lookback_publish(c, T, st, spin_limit);
-    uint64_t base = 0;
-    bool based    = false;
-    auto finish   = [&]() -> uint64_t {
-      if (!based) {
-        base = fsst_lookback_wait(c, n_chunks, T, st, spin_limit, sm);
-        fsst_offsets(ch, c, n_chunks, rows, T, base, offsets, total_rows, sm);
-        based = true;
-      } else {
-        __syncthreads();
-      }
-      return base;
-    };
-    const bool emitted = T != 0 && fsst_emit_staged(sm, rows, c_h, c_hi, T, finish, chars, chars_cap, stage);
-    if (!based) finish();
-    if (T == 0 || emitted || base >= chars_cap) return;
-    fsst_emit_rows(sm, seg, dict_end, rows, T, base, chars, chars_cap);
-  } else {
-    const uint32_t T    = fsst_lengths_rows(sm, ok, seg, dict_end, rows);
-    const uint64_t base = fsst_lookback(c, n_chunks, T, st, spin_limit, sm);
-    fsst_offsets(ch, c, n_chunks, rows, T, base, offsets, total_rows, sm);
-    if (T == 0 || base >= chars_cap) return;
-    fsst_emit_rows(sm, seg, dict_end, rows, T, base, chars, chars_cap);
-  }
+  // ---- rows: output positions.  A row's chars follow those of the rows below
+  // it, which lie after it in storage order ----
+  const uint32_t k0 = n_all - n0;  // one past row 2t's rank (the rank's place when it has no bytes)
+  const uint32_t k1 = k0 - ne0;
+  const uint32_t e0 = sm.comp[k0], e1 = sm.comp[k1];
+  if (ne0) sm.dec[k0] = T - e0 - e1;  // rank k0 - 1 == k1: output position T - e0, prefix e1
+  if (ne1) sm.dec[k1] = T - e1 - sm.comp[k1 - 1u];
+  if (tid == 0) sm.dec[0] = T;  // bytes before the first row's, which decode to nothing
+  lds_barrier();
+
+  // ---- second walk ----
+  fsst_emit_run(gr, sm, y_hi, lits, T, chars, chars_cap, [&]() -> uint64_t {
+    const uint64_t base = fsst_lookback_wait(c, n_chunks, T, st, spin_limit, sm);
+    fsst_row_offsets(c, n_chunks, ch.col_row, rows, T, base, T - e0, T - e1, offsets, total_rows);
+    return base;
+  });
 }
 
 }  // namespace sdr

@@ -61,16 +61,6 @@ __device__ __forceinline__ uint32_t lds_u16(const uint32_t* lds, uint32_t byte)
   return __builtin_amdgcn_alignbit(lds[w + 1], lds[w], (byte & 3u) * 8u) & 0xFFFFu;
 }
 
-// Inclusive prefix sum within each 16-lane row of the wave.
-__device__ __forceinline__ uint32_t row_incl_sum_u32(uint32_t v)
-{
-  v += dpp_u32<0x111>(v);  // row_shr:1
-  v += dpp_u32<0x112>(v);  // row_shr:2
-  v += dpp_u32<0x114>(v);  // row_shr:4
-  v += dpp_u32<0x118>(v);  // row_shr:8
-  return v;
-}
-
 // Stage pass `t0` (n entries) and compute every chunk's row base from
 // `base`.  With `detect`, also record the first exact match and the first
 // zero/overshoot entry of the pass in sm.match / sm.bad (UINT32_MAX: none).

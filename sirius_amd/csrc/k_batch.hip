@@ -27,7 +27,7 @@ namespace sdr {
 // 4 KiB of bitpacking or ALP codes, or the ALP-RD left stream plus 4 KiB of
 // its right stream.
 constexpr uint32_t BATCH_BP_STAGE = 4096;
-static_assert(BATCH_PREP_THREADS == FSST_THREADS, "pre-pass workgroup size");
+static_assert(BATCH_PREP_THREADS == PREP_THREADS, "pre-pass workgroup size");
 static_assert(BATCH_WAVES == WAVES_PER_BLOCK, "fixed-width group block");
 
 template <typename T>
@@ -108,11 +108,11 @@ __global__ __launch_bounds__(BLOCK_THREADS) void k_bgroup_copy(const BatchItem* 
 // predecessors in its column are held by blocks that started earlier, which
 // the look-back's progress needs (the per-column kernel's ticket does the
 // same).  One chunk per block, with no loop around it, keeps the kernel at
-// 80 VGPRs: six workgroups per CU with the 11 KiB window.
+// 80 VGPRs: three workgroups of eight waves per CU.
 __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_bgroup_fsst(
   const BatchItem* __restrict__ items, BatchQueue* __restrict__ q, uint32_t g)
 {
-  __shared__ FsstSmemT<FSST_OUT_BATCH> sm;
+  __shared__ FsstSmem sm;
   __shared__ uint32_t s_idx;
   (void)items;  // the FSST group's entries are q->fsst_entries
   // read before the claim, so they arrive while it does
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6)
   // launch), so its wait falls behind the loads of the symbol table and
   // the compressed bytes
   const FsstColumn col = sload(q->fsst_cols + e.col);
-  fsst_chunk<FSST_OUT_BATCH>(ch, ci, q->fsst_tabs + (ch.seg == FSST_GAP ? 0u : ch.seg), e.chunk, col.n_chunks,
+  fsst_chunk(ch, ci, q->fsst_tabs + (ch.seg == FSST_GAP ? 0u : ch.seg), e.chunk, col.n_chunks,
                              col.state, col.offsets, col.chars, col.chars_cap, col.total_rows, spin, sm);
 }
 
@@ -146,7 +146,7 @@ __global__ void k_batch_reset(BatchQueue* q)
   if (blockIdx.x == 0 && threadIdx.x == 0) q->error = 0;
 }
 
-__global__ __launch_bounds__(FSST_THREADS) void k_batch_fsst_prep(const BatchQueue* __restrict__ q)
+__global__ __launch_bounds__(PREP_THREADS) void k_batch_fsst_prep(const BatchQueue* __restrict__ q)
 {
   __shared__ FsstPrepSmem sm;
   const uint32_t n = q->n_fsst_segs;

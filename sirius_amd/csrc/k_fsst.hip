@@ -11,19 +11,19 @@ __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6)
                                                        int32_t* __restrict__ offsets, uint8_t* __restrict__ chars,
                                                        uint64_t chars_cap, uint32_t total_rows, uint32_t spin_limit)
 {
-  __shared__ FsstSmemT<FSST_OUT_COLUMN> sm;
+  __shared__ FsstSmem sm;
   __shared__ uint32_t s_ticket;
   if (threadIdx.x == 0) s_ticket = atomicAdd(&st->ticket, 1u);
   __syncthreads();
   const uint32_t c = s_ticket;
   if (c >= n_chunks) return;  // grid size equals chunk count; never taken
   const FsstChunk ch = chunks[c];
-  fsst_chunk<FSST_OUT_COLUMN>(ch, info[c], tabs + (ch.seg == FSST_GAP ? 0u : ch.seg), c, n_chunks, st, offsets,
+  fsst_chunk(ch, info[c], tabs + (ch.seg == FSST_GAP ? 0u : ch.seg), c, n_chunks, st, offsets,
                               chars, chars_cap, total_rows, spin_limit, sm);
 }
 
 // Segment pre-pass: one workgroup per segment (grid-stride).
-__global__ __launch_bounds__(FSST_THREADS) void k_fsst_prep(const FsstSeg* __restrict__ segs, uint32_t n_segs,
+__global__ __launch_bounds__(PREP_THREADS) void k_fsst_prep(const FsstSeg* __restrict__ segs, uint32_t n_segs,
                                                             const uint32_t* __restrict__ d_n_segs,
                                                             FsstChunk* __restrict__ chunks,
                                                             FsstChunkInfo* __restrict__ info,
@@ -57,7 +57,7 @@ __global__ void k_dfsst_headers(const FsstSeg* __restrict__ segs, uint32_t n, ui
   }
 }
 
-__global__ __launch_bounds__(FSST_THREADS) void k_dfsst_prep(const DictFsstSeg* __restrict__ dseg, uint32_t n,
+__global__ __launch_bounds__(PREP_THREADS) void k_dfsst_prep(const DictFsstSeg* __restrict__ dseg, uint32_t n,
                                                              uint32_t* __restrict__ e_byte,
                                                              uint32_t* __restrict__ e_dec,
                                                              FsstSymTab* __restrict__ tabs, uint32_t* __restrict__ out)
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(FSST_THREADS) void k_dfsst_prep(const DictFsstSeg* 
 }
 
 // grid.y: segments; grid.x blocks share a segment's entries
-__global__ __launch_bounds__(FSST_THREADS) void k_dfsst_predecode(const DictFsstSeg* __restrict__ dseg,
+__global__ __launch_bounds__(PREP_THREADS) void k_dfsst_predecode(const DictFsstSeg* __restrict__ dseg,
                                                                   const uint32_t* __restrict__ e_byte,
                                                                   const FsstSymTab* __restrict__ tabs)
 {
@@ -132,7 +132,7 @@ hipError_t launch_dfsst_prep(const DictFsstSeg* d_dseg, uint32_t n_dseg, uint32_
                              FsstSymTab* d_tabs, uint32_t* d_out, hipStream_t s)
 {
   if (n_dseg == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_dfsst_prep, dim3(n_dseg < 4096u ? n_dseg : 4096u), dim3(FSST_THREADS), 0, s, d_dseg, n_dseg,
+  hipLaunchKernelGGL(k_dfsst_prep, dim3(n_dseg < 4096u ? n_dseg : 4096u), dim3(PREP_THREADS), 0, s, d_dseg, n_dseg,
                      d_e_byte, d_e_dec, d_tabs, d_out);
   return hipGetLastError();
 }
@@ -141,7 +141,7 @@ hipError_t launch_dfsst_predecode(const DictFsstSeg* d_dseg, uint32_t n_dseg, co
                                   const FsstSymTab* d_tabs, hipStream_t s)
 {
   if (n_dseg == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_dfsst_predecode, dim3(8, n_dseg), dim3(FSST_THREADS), 0, s, d_dseg, d_e_byte, d_tabs);
+  hipLaunchKernelGGL(k_dfsst_predecode, dim3(8, n_dseg), dim3(PREP_THREADS), 0, s, d_dseg, d_e_byte, d_tabs);
   return hipGetLastError();
 }
 
@@ -170,7 +170,7 @@ hipError_t launch_fsst_prep(const FsstSeg* d_segs, uint32_t n_segs, const uint32
                             FsstChunk* d_chunks, FsstChunkInfo* d_info, FsstSymTab* d_tabs, hipStream_t s)
 {
   if (grid == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fsst_prep, dim3(grid), dim3(FSST_THREADS), 0, s, d_segs, n_segs, d_n_segs, d_chunks, d_info,
+  hipLaunchKernelGGL(k_fsst_prep, dim3(grid), dim3(PREP_THREADS), 0, s, d_segs, n_segs, d_n_segs, d_chunks, d_info,
                      d_tabs);
   return hipGetLastError();
 }

@@ -49,6 +49,11 @@ __device__ __forceinline__ gptr<T> gbl(T* p)
   return (gptr<T>)(p);
 }
 
+// An LDS object as the argument of a function that is called, not inlined: a
+// generic reference would make the callee's accesses flat.
+template <typename T>
+using LdsPtr = __attribute__((address_space(3))) T*;
+
 // A whole descriptor read through a global pointer (struct copies through an
 // address-space-qualified lvalue are not allowed).
 template <typename T>
@@ -179,28 +184,36 @@ __device__ __forceinline__ uint64_t su_t(const uint8_t* p)
   else return su64(p);
 }
 
-// ---- wave scans (DPP row shifts + cross-row readlane) ----------------------
+// ---- wave scans (DPP row shifts, then row broadcasts) ----------------------
 
+// v moved by a DPP row shift; lanes without a source read 0, which lets the
+// compiler fold the move into the add that uses it.
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_u32(uint32_t v)
 {
   return static_cast<uint32_t>(
-    __builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xF, 0xF, false));
+    __builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xF, 0xF, true));
 }
 
-// Inclusive prefix sum over the 64 lanes (wrapping).
-__device__ __forceinline__ uint32_t wave_incl_sum_u32(uint32_t v)
+// Inclusive prefix sum within each 16-lane row of the wave.
+__device__ __forceinline__ uint32_t row_incl_sum_u32(uint32_t v)
 {
   v += dpp_u32<0x111>(v);  // row_shr:1
   v += dpp_u32<0x112>(v);  // row_shr:2
   v += dpp_u32<0x114>(v);  // row_shr:4
   v += dpp_u32<0x118>(v);  // row_shr:8
-  uint32_t r15 = __builtin_amdgcn_readlane(v, 15);
-  uint32_t r31 = __builtin_amdgcn_readlane(v, 31);
-  uint32_t r47 = __builtin_amdgcn_readlane(v, 47);
-  uint32_t row = lane_id() >> 4;
-  uint32_t add = (row >= 1 ? r15 : 0u) + (row >= 2 ? r31 : 0u) + (row >= 3 ? r47 : 0u);
-  return v + add;
+  return v;
+}
+
+// Inclusive prefix sum over the 64 lanes (wrapping): six DPP adds, the last
+// two adding lane 15 of rows 0 and 2 to the row above, then lane 31 to rows
+// 2 and 3.
+__device__ __forceinline__ uint32_t wave_incl_sum_u32(uint32_t v)
+{
+  v = row_incl_sum_u32(v);
+  v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x142, 0xA, 0xF, false));
+  v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x143, 0xC, 0xF, false));
+  return v;
 }
 
 template <int CTRL>
