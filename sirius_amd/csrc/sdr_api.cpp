@@ -11,6 +11,8 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <iterator>
+#include <map>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -172,12 +174,11 @@ int copy_stream(int dev, hipStream_t* out)
 }
 }  // namespace
 
-int desc_acquire(const void* h_src, size_t bytes, hipStream_t s, void** d_out, void** token)
+namespace {
+// A held slot of device `dev` with buffers of at least `bytes`.
+int slot_hold(int dev, size_t bytes, DescSlot** out)
 {
-  *d_out = nullptr;
-  *token = nullptr;
-  int dev = 0;
-  HIP_TRY(hipGetDevice(&dev));
+  *out = nullptr;
   DescSlot* pick = nullptr;
   bool fresh = false, wait = false;
   {
@@ -237,6 +238,44 @@ int desc_acquire(const void* h_src, size_t bytes, hipStream_t s, void** d_out, v
     if (e == hipSuccess) pick->cap = cap;
   }
   if (e != hipSuccess) return unhold(fail(SDR_E_HIP, "descriptor slot: %s", hipGetErrorString(e)));
+  *out = pick;
+  return SDR_OK;
+}
+
+// Give a held slot back unused.
+int slot_unhold(DescSlot* sl, int rc)
+{
+  std::lock_guard<std::mutex> lk(g_desc_mu);
+  sl->held = false;
+  return rc;
+}
+}  // namespace
+
+int pinned_acquire(size_t bytes, void** h_out, void** token)
+{
+  *h_out  = nullptr;
+  *token  = nullptr;
+  int dev = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  DescSlot* sl = nullptr;
+  const int rc = slot_hold(dev, bytes, &sl);
+  if (rc) return rc;
+  *h_out = sl->h;
+  *token = sl;
+  return SDR_OK;
+}
+
+int desc_acquire(const void* h_src, size_t bytes, hipStream_t s, void** d_out, void** token)
+{
+  *d_out  = nullptr;
+  *token  = nullptr;
+  int dev = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  DescSlot* pick = nullptr;
+  const int hrc  = slot_hold(dev, bytes, &pick);
+  if (hrc) return hrc;
+  auto unhold  = [&](int rc) { return slot_unhold(pick, rc); };
+  hipError_t e = hipSuccess;
   std::memcpy(pick->h, h_src, bytes);
   // The copy goes on the copy stream only while the caller's stream still
   // has work queued: on an idle stream the cross-stream wait would only add
@@ -330,20 +369,83 @@ int check_validity_runs(const sdr_run* runs, uint32_t n, uint32_t total_rows)
   return SDR_OK;
 }
 
-// Overlay the UNCOMPRESSED validity bytes on an all-valid mask and count the
-// nulls into *d_count (src/cuda/scan/gpu_native_decode.cu:396-476, :519-538).
-int build_null_mask(const sdr_run* runs, uint32_t n, uint32_t total_rows, uint8_t* d_mask,
-                    unsigned long long* d_count, hipStream_t s)
+// The mask of a column: its UNCOMPRESSED validity bytes over an all-valid mask
+// (src/cuda/scan/gpu_native_decode.cu:396-476, :519-538), as pieces of at most
+// MASK_UNIT_BYTES in mask order.
+void add_mask_units(const sdr_run* runs, uint32_t n, uint32_t total_rows, uint8_t* d_mask, std::vector<MaskUnit>& out)
 {
-  HIP_TRY(launch_fill_u8(d_mask, 0xFF, (total_rows + 7u) / 8u, s));
+  struct Span {
+    uint32_t b0, b1;  // mask bytes
+    const uint8_t* src;
+  };
+  std::vector<Span> spans;
+  bool sorted = true;
   for (uint32_t r = 0; r < n; ++r)
     for (uint32_t k = 0; k < runs[r].n_segments; ++k) {
       const sdr_segment& g = runs[r].segments[k];
       if (!g.row_count) continue;
-      HIP_TRY(hipMemcpyAsync(d_mask + g.row_offset / 8u, g.d_bytes, (g.row_count + 7u) / 8u,
-                             hipMemcpyDeviceToDevice, s));
+      const uint32_t b0 = g.row_offset / 8u, b1 = b0 + (g.row_count + 7u) / 8u;
+      sorted = sorted && (spans.empty() || spans.back().b1 <= b0);
+      spans.push_back({b0, b1, g.d_bytes});
     }
-  HIP_TRY(launch_count_nulls(d_mask, total_rows, d_count, s));
+  if (!sorted) {
+    // a later segment wins: from the last one back, each keeps the bytes that
+    // none after it covers
+    std::map<uint32_t, uint32_t> taken;  // disjoint [first, second)
+    std::vector<Span> kept;
+    for (size_t i = spans.size(); i-- > 0;) {
+      uint32_t at = spans[i].b0;
+      auto it     = taken.upper_bound(at);
+      if (it != taken.begin() && std::prev(it)->second > at) at = std::prev(it)->second;
+      for (; at < spans[i].b1; it = taken.lower_bound(at)) {
+        const uint32_t to = it == taken.end() ? spans[i].b1 : std::min(spans[i].b1, it->first);
+        if (to > at) {
+          kept.push_back({at, to, spans[i].src + (at - spans[i].b0)});
+          taken[at] = to;
+        }
+        at = it == taken.end() ? to : std::max(to, it->second);
+      }
+    }
+    std::sort(kept.begin(), kept.end(), [](const Span& a, const Span& b) { return a.b0 < b.b0; });
+    spans.swap(kept);
+  }
+  const uint32_t end  = static_cast<uint32_t>((uint64_t{total_rows} + 7u) / 8u);
+  const uint32_t past = total_rows & 7u ? (0xFFu << (total_rows & 7u)) & 0xFFu : 0u;
+  auto add            = [&](uint32_t b0, uint32_t b1, const uint8_t* src) {
+    for (; b0 < b1; b0 += MASK_UNIT_BYTES) {
+      const uint32_t m = std::min(MASK_UNIT_BYTES, b1 - b0);
+      out.push_back({src, d_mask + b0, m, b0 + m == end ? past : 0u});
+      if (src) src += m;
+    }
+  };
+  uint32_t at = 0;
+  for (const Span& sp : spans) {
+    add(at, sp.b0, nullptr);
+    add(sp.b0, sp.b1, sp.src);
+    at = sp.b1;
+  }
+  add(at, end, nullptr);
+}
+
+int masks_launch(const std::vector<MaskUnit>& units, hipStream_t s, const uint32_t** counts, void** token)
+{
+  // the counts are written to pinned memory by the kernel, and a long list of
+  // pieces is read from it: no copy and no clear on the stream
+  const size_t n = units.size(), b_counts = (n * sizeof(uint32_t) + 15u) & ~size_t{15};
+  const bool host = n <= MASKS_INLINE;
+  void* h         = nullptr;
+  const int rc    = pinned_acquire(b_counts + (host ? 0u : n * sizeof(MaskUnit)), &h, token);
+  if (rc) return rc;
+  auto* hc = static_cast<uint32_t*>(h);
+  auto* hu = reinterpret_cast<MaskUnit*>(static_cast<uint8_t*>(h) + b_counts);
+  if (!host) std::memcpy(hu, units.data(), n * sizeof(MaskUnit));
+  const hipError_t e =
+    launch_null_mask(host ? units.data() : hu, static_cast<uint32_t>(n), hc, nullptr, s, host);
+  if (e != hipSuccess) {
+    (void)desc_release(*token, s);
+    return fail(SDR_E_HIP, "null mask launch: %s", hipGetErrorString(e));
+  }
+  *counts = hc;
   return SDR_OK;
 }
 
@@ -509,29 +611,27 @@ int decode_table(sdr_column* cols, uint32_t n_cols, hipStream_t s, uint32_t mode
   }
   rc = decode_runs(targets, s, mode);
   if (rc) return rc;
-  // validity: one counter per column, one synchronisation for all of them
+  // validity: one launch and one synchronisation for all columns
   std::vector<uint32_t> masked;
   for (uint32_t c = 0; c < n_cols; ++c)
     if (cols[c].has_nulls && cols[c].n_validity && cols[c].total_rows) masked.push_back(c);
   if (!masked.empty()) {
-    unsigned long long* d_cnt = nullptr;
-    rc = device_alloc(reinterpret_cast<void**>(&d_cnt), masked.size() * sizeof(unsigned long long), s);
-    if (rc) return rc;
-    HIP_TRY(hipMemsetAsync(d_cnt, 0, masked.size() * sizeof(unsigned long long), s));
-    for (size_t i = 0; i < masked.size(); ++i) {
-      sdr_column& col = cols[masked[i]];
-      rc = build_null_mask(col.validity, col.n_validity, col.total_rows, col.d_null_mask, d_cnt + i, s);
-      if (rc) {
-        device_free(d_cnt, s);
-        return rc;
-      }
+    std::vector<MaskUnit> units;
+    std::vector<size_t> ends;
+    for (uint32_t c : masked) {
+      add_mask_units(cols[c].validity, cols[c].n_validity, cols[c].total_rows, cols[c].d_null_mask, units);
+      ends.push_back(units.size());
     }
-    std::vector<unsigned long long> h(masked.size());
-    hipError_t e = hipMemcpyAsync(h.data(), d_cnt, h.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
-    device_free(d_cnt, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    const uint32_t* counts = nullptr;
+    void* token            = nullptr;
+    rc                     = masks_launch(units, s, &counts, &token);
+    if (rc) return rc;
+    const hipError_t e = hipStreamSynchronize(s);
+    for (size_t i = 0, u = 0; e == hipSuccess && i < masked.size(); ++i)
+      for (; u < ends[i]; ++u) cols[masked[i]].null_count += counts[u];
+    rc = desc_release(token, s);
     if (e != hipSuccess) return fail(SDR_E_HIP, "null count: %s", hipGetErrorString(e));
-    for (size_t i = 0; i < masked.size(); ++i) cols[masked[i]].null_count = static_cast<int64_t>(h[i]);
+    if (rc) return rc;
   }
   hipError_t e = hipPeekAtLastError();
   if (e != hipSuccess) return fail(SDR_E_HIP, "sticky launch error: %s", hipGetErrorString(e));
@@ -580,8 +680,17 @@ int plan_create(const sdr_column* cols, uint32_t n_cols, uint32_t mode, hipStrea
   build_batches(targets, p->batches, p->all);
   hipError_t e = hipSuccess;
   if (!p->all.empty()) e = hipMalloc(reinterpret_cast<void**>(&p->d_segs), p->all.size() * sizeof(FixedSeg));
-  if (e == hipSuccess && !p->masked.empty())
-    e = hipMalloc(reinterpret_cast<void**>(&p->d_counts), p->masked.size() * sizeof(unsigned long long));
+  std::vector<MaskUnit> units;
+  for (const sdr_column& col : p->masked) {
+    add_mask_units(col.validity, col.n_validity, col.total_rows, col.d_null_mask, units);
+    p->mask_ends.push_back(static_cast<uint32_t>(units.size()));
+  }
+  if (e == hipSuccess && !units.empty())
+    e = hipMalloc(reinterpret_cast<void**>(&p->d_units), units.size() * sizeof(MaskUnit));
+  if (e == hipSuccess && !units.empty())
+    e = hipMalloc(reinterpret_cast<void**>(&p->d_counts), units.size() * sizeof(uint32_t));
+  if (e == hipSuccess && !units.empty())
+    e = hipMemcpyAsync(p->d_units, units.data(), units.size() * sizeof(MaskUnit), hipMemcpyHostToDevice, s);
   if (e == hipSuccess && p->d_segs)
     e = hipMemcpyAsync(p->d_segs, p->all.data(), p->all.size() * sizeof(FixedSeg), hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -600,12 +709,8 @@ int plan_launch(sdr_plan* p, uint32_t codec, hipStream_t s)
   hipError_t e = launch_batches(p->batches, p->all, p->d_segs, p->mode, codec, s, nullptr);
   if (e != hipSuccess) return fail(SDR_E_HIP, "kernel launch failed: %s", hipGetErrorString(e));
   if (codec == 0 && !p->masked.empty()) {
-    HIP_TRY(launch_fill_u8(reinterpret_cast<uint8_t*>(p->d_counts), 0, p->masked.size() * sizeof(unsigned long long), s));
-    for (size_t i = 0; i < p->masked.size(); ++i) {
-      const sdr_column& col = p->masked[i];
-      int rc = build_null_mask(col.validity, col.n_validity, col.total_rows, col.d_null_mask, p->d_counts + i, s);
-      if (rc) return rc;
-    }
+    e = launch_null_mask(p->d_units, p->mask_ends.back(), p->d_counts, nullptr, s, false);
+    if (e != hipSuccess) return fail(SDR_E_HIP, "null mask launch: %s", hipGetErrorString(e));
   }
   return SDR_OK;
 }
@@ -615,6 +720,7 @@ int plan_launch(sdr_plan* p, uint32_t codec, hipStream_t s)
 sdr_plan::~sdr_plan()
 {
   if (d_segs) (void)hipFree(d_segs);
+  if (d_units) (void)hipFree(d_units);
   if (d_counts) (void)hipFree(d_counts);
 }
 
@@ -690,16 +796,18 @@ int sdr_plan_null_counts(sdr_plan* plan, int64_t* counts, uint32_t n_cols, sdr_s
   if (!plan || (n_cols && !counts)) return fail(SDR_E_INVALID_ARG, "NULL argument");
   if (n_cols < plan->n_cols) return fail(SDR_E_INVALID_ARG, "counts holds %u entries, plan has %u columns", n_cols, plan->n_cols);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  std::vector<unsigned long long> h(plan->masked.size());
-  if (!h.empty()) {
-    HIP_TRY(hipMemcpyAsync(h.data(), plan->d_counts, h.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-  }
+  std::vector<uint32_t> h(plan->mask_ends.empty() ? 0 : plan->mask_ends.back());  // null count of each mask piece
+  if (!h.empty())
+    HIP_TRY(hipMemcpyAsync(h.data(), plan->d_counts, h.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
   for (uint32_t c = 0; c < plan->n_cols; ++c) counts[c] = 0;
   // masked columns are recorded in column order
-  size_t mi = 0;
+  size_t mi = 0, u = 0;
   for (uint32_t c = 0; c < plan->n_cols && mi < plan->masked.size(); ++c)
-    if (plan->col_masked.size() > c && plan->col_masked[c]) counts[c] = static_cast<int64_t>(h[mi++]);
+    if (plan->col_masked.size() > c && plan->col_masked[c]) {
+      for (; u < plan->mask_ends[mi]; ++u) counts[c] += h[u];
+      ++mi;
+    }
   return SDR_OK;
 }
 

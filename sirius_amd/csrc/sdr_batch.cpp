@@ -34,6 +34,8 @@ struct sdr_batch {
     sdr_string_column* str;
   };
   std::vector<MaskJob> masks;
+  std::vector<sdr::MaskUnit> mask_units;  // the masks' pieces of the last upload
+  std::vector<size_t> mask_ends;          // ... and where each mask's end
   // device arena and pinned staging
   uint8_t* d_arena     = nullptr;
   size_t arena_bytes   = 0;
@@ -45,7 +47,7 @@ struct sdr_batch {
   size_t readback_cap  = 0;
   size_t readback_bytes = 0;
   size_t used_bytes    = 0;
-  size_t off_items = 0, off_cols = 0, off_chunks = 0, off_segs = 0, off_state = 0, off_nulls = 0;
+  size_t off_items = 0, off_cols = 0, off_chunks = 0, off_segs = 0, off_state = 0, off_nulls = 0, off_units = 0;
   uint32_t n_status    = 0;
   hipEvent_t launch_done = nullptr;
   size_t n_entries     = 0;                         // queue entries of the last upload
@@ -372,10 +374,19 @@ int batch_upload(sdr_batch* b, hipStream_t s)
   off                         = al(off + b->cols.size() * sizeof(FsstColumn));
   b->off_segs                 = off;
   off                         = al(off + n_segs * sizeof(FsstSeg));
+  b->mask_units.clear();
+  b->mask_ends.clear();
+  for (const auto& m : b->masks) {
+    if (m.fixed) add_mask_units(m.fixed->validity, m.fixed->n_validity, m.fixed->total_rows, m.fixed->d_null_mask, b->mask_units);
+    else add_mask_units(m.str->validity, m.str->n_validity, m.str->total_rows, m.str->d_null_mask, b->mask_units);
+    b->mask_ends.push_back(b->mask_units.size());
+  }
+  b->off_units                = off;
+  off                         = al(off + b->mask_units.size() * sizeof(MaskUnit));
   b->off_state                = off;
   off                         = al(off + state_words * sizeof(uint64_t));
   b->off_nulls                = off;
-  off                         = al(off + std::max<size_t>(1, b->masks.size()) * sizeof(unsigned long long));
+  off                         = al(off + b->mask_units.size() * sizeof(uint32_t));
   const size_t readback_end   = off;
   // written on the device by the FSST segment pre-pass: neither uploaded nor read back
   b->off_chunks               = off;
@@ -384,7 +395,7 @@ int batch_upload(sdr_batch* b, hipStream_t s)
   off                         = al(off + n_chunks * sizeof(FsstChunkInfo));
   const size_t off_tabs       = off;
   off                         = al(off + n_segs * sizeof(FsstSymTab));
-  const size_t upload_bytes   = b->off_state;  // the state and null counters are cleared on the device
+  const size_t upload_bytes   = b->off_state;  // the state is cleared on the device, the null counts are written there
   b->used_bytes               = off;
   if (off > b->arena_bytes) {
     if (b->d_arena) HIP_TRY(hipFree(b->d_arena));
@@ -462,6 +473,8 @@ int batch_upload(sdr_batch* b, hipStream_t s)
     st += 2 + c.n_chunks;
   }
   if (!dcols.empty()) std::memcpy(h + b->off_cols, dcols.data(), dcols.size() * sizeof(FsstColumn));
+  if (!b->mask_units.empty())
+    std::memcpy(h + b->off_units, b->mask_units.data(), b->mask_units.size() * sizeof(MaskUnit));
   if (!fsegs.empty()) std::memcpy(h + b->off_fsegs, fsegs.data(), fsegs.size() * sizeof(FixedSeg));
   if (mask & (1u << BG_FSST)) {  // every chunk of every string column, column by column
     auto* fe = reinterpret_cast<FsstEntry*>(h + off_fentries);
@@ -655,18 +668,9 @@ int batch_launch(sdr_batch* b, hipStream_t s)
   for (const auto& c : b->cols)
     if (c.total_rows == 0 && c.offsets) HIP_TRY(launch_fill_u8(reinterpret_cast<uint8_t*>(c.offsets), 0, sizeof(int32_t), s));
   // validity masks (UNCOMPRESSED overlays) after the data decode
-  auto* d_nulls = reinterpret_cast<unsigned long long*>(b->d_arena + b->off_nulls);
-  if (!b->masks.empty()) {
-    HIP_TRY(launch_fill_u8(reinterpret_cast<uint8_t*>(d_nulls), 0, b->masks.size() * sizeof(unsigned long long), s));
-    for (size_t i = 0; i < b->masks.size(); ++i) {
-      const auto& m = b->masks[i];
-      if (m.fixed)
-        rc = build_null_mask(m.fixed->validity, m.fixed->n_validity, m.fixed->total_rows, m.fixed->d_null_mask, d_nulls + i, s);
-      else
-        rc = build_null_mask(m.str->validity, m.str->n_validity, m.str->total_rows, m.str->d_null_mask, d_nulls + i, s);
-      if (rc) return rc;
-    }
-  }
+  HIP_TRY(launch_null_mask(reinterpret_cast<const MaskUnit*>(b->d_arena + b->off_units),
+                           static_cast<uint32_t>(b->mask_units.size()),
+                           reinterpret_cast<uint32_t*>(b->d_arena + b->off_nulls), nullptr, s, false));
   // the host reads string totals and null counts from a pinned copy once
   // the launch has finished (batch_collect)
   if (!b->cols.empty() || !b->masks.empty())  // otherwise there is nothing to write back
@@ -695,8 +699,7 @@ int batch_collect(sdr_batch* b)
   if (!b->launched) return SDR_OK;
   b->launched = false;
   const auto* st = reinterpret_cast<const uint64_t*>(b->h_readback);
-  const auto* nulls =
-    reinterpret_cast<const unsigned long long*>(b->h_readback + (b->off_nulls - b->off_state));
+  const auto* nulls = reinterpret_cast<const uint32_t*>(b->h_readback + (b->off_nulls - b->off_state));
   int rc = SDR_OK;
   size_t w = 0;
   for (auto& c : b->cols) {
@@ -711,9 +714,11 @@ int batch_collect(sdr_batch* b)
              : fail(SDR_E_OVERFLOW, "total_chars (%llu) exceeds capacity (%llu) or int32 max",
                     static_cast<unsigned long long>(total), static_cast<unsigned long long>(c.cap));
   }
-  for (size_t i = 0; i < b->masks.size(); ++i) {
-    if (b->masks[i].fixed) b->masks[i].fixed->null_count = static_cast<int64_t>(nulls[i]);
-    else b->masks[i].str->null_count = static_cast<int64_t>(nulls[i]);
+  for (size_t i = 0, u = 0; i < b->masks.size(); ++i) {
+    int64_t n = 0;
+    for (; u < b->mask_ends[i]; ++u) n += nulls[u];
+    if (b->masks[i].fixed) b->masks[i].fixed->null_count = n;
+    else b->masks[i].str->null_count = n;
   }
   return rc;
 }

@@ -31,13 +31,20 @@ int upload_async(void* d_dst, const void* h_src, size_t bytes, hipStream_t s);
 // the slot free once the work enqueued on s so far has completed.
 int desc_acquire(const void* h_src, size_t bytes, hipStream_t s, void** d_out, void** token);
 int desc_release(void* token, hipStream_t s);
+// A slot's pinned buffer of at least `bytes` (device-accessible), nothing
+// copied; given back with desc_release.
+int pinned_acquire(size_t bytes, void** h_out, void** token);
 
 bool type_ok_for(uint32_t codec, uint32_t ts);
 bool codec_fixed(uint32_t codec);
 int check_runs(const sdr_run* runs, uint32_t n, uint32_t total_rows, const char* what);
 int check_validity_runs(const sdr_run* runs, uint32_t n, uint32_t total_rows);
-int build_null_mask(const sdr_run* runs, uint32_t n, uint32_t total_rows, uint8_t* d_mask,
-                    unsigned long long* d_count, hipStream_t s);
+// Append the pieces of a column's null mask: its validity segments (a later
+// one wins where two share a byte) and all-valid rows where none lies.
+void add_mask_units(const sdr_run* runs, uint32_t n, uint32_t total_rows, uint8_t* d_mask, std::vector<MaskUnit>& out);
+// The launch of a call's pieces.  counts[i] is piece i's null count once `s`
+// has been synchronised; desc_release(token, s) then ends the use of counts.
+int masks_launch(const std::vector<MaskUnit>& units, hipStream_t s, const uint32_t** counts, void** token);
 
 // One fixed-width run and where its rows go.
 struct RunTarget {
@@ -79,6 +86,8 @@ struct sdr_plan {
   sdr::FixedSeg* d_segs = nullptr;
   std::vector<sdr_column> masked;  // columns with a null mask, in column order
   std::vector<bool> col_masked;
-  unsigned long long* d_counts = nullptr;
+  std::vector<uint32_t> mask_ends;  // per masked column: its pieces end here in the list of all
+  sdr::MaskUnit* d_units = nullptr;
+  uint32_t* d_counts     = nullptr;  // null count of each piece
   ~sdr_plan();
 };

@@ -46,9 +46,24 @@ struct RowRange {
 };
 hipError_t launch_rowids(const RowRange* d_ranges, uint32_t n, uint32_t max_count, int64_t* out, hipStream_t s);
 
-// Validity: fill mask bytes, then count zero bits among the first `rows`.
 hipError_t launch_fill_u8(uint8_t* p, uint8_t v, uint64_t n, hipStream_t s);
-hipError_t launch_count_nulls(const uint8_t* mask, uint32_t rows, unsigned long long* d_count,
-                              hipStream_t s);
+
+// Validity: a piece of a null mask, copied from a validity segment (src null:
+// set to all valid) with its zero bits counted.  `past` has the bits of the
+// piece's last byte that are past the column's rows.
+struct MaskUnit {
+  const uint8_t* src;
+  uint8_t* dst;
+  uint32_t bytes;
+  uint32_t past;
+};
+static_assert(sizeof(MaskUnit) == 24, "MaskUnit layout");
+constexpr uint32_t MASK_UNIT_BYTES = 8192;  // the largest piece: one 256-thread block
+constexpr uint32_t MASKS_INLINE    = 120;   // pieces a launch can carry in its kernel arguments
+// Build n pieces, one block each; piece i's null count is stored at counts[i],
+// or (counts null) added to *total.  `units`: memory the device reads, or
+// with `host` host memory whose pieces travel in the kernel arguments.
+hipError_t launch_null_mask(const MaskUnit* units, uint32_t n, uint32_t* counts, unsigned long long* total,
+                            hipStream_t s, bool host);
 
 }  // namespace sdr

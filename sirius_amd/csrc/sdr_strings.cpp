@@ -332,18 +332,27 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
     }
   }
   const bool masked = (col->has_nulls && col->d_null_mask) || dc.any_inline;
+  std::vector<MaskUnit> units;
+  const uint32_t* counts = nullptr;  // null count of each piece of the mask
+  void* counts_token     = nullptr;
+  // nulls counted on the device: DICT_FSST's inline ones (or every one, when
+  // nothing may be allocated for the pieces' counts)
+  const bool device_nulls = masked && (dc.any_inline || scratch_mem);
   if (e == hipSuccess && masked) {
-    e = launch_fill_u8(reinterpret_cast<uint8_t*>(d_nulls), 0, sizeof(unsigned long long), s);
-    if (e == hipSuccess) {
-      rc = build_null_mask(col->validity, col->has_nulls ? col->n_validity : 0u, n, col->d_null_mask, d_nulls, s);
+    add_mask_units(col->validity, col->has_nulls ? col->n_validity : 0u, n, col->d_null_mask, units);
+    if (device_nulls) e = launch_fill_u8(reinterpret_cast<uint8_t*>(d_nulls), 0, sizeof(unsigned long long), s);
+    if (e == hipSuccess && scratch_mem) {
+      e = launch_null_mask(units.data(), static_cast<uint32_t>(units.size()), nullptr, d_nulls, s, true);
+    } else if (e == hipSuccess) {
+      rc = masks_launch(units, s, &counts, &counts_token);
       if (rc) {
         release_all();
         return rc;
       }
-      // DICT_FSST inline NULLs (dict_fsst.cu:426-446) on top of the validity
-      if (dc.any_inline)
-        e = launch_dfsst_nulls(d_segs, n_ranges, dc.d_desc, dc.d_range, col->d_null_mask, n, d_nulls, s);
     }
+    // DICT_FSST inline NULLs (dict_fsst.cu:426-446) on top of the validity
+    if (e == hipSuccess && dc.any_inline)
+      e = launch_dfsst_nulls(d_segs, n_ranges, dc.d_desc, dc.d_range, col->d_null_mask, n, d_nulls, s);
   }
   struct {
     uint32_t ticket, error;
@@ -351,10 +360,13 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
   } h{};
   unsigned long long h_nulls = 0;
   if (e == hipSuccess) e = hipMemcpyAsync(&h, d_state, sizeof(h), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess && masked) e = hipMemcpyAsync(&h_nulls, d_nulls, sizeof(h_nulls), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess && device_nulls) e = hipMemcpyAsync(&h_nulls, d_nulls, sizeof(h_nulls), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
+  for (size_t u = 0; e == hipSuccess && counts && u < units.size(); ++u) h_nulls += counts[u];
+  rc = desc_release(counts_token, s);
   release_all();
   if (e != hipSuccess) return fail(SDR_E_HIP, "string decode: %s", hipGetErrorString(e));
+  if (rc) return rc;
   if (h.error) return fail(SDR_E_HIP, "string decode: offset look-back did not complete");
   col->chars_used = h.total;
   col->null_count = masked ? static_cast<int64_t>(h_nulls) : 0;
