@@ -907,148 +907,174 @@ __device__ __forceinline__ uint32_t dfsst_entry_len(const uint8_t* p, uint32_t n
   return dl;
 }
 
-// Block sum of one u64 per thread (every thread gets it).
-template <class SM>
-__device__ __forceinline__ uint64_t block_sum_u64(uint64_t v, SM& sm)
+// The offsets of thread t's rows 2t and 2t + 1, and the column's closing one.
+__device__ __forceinline__ void fsst_row_offsets(uint32_t c, uint32_t n_chunks, uint32_t col_row, uint32_t rows,
+                                                 uint64_t T, uint64_t base, uint32_t o0, uint32_t o1, int32_t* offsets,
+                                                 uint32_t total_rows)
 {
-  const uint64_t w = readlane_u64(wave_incl_sum_u64(v), WAVE - 1);
-  if (lane_id() == 0) {
-    sm.part[2u * (threadIdx.x / WAVE)]      = static_cast<uint32_t>(w);
-    sm.part[2u * (threadIdx.x / WAVE) + 1u] = static_cast<uint32_t>(w >> 32);
-  }
-  __syncthreads();
-  uint64_t t = 0;
-#pragma unroll
-  for (uint32_t k = 0; k < FSST_WAVES; ++k)
-    t += static_cast<uint64_t>(sm.part[2u * k]) | (static_cast<uint64_t>(sm.part[2u * k + 1u]) << 32);
-  __syncthreads();
-  return t;
+  const uint32_t r        = 2u * threadIdx.x;
+  const gptr<int32_t> off = gbl(offsets) + col_row;
+  if (r < rows) off[r] = static_cast<int32_t>(static_cast<uint32_t>(base) + o0);
+  if (r + 1u < rows) off[r + 1u] = static_cast<int32_t>(static_cast<uint32_t>(base) + o1);
+  if (c == n_chunks - 1u && threadIdx.x == 0)
+    gbl(offsets)[total_rows] = static_cast<int32_t>(static_cast<uint32_t>(base + T));
 }
 
-// Chars of a plain chunk from dec[] (row starts) and comp[] (each row's
-// first byte in the segment), one row per thread, in 8 KiB LDS pieces
-// flushed as in fsst_emit_rows.
-template <class SM>
-__device__ __forceinline__ void plain_emit_rows(SM& sm, const uint8_t* seg, const uint8_t* end,
-                                                         uint32_t rows, uint32_t T, uint64_t base, uint8_t* chars,
-                                                         uint64_t chars_cap)
+// One row's bytes into the window over chunk output bytes [w0, w0 +
+// FSST_WINDOW) (cleared): source bytes [src, src + len) are output bytes
+// [d, d + len); those at or past `end` are zeros.  A word of the window at a
+// time, four in flight: its four bytes come from two aligned words of the
+// source, of which only those that hold the row's bytes are read, and are
+// ORed in, since a row's first and last word are shared with its neighbours.
+__device__ __forceinline__ void plain_copy_row(FsstSmem& sm, const uint8_t* src, uint32_t len, const uint8_t* end,
+                                               uint32_t d, uint32_t w0)
 {
-  const uint32_t tid = threadIdx.x;
-  const uintptr_t cb = reinterpret_cast<uintptr_t>(chars);
-  const uintptr_t g0 = cb + base;
-  const uintptr_t g1 = cb + ((base + T < chars_cap) ? base + T : chars_cap);
-  for (uintptr_t pa = g0 & ~uintptr_t{15}; pa < g1; pa += FSST_PIECE) {
-    const uintptr_t pb = pa + FSST_PIECE;
+  const uint64_t left = src < end ? static_cast<uint64_t>(end - src) : 0u;
+  const uint32_t have = len < left ? len : static_cast<uint32_t>(left);
+  const uint32_t j0   = d < w0 ? w0 - d : 0u;
+  const uint32_t lim  = w0 + FSST_WINDOW > d ? w0 + FSST_WINDOW - d : 0u;
+  const uint32_t j1   = have < lim ? have : lim;
+  if (j0 >= j1) return;
+  const uint32_t p      = d + j0 - w0;  // first window byte
+  const uint32_t sh     = p & 3u;
+  const uint32_t nb     = sh + (j1 - j0);  // bytes from the first window word's start
+  const uintptr_t a     = reinterpret_cast<uintptr_t>(src) + j0 - sh;
+  const uint32_t ph     = static_cast<uint32_t>(a & 3u);
+  const gptr<const uint32_t> w = gbl(reinterpret_cast<const uint32_t*>(a - ph));
+  // source word i holds bytes 4i - ph .. 4i - ph + 3 from `a`; the row's are [sh, nb)
+  auto load = [&](uint32_t i) -> uint32_t { return 4u * i + 3u >= sh + ph && 4u * i < nb + ph ? w[i] : 0u; };
+  uint32_t* o    = reinterpret_cast<uint32_t*>(sm.out + (p - sh));
+  uint32_t carry = load(0);
 #pragma unroll 1
-    for (uint32_t k = 0; k < ROWS_PER_THR; ++k) {
-      const uint32_t r = k * FSST_THREADS + tid;
-      if (r >= rows) continue;
-      const uint32_t d0 = sm.dec[r], dl = sm.dec[r + 1] - d0;
-      const uintptr_t o0 = g0 + d0;
-      if (dl == 0 || o0 + dl <= pa || o0 >= pb) continue;
-      const uint32_t j0 = o0 < pa ? static_cast<uint32_t>(pa - o0) : 0u;
-      const uint32_t j1 = o0 + dl > pb ? static_cast<uint32_t>(pb - o0) : dl;
-      const uint8_t* src = seg + sm.comp[r];
-      uint8_t* dst       = sm.out + (o0 - pa);
-      if (src + dl <= end) {
-        ByteReader br(src + j0);
-        for (uint32_t j = j0; j < j1; ++j) dst[j] = static_cast<uint8_t>(br.next());
-      } else {
-        for (uint32_t j = j0; j < j1; ++j) dst[j] = static_cast<uint8_t>(byte_at(src + j, end));
+  for (uint32_t k = 0; 4u * k < nb; k += 4) {
+    uint32_t n[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) n[i] = load(k + i + 1u);
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+      const uint32_t at = 4u * (k + i);
+      uint32_t v        = __builtin_amdgcn_alignbyte(n[i], carry, ph);
+      carry             = n[i];
+      if (at < nb) {
+        if (at == 0) v &= ~0u << (8u * sh);
+        if (nb - at < 4u) v &= (1u << (8u * (nb - at))) - 1u;
+        __hip_atomic_fetch_or(o + k + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
     }
-    __syncthreads();
-    const uintptr_t lo = pa > g0 ? pa : g0;
-    const uintptr_t hi = pb < g1 ? pb : g1;
-    for (uintptr_t blk = pa + uintptr_t{tid} * 16u; blk < hi; blk += uintptr_t{FSST_THREADS} * 16u) {
-      if (blk >= lo && blk + 16u <= hi) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(&sm.out[blk - pa]);
-        __builtin_nontemporal_store(v, gbl(reinterpret_cast<u32x4*>(blk)));
-      } else {
-        for (uintptr_t x = blk; x < blk + 16u; ++x)
-          if (x >= lo && x < hi) *gbl(reinterpret_cast<uint8_t*>(x)) = sm.out[x - pa];
-      }
-    }
-    __syncthreads();
   }
 }
 
-// Decode chunk c of a valid DICTIONARY or UNCOMPRESSED segment: per-row
-// lengths (dictionary.cu:84-108, uncompressed.cu:56-81), the chunk's
-// look-back for its chars offset, offsets, then the bytes (dictionary.cu:
-// 117-140, uncompressed.cu:88-120).  Every thread must call it.
-// A leaf call with scalar arguments: descriptors passed by value, or a
-// call from here, would need a stack in scratch memory.
-template <class SM>
+// Decode chunk c of a valid DICTIONARY, UNCOMPRESSED or DICT_FSST segment: per-
+// row lengths (dictionary.cu:84-108, uncompressed.cu:56-81), the chunk's
+// look-back for its chars offset, offsets, and the bytes (dictionary.cu:
+// 117-140, uncompressed.cu:88-120).  Every thread must call it.  A called
+// function with scalar arguments, so that the FSST path keeps its registers.
+//
+// Bound by latency: a row's length is two dependent loads away, its bytes a
+// third.  Thread t owns rows 2t and 2t + 1, whose loads overlap, and each row
+// is copied a word at a time into the LDS window that the FSST path fills (a
+// byte at a time into 8 KiB pieces, with flat accesses to LDS, took 180 us for
+// 8 Mi label rows, 128 us for 2 M rows of 27 chars; now 119 us and 57 us).
 __device__ __attribute__((noinline)) void plain_chunk(const uint8_t* seg, uint32_t bytes_size, uint32_t dict_end,
                                                      uint32_t flags, uint32_t ibo, uint32_t ibc, uint32_t row_begin,
                                                      uint32_t rows, uint32_t col_row, uint32_t c, uint32_t n_chunks,
                                                      FsstState* __restrict__ st, int32_t* __restrict__ offsets,
                                                      uint8_t* __restrict__ chars, uint64_t chars_cap,
-                                                     uint32_t total_rows, uint32_t spin_limit, SM& sm)
+                                                     uint32_t total_rows, uint32_t spin_limit, LdsPtr<FsstSmem> smp)
 {
+  FsstSmem& sm        = *(FsstSmem*)smp;
   const uint32_t tid  = threadIdx.x;
   const uint8_t* end  = seg + bytes_size;
   const bool dict     = flags & FI_DICT;
   const bool dfsst    = flags & FI_DFSST;
   const uint32_t w    = flags & FI_WIDTH;
-  const FsstChunk ch{0u, row_begin, rows, col_row};
   DictFsstSeg dd{};
   if (dfsst) {  // seg is the segment's descriptor; rows copy from its entries
-    dd  = gload(reinterpret_cast<const DictFsstSeg*>(seg));
+    dd  = uniform(gload(reinterpret_cast<const DictFsstSeg*>(seg)));
     seg = dd.src;
     end = dd.src + dd.src_size;
   }
-  __syncthreads();  // the previous user of sm is done
-  uint32_t T   = 0;
-  uint64_t own = 0;
-#pragma unroll 1
-  for (uint32_t k = 0; k < ROWS_PER_THR; ++k) {
-    const uint32_t r = k * FSST_THREADS + tid;
-    uint32_t len = 0, src = 0;
+  // the rows' entries [e0, e1): two loads, both rows' in flight together
+  uint32_t idx[ROWS_PER_THR], e0[ROWS_PER_THR] = {}, e1[ROWS_PER_THR] = {};
+#pragma unroll
+  for (uint32_t i = 0; i < ROWS_PER_THR; ++i) {
+    const uint32_t r = ROWS_PER_THR * tid + i, sr = row_begin + r;
+    idx[i]           = 0;
     if (r < rows) {
-      const uint32_t sr = ch.row_begin + r;
-      uint32_t e0 = 0, e1 = 0;
-      if (dfsst) {
-        const uint32_t idx = dfsst_index(dd, sr);
-        if (idx != 0u && idx < dd.dict_count) {
-          e0 = gbl(dd.e)[idx];
-          e1 = gbl(dd.e)[idx + 1u];
-        }
-        dict_end = e1 >= e0 ? e1 : 0u;  // the entries are front to back: a row starts at e0
-      } else if (dict) {
-        const uint32_t sel = stream_bits32(seg + 20, end, uint64_t{sr} * w, w);
-        if (sel != 0u && sel < ibc) {
-          e1 = ld_u32_any(seg + ibo + 4ull * sel);
-          e0 = ld_u32_any(seg + ibo + 4ull * (sel - 1u));
-        }
-      } else {
-        const int32_t v1 = static_cast<int32_t>(ld_u32_any(seg + 8 + 4ull * sr));
-        const int32_t v0 = sr ? static_cast<int32_t>(ld_u32_any(seg + 8 + 4ull * (sr - 1u))) : 0;
-        e1 = v1 < 0 ? 0u - static_cast<uint32_t>(v1) : static_cast<uint32_t>(v1);
-        e0 = v0 < 0 ? 0u - static_cast<uint32_t>(v0) : static_cast<uint32_t>(v0);
-      }
-      if (e1 <= dict_end && e1 >= e0) {
-        len = e1 - e0;
-        src = dfsst ? e0 : dict_end - e1;
-      }
-      sm.comp[r] = src;
+      if (dfsst) idx[i] = dfsst_index(dd, sr);
+      else if (dict) idx[i] = stream_bits32(seg + 20, end, uint64_t{sr} * w, w);
+      else idx[i] = sr + 1u;
     }
-    own += len;
-    uint32_t tot      = 0;
-    const uint32_t ex = block_excl_scan(len, sm.wave, &tot);
-    if (r < rows) sm.dec[r] = T + ex;
-    T += tot;
   }
-  if (tid == 0) sm.dec[rows] = T;
-  // Rows are bounded by the segment, but a chunk of long rows can pass
-  // 2^31 chars: publish a saturated total so the column reports overflow.
-  const uint64_t T64 = block_sum_u64(own, sm);
-  const uint64_t Tp  = T64 > 0x7FFFFFFFull ? 0x80000000ull : T64;
-  const uint64_t b   = fsst_lookback(c, n_chunks, Tp, st, spin_limit, sm);
-  fsst_offsets(ch, c, n_chunks, rows, static_cast<uint32_t>(Tp), b, offsets, total_rows, sm);
-  if (T64 == 0 || Tp != T64 || b >= chars_cap) return;
-  plain_emit_rows(sm, seg, end, rows, T, b, chars, chars_cap);
+#pragma unroll
+  for (uint32_t i = 0; i < ROWS_PER_THR; ++i) {
+    const uint32_t k = idx[i];
+    if (dfsst) {
+      if (k != 0u && k < dd.dict_count) {
+        e0[i] = gbl(dd.e)[k];
+        e1[i] = gbl(dd.e)[k + 1u];
+      }
+    } else if (dict) {
+      if (k != 0u && k < ibc) {
+        e1[i] = ld_u32_any(seg + ibo + 4ull * k);
+        e0[i] = ld_u32_any(seg + ibo + 4ull * (k - 1u));
+      }
+    } else if (k) {
+      const int32_t v1 = static_cast<int32_t>(ld_u32_any(seg + 8 + 4ull * (k - 1u)));
+      const int32_t v0 = k > 1u ? static_cast<int32_t>(ld_u32_any(seg + 8 + 4ull * (k - 2u))) : 0;
+      e1[i] = v1 < 0 ? 0u - static_cast<uint32_t>(v1) : static_cast<uint32_t>(v1);
+      e0[i] = v0 < 0 ? 0u - static_cast<uint32_t>(v0) : static_cast<uint32_t>(v0);
+    }
+  }
+  uint32_t len[ROWS_PER_THR], src[ROWS_PER_THR];
+#pragma unroll
+  for (uint32_t i = 0; i < ROWS_PER_THR; ++i) {
+    // a DICT_FSST segment's entries are front to back, the others' back to
+    // front; a row whose end passes dict_end or falls below its start is empty
+    const bool sound = e1[i] >= e0[i] && (dfsst || e1[i] <= dict_end);
+    len[i]           = sound ? e1[i] - e0[i] : 0u;
+    src[i]           = dfsst ? e0[i] : dict_end - e1[i];
+  }
+  // 64-bit prefixes as two scans of 16-bit halves: the rows are bounded by
+  // the segment, but a chunk of long rows can pass 2^31 chars
+  static_assert(ROWS_PER_THR == 2, "row arithmetic");
+  uint32_t plo, phi, tlo, thi;
+  block_excl_scan2((len[0] & 0xFFFFu) + (len[1] & 0xFFFFu), (len[0] >> 16) + (len[1] >> 16), sm.wave, plo, phi, tlo,
+                   thi);
+  const uint64_t T64 = tlo + (uint64_t{thi} << 16);
+  // publish a saturated total then, so the column reports overflow
+  const uint64_t Tp = T64 > 0x7FFFFFFFull ? 0x80000000ull : T64;
+  const uint32_t T  = static_cast<uint32_t>(Tp);
+  const uint32_t o0 = plo + (phi << 16), o1 = o0 + len[0];
+  fsst_lookback_publish(c, Tp, st, spin_limit);
+  if (Tp != T64) {  // nothing but the offsets can be written
+    const uint64_t base = fsst_lookback_wait(c, n_chunks, Tp, st, spin_limit, sm);
+    fsst_row_offsets(c, n_chunks, col_row, rows, Tp, base, o0, o1, offsets, total_rows);
+    return;
+  }
+  uint64_t base = 0;
+#pragma unroll 1
+  for (uint32_t w0 = 0;;) {
+    const uint32_t nw = T - w0 < FSST_WINDOW ? T - w0 : FSST_WINDOW;
+    window_clear(sm, nw);
+    __syncthreads();
+#pragma unroll 1
+    for (uint32_t i = 0; i < ROWS_PER_THR; ++i)
+      plain_copy_row(sm, seg + (i ? src[1] : src[0]), i ? len[1] : len[0], end, i ? o1 : o0, w0);
+    if (w0) {
+      __syncthreads();
+    } else {
+      base = fsst_lookback_wait(c, n_chunks, Tp, st, spin_limit, sm);  // synchronises the workgroup
+      fsst_row_offsets(c, n_chunks, col_row, rows, Tp, base, o0, o1, offsets, total_rows);
+    }
+    const uint64_t at = base + w0;
+    if (at >= chars_cap) return;
+    window_store(sm, reinterpret_cast<uintptr_t>(chars) + at,
+                 at + nw <= chars_cap ? nw : static_cast<uint32_t>(chars_cap - at));
+    w0 += nw;
+    if (w0 >= T) return;
+    __syncthreads();  // the stores have read the window
+  }
 }
 
 // Import the symbol table serialised at seg + symoff (at most
@@ -1334,21 +1360,7 @@ __device__ __forceinline__ uint32_t fsst_issue_front(FsstSmem& sm, bool ok, cons
   return h * 8u + static_cast<uint32_t>((uint64_t{row_begin} * width) & 7u);
 }
 
-// The offsets of thread t's rows 2t and 2t + 1, and the column's closing one.
-__device__ __forceinline__ void fsst_row_offsets(uint32_t c, uint32_t n_chunks, uint32_t col_row, uint32_t rows,
-                                                 uint64_t T, uint64_t base, uint32_t o0, uint32_t o1, int32_t* offsets,
-                                                 uint32_t total_rows)
-{
-  const uint32_t r        = 2u * threadIdx.x;
-  const gptr<int32_t> off = gbl(offsets) + col_row;
-  if (r < rows) off[r] = static_cast<int32_t>(static_cast<uint32_t>(base) + o0);
-  if (r + 1u < rows) off[r + 1u] = static_cast<int32_t>(static_cast<uint32_t>(base) + o1);
-  if (c == n_chunks - 1u && threadIdx.x == 0)
-    gbl(offsets)[total_rows] = static_cast<int32_t>(static_cast<uint32_t>(base + T));
-}
-
-// The row starts of a run: thread t's rows end at run positions e0, e1 in
-// row order (compressed bytes of the run up to and including the row).
+// A row that has bytes starts at stage position y.
 __device__ __forceinline__ void fsst_mark_row(FsstSmem& sm, uint32_t y)
 {
   __hip_atomic_fetch_or(&sm.bits[y >> 5], 1u << (y & 31u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -1542,7 +1554,7 @@ __device__ __forceinline__ void fsst_chunk(const FsstChunk ch, const FsstChunkIn
   const uint32_t rows = ch.rows;
   if (ok && (ci.flags & (FI_DICT | FI_UNC | FI_DFSST))) {  // uniform per chunk
     plain_chunk(ci.bytes, ci.bytes_size, ci.dict_end, ci.flags, ci.c_lo, ci.c_hi, ch.row_begin, rows, ch.col_row, c,
-                n_chunks, st, offsets, chars, chars_cap, total_rows, spin_limit, sm);
+                n_chunks, st, offsets, chars, chars_cap, total_rows, spin_limit, (LdsPtr<FsstSmem>)(&sm));
     return;
   }
   // Rows are stored back to front ending at dict_end: the chunk's bytes are
