@@ -702,6 +702,12 @@ __device__ __forceinline__ void fsst_lookback_publish(uint32_t c, uint64_t T, Fs
   }
 }
 
+__device__ __forceinline__ void fsst_lookback_failed(FsstState* st)
+{
+  __hip_atomic_fetch_or(gbl(&st->error), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (FsstResult* const r = *gbl(&st->result)) *gbl(&r->error) = 1u;
+}
+
 // The wait half: synchronises the workgroup and returns the exclusive prefix
 // to every thread.
 template <class SM>
@@ -715,7 +721,7 @@ __device__ __forceinline__ uint64_t fsst_lookback_wait(uint32_t c, uint32_t n_ch
     if (c == 0) {
       // published inclusive already
     } else if (spin_limit == 0) {  // no waiting allowed: report the look-back as failed
-      if (lane == 0) __hip_atomic_fetch_or(gbl(&st->error), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (lane == 0) fsst_lookback_failed(st);
     } else {
       uint32_t p = c - 1, spins = 0;
       for (;;) {
@@ -728,7 +734,7 @@ __device__ __forceinline__ uint64_t fsst_lookback_wait(uint32_t c, uint32_t n_ch
         const uint64_t need = stop == WAVE - 1 ? ~0ull : ((2ull << stop) - 1ull);
         if (ballot(valid && flag == 0) & need) {  // a predecessor has not published yet
           if (++spins > spin_limit) {              // never expected: give up rather than hang
-            if (lane == 0) __hip_atomic_fetch_or(gbl(&st->error), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (lane == 0) fsst_lookback_failed(st);
             break;
           }
           __builtin_amdgcn_s_sleep(1);
@@ -743,7 +749,10 @@ __device__ __forceinline__ uint64_t fsst_lookback_wait(uint32_t c, uint32_t n_ch
     }
     if (lane == 0) {
       sm.base = excl64;
-      if (c == n_chunks - 1) *gbl(&st->total) = excl64 + T;
+      if (c == n_chunks - 1) {
+        *gbl(&st->total) = excl64 + T;
+        if (FsstResult* const r = *gbl(&st->result)) *gbl(&r->total) = excl64 + T;
+      }
     }
   }
   __syncthreads();

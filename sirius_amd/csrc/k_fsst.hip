@@ -22,26 +22,27 @@ __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6)
                               chars, chars_cap, total_rows, spin_limit, sm);
 }
 
-// Segment pre-pass: one workgroup per segment (grid-stride).
+// Segment pre-pass: one workgroup per segment (grid-stride), which also clears
+// the look-back status of its chunks (a launch of its own for that, and a copy
+// of the ranges to the device before it, were 10 us of a 76 us call).
 __global__ __launch_bounds__(PREP_THREADS) void k_fsst_prep(const FsstSeg* __restrict__ segs, uint32_t n_segs,
-                                                            const uint32_t* __restrict__ d_n_segs,
                                                             FsstChunk* __restrict__ chunks,
                                                             FsstChunkInfo* __restrict__ info,
-                                                            FsstSymTab* __restrict__ tabs)
+                                                            FsstSymTab* __restrict__ tabs, FsstState* __restrict__ st,
+                                                            FsstResult* __restrict__ result)
 {
   __shared__ FsstPrepSmem sm;
-  const uint32_t n = d_n_segs ? *d_n_segs : n_segs;
-  for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) fsst_prep_segment(segs[i], i, chunks, info, tabs + i, sm);
-}
-
-__global__ void k_fsst_reset(FsstState* st, uint32_t n_chunks)
-{
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_chunks; i += gridDim.x * blockDim.x)
-    st->status[i] = 0;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     st->ticket = 0;
     st->error  = 0;
     st->total  = 0;
+    st->result = result;
+  }
+  for (uint32_t i = blockIdx.x; i < n_segs; i += gridDim.x) {
+    const FsstSeg sg = uniform(gload(segs + i));
+    for (uint32_t k = threadIdx.x; k * FSST_CHUNK_ROWS < sg.row_count; k += PREP_THREADS)
+      gbl(st->status)[sg.first_chunk + k] = 0;
+    fsst_prep_segment(sg, i, chunks, info, tabs + i, sm);
   }
 }
 
@@ -157,21 +158,12 @@ hipError_t launch_dfsst_nulls(const FsstSeg* d_segs, uint32_t n_ranges, const Di
   return hipGetLastError();
 }
 
-hipError_t launch_fsst_reset(FsstState* d_state, uint32_t n_chunks, hipStream_t s)
+hipError_t launch_fsst_prep(const FsstSeg* segs, uint32_t n_segs, FsstChunk* d_chunks, FsstChunkInfo* d_info,
+                            FsstSymTab* d_tabs, FsstState* d_state, FsstResult* result, hipStream_t s)
 {
-  uint32_t blocks = (n_chunks + 255) / 256;
-  if (blocks == 0) blocks = 1;
-  if (blocks > 1024) blocks = 1024;
-  hipLaunchKernelGGL(k_fsst_reset, dim3(blocks), dim3(256), 0, s, d_state, n_chunks);
-  return hipGetLastError();
-}
-
-hipError_t launch_fsst_prep(const FsstSeg* d_segs, uint32_t n_segs, const uint32_t* d_n_segs, uint32_t grid,
-                            FsstChunk* d_chunks, FsstChunkInfo* d_info, FsstSymTab* d_tabs, hipStream_t s)
-{
-  if (grid == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fsst_prep, dim3(grid), dim3(PREP_THREADS), 0, s, d_segs, n_segs, d_n_segs, d_chunks, d_info,
-                     d_tabs);
+  if (n_segs == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_fsst_prep, dim3(n_segs < 4096u ? n_segs : 4096u), dim3(PREP_THREADS), 0, s, segs, n_segs,
+                     d_chunks, d_info, d_tabs, d_state, result);
   return hipGetLastError();
 }
 

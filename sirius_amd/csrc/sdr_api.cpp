@@ -142,7 +142,8 @@ namespace {
 struct DescSlot {
   void* h         = nullptr;
   void* d         = nullptr;
-  size_t cap      = 0;
+  size_t cap_h    = 0;
+  size_t cap_d    = 0;
   hipEvent_t done = nullptr;
   hipEvent_t up   = nullptr;  // recorded after the slot's upload on the copy stream
   int dev         = -1;
@@ -175,8 +176,9 @@ int copy_stream(int dev, hipStream_t* out)
 }  // namespace
 
 namespace {
-// A held slot of device `dev` with buffers of at least `bytes`.
-int slot_hold(int dev, size_t bytes, DescSlot** out)
+// A held slot of device `dev` with at least `h_bytes` of pinned and `d_bytes`
+// of device memory.
+int slot_hold(int dev, size_t h_bytes, size_t d_bytes, DescSlot** out)
 {
   *out = nullptr;
   DescSlot* pick = nullptr;
@@ -191,8 +193,11 @@ int slot_hold(int dev, size_t bytes, DescSlot** out)
       if (sl->dev != dev) continue;
       ++n_dev;
       if (sl->held) continue;
+      const bool fits = sl->cap_h >= h_bytes && sl->cap_d >= d_bytes;
+      if (pick && !fits) continue;
       if (hipEventQuery(sl->done) == hipSuccess) {
-        if (!pick || (sl->cap >= bytes && pick->cap < bytes)) pick = sl;
+        pick = sl;
+        if (fits) break;
       } else if (!oldest || sl->seq < oldest->seq) {
         oldest = sl;
       }
@@ -226,16 +231,25 @@ int slot_hold(int dev, size_t bytes, DescSlot** out)
     }
   }
   if (wait) e = hipEventSynchronize(pick->done);
-  if (e == hipSuccess && pick->cap < bytes) {  // its event has completed: nothing still reads the old buffers
-    if (pick->h) e = hipHostFree(pick->h);
-    if (e == hipSuccess && pick->d) e = hipFree(pick->d);
-    pick->h = pick->d = nullptr;
-    pick->cap         = 0;
-    size_t cap        = DESC_MIN_BYTES;
+  // its event has completed: nothing still reads buffers that are too small
+  auto grown = [](size_t bytes) {
+    size_t cap = DESC_MIN_BYTES;
     while (cap < bytes) cap *= 2;
-    if (e == hipSuccess) e = hipHostMalloc(&pick->h, cap, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipMalloc(&pick->d, cap);
-    if (e == hipSuccess) pick->cap = cap;
+    return cap;
+  };
+  if (e == hipSuccess && pick->cap_h < h_bytes) {
+    if (pick->h) e = hipHostFree(pick->h);
+    pick->h     = nullptr;
+    pick->cap_h = 0;
+    if (e == hipSuccess) e = hipHostMalloc(&pick->h, grown(h_bytes), hipHostMallocDefault);
+    if (e == hipSuccess) pick->cap_h = grown(h_bytes);
+  }
+  if (e == hipSuccess && pick->cap_d < d_bytes) {
+    if (pick->d) e = hipFree(pick->d);
+    pick->d     = nullptr;
+    pick->cap_d = 0;
+    if (e == hipSuccess) e = hipMalloc(&pick->d, grown(d_bytes));
+    if (e == hipSuccess) pick->cap_d = grown(d_bytes);
   }
   if (e != hipSuccess) return unhold(fail(SDR_E_HIP, "descriptor slot: %s", hipGetErrorString(e)));
   *out = pick;
@@ -251,18 +265,23 @@ int slot_unhold(DescSlot* sl, int rc)
 }
 }  // namespace
 
-int pinned_acquire(size_t bytes, void** h_out, void** token)
+int slot_acquire(size_t h_bytes, size_t d_bytes, void** h_out, void** d_out, void** token)
 {
-  *h_out  = nullptr;
-  *token  = nullptr;
+  *h_out = *d_out = *token = nullptr;
   int dev = 0;
   HIP_TRY(hipGetDevice(&dev));
   DescSlot* sl = nullptr;
-  const int rc = slot_hold(dev, bytes, &sl);
+  const int rc = slot_hold(dev, h_bytes, d_bytes, &sl);
   if (rc) return rc;
   *h_out = sl->h;
+  *d_out = sl->d;
   *token = sl;
   return SDR_OK;
+}
+
+void slot_release_idle(void* token)
+{
+  if (token) (void)slot_unhold(static_cast<DescSlot*>(token), SDR_OK);
 }
 
 int desc_acquire(const void* h_src, size_t bytes, hipStream_t s, void** d_out, void** token)
@@ -272,7 +291,7 @@ int desc_acquire(const void* h_src, size_t bytes, hipStream_t s, void** d_out, v
   int dev = 0;
   HIP_TRY(hipGetDevice(&dev));
   DescSlot* pick = nullptr;
-  const int hrc  = slot_hold(dev, bytes, &pick);
+  const int hrc  = slot_hold(dev, bytes, bytes, &pick);
   if (hrc) return hrc;
   auto unhold  = [&](int rc) { return slot_unhold(pick, rc); };
   hipError_t e = hipSuccess;
@@ -433,8 +452,8 @@ int masks_launch(const std::vector<MaskUnit>& units, hipStream_t s, const uint32
   // pieces is read from it: no copy and no clear on the stream
   const size_t n = units.size(), b_counts = (n * sizeof(uint32_t) + 15u) & ~size_t{15};
   const bool host = n <= MASKS_INLINE;
-  void* h         = nullptr;
-  const int rc    = pinned_acquire(b_counts + (host ? 0u : n * sizeof(MaskUnit)), &h, token);
+  void *h = nullptr, *d = nullptr;
+  const int rc = slot_acquire(b_counts + (host ? 0u : n * sizeof(MaskUnit)), 0, &h, &d, token);
   if (rc) return rc;
   auto* hc = static_cast<uint32_t*>(h);
   auto* hu = reinterpret_cast<MaskUnit*>(static_cast<uint8_t*>(h) + b_counts);
@@ -629,9 +648,11 @@ int decode_table(sdr_column* cols, uint32_t n_cols, hipStream_t s, uint32_t mode
     const hipError_t e = hipStreamSynchronize(s);
     for (size_t i = 0, u = 0; e == hipSuccess && i < masked.size(); ++i)
       for (; u < ends[i]; ++u) cols[masked[i]].null_count += counts[u];
-    rc = desc_release(token, s);
-    if (e != hipSuccess) return fail(SDR_E_HIP, "null count: %s", hipGetErrorString(e));
-    if (rc) return rc;
+    if (e != hipSuccess) {
+      (void)desc_release(token, s);
+      return fail(SDR_E_HIP, "null count: %s", hipGetErrorString(e));
+    }
+    slot_release_idle(token);
   }
   hipError_t e = hipPeekAtLastError();
   if (e != hipSuccess) return fail(SDR_E_HIP, "sticky launch error: %s", hipGetErrorString(e));

@@ -360,9 +360,9 @@ int batch_upload(sdr_batch* b, hipStream_t s)
     n_chunks += c.n_chunks;
     n_segs += c.segs.size();
   }
-  // FsstState = {ticket, error, total, status[n]}: 16 + 8 n bytes per column
+  // FsstState: FSST_STATE_WORDS + n words per column (its result is cleared to null: totals are read back)
   size_t state_words = 0;
-  for (auto& c : b->cols) state_words += 2 + c.n_chunks;
+  for (auto& c : b->cols) state_words += FSST_STATE_WORDS + c.n_chunks;
   size_t off                  = al(sizeof(BatchQueue));
   b->off_items                = off;
   off                         = al(off + n_entries * sizeof(BatchItem));
@@ -470,7 +470,7 @@ int batch_upload(sdr_batch* b, hipStream_t s)
     }
     ck += c.n_chunks;
     sg += c.segs.size();
-    st += 2 + c.n_chunks;
+    st += FSST_STATE_WORDS + c.n_chunks;
   }
   if (!dcols.empty()) std::memcpy(h + b->off_cols, dcols.data(), dcols.size() * sizeof(FsstColumn));
   if (!b->mask_units.empty())
@@ -705,7 +705,7 @@ int batch_collect(sdr_batch* b)
   for (auto& c : b->cols) {
     const uint32_t err   = static_cast<uint32_t>(st[w] >> 32);
     const uint64_t total = st[w + 1];
-    w += 2 + c.n_chunks;
+    w += FSST_STATE_WORDS + c.n_chunks;
     c.user->chars_used = total;
     c.status           = err ? SDR_E_HIP : (total > 0x7FFFFFFFull || total > c.cap) ? SDR_E_OVERFLOW : SDR_OK;
     if (c.status && !rc)

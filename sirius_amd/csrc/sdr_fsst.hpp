@@ -107,21 +107,30 @@ hipError_t launch_dfsst_nulls(const FsstSeg* d_segs, uint32_t n_ranges, const Di
                               const uint32_t* d_range_dseg, uint8_t* d_mask, uint32_t total_rows,
                               unsigned long long* d_count, hipStream_t s);
 
+// What a column decode reports to the host, in pinned memory.
+struct FsstResult {
+  uint64_t total;  // decoded chars
+  uint64_t error;  // the look-back did not complete
+};
+
 // Device state of one column decode: ticket counter, look-back status per
-// chunk, error flag and the decoded chars total.
+// chunk, error flag and the decoded chars total, which the last chunk also
+// writes to `result` when that is set.
 struct FsstState {
   uint32_t ticket;
   uint32_t error;
   uint64_t total;
+  FsstResult* result;
   uint64_t status[1];  // n_chunks entries
 };
+constexpr uint32_t FSST_STATE_WORDS = 3;  // 8-byte words before status
 
-hipError_t launch_fsst_reset(FsstState* d_state, uint32_t n_chunks, hipStream_t s);
-// Segment pre-pass over n_segs ranges (or *d_n_segs when given, for a
-// launch recorded before the count is known): writes the chunk list, the
-// chunks' FsstChunkInfo and the segments' symbol tables.
-hipError_t launch_fsst_prep(const FsstSeg* d_segs, uint32_t n_segs, const uint32_t* d_n_segs, uint32_t grid,
-                            FsstChunk* d_chunks, FsstChunkInfo* d_info, FsstSymTab* d_tabs, hipStream_t s);
+// Segment pre-pass over n_segs ranges: writes the chunk list, the chunks'
+// FsstChunkInfo and the segments' symbol tables, and sets up the state (its
+// result may be null).  The ranges may be pinned host memory: each is read
+// once, by the block that handles it.
+hipError_t launch_fsst_prep(const FsstSeg* segs, uint32_t n_segs, FsstChunk* d_chunks, FsstChunkInfo* d_info,
+                            FsstSymTab* d_tabs, FsstState* d_state, FsstResult* result, hipStream_t s);
 hipError_t launch_fsst(const FsstChunk* d_chunks, uint32_t first, uint32_t n, uint32_t n_chunks_total,
                        const FsstChunkInfo* d_info, const FsstSymTab* d_tabs, FsstState* d_state,
                        int32_t* d_offsets, uint8_t* d_chars, uint64_t chars_cap, uint32_t total_rows,

@@ -31,9 +31,11 @@ int upload_async(void* d_dst, const void* h_src, size_t bytes, hipStream_t s);
 // the slot free once the work enqueued on s so far has completed.
 int desc_acquire(const void* h_src, size_t bytes, hipStream_t s, void** d_out, void** token);
 int desc_release(void* token, hipStream_t s);
-// A slot's pinned buffer of at least `bytes` (device-accessible), nothing
-// copied; given back with desc_release.
-int pinned_acquire(size_t bytes, void** h_out, void** token);
+// A slot's pinned (device-accessible) and device buffers of at least these
+// sizes, nothing copied; given back with desc_release, or, when no work on
+// them can be pending (the stream was synchronised), slot_release_idle.
+int slot_acquire(size_t h_bytes, size_t d_bytes, void** h_out, void** d_out, void** token);
+void slot_release_idle(void* token);
 
 bool type_ok_for(uint32_t codec, uint32_t ts);
 bool codec_fixed(uint32_t codec);

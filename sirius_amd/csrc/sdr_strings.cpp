@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <cstring>
 #include <mutex>
 #include <vector>
 
@@ -18,7 +19,7 @@
 // (sdr_decode_strings_column_noalloc): a fixed array in the code object, one
 // copy per GPU, held until the process ends.  Host code never uses its name
 // as an address: the per-device address comes from hipGetSymbolAddress.
-static __device__ __align__(256) uint8_t scratch[SDR_NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) uint8_t scratch[SDR_NOALLOC_SCRATCH_BYTES + 256];  // and FsstState::result
 
 namespace sdr {
 
@@ -273,18 +274,35 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
   const size_t tab_bytes   = al(std::max<size_t>(1, hsegs.size()) * sizeof(FsstSymTab));
   const size_t state_bytes = al(sizeof(FsstState) + sizeof(uint64_t) * n_chunks);
   const size_t total_bytes = seg_bytes + chunk_bytes + info_bytes + tab_bytes + state_bytes + sizeof(unsigned long long);
-  uint8_t* d = nullptr;
+  // The call's device memory and, in pinned memory, the ranges, which the
+  // pre-pass reads in place, and the result, which the kernels write: both in
+  // a slot that later calls reuse (device memory past STRINGS_KEEP_BYTES, or
+  // none when nothing may be allocated, is not the slot's).
+  constexpr size_t STRINGS_KEEP_BYTES = 32u << 20;
+  uint8_t* d = scratch_mem;
+  void *h_slot = nullptr, *d_slot = nullptr, *slot = nullptr;
+  const bool own = !scratch_mem && total_bytes > STRINGS_KEEP_BYTES;
   if (scratch_mem) {
-    if (total_bytes > SDR_NOALLOC_SCRATCH_BYTES)
+    // FsstState::result, unused here, does not count against the limit
+    const size_t counted = total_bytes - state_bytes + al(sizeof(FsstState) - sizeof(FsstResult*) + sizeof(uint64_t) * n_chunks);
+    if (counted > SDR_NOALLOC_SCRATCH_BYTES)
       return fail(SDR_E_CAPACITY, "string decode needs %llu bytes of descriptors; the no-allocation scratch holds %u",
-                  static_cast<unsigned long long>(total_bytes), SDR_NOALLOC_SCRATCH_BYTES);
-    d = scratch_mem;
+                  static_cast<unsigned long long>(counted), SDR_NOALLOC_SCRATCH_BYTES);
   } else {
-    rc = device_alloc(reinterpret_cast<void**>(&d), total_bytes, s);
-    if (rc) return rc;
+    rc = slot_acquire(sizeof(FsstResult) + hsegs.size() * sizeof(FsstSeg), own ? 0 : total_bytes, &h_slot, &d_slot, &slot);
+    if (!rc && own) rc = device_alloc(reinterpret_cast<void**>(&d), total_bytes, s);
+    if (rc) {
+      slot_release_idle(slot);
+      return rc;
+    }
+    if (!own) d = static_cast<uint8_t*>(d_slot);
   }
+  auto* result = static_cast<FsstResult*>(h_slot);
+  bool synced  = false;  // nothing enqueued on the slot's memory is pending
   auto release = [&]() {
-    if (!scratch_mem) device_free(d, s);
+    if (own) device_free(d, s);
+    if (synced) slot_release_idle(slot);
+    else (void)desc_release(slot, s);
   };
   auto* d_segs   = reinterpret_cast<FsstSeg*>(d);
   auto* d_chunks = reinterpret_cast<FsstChunk*>(d + seg_bytes);
@@ -295,14 +313,22 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
   auto* d_nulls  = reinterpret_cast<unsigned long long*>(d_rest + state_bytes);
 
   hipError_t e = hipSuccess;
+  const FsstSeg* prep_segs = d_segs;
   if (scratch_mem) {
     e = hipMemcpyAsync(d_segs, hsegs.data(), hsegs.size() * sizeof(FsstSeg), hipMemcpyHostToDevice, s);
     if (e != hipSuccess) return fail(SDR_E_HIP, "string decode: %s", hipGetErrorString(e));
   } else {
-    rc = upload_async(d_segs, hsegs.data(), hsegs.size() * sizeof(FsstSeg), s);
-    if (rc) {
-      release();
-      return rc;
+    *result = FsstResult{0, 0};
+    if (dfsst) {  // its passes read the ranges many times
+      rc = upload_async(d_segs, hsegs.data(), hsegs.size() * sizeof(FsstSeg), s);
+      if (rc) {
+        release();
+        return rc;
+      }
+    } else {
+      auto* hs = reinterpret_cast<FsstSeg*>(result + 1);
+      std::memcpy(hs, hsegs.data(), hsegs.size() * sizeof(FsstSeg));
+      prep_segs = hs;
     }
   }
   DictFsstCall dc;
@@ -318,9 +344,7 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
     dc.release(s);
     release();
   };
-  e = launch_fsst_reset(d_state, n_chunks, s);
-  if (e == hipSuccess)
-    e = launch_fsst_prep(d_segs, n_ranges, nullptr, std::min<uint32_t>(n_ranges, 4096u), d_chunks, d_info, d_tabs, s);
+  e = launch_fsst_prep(prep_segs, n_ranges, d_chunks, d_info, d_tabs, d_state, result, s);
   if (e == hipSuccess) {
     if (mode == SDR_LAUNCH_PER_SEGMENT) {
       for (uint32_t i = 0; e == hipSuccess && i < n_ranges; ++i)
@@ -359,14 +383,19 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
     uint64_t total;
   } h{};
   unsigned long long h_nulls = 0;
-  if (e == hipSuccess) e = hipMemcpyAsync(&h, d_state, sizeof(h), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess && scratch_mem) e = hipMemcpyAsync(&h, d_state, sizeof(h), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess && device_nulls) e = hipMemcpyAsync(&h_nulls, d_nulls, sizeof(h_nulls), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  for (size_t u = 0; e == hipSuccess && counts && u < units.size(); ++u) h_nulls += counts[u];
-  rc = desc_release(counts_token, s);
+  synced = e == hipSuccess;
+  if (synced && result) {
+    h.total = result->total;
+    h.error = static_cast<uint32_t>(result->error);
+  }
+  for (size_t u = 0; synced && counts && u < units.size(); ++u) h_nulls += counts[u];
+  if (synced) slot_release_idle(counts_token);
+  else (void)desc_release(counts_token, s);
   release_all();
   if (e != hipSuccess) return fail(SDR_E_HIP, "string decode: %s", hipGetErrorString(e));
-  if (rc) return rc;
   if (h.error) return fail(SDR_E_HIP, "string decode: offset look-back did not complete");
   col->chars_used = h.total;
   col->null_count = masked ? static_cast<int64_t>(h_nulls) : 0;
