@@ -158,6 +158,22 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* s_wave
   return before + incl - v;
 }
 
+// Exclusive scan of one value per thread with one barrier, for LDS alone
+// (global loads stay in flight); s_wave must not be written again before the
+// caller's next barrier.
+__device__ __forceinline__ uint32_t block_excl_scan_lds(uint32_t v, uint32_t* s_wave, uint32_t* total)
+{
+  static_assert(FSST_WAVES <= 16, "one DPP row of wave sums");
+  const uint32_t incl = wave_incl_sum_u32(v);
+  const uint32_t w    = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)));
+  if (lane_id() == WAVE - 1u) s_wave[w] = incl;
+  lds_barrier();
+  const uint32_t ws = s_wave[lane_id() & (FSST_WAVES - 1u)];  // every wave scans the wave sums
+  const uint32_t wi = row_incl_sum_u32(ws);
+  *total            = __builtin_amdgcn_readlane(wi, FSST_WAVES - 1u);
+  return __builtin_amdgcn_readlane(wi, w) - __builtin_amdgcn_readlane(ws, w) + incl - v;
+}
+
 // Exclusive scans of two values per thread with one barrier, for LDS alone
 // (global loads stay in flight); s_wave[2 * FSST_WAVES] must not be written
 // again before the caller's next barrier.
@@ -188,13 +204,13 @@ __device__ __forceinline__ void block_excl_scan2(uint32_t a, uint32_t b, uint32_
 // in 256-thread workgroups with an 11 KiB window: 70 VALU and 52 LDS cycles
 // per 64 bytes, 560 us for 16 Mi rows of 27 chars (12.9 compressed).  Row
 // starts as a bitmap, packed prefix sums and two lookups and two to three ORs
-// per byte take it to 39 VALU and 32 LDS cycles and 318 us.  512 threads with
-// two groups each keep a 16 KiB run in registers, so nothing is read twice;
-// three such workgroups share a CU (51 KB of LDS, 80 VGPRs), whose 38 KiB
-// window builds most chunks in one piece.  Rows of 70 and 200 chars, whose
-// chunks take several runs, went from 945 to 305 and from 2956 to 440 us (137
-// and 197 MB of chars); the row-wise path is left to malformed chunks and to
-// rows that no run holds.
+// per byte take it to 32 VALU and 31 LDS cycles and 294 us, both busy 58% of
+// the time.  512 threads with two groups each keep a 16 KiB run in registers,
+// so nothing is read twice; three such workgroups share a CU (51 KB of LDS, 80
+// VGPRs), whose 38 KiB window builds most chunks in one piece.  Rows of 70 and
+// 200 chars, whose chunks take several runs, went from 945 to 221 and from 2956
+// to 324 us (137 and 197 MB of chars); the row-wise path is left to malformed
+// chunks and to rows that no run holds.
 constexpr uint32_t FSST_SYMSTAGE = 17u + 8u * FSST_NSYM;  // the largest symbol table (2057 bytes)
 // Compressed bytes that the staged path takes at a time, the head of up to
 // 15 bytes before them included: GROUPS_PER_THR 16-byte groups per thread.
@@ -207,8 +223,8 @@ constexpr uint32_t FSST_WINDOW = 38u << 10;
 static __device__ __attribute__((aligned(16))) const uint32_t fsst_zero_group[4] = {0u, 0u, 0u, 0u};
 
 constexpr uint32_t ROW_HUGE = 1u << 20;  // a staged row is shorter than this
-// The first walk's packed prefixes: decoded bytes (at most 8 * FSST_CSTAGE,
-// bits 0-17) with a count of at most 1024 rows above.
+// Packed prefixes: decoded bytes (at most 8 * FSST_CSTAGE, bits 0-17) or a
+// run's compressed bytes, with a count of at most 1024 rows above.
 constexpr uint32_t PK_LEN = 18;
 // len[] of the escape code in a staged chunk's table, so that the lengths a
 // group looks up tell whether it holds an escape.
@@ -219,15 +235,16 @@ struct FsstSmem {
   __attribute__((aligned(16))) uint64_t sym[256];  // symbol bytes, zero above its length
   uint8_t len[256];
   // row-wise path: comp[] is the segment-relative inclusive compressed prefix,
-  // dec[] the chunk-relative exclusive decoded offset.  Staged path, rows with
-  // compressed bytes in storage order (rank): comp[k] is the decoded prefix at
-  // row k's first byte, dec[k + 1] what takes a decoded prefix inside row k to
-  // its output position.
+  // dec[] the chunk-relative exclusive decoded offset.  Staged path: comp[g] is
+  // the decoded prefix at group g's first byte; of the rows with compressed
+  // bytes in storage order (rank), dec[k + 1] is what takes a decoded prefix
+  // inside row k to its output position.
   uint32_t comp[FSST_CHUNK_ROWS + 1];
   uint32_t dec[FSST_CHUNK_ROWS + 4];
   uint32_t bits[FSST_CSTAGE / 32];  // bit y: a row's first byte is stage position y
   // output window (and the slack its last symbol's words reach); before that,
-  // the compressed-length fields
+  // the compressed-length fields, then the groups' packed prefixes (byte y:
+  // decoded bytes of stage position y's group before it)
   __attribute__((aligned(16))) uint8_t out[FSST_WINDOW + 48];
   uint32_t wave[2 * FSST_WAVES];
   uint32_t part[2 * FSST_WAVES];
@@ -438,33 +455,40 @@ __device__ __forceinline__ uint32_t fsst_group_lengths(FsstGroup& gr, const Fsst
   }
   gr.m               = live ? (sm.bits[g >> 1] >> (16u * (g & 1u))) & 0xFFFFu : 0u;
   gr.lit             = 0;
-  const bool has_esc = ((L[0] | L[1] | L[2] | L[3]) & 0x80808080u) != 0;
-  const bool edge    = 16u * g < c_h || 16u * g + 16u > y_hi;
-  const bool after   = (prev >> 24) == FSST_ESC && 16u * g > c_h;
+  const uint32_t y   = 16u * g;
+  const bool has_esc = live && ((L[0] | L[1] | L[2] | L[3]) & 0x80808080u) != 0;
+  const bool after   = live && (prev >> 24) == FSST_ESC && y > c_h;
   *lits              = false;
-  if (ballot(live && (has_esc || edge || after)) != 0) {
-    const uint32_t y     = 16u * g;
-    const uint32_t lo    = c_h > y ? c_h - y : 0u;  // c_h < 16
-    const uint32_t hi    = live ? (y_hi - y < 16u ? y_hi - y : 16u) : lo;
-    const uint32_t valid = ((1u << hi) - 1u) & ~((1u << lo) - 1u);
-    uint32_t e           = 0;
+  uint32_t valid     = 0xFFFFu;  // the bytes that are the run's
+  if (ballot(live && (y < c_h || y + 16u > y_hi)) != 0) {
+    const uint32_t lo = c_h > y ? c_h - y : 0u;  // c_h < 16
+    const uint32_t hi = live ? (y_hi - y < 16u ? y_hi - y : 16u) : lo;
+    valid             = ((1u << hi) - 1u) & ~((1u << lo) - 1u);
+#pragma unroll
+    for (uint32_t d = 0; d < 4; ++d) {
+      const uint32_t in = spread4(valid >> (4u * d)) * 0xFFu;
+      L[d] &= in;
+      gr.q[d] |= ~in;
+    }
+  }
+  if (ballot(has_esc || after) != 0) {
+    uint32_t e = 0;
 #pragma unroll
     for (uint32_t j = 0; j < 16; ++j) e |= group_byte(gr.q, j) == FSST_ESC ? 1u << j : 0u;
     e &= valid;
     bool esc = false;  // an odd run of 255s of the row ends just before the group
-    if (live && after && !(gr.m & 1u)) {
+    if (after && !(gr.m & 1u)) {
       for (uint32_t x = y; x > c_h; --x) {
         if (ld_u8(stage + x - 1u) != FSST_ESC) break;
         esc = !esc;
         if ((sm.bits[(x - 1u) >> 5] >> ((x - 1u) & 31u)) & 1u) break;  // the row's first byte
       }
     }
-    gr.lit = literal_mask(e, gr.m, esc) & valid;
+    gr.lit = live ? literal_mask(e, gr.m, esc) & valid : 0u;
 #pragma unroll
     for (uint32_t d = 0; d < 4; ++d) {
-      const uint32_t one = spread4(gr.lit >> (4u * d)), in = spread4(valid >> (4u * d)) * 0xFFu;
-      L[d]               = (L[d] & 0x7F7F7F7Fu & in & ~(one * 0xFFu)) | one;
-      gr.q[d] |= ~in;
+      const uint32_t one = spread4(gr.lit >> (4u * d));
+      L[d]               = (L[d] & 0x7F7F7F7Fu & ~(one * 0xFFu)) | one;
     }
     *lits = ballot(gr.lit != 0) != 0;
   }
@@ -479,49 +503,61 @@ __device__ __forceinline__ uint32_t fsst_group_lengths(FsstGroup& gr, const Fsst
   return live ? t & 0xFFu : 0u;
 }
 
-// Both groups' first walk, the run's decoded total *T, and sm.comp[] (the
-// decoded prefix at every first byte of a row, and after the last byte).  The caller's next barrier makes sm.comp[] visible.
-__device__ __forceinline__ void fsst_walk_lengths(FsstGroup (&gr)[GROUPS_PER_THR], FsstSmem& sm,
-                                                  const uint32_t (&prev)[GROUPS_PER_THR], uint32_t c_h, uint32_t y_hi,
-                                                  const uint8_t* stage, bool (&lits)[GROUPS_PER_THR], uint32_t* T)
+// Both groups' first walk and the run's decoded total T.  Leaves every group's
+// decoded prefix in sm.comp[] and its packed prefixes in sm.out, so that after
+// the caller's next barrier run_prefix() tells the decoded prefix at any stage
+// position.  (Each lane collecting it for the rows that start in its groups,
+// one loop iteration per row, cost a tenth of the kernel's instructions.)
+__device__ __forceinline__ uint32_t fsst_walk_lengths(FsstGroup (&gr)[GROUPS_PER_THR], FsstSmem& sm,
+                                                      const uint32_t (&prev)[GROUPS_PER_THR], uint32_t c_h,
+                                                      uint32_t y_hi, const uint8_t* stage,
+                                                      bool (&lits)[GROUPS_PER_THR])
 {
   const uint32_t tid  = threadIdx.x;
   const uint32_t lane = lane_id();
   const uint32_t w    = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(tid >> 6)));
-  uint32_t v[GROUPS_PER_THR], incl[GROUPS_PER_THR];
+  uint32_t v[GROUPS_PER_THR] = {}, incl[GROUPS_PER_THR] = {};
 #pragma unroll
   for (uint32_t k = 0; k < GROUPS_PER_THR; ++k) {
-    // the word before the group: the lane below holds it, lane 0 loaded it
-    uint32_t pw = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
-      static_cast<int>(prev[k]), static_cast<int>(gr[k].q[3]), 0x138, 0xF, 0xF, false));  // wave_shr:1
-    v[k] = fsst_group_lengths(gr[k], sm, k * FSST_THREADS + tid, pw, c_h, y_hi, stage, &lits[k]);
-    v[k] |= static_cast<uint32_t>(__builtin_popcount(gr[k].m)) << PK_LEN;
-    incl[k] = wave_incl_sum_u32(v[k]);
+    lits[k] = false;
+    gr[k].m = gr[k].lit = 0;
+    if (16u * (k * FSST_THREADS + w * WAVE) < y_hi) {  // the wave has groups of the run
+      // the word before the group: the lane below holds it, lane 0 loaded it
+      const uint32_t pw = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+        static_cast<int>(prev[k]), static_cast<int>(gr[k].q[3]), 0x138, 0xF, 0xF, false));  // wave_shr:1
+      v[k] = fsst_group_lengths(gr[k], sm, k * FSST_THREADS + tid, pw, c_h, y_hi, stage, &lits[k]);
+      v[k] |= static_cast<uint32_t>(__builtin_popcount(gr[k].m)) << PK_LEN;
+      incl[k] = wave_incl_sum_u32(v[k]);
+    }
     if (lane == WAVE - 1) sm.part[k * FSST_WAVES + w] = incl[k];
   }
   lds_barrier();
   // every wave scans the 2 x FSST_WAVES wave sums in one 16-lane row
   static_assert(GROUPS_PER_THR * FSST_WAVES == 16, "one DPP row of wave sums");
-  const uint32_t ws  = sm.part[lane & 15u];
-  const uint32_t wi  = row_incl_sum_u32(ws);
-  const uint32_t tot = __builtin_amdgcn_readlane(wi, 15);
-  *T = tot & ((1u << PK_LEN) - 1u);
+  const uint32_t ws = sm.part[lane & 15u];
+  const uint32_t wi = row_incl_sum_u32(ws);
+  const uint32_t T  = static_cast<uint32_t>(__builtin_amdgcn_readlane(wi, 15)) & ((1u << PK_LEN) - 1u);
 #pragma unroll
   for (uint32_t k = 0; k < GROUPS_PER_THR; ++k) {
     const uint32_t i  = k * FSST_WAVES + w;
     const uint32_t ex = __builtin_amdgcn_readlane(wi, i) - __builtin_amdgcn_readlane(ws, i) + incl[k] - v[k];
     gr[k].d           = ex & ((1u << PK_LEN) - 1u);
     gr[k].r           = ex >> PK_LEN;
-    const uint64_t lo = gr[k].p[0] | uint64_t{gr[k].p[1]} << 32, hi = gr[k].p[2] | uint64_t{gr[k].p[3]} << 32;
-    uint32_t m = gr[k].m, rank = gr[k].r;
-    while (m) {
-      const uint32_t j = static_cast<uint32_t>(__builtin_ctz(m));
-      m &= m - 1u;
-      sm.comp[rank++] = gr[k].d + (static_cast<uint32_t>((j & 8u ? hi : lo) >> (8u * (j & 7u))) & 0xFFu);
+    const uint32_t g  = k * FSST_THREADS + tid;
+    if (16u * g < y_hi) {
+      sm.comp[g]                               = gr[k].d;
+      reinterpret_cast<u32x4*>(sm.out)[g] = u32x4{gr[k].p[0], gr[k].p[1], gr[k].p[2], gr[k].p[3]};
     }
   }
-  if (tid == 0) sm.comp[tot >> PK_LEN] = tot & ((1u << PK_LEN) - 1u);
+  if (tid == 0 && !(y_hi & 15u)) {  // the position after the last byte starts a group of its own
+    sm.comp[y_hi >> 4] = T;
+    sm.out[y_hi]       = 0;
+  }
+  return T;
 }
+
+// The decoded prefix of the run at stage position y.
+__device__ __forceinline__ uint32_t run_prefix(const FsstSmem& sm, uint32_t y) { return sm.comp[y >> 4] + sm.out[y]; }
 
 // OR symbol bytes v at window position o.
 __device__ __forceinline__ void window_or(uint8_t* out, uint32_t o, uint64_t v)
@@ -536,20 +572,22 @@ __device__ __forceinline__ void window_or(uint8_t* out, uint32_t o, uint64_t v)
 }
 
 // Second walk of one group into the window over output bytes [w0, w0 +
-// FSST_WINDOW) of the run's T.  MULTI: the run's output takes several windows;
+// FSST_WINDOW) of the run.  MULTI: the run's output takes several windows;
 // a wave skips a window that none of its groups reaches, and words outside
 // the window go to a word past it.
 template <bool MULTI>
 __device__ __forceinline__ void fsst_group_emit(const FsstGroup& gr, FsstSmem& sm, uint32_t g, uint32_t y_hi, bool lits,
-                                                uint32_t T, uint32_t w0)
+                                                uint32_t w0)
 {
   bool live         = 16u * g < y_hi;
   const uint32_t pc = static_cast<uint32_t>(__builtin_popcount(gr.m));
   if constexpr (MULTI) {
-    // the rows that the group touches are output bytes [lo, hi)
-    const uint32_t lo = live ? T - sm.comp[gr.r + pc] : 0u;
-    const uint32_t hi = live && gr.r ? T - sm.comp[gr.r - 1u] : T;
-    live              = live && lo < w0 + FSST_WINDOW && hi > w0;
+    // rows that follow lie below in the output: the group's bytes are inside
+    // [lo, hi), 128 of them at most in a row (lo may be negative: a row may
+    // start inside the group)
+    const int32_t lo = live ? static_cast<int32_t>(sm.dec[gr.r + pc] + gr.d - w0) : 0;
+    const int32_t hi = live ? static_cast<int32_t>(sm.dec[gr.r] + gr.d + 128u - w0) : 0;
+    live             = live && lo < static_cast<int32_t>(FSST_WINDOW) && hi > 0;
   } else if (!lits && !ballot(live && pc > 3u)) {
     if (!live) return;
     // at most four rows cross a group: what takes a prefix to its output
@@ -1376,8 +1414,8 @@ __device__ __forceinline__ void fsst_mark_row(FsstSmem& sm, uint32_t y)
 }
 
 // A run's chars from its walked groups: window by window when they pass
-// FSST_WINDOW.  The window is cleared for the first one, and sm.comp[] and
-// sm.dec[] are complete.  `get_base()` gives the chars offset of the run (it
+// FSST_WINDOW.  The window is cleared for the first one, and sm.dec[] is
+// complete.  `get_base()` gives the chars offset of the run (it
 // is called once, after the first window's ORs, and synchronises the
 // workgroup).
 template <class GetBase>
@@ -1395,7 +1433,7 @@ __device__ __forceinline__ void fsst_emit_run(FsstGroup (&gr)[GROUPS_PER_THR], F
   if (T <= FSST_WINDOW) {
 #pragma unroll
     for (uint32_t k = 0; k < GROUPS_PER_THR; ++k)
-      fsst_group_emit<false>(gr[k], sm, k * FSST_THREADS + tid, y_hi, lits[k], T, 0u);
+      fsst_group_emit<false>(gr[k], sm, k * FSST_THREADS + tid, y_hi, lits[k], 0u);
     const uint64_t at = get_base();
     if (at < chars_cap)
       window_store(sm, reinterpret_cast<uintptr_t>(chars) + at,
@@ -1413,7 +1451,7 @@ __device__ __forceinline__ void fsst_emit_run(FsstGroup (&gr)[GROUPS_PER_THR], F
     }
 #pragma unroll
     for (uint32_t k = 0; k < GROUPS_PER_THR; ++k)
-      fsst_group_emit<true>(gr[k], sm, k * FSST_THREADS + tid, y_hi, lits[k], T, w0);
+      fsst_group_emit<true>(gr[k], sm, k * FSST_THREADS + tid, y_hi, lits[k], w0);
     if (w0) __syncthreads();
     else base = get_base();
     const uint64_t at = base + w0;
@@ -1509,19 +1547,22 @@ __device__ __attribute__((noinline)) void fsst_chunk_runs(const uint8_t* seg, ui
     if (in1 && ne1) fsst_mark_row(sm, y_hi - (x2 - xa));
     __syncthreads();
     bool lits[GROUPS_PER_THR];
-    uint32_t T = 0;
-    fsst_walk_lengths(gr, sm, prev, c_h, y_hi, stage, lits, &T);
-    window_clear(sm, T < FSST_WINDOW ? T : FSST_WINDOW);
+    const uint32_t T = fsst_walk_lengths(gr, sm, prev, c_h, y_hi, stage, lits);
     __syncthreads();
-    if (in0 || in1) {  // as in fsst_chunk
-      const uint32_t k0 = nb - (in0 ? n0 : n1), k1 = nb - n1;
-      const uint32_t e0 = sm.comp[k0], e1 = sm.comp[k1];
-      if (in0) o0 = static_cast<uint32_t>(t_before) + T - e0;
-      if (in1) o1 = static_cast<uint32_t>(t_before) + T - e1;
-      if (in0 && ne0) sm.dec[k0] = T - e0 - e1;
-      if (in1 && ne1) sm.dec[k1] = T - e1 - sm.comp[k1 - 1u];
+    // as in fsst_chunk, for the rows that are the run's
+    if (in0) {
+      const uint32_t e0 = run_prefix(sm, y_hi - (x0 - xa)), e1 = run_prefix(sm, y_hi - (x1 - xa));
+      o0 = static_cast<uint32_t>(t_before) + T - e0;
+      if (ne0) sm.dec[nb - n0] = T - e0 - e1;
+    }
+    if (in1) {
+      const uint32_t e1 = run_prefix(sm, y_hi - (x1 - xa)), e2 = run_prefix(sm, y_hi - (x2 - xa));
+      o1 = static_cast<uint32_t>(t_before) + T - e1;
+      if (ne1) sm.dec[nb - n1] = T - e1 - e2;
     }
     if (tid == 0) sm.dec[0] = T;
+    __syncthreads();
+    window_clear(sm, T < FSST_WINDOW ? T : FSST_WINDOW);
     __syncthreads();
     if (measured) {
       fsst_emit_run(gr, sm, y_hi, lits, T, chars, chars_cap, [&]() -> uint64_t {
@@ -1602,31 +1643,32 @@ __device__ __forceinline__ void fsst_chunk(const FsstChunk ch, const FsstChunkIn
   const uint32_t cl0 = fsst_field(lw, bit0, lfast, seg, end, ch.row_begin, width, 2u * tid, rows);
   const uint32_t cl1 = fsst_field(lw, bit0, lfast, seg, end, ch.row_begin, width, 2u * tid + 1u, rows);
   const uint32_t ne0 = cl0 ? 1u : 0u, ne1 = cl1 ? 1u : 0u;  // rows with bytes
-  uint32_t x0, n0, x_all, n_all;
-  block_excl_scan2(cl0 + cl1, ne0 + ne1, sm.wave, x0, n0, x_all, n_all);
-  if (ne0) fsst_mark_row(sm, y_hi - (x0 + cl0));
-  if (ne1) fsst_mark_row(sm, y_hi - (x0 + cl0 + cl1));
+  uint32_t all;
+  const uint32_t pre = block_excl_scan_lds((cl0 + cl1) | (ne0 + ne1) << PK_LEN, sm.wave, &all);
+  // stage positions: row 2t ends at ya, row 2t + 1 at yb and starts at yc
+  const uint32_t ya = y_hi - (pre & ((1u << PK_LEN) - 1u)), yb = ya - cl0, yc = yb - cl1;
+  if (ne0) fsst_mark_row(sm, yb);
+  if (ne1) fsst_mark_row(sm, yc);
   if (tid == 0) sm.len[FSST_ESC] = LEN_ESC;
   lds_barrier();
 
   // ---- first walk ----
   bool lits[GROUPS_PER_THR];
-  uint32_t T = 0;
-  fsst_walk_lengths(gr, sm, prev, c_h, y_hi, stage, lits, &T);
+  const uint32_t T = fsst_walk_lengths(gr, sm, prev, c_h, y_hi, stage, lits);
   // The aggregate is published now; the look-back's wait, and the offsets,
   // come once the first window's chars are in LDS.
   fsst_lookback_publish(c, T, st, spin_limit);
-  window_clear(sm, T < FSST_WINDOW ? T : FSST_WINDOW);
   lds_barrier();
 
   // ---- rows: output positions.  A row's chars follow those of the rows below
   // it, which lie after it in storage order ----
-  const uint32_t k0 = n_all - n0;  // one past row 2t's rank (the rank's place when it has no bytes)
-  const uint32_t k1 = k0 - ne0;
-  const uint32_t e0 = sm.comp[k0], e1 = sm.comp[k1];
-  if (ne0) sm.dec[k0] = T - e0 - e1;  // rank k0 - 1 == k1: output position T - e0, prefix e1
-  if (ne1) sm.dec[k1] = T - e1 - sm.comp[k1 - 1u];
+  const uint32_t e0 = run_prefix(sm, ya), e1 = run_prefix(sm, yb), e2 = run_prefix(sm, yc);
+  const uint32_t k0 = (all >> PK_LEN) - (pre >> PK_LEN);  // one past row 2t's rank
+  if (ne0) sm.dec[k0] = T - e0 - e1;        // output position T - e0, prefix e1
+  if (ne1) sm.dec[k0 - ne0] = T - e1 - e2;
   if (tid == 0) sm.dec[0] = T;  // bytes before the first row's, which decode to nothing
+  lds_barrier();
+  window_clear(sm, T < FSST_WINDOW ? T : FSST_WINDOW);
   lds_barrier();
 
   // ---- second walk ----
