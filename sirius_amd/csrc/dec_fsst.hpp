@@ -38,8 +38,6 @@ namespace sdr {
 constexpr uint32_t FSST_THREADS   = 512;  // a chunk's workgroup
 constexpr uint32_t FSST_WAVES     = FSST_THREADS / WAVE;
 constexpr uint32_t ROWS_PER_THR   = FSST_CHUNK_ROWS / FSST_THREADS;
-constexpr uint32_t PREP_THREADS   = 256;  // the segment pre-passes' workgroups: one symbol code per thread
-constexpr uint32_t PREP_WAVES     = PREP_THREADS / WAVE;
 constexpr uint32_t FSST_PIECE     = 8192;  // LDS output piece of the row-wise path
 constexpr uint32_t FSST_ESC       = 255;
 constexpr uint32_t FSST_NSYM      = 255;
@@ -820,12 +818,18 @@ __device__ __forceinline__ void fsst_offsets(const FsstChunk& ch, uint32_t c, ui
 
 // ---- segment pre-pass ----
 
+constexpr uint32_t PREP_STAGE = 16384;  // segment bytes of the length stream staged at a time
+
+// A pre-pass workgroup of NT threads, 256 or more (a symbol table is imported
+// one code per thread).
+template <uint32_t NT>
 struct FsstPrepSmem {
   __attribute__((aligned(16))) uint8_t st[FSST_SYMSTAGE + 48];
+  __attribute__((aligned(16))) uint32_t fields[(PREP_STAGE + 128) / 4];
   uint8_t len[256];  // code lengths of a DICT_FSST dictionary's table
-  uint32_t sum[PREP_THREADS];
-  uint32_t huge[PREP_THREADS];
-  uint32_t wave[PREP_WAVES];
+  uint32_t sum[NT];
+  uint32_t huge[NT];
+  uint32_t wave[NT / WAVE];
 };
 
 // Sum of the w-bit fields [f0, f1) of the length stream at `base`, and
@@ -854,6 +858,27 @@ __device__ __forceinline__ uint32_t fields_sum(const uint8_t* base, const uint8_
   return s;
 }
 
+// Sum of the first n (at most 16) w-bit fields (1 <= w <= 32) from bit `bit` of
+// a stream staged in LDS, and the largest of them into *mx.  All 16 are read,
+// so that no branch or earlier read holds one back (a word cursor, or a branch
+// around each field, took 250 cycles a field): up to 68 bytes past the first
+// field must be readable.
+__device__ __forceinline__ uint32_t lds_fields_sum(const uint32_t* lds, uint32_t bit, uint32_t n, uint32_t w,
+                                                   uint32_t* mx)
+{
+  uint32_t v[16], s = 0, m = 0;
+#pragma unroll
+  for (uint32_t f = 0; f < 16; ++f) v[f] = lds_bits32(lds, bit + f * w, w);
+#pragma unroll
+  for (uint32_t f = 0; f < 16; ++f) {
+    const uint32_t x = f < n ? v[f] : 0u;
+    s += x;
+    m = x > m ? x : m;
+  }
+  *mx = m;
+  return s;
+}
+
 // ---- DICTIONARY and UNCOMPRESSED strings ----
 //
 // DICTIONARY (strings/dictionary.cu:17-33): a 20-byte header {dict_size,
@@ -876,6 +901,7 @@ __device__ __forceinline__ uint32_t fields_sum(const uint8_t* base, const uint8_
 // the reference's passes' intent (its length pass gives 0).
 
 // Per-chunk info of a plain segment, one thread per chunk.
+template <uint32_t NT>
 __device__ __forceinline__ void plain_prep_segment(const FsstSeg& sg, FsstChunkInfo* __restrict__ info)
 {
   const uint8_t* seg = sg.bytes;
@@ -895,7 +921,7 @@ __device__ __forceinline__ void plain_prep_segment(const FsstSeg& sg, FsstChunkI
     ok       = dict_end <= sg.bytes_size;
   }
   const uint32_t flags = (dict ? FI_DICT | (width & FI_WIDTH) : FI_UNC) | (ok ? FI_OK : 0u);
-  for (uint32_t k = threadIdx.x; k * FSST_CHUNK_ROWS < sg.row_count; k += PREP_THREADS) {
+  for (uint32_t k = threadIdx.x; k * FSST_CHUNK_ROWS < sg.row_count; k += NT) {
     FsstChunkInfo ci;
     ci.bytes      = seg;
     ci.c_lo       = ibo;
@@ -1130,8 +1156,9 @@ __device__ __attribute__((noinline)) void plain_chunk(const uint8_t* seg, uint32
 // length of the calling thread's code.  A table whose version word does not
 // match decodes every code to nothing.  Every thread of the block must call
 // it.
+template <uint32_t NT>
 __device__ __forceinline__ uint32_t import_symtab(const uint8_t* seg, uint32_t bytes_size, uint32_t symoff, bool ok,
-                                                  FsstSymTab* __restrict__ tab, FsstPrepSmem& sm)
+                                                  FsstSymTab* __restrict__ tab, FsstPrepSmem<NT>& sm)
 {
   const uint32_t tid = threadIdx.x;
   __syncthreads();  // the previous segment's use of sm is done
@@ -1139,11 +1166,13 @@ __device__ __forceinline__ uint32_t import_symtab(const uint8_t* seg, uint32_t b
   if (ok) {
     sym_n = bytes_size - symoff;
     if (sym_n > FSST_SYMSTAGE) sym_n = FSST_SYMSTAGE;
-    sym_h = block_stage<PREP_THREADS>(reinterpret_cast<uint32_t*>(sm.st), seg + symoff, sym_n);
+    sym_h = block_issue<NT>(reinterpret_cast<uint32_t*>(sm.st), seg + symoff, sym_n);
   }
+  __builtin_amdgcn_s_waitcnt(WAITCNT_VMEM_DONE);  // and for what the caller issued
   __syncthreads();
   uint32_t len = 0;
   uint64_t sym = 0;
+  if (tid >= 256u) return 0;  // one code per thread (uniform per wave)
   if (ok) {
     auto sb = [&](uint32_t i) -> uint32_t { return i < sym_n ? sm.st[sym_h + i] : 0u; };
     uint64_t version = 0;
@@ -1188,9 +1217,10 @@ __device__ __forceinline__ uint32_t import_symtab(const uint8_t* seg, uint32_t b
 // entry offsets (entry 0 empty), otherwise the byte offsets again, into
 // e_dec; out = {decoded total, inline-NULL flag}.  32-bit sums, as the
 // reference's scans.
+template <uint32_t NT>
 __device__ __forceinline__ void dfsst_prep_segment(const DictFsstSeg& d, uint32_t* __restrict__ e_byte,
                                                    uint32_t* __restrict__ e_dec, FsstSymTab* __restrict__ tab,
-                                                   uint32_t* __restrict__ out, FsstPrepSmem& sm)
+                                                   uint32_t* __restrict__ out, FsstPrepSmem<NT>& sm)
 {
   const uint32_t tid = threadIdx.x;
   if (!d.valid) {  // uniform per block
@@ -1201,12 +1231,12 @@ __device__ __forceinline__ void dfsst_prep_segment(const DictFsstSeg& d, uint32_
   const uint8_t* end  = seg + d.bytes_size;
   const bool fsst     = d.mode != 0u && d.dict_count > 1u;
   const uint32_t mylen = import_symtab(seg, d.bytes_size, d.off_symtab, fsst && d.off_symtab < d.bytes_size, tab, sm);
-  sm.len[tid] = static_cast<uint8_t>(mylen);
+  if (tid < 256u) sm.len[tid] = static_cast<uint8_t>(mylen);
   __syncthreads();
   const uint8_t* slens = seg + d.off_slens;
   const uint8_t* dict  = seg + d.off_dict;
   uint32_t carry_b = 0, carry_d = 0, first_len = 0;
-  for (uint32_t k0 = 0; k0 < d.dict_count; k0 += 4u * PREP_THREADS) {
+  for (uint32_t k0 = 0; k0 < d.dict_count; k0 += 4u * NT) {
     uint32_t v[4], dl[4], sb = 0, sd = 0;
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {
@@ -1215,7 +1245,7 @@ __device__ __forceinline__ void dfsst_prep_segment(const DictFsstSeg& d, uint32_
       sb += v[i];
     }
     uint32_t tb = 0;
-    uint32_t run = carry_b + block_excl_scan<PREP_WAVES>(sb, sm.wave, &tb);
+    uint32_t run = carry_b + block_excl_scan<NT / WAVE>(sb, sm.wave, &tb);
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {
       const uint32_t k = k0 + 4u * tid + i;
@@ -1226,7 +1256,7 @@ __device__ __forceinline__ void dfsst_prep_segment(const DictFsstSeg& d, uint32_
       sd += dl[i];
     }
     uint32_t td = 0;
-    uint32_t rd = carry_d + block_excl_scan<PREP_WAVES>(sd, sm.wave, &td);
+    uint32_t rd = carry_d + block_excl_scan<NT / WAVE>(sd, sm.wave, &td);
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {
       const uint32_t k = k0 + 4u * tid + i;
@@ -1278,22 +1308,23 @@ __device__ __forceinline__ void dfsst_predecode(const DictFsstSeg& d, const uint
   }
 }
 
-// Range `si` with the calling PREP_THREADS-thread workgroup: its chunk descriptors
+// Range `si` with the calling NT-thread workgroup: its chunk descriptors
 // into chunks[first_chunk + k]; for a segment, header checks
 // (fsst.cu:79-87), the symbol table import, one code per thread
 // (detail/fsst.cuh:50-96), into `tab`, and for each chunk k its
 // compressed-length prefix bounds (fsst.cu:132-188) and flags into
 // info[first_chunk + k].  Bytes past the segment read as zero; no symbol
 // table parse reads past byte 2057.
+template <uint32_t NT>
 __device__ __forceinline__ void fsst_prep_segment(const FsstSeg sg, uint32_t si, FsstChunk* __restrict__ chunks,
                                                   FsstChunkInfo* __restrict__ info, FsstSymTab* __restrict__ tab,
-                                                  FsstPrepSmem& sm)
+                                                  FsstPrepSmem<NT>& sm)
 {
   const uint32_t tid = threadIdx.x;
   const uint8_t* seg = sg.bytes;
   const uint8_t* end = seg + sg.bytes_size;
   const bool gap     = seg == nullptr;
-  for (uint32_t k = tid; k * FSST_CHUNK_ROWS < sg.row_count; k += PREP_THREADS) {
+  for (uint32_t k = tid; k * FSST_CHUNK_ROWS < sg.row_count; k += NT) {
     const uint32_t r0 = k * FSST_CHUNK_ROWS;
     const uint32_t n  = sg.row_count - r0 < FSST_CHUNK_ROWS ? sg.row_count - r0 : FSST_CHUNK_ROWS;
     const FsstChunk fc{gap ? FSST_GAP : si, gap ? 0u : r0, n, sg.col_row + r0};
@@ -1301,11 +1332,11 @@ __device__ __forceinline__ void fsst_prep_segment(const FsstSeg sg, uint32_t si,
   }
   if (gap) return;  // uniform: nothing else of a gap is read
   if (sg.codec == SDR_CODEC_DICTIONARY || sg.codec == SDR_CODEC_UNCOMPRESSED) {
-    plain_prep_segment(sg, info);
+    plain_prep_segment<NT>(sg, info);
     return;  // uniform per segment
   }
   if (sg.codec == SDR_CODEC_DICT_FSST) {  // bytes: the range's DictFsstSeg; pad: 1 if valid
-    for (uint32_t k = tid; k * FSST_CHUNK_ROWS < sg.row_count; k += PREP_THREADS) {
+    for (uint32_t k = tid; k * FSST_CHUNK_ROWS < sg.row_count; k += NT) {
       FsstChunkInfo ci{sg.bytes, 0u, 0u, 0u, FI_DFSST | (sg.pad ? FI_OK : 0u), 0u, 0u};
       const gptr<u32x4> dst = gbl(reinterpret_cast<u32x4*>(info + sg.first_chunk + k));
       const u32x8 cv        = __builtin_bit_cast(u32x8, ci);
@@ -1314,32 +1345,63 @@ __device__ __forceinline__ void fsst_prep_segment(const FsstSeg sg, uint32_t si,
     }
     return;  // uniform per segment
   }
-  bool ok = false;
-  uint32_t dict_end = 0, width = 0, symoff = 0;
+  // The front of the segment, nearly always its whole length stream, goes to
+  // LDS while the header that describes it arrives, the symbol table behind
+  // it: two round trips.  (Each lane reading its fields' words from memory, one
+  // dependent load after another, chunk by chunk, took 13 us for a row group
+  // and 20 us for 956 segments; now 8.7 us and 18.5 us.)
+  const uint32_t rows = sg.row_count;
+  const uint32_t nch  = (rows + FSST_CHUNK_ROWS - 1u) / FSST_CHUNK_ROWS;
+  const uint32_t wv   = tid / WAVE;
+  const uint32_t lane = lane_id();
+  bool ok             = false;
+  uint32_t dict_end = 0, width = 0, symoff = 0, skew = 0;
+  uint32_t b0 = 0, bn = sg.bytes_size < PREP_STAGE ? sg.bytes_size : PREP_STAGE;  // staged: bytes [b0, b0 + bn)
+  __syncthreads();  // the previous segment's use of sm is done
   if (sg.bytes_size >= 16u) {
+    skew     = block_issue<NT>(sm.fields, seg, bn);
     dict_end = su32(seg + 4);
     width    = su32(seg + 8);
     symoff   = su32(seg + 12);
     ok       = dict_end <= sg.bytes_size && symoff < dict_end && width <= 32u;
   }
-  import_symtab(seg, sg.bytes_size, symoff, ok, tab, sm);
+  import_symtab(seg, sg.bytes_size, symoff, ok, tab, sm);  // waits for both
 
-  // chunk bounds: wave w sums chunks w, w + 4, ..., 16 fields per lane
-  const uint32_t rows = sg.row_count;
-  const uint32_t nch  = (rows + FSST_CHUNK_ROWS - 1u) / FSST_CHUNK_ROWS;
-  const uint32_t wv   = tid / WAVE;
-  const uint32_t lane = lane_id();
-  uint32_t carry      = 0;
-  for (uint32_t k0 = 0; k0 < nch; k0 += PREP_THREADS) {
-    const uint32_t cnt = nch - k0 < PREP_THREADS ? nch - k0 : PREP_THREADS;
+  // chunk bounds: wave w sums chunks w, w + NT / WAVE, ..., 16 fields per lane; a
+  // stream that leaves the segment (malformed) is read from memory, bounded
+  const uint64_t stream_end = 16u + ((uint64_t{rows} * width + 7u) >> 3);
+  const bool inside         = ok && width && stream_end <= sg.bytes_size;
+  uint32_t carry            = 0;
+  for (uint32_t k0 = 0; k0 < nch;) {
+    uint32_t cnt = nch - k0 < NT ? nch - k0 : NT;
+    if (inside) {
+      if (k0) {  // the next piece of the stream
+        b0 = 16u + 128u * width * k0;  // 1024 fields take 128 * width bytes
+        bn = stream_end - b0 < PREP_STAGE ? static_cast<uint32_t>(stream_end - b0) : PREP_STAGE;
+        skew = block_stage<NT>(sm.fields, seg + b0, bn);
+        __syncthreads();
+      }
+      if (b0 + bn < stream_end) {  // the chunks that are staged whole
+        const uint32_t whole = (b0 + bn - 16u) / (128u * width) - k0;
+        cnt                  = whole < cnt ? whole : cnt;
+      }
+    }
     if (ok)
-      for (uint32_t k = k0 + wv; k < k0 + cnt; k += PREP_WAVES) {
+      for (uint32_t k = k0 + wv; k < k0 + cnt; k += NT / WAVE) {
         const uint32_t r0 = k * FSST_CHUNK_ROWS;
         const uint32_t r1 = rows - r0 < FSST_CHUNK_ROWS ? rows : r0 + FSST_CHUNK_ROWS;
         const uint32_t f0 = r0 + 16u * lane < r1 ? r0 + 16u * lane : r1;
         const uint32_t f1 = f0 + 16u < r1 ? f0 + 16u : r1;
         bool hg           = false;
-        const uint32_t s  = fields_sum(seg + 16, end, f0, f1, width, &hg);
+        uint32_t s        = 0;
+        if (inside) {
+          uint32_t mx      = 0;
+          const uint64_t p = 8u * (uint64_t{skew} + 16u - b0) + uint64_t{f0} * width;  // modulo 2^64: f0's bit is staged
+          s                = lds_fields_sum(sm.fields, static_cast<uint32_t>(p), f1 - f0, width, &mx);
+          hg = mx >= ROW_HUGE;
+        } else {
+          s = fields_sum(seg + 16, end, f0, f1, width, &hg);
+        }
         const uint32_t tt = __builtin_amdgcn_readlane(wave_incl_sum_u32(s), WAVE - 1);
         const bool any_hg = ballot(hg) != 0;
         if (lane == 0) {
@@ -1350,7 +1412,7 @@ __device__ __forceinline__ void fsst_prep_segment(const FsstSeg sg, uint32_t si,
     __syncthreads();
     const uint32_t v  = (ok && tid < cnt) ? sm.sum[tid] : 0u;
     uint32_t T        = 0;
-    const uint32_t ex = block_excl_scan<PREP_WAVES>(v, sm.wave, &T);
+    const uint32_t ex = block_excl_scan<NT / WAVE>(v, sm.wave, &T);
     if (tid < cnt) {
       const uint32_t k  = k0 + tid;
       const uint32_t r1 = rows - k * FSST_CHUNK_ROWS < FSST_CHUNK_ROWS ? rows : (k + 1u) * FSST_CHUNK_ROWS;
@@ -1374,25 +1436,33 @@ __device__ __forceinline__ void fsst_prep_segment(const FsstSeg sg, uint32_t si,
       dst[1]                = cv.hi;
     }
     carry += T;
-    __syncthreads();  // sum[] and huge[] are read before the next batch refills them
+    k0 += cnt;
+    __syncthreads();  // sum[], huge[] and fields[] are read before the next piece refills them
   }
 }
 
 // ---- chunk decode ----
 
-// Row r's compressed-length field (0 past the chunk's rows); lw: the fields
-// staged in LDS from bit bit0 when they all lie inside the segment (lfast).
-__device__ __forceinline__ uint32_t fsst_field(const uint32_t* lw, uint32_t bit0, bool lfast, const uint8_t* seg,
-                                               const uint8_t* end, uint32_t row_begin, uint32_t width, uint32_t r,
-                                               uint32_t rows)
+// The compressed-length fields of rows r and r + 1 (0 past the chunk's rows);
+// lw: the fields staged in LDS from bit bit0 when they all lie inside the
+// segment (lfast), read without a branch around them.
+__device__ __forceinline__ void fsst_fields2(const uint32_t* lw, uint32_t bit0, bool lfast, const uint8_t* seg,
+                                             const uint8_t* end, uint32_t row_begin, uint32_t width, uint32_t r,
+                                             uint32_t rows, uint32_t& a, uint32_t& b)
 {
-  if (!width || r >= rows) return 0u;
-  return lfast ? lds_bits32(lw, bit0 + r * width, width)
-               : stream_bits32(seg + 16, end, uint64_t{row_begin + r} * width, width);
+  if (lfast) {
+    a = lds_bits32(lw, bit0 + r * width, width);
+    b = lds_bits32(lw, bit0 + (r + 1u) * width, width);
+  } else {
+    a = stream_bits32(seg + 16, end, uint64_t{row_begin + r} * width, width);
+    b = stream_bits32(seg + 16, end, uint64_t{row_begin + r + 1u} * width, width);
+  }
+  a = r < rows ? a : 0u;
+  b = r + 1u < rows ? b : 0u;
 }
 
 // The segment's symbol table and the chunk's length fields on their way to
-// LDS (LDS-direct loads); returns bit0 of fsst_field.
+// LDS (LDS-direct loads); returns bit0 of fsst_fields2.
 __device__ __forceinline__ uint32_t fsst_issue_front(FsstSmem& sm, bool ok, const FsstSymTab* tab, bool lfast,
                                                      const uint8_t* seg, uint32_t row_begin, uint32_t rows,
                                                      uint32_t width)
@@ -1485,8 +1555,8 @@ __device__ __attribute__((noinline)) void fsst_chunk_runs(const uint8_t* seg, ui
   __syncthreads();
   const uint32_t* lw = reinterpret_cast<const uint32_t*>(sm.out);
   const uint32_t r0 = 2u * tid, r1 = r0 + 1u;
-  const uint32_t cl0 = fsst_field(lw, bit0, lfast, seg, end, row_begin, width, r0, rows);
-  const uint32_t cl1 = fsst_field(lw, bit0, lfast, seg, end, row_begin, width, r1, rows);
+  uint32_t cl0, cl1;
+  fsst_fields2(lw, bit0, lfast, seg, end, row_begin, width, r0, rows, cl0, cl1);
   const uint32_t ne0 = cl0 ? 1u : 0u, ne1 = cl1 ? 1u : 0u;  // rows with bytes
   constexpr uint32_t RUN_MAX = FSST_CSTAGE - 15u;            // whatever the run's alignment
   const uint32_t wide        = cl0 > RUN_MAX || cl1 > RUN_MAX ? 1u << 16 : 0u;
@@ -1640,8 +1710,8 @@ __device__ __forceinline__ void fsst_chunk(const FsstChunk ch, const FsstChunkIn
   // rows 2t, 2t + 1 ----
   static_assert(ROWS_PER_THR == 2, "the staged path's row arithmetic");
   const uint32_t* lw = reinterpret_cast<const uint32_t*>(sm.out);
-  const uint32_t cl0 = fsst_field(lw, bit0, lfast, seg, end, ch.row_begin, width, 2u * tid, rows);
-  const uint32_t cl1 = fsst_field(lw, bit0, lfast, seg, end, ch.row_begin, width, 2u * tid + 1u, rows);
+  uint32_t cl0, cl1;
+  fsst_fields2(lw, bit0, lfast, seg, end, ch.row_begin, width, 2u * tid, rows, cl0, cl1);
   const uint32_t ne0 = cl0 ? 1u : 0u, ne1 = cl1 ? 1u : 0u;  // rows with bytes
   uint32_t all;
   const uint32_t pre = block_excl_scan_lds((cl0 + cl1) | (ne0 + ne1) << PK_LEN, sm.wave, &all);

@@ -27,7 +27,6 @@ namespace sdr {
 // 4 KiB of bitpacking or ALP codes, or the ALP-RD left stream plus 4 KiB of
 // its right stream.
 constexpr uint32_t BATCH_BP_STAGE = 4096;
-static_assert(BATCH_PREP_THREADS == PREP_THREADS, "pre-pass workgroup size");
 static_assert(BATCH_WAVES == WAVES_PER_BLOCK, "fixed-width group block");
 
 template <typename T>
@@ -146,9 +145,9 @@ __global__ void k_batch_reset(BatchQueue* q)
   if (blockIdx.x == 0 && threadIdx.x == 0) q->error = 0;
 }
 
-__global__ __launch_bounds__(PREP_THREADS) void k_batch_fsst_prep(const BatchQueue* __restrict__ q)
+__global__ __launch_bounds__(BATCH_PREP_THREADS) void k_batch_fsst_prep(const BatchQueue* __restrict__ q)
 {
-  __shared__ FsstPrepSmem sm;
+  __shared__ FsstPrepSmem<BATCH_PREP_THREADS> sm;
   const uint32_t n = q->n_fsst_segs;
   for (uint32_t i = blockIdx.x; i < n; i += gridDim.x)
     fsst_prep_segment(gload(q->fsst_segs + i), i, q->fsst_chunks, q->fsst_info, q->fsst_tabs + i, sm);

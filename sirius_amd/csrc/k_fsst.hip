@@ -3,6 +3,8 @@
 #include "dec_fsst.hpp"
 #include "sdr_tune.hpp"
 
+#include <cstring>
+
 namespace sdr {
 
 __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_fsst(const FsstChunk* __restrict__ chunks, uint32_t n_chunks,
@@ -25,13 +27,32 @@ __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6)
 // Segment pre-pass: one workgroup per segment (grid-stride), which also clears
 // the look-back status of its chunks (a launch of its own for that, and a copy
 // of the ranges to the device before it, were 10 us of a 76 us call).
-__global__ __launch_bounds__(PREP_THREADS) void k_fsst_prep(const FsstSeg* __restrict__ segs, uint32_t n_segs,
-                                                            FsstChunk* __restrict__ chunks,
+//
+// Up to RANGES_INLINE ranges travel in the kernel arguments; more are read
+// where they are, a device array or pinned memory.
+//
+// Few ranges have the chip to themselves: twice the waves share a segment's
+// chunks (seven segments 10.6 -> 8.7 us).  956 segments fill it with 256-thread
+// workgroups, and larger ones only start later (18.9 -> 22 us).
+constexpr uint32_t RANGES_INLINE = 100;
+struct DevRanges {
+  static constexpr uint32_t THREADS = 256;
+  const FsstSeg* p;
+  __device__ __forceinline__ FsstSeg at(uint32_t i) const { return uniform(gload(p + i)); }
+};
+struct RangesInline {
+  static constexpr uint32_t THREADS = 512;
+  FsstSeg seg[RANGES_INLINE];
+  __device__ __forceinline__ FsstSeg at(uint32_t i) const { return uniform(seg[i]); }
+};
+
+template <class Src>
+__global__ __launch_bounds__(Src::THREADS) void k_fsst_prep(Src src, uint32_t n_segs, FsstChunk* __restrict__ chunks,
                                                             FsstChunkInfo* __restrict__ info,
                                                             FsstSymTab* __restrict__ tabs, FsstState* __restrict__ st,
                                                             FsstResult* __restrict__ result)
 {
-  __shared__ FsstPrepSmem sm;
+  __shared__ FsstPrepSmem<Src::THREADS> sm;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     st->ticket = 0;
     st->error  = 0;
@@ -39,14 +60,16 @@ __global__ __launch_bounds__(PREP_THREADS) void k_fsst_prep(const FsstSeg* __res
     st->result = result;
   }
   for (uint32_t i = blockIdx.x; i < n_segs; i += gridDim.x) {
-    const FsstSeg sg = uniform(gload(segs + i));
-    for (uint32_t k = threadIdx.x; k * FSST_CHUNK_ROWS < sg.row_count; k += PREP_THREADS)
+    const FsstSeg sg = src.at(i);
+    for (uint32_t k = threadIdx.x; k * FSST_CHUNK_ROWS < sg.row_count; k += Src::THREADS)
       gbl(st->status)[sg.first_chunk + k] = 0;
     fsst_prep_segment(sg, i, chunks, info, tabs + i, sm);
   }
 }
 
 // ---- DICT_FSST passes ----
+
+constexpr uint32_t DFSST_PREP_THREADS = 512;  // 66 dictionaries: 256 threads 38 us, 512 24 us
 
 __global__ void k_dfsst_headers(const FsstSeg* __restrict__ segs, uint32_t n, uint32_t* __restrict__ hdr)
 {
@@ -58,12 +81,12 @@ __global__ void k_dfsst_headers(const FsstSeg* __restrict__ segs, uint32_t n, ui
   }
 }
 
-__global__ __launch_bounds__(PREP_THREADS) void k_dfsst_prep(const DictFsstSeg* __restrict__ dseg, uint32_t n,
+__global__ __launch_bounds__(DFSST_PREP_THREADS) void k_dfsst_prep(const DictFsstSeg* __restrict__ dseg, uint32_t n,
                                                              uint32_t* __restrict__ e_byte,
                                                              uint32_t* __restrict__ e_dec,
                                                              FsstSymTab* __restrict__ tabs, uint32_t* __restrict__ out)
 {
-  __shared__ FsstPrepSmem sm;
+  __shared__ FsstPrepSmem<DFSST_PREP_THREADS> sm;
   for (uint32_t j = blockIdx.x; j < n; j += gridDim.x) {
     const DictFsstSeg d = gload(dseg + j);
     dfsst_prep_segment(d, e_byte, e_dec, tabs + d.range, out + 2u * j, sm);
@@ -71,10 +94,12 @@ __global__ __launch_bounds__(PREP_THREADS) void k_dfsst_prep(const DictFsstSeg* 
   }
 }
 
+constexpr uint32_t PREDECODE_THREADS = 256;  // one code of the table per thread
+
 // grid.y: segments; grid.x blocks share a segment's entries
-__global__ __launch_bounds__(PREP_THREADS) void k_dfsst_predecode(const DictFsstSeg* __restrict__ dseg,
-                                                                  const uint32_t* __restrict__ e_byte,
-                                                                  const FsstSymTab* __restrict__ tabs)
+__global__ __launch_bounds__(PREDECODE_THREADS) void k_dfsst_predecode(const DictFsstSeg* __restrict__ dseg,
+                                                                       const uint32_t* __restrict__ e_byte,
+                                                                       const FsstSymTab* __restrict__ tabs)
 {
   __shared__ uint64_t sym[256];
   __shared__ uint8_t len[256];
@@ -133,7 +158,7 @@ hipError_t launch_dfsst_prep(const DictFsstSeg* d_dseg, uint32_t n_dseg, uint32_
                              FsstSymTab* d_tabs, uint32_t* d_out, hipStream_t s)
 {
   if (n_dseg == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_dfsst_prep, dim3(n_dseg < 4096u ? n_dseg : 4096u), dim3(PREP_THREADS), 0, s, d_dseg, n_dseg,
+  hipLaunchKernelGGL(k_dfsst_prep, dim3(n_dseg < 4096u ? n_dseg : 4096u), dim3(DFSST_PREP_THREADS), 0, s, d_dseg, n_dseg,
                      d_e_byte, d_e_dec, d_tabs, d_out);
   return hipGetLastError();
 }
@@ -142,7 +167,7 @@ hipError_t launch_dfsst_predecode(const DictFsstSeg* d_dseg, uint32_t n_dseg, co
                                   const FsstSymTab* d_tabs, hipStream_t s)
 {
   if (n_dseg == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_dfsst_predecode, dim3(8, n_dseg), dim3(PREP_THREADS), 0, s, d_dseg, d_e_byte, d_tabs);
+  hipLaunchKernelGGL(k_dfsst_predecode, dim3(8, n_dseg), dim3(PREDECODE_THREADS), 0, s, d_dseg, d_e_byte, d_tabs);
   return hipGetLastError();
 }
 
@@ -159,11 +184,19 @@ hipError_t launch_dfsst_nulls(const FsstSeg* d_segs, uint32_t n_ranges, const Di
 }
 
 hipError_t launch_fsst_prep(const FsstSeg* segs, uint32_t n_segs, FsstChunk* d_chunks, FsstChunkInfo* d_info,
-                            FsstSymTab* d_tabs, FsstState* d_state, FsstResult* result, hipStream_t s)
+                            FsstSymTab* d_tabs, FsstState* d_state, FsstResult* result, hipStream_t s, bool host)
 {
   if (n_segs == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fsst_prep, dim3(n_segs < 4096u ? n_segs : 4096u), dim3(PREP_THREADS), 0, s, segs, n_segs,
-                     d_chunks, d_info, d_tabs, d_state, result);
+  const dim3 grid(n_segs < 4096u ? n_segs : 4096u);
+  if (host && n_segs <= RANGES_INLINE) {
+    RangesInline ri{};
+    std::memcpy(ri.seg, segs, size_t{n_segs} * sizeof(FsstSeg));
+    hipLaunchKernelGGL((k_fsst_prep<RangesInline>), grid, dim3(RangesInline::THREADS), 0, s, ri, n_segs, d_chunks, d_info, d_tabs, d_state,
+                       result);
+  } else {
+    hipLaunchKernelGGL((k_fsst_prep<DevRanges>), grid, dim3(DevRanges::THREADS), 0, s, DevRanges{segs}, n_segs, d_chunks, d_info, d_tabs,
+                       d_state, result);
+  }
   return hipGetLastError();
 }
 

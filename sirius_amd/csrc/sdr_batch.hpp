@@ -100,7 +100,7 @@ struct BatchQueue {
 // recorded launch serves every batch.
 constexpr uint32_t BATCH_RESET_GRID    = 64;
 constexpr uint32_t BATCH_PREP_GRID     = 512;
-constexpr uint32_t BATCH_PREP_THREADS  = 256;  // the FSST pre-pass workgroup
+constexpr uint32_t BATCH_PREP_THREADS  = 512;  // the FSST pre-pass workgroup
 constexpr uint32_t BATCH_WAVES         = 4;    // wavefronts of a fixed-width group block
 constexpr uint32_t BATCH_XCDS          = 8;    // XCDs workgroups are dispatched to round-robin;
                                                // fixed-width group grids are a multiple

@@ -127,10 +127,10 @@ constexpr uint32_t FSST_STATE_WORDS = 3;  // 8-byte words before status
 
 // Segment pre-pass over n_segs ranges: writes the chunk list, the chunks'
 // FsstChunkInfo and the segments' symbol tables, and sets up the state (its
-// result may be null).  The ranges may be pinned host memory: each is read
-// once, by the block that handles it.
+// result may be null).  With `host` the ranges are pinned host memory: a few
+// travel in the kernel arguments, each of many is read by its block.
 hipError_t launch_fsst_prep(const FsstSeg* segs, uint32_t n_segs, FsstChunk* d_chunks, FsstChunkInfo* d_info,
-                            FsstSymTab* d_tabs, FsstState* d_state, FsstResult* result, hipStream_t s);
+                            FsstSymTab* d_tabs, FsstState* d_state, FsstResult* result, hipStream_t s, bool host);
 hipError_t launch_fsst(const FsstChunk* d_chunks, uint32_t first, uint32_t n, uint32_t n_chunks_total,
                        const FsstChunkInfo* d_info, const FsstSymTab* d_tabs, FsstState* d_state,
                        int32_t* d_offsets, uint8_t* d_chars, uint64_t chars_cap, uint32_t total_rows,

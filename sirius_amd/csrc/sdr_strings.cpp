@@ -344,7 +344,7 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
     dc.release(s);
     release();
   };
-  e = launch_fsst_prep(prep_segs, n_ranges, d_chunks, d_info, d_tabs, d_state, result, s);
+  e = launch_fsst_prep(prep_segs, n_ranges, d_chunks, d_info, d_tabs, d_state, result, s, prep_segs != d_segs);
   if (e == hipSuccess) {
     if (mode == SDR_LAUNCH_PER_SEGMENT) {
       for (uint32_t i = 0; e == hipSuccess && i < n_ranges; ++i)
