@@ -247,6 +247,8 @@ struct FsstSmem {
   uint32_t wave[2 * FSST_WAVES];
   uint32_t part[2 * FSST_WAVES];
   uint64_t base;
+  __device__ __forceinline__ uint32_t* plain_part() { return comp; }
+  __device__ __forceinline__ uint64_t* plain_sum() { return sym; }
 };
 
 // Walk the n compressed bytes of one row with DuckDB's serial semantics:
@@ -655,7 +657,8 @@ __device__ __forceinline__ void fsst_group_emit(const FsstGroup& gr, FsstSmem& s
 }
 
 // Clear the window's bytes [0, n) and the words a last symbol may reach.
-__device__ __forceinline__ void window_clear(FsstSmem& sm, uint32_t n)
+template <class SM>
+__device__ __forceinline__ void window_clear(SM& sm, uint32_t n)
 {
   for (uint32_t i = threadIdx.x * 8u; i < n + 12u; i += FSST_THREADS * 8u)
     *reinterpret_cast<uint64_t*>(&sm.out[i]) = 0u;
@@ -676,8 +679,8 @@ __device__ __forceinline__ u32x4 funnel16(const u32x4& a, const u32x4& b, uint32
 // (16-byte aligned) starts at window byte 16 i - skew, so its bytes come from
 // the aligned window blocks i - 1 and i at an offset that is the same for the
 // whole chunk.
-template <uint32_t WORD>
-__device__ __forceinline__ void window_store_blocks(const FsstSmem& sm, uintptr_t dst, uint32_t i0, uint32_t i1,
+template <uint32_t WORD, class SM>
+__device__ __forceinline__ void window_store_blocks(const SM& sm, uintptr_t dst, uint32_t i0, uint32_t i1,
                                                     uint32_t byte)
 {
   const u32x4* w = reinterpret_cast<const u32x4*>(sm.out);
@@ -691,7 +694,8 @@ __device__ __forceinline__ void window_store_blocks(const FsstSmem& sm, uintptr_
 
 // The window's n bytes to global address g: 16-byte stores, single bytes
 // where the first and last 16-byte blocks are shared with other chunks.
-__device__ __forceinline__ void window_store(const FsstSmem& sm, uintptr_t g, uint32_t n)
+template <class SM>
+__device__ __forceinline__ void window_store(const SM& sm, uintptr_t g, uint32_t n)
 {
   const uint32_t skew = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(g & 15u)));
   const uintptr_t dst = g - skew;
@@ -921,7 +925,7 @@ __device__ __forceinline__ void plain_prep_segment(const FsstSeg& sg, FsstChunkI
     ok       = dict_end <= sg.bytes_size;
   }
   const uint32_t flags = (dict ? FI_DICT | (width & FI_WIDTH) : FI_UNC) | (ok ? FI_OK : 0u);
-  for (uint32_t k = threadIdx.x; k * FSST_CHUNK_ROWS < sg.row_count; k += NT) {
+  for (uint32_t k = threadIdx.x; uint64_t{k} * sg.chunk_rows < sg.row_count; k += NT) {
     FsstChunkInfo ci;
     ci.bytes      = seg;
     ci.c_lo       = ibo;
@@ -993,160 +997,382 @@ __device__ __forceinline__ void fsst_row_offsets(uint32_t c, uint32_t n_chunks, 
     gbl(offsets)[total_rows] = static_cast<int32_t>(static_cast<uint32_t>(base + T));
 }
 
-// One row's bytes into the window over chunk output bytes [w0, w0 +
-// FSST_WINDOW) (cleared): source bytes [src, src + len) are output bytes
-// [d, d + len); those at or past `end` are zeros.  A word of the window at a
-// time, four in flight: its four bytes come from two aligned words of the
-// source, of which only those that hold the row's bytes are read, and are
-// ORed in, since a row's first and last word are shared with its neighbours.
-__device__ __forceinline__ void plain_copy_row(FsstSmem& sm, const uint8_t* src, uint32_t len, const uint8_t* end,
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
+
+// The w-bit field (1 <= w <= 32) at bit `bit` from the word p, of a stream that
+// holds all of it.
+__device__ __forceinline__ uint32_t bits32_inside(gptr<const uint32_t> p, uint32_t bit, uint32_t w)
+{
+  const uint32_t k = bit >> 5, off = bit & 31u;
+  const uint32_t lo = p[k], hi = p[k + (off + w > 32u ? 1u : 0u)];
+  return __builtin_amdgcn_ubfe(__builtin_amdgcn_alignbit(hi, lo, off), 0u, w);
+}
+
+// A row's bytes into the window over chunk output bytes [w0, w0 + FSST_WINDOW)
+// (cleared): bytes [src, src + len) of `seg` are output bytes [d, d + len);
+// those at or past `size` (not 0) are zeros.  Sixteen bytes a load, funnelled
+// into words of the window and ORed in, since a row's first and last word are
+// shared with its neighbours.
+template <class SM>
+__device__ __forceinline__ void plain_copy_row(SM& sm, const uint8_t* seg, uint32_t size, uint32_t src, uint32_t len,
                                                uint32_t d, uint32_t w0)
 {
-  const uint64_t left = src < end ? static_cast<uint64_t>(end - src) : 0u;
-  const uint32_t have = len < left ? len : static_cast<uint32_t>(left);
-  const uint32_t j0   = d < w0 ? w0 - d : 0u;
-  const uint32_t lim  = w0 + FSST_WINDOW > d ? w0 + FSST_WINDOW - d : 0u;
-  const uint32_t j1   = have < lim ? have : lim;
+  const uint32_t skew          = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(seg) & 3u);
+  const gptr<const uint32_t> w = gbl(reinterpret_cast<const uint32_t*>(seg - skew));
+  const uint32_t w_last        = static_cast<uint32_t>((uint64_t{skew} + size - 1u) >> 2);  // the last that may be read
+  const uint32_t left          = src < size ? size - src : 0u;
+  const uint32_t have          = len < left ? len : left;
+  const uint32_t j0            = d < w0 ? w0 - d : 0u;
+  const uint32_t lim           = w0 + FSST_WINDOW > d ? w0 + FSST_WINDOW - d : 0u;
+  const uint32_t j1            = have < lim ? have : lim;
   if (j0 >= j1) return;
-  const uint32_t p      = d + j0 - w0;  // first window byte
-  const uint32_t sh     = p & 3u;
-  const uint32_t nb     = sh + (j1 - j0);  // bytes from the first window word's start
-  const uintptr_t a     = reinterpret_cast<uintptr_t>(src) + j0 - sh;
-  const uint32_t ph     = static_cast<uint32_t>(a & 3u);
-  const gptr<const uint32_t> w = gbl(reinterpret_cast<const uint32_t*>(a - ph));
-  // source word i holds bytes 4i - ph .. 4i - ph + 3 from `a`; the row's are [sh, nb)
-  auto load = [&](uint32_t i) -> uint32_t { return 4u * i + 3u >= sh + ph && 4u * i < nb + ph ? w[i] : 0u; };
-  uint32_t* o    = reinterpret_cast<uint32_t*>(sm.out + (p - sh));
-  uint32_t carry = load(0);
+  // Source words k0, k0 + 1, ...: k0 holds the first byte.  Words k0 + k - 1 and
+  // k0 + k make window word o + k, from byte ph on; f: the first pair makes none
+  // of the row's.
+  const uint32_t p  = d + j0 - w0;  // first window byte
+  const uint32_t x  = src + j0;
+  const uint32_t x3 = (x & 3u) + skew;
+  const uint32_t sh = p & 3u;
+  const uint32_t nb = sh + (j1 - j0);  // bytes from the first window word's start
+  const uint32_t ph = x3 - sh;         // the funnel takes it modulo 4
+  const uint32_t f  = (x3 & 3u) >= sh ? 1u : 0u;
+  const uint32_t o  = (p >> 2) - f;
+  const uint32_t k0 = (x >> 2) + (x3 >> 2);
+  const uint32_t nw = ((nb + 3u) >> 2) + f;
+  uint32_t carry    = 0;
 #pragma unroll 1
-  for (uint32_t k = 0; 4u * k < nb; k += 4) {
-    uint32_t n[4];
+  for (uint32_t k = 0; k < nw; k += 4) {
+    u32x4 n;
+    if (ballot(k0 + k + 3u > w_last) == 0) {
+      n = *(gptr<const u32x4_a4>)(w + k0 + k);
+    } else {
 #pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) n[i] = load(k + i + 1u);
+      for (uint32_t j = 0; j < 4; ++j) n[j] = w[k0 + k + j < w_last ? k0 + k + j : w_last];
+    }
 #pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-      const uint32_t at = 4u * (k + i);
-      uint32_t v        = __builtin_amdgcn_alignbyte(n[i], carry, ph);
-      carry             = n[i];
+    for (uint32_t j = 0; j < 4; ++j) {
+      const uint32_t at = 4u * (k + j - f);  // wraps where f drops the first
+      uint32_t v        = __builtin_amdgcn_alignbyte(n[j], carry, ph);
+      carry             = n[j];
       if (at < nb) {
         if (at == 0) v &= ~0u << (8u * sh);
         if (nb - at < 4u) v &= (1u << (8u * (nb - at))) - 1u;
-        __hip_atomic_fetch_or(o + k + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_or(reinterpret_cast<uint32_t*>(sm.out) + (o + k + j), v, __ATOMIC_RELAXED,
+                              __HIP_MEMORY_SCOPE_WORKGROUP);
       }
     }
   }
 }
 
+// plain_copy_row for B rows of which each lies whole in the window, which begins
+// with the chunk's output, and in the segment: row i's bytes [src[i], src[i] +
+// len[i]) are window bytes [d[i], d[i] + len[i]).  The copy costs instructions
+// as much as loads, so what is not needed then is left out, and the first
+// word's mask is applied to the source, the last word's made once.  Where a
+// lane needs no further words it loads its row's first again (a row without
+// bytes, the segment's): no branch holds a load back.
+template <uint32_t B, class SM>
+__device__ __forceinline__ void plain_copy_whole(SM& sm, const uint8_t* seg, uint32_t size, const uint32_t* src,
+                                                 const uint32_t* len, const uint32_t* d)
+{
+  const uint32_t skew          = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(seg) & 3u);
+  const gptr<const uint8_t> w  = gbl(seg - skew);
+  const uint32_t w_last        = (skew + size - 1u) >> 2;  // the last word that may be read
+  // Source words k0 + k: k0 holds the row's first byte.  Words k0 + k - 1 and
+  // k0 + k make, from byte ph on, window word o + k; the first pair makes none of
+  // the row's if `skip`, the one with 4 k = `last` its last, of which `tail` are
+  // its bytes.
+  uint32_t k0[B], ph[B], o[B], last[B], tail[B], carry[B] = {}, most = 0;
+  bool skip[B];
+#pragma unroll
+  for (uint32_t i = 0; i < B; ++i) {
+    const uint32_t sh = d[i] & 3u;
+    const uint32_t x  = src[i] + skew;
+    skip[i]           = (x & 3u) >= sh;
+    const uint32_t f4 = skip[i] ? 4u : 0u;
+    const uint32_t e  = sh + len[i] + f4;  // where the row ends, from word o on
+    ph[i]             = x - sh;            // the funnel takes it modulo 4
+    o[i]              = (d[i] >> 2) - (f4 >> 2);
+    k0[i]             = len[i] ? x >> 2 : 0u;
+    last[i]           = (e - 1u) & ~3u;
+    tail[i]           = ~0u >> (8u * ((0u - e) & 3u));
+    if (len[i] == 0u) {  // no word of the window
+      skip[i] = true;
+      last[i] = 0u;
+    }
+    most = last[i] > most ? last[i] : most;
+  }
+#pragma unroll 1
+  for (uint32_t k = 0;; k += 4) {
+    u32x4 n[B];
+    uint32_t at[B];
+    bool past = false;
+#pragma unroll
+    for (uint32_t i = 0; i < B; ++i) {
+      at[i] = k0[i] + (4u * k <= last[i] ? k : 0u);
+      past  = past || at[i] + 3u > w_last;
+    }
+    if (ballot(past) == 0) {
+#pragma unroll
+      for (uint32_t i = 0; i < B; ++i) n[i] = *(gptr<const u32x4_a4>)(w + 4u * at[i]);
+    } else {
+#pragma unroll
+      for (uint32_t i = 0; i < B; ++i)
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j)
+          n[i][j] = *(gptr<const uint32_t>)(w + 4u * (at[i] + j < w_last ? at[i] + j : w_last));
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < B; ++i) {
+      if (k == 0) n[i][0] &= ~0u << (8u * ((src[i] + skew) & 3u));  // uniform
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j) {
+        const uint32_t t = 4u * (k + j);
+        const uint32_t v = __builtin_amdgcn_alignbyte(n[i][j], carry[i], ph[i]) & (t == last[i] ? tail[i] : ~0u);
+        carry[i]         = n[i][j];
+        if (t <= last[i] && !(j == 0 && k == 0 && skip[i]))
+          __hip_atomic_fetch_or(reinterpret_cast<uint32_t*>(sm.out) + (o[i] + k + j), v, __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+    }
+    if (4u * (k + 4u) > most) break;
+  }
+}
+
+// LDS of a workgroup that decodes no FSST chunk.
+struct PlainSmem {
+  __attribute__((aligned(16))) uint8_t out[FSST_WINDOW + 48];
+  uint32_t part[WAVE];
+  uint64_t sum[FSST_WAVES];
+  uint64_t base;
+  __device__ __forceinline__ uint32_t* plain_part() { return part; }
+  __device__ __forceinline__ uint64_t* plain_sum() { return sum; }
+};
+
+struct PlainArgs {
+  const uint8_t* seg;
+  uint32_t bytes_size, dict_end, flags, ibo, ibc, row_begin, rows, col_row, c, n_chunks;
+  FsstState* st;
+  int32_t* offsets;
+  uint8_t* chars;
+  uint64_t chars_cap;
+  uint32_t total_rows, spin_limit;
+};
+
 // Decode chunk c of a valid DICTIONARY, UNCOMPRESSED or DICT_FSST segment: per-
 // row lengths (dictionary.cu:84-108, uncompressed.cu:56-81), the chunk's
 // look-back for its chars offset, offsets, and the bytes (dictionary.cu:
-// 117-140, uncompressed.cu:88-120).  Every thread must call it.  A called
-// function with scalar arguments, so that the FSST path keeps its registers.
+// 117-140, uncompressed.cu:88-120).  Every thread must call it.
 //
-// Bound by latency: a row's length is two dependent loads away, its bytes a
-// third.  Thread t owns rows 2t and 2t + 1, whose loads overlap, and each row
-// is copied a word at a time into the LDS window that the FSST path fills (a
-// byte at a time into 8 KiB pieces, with flat accesses to LDS, took 180 us for
-// 8 Mi label rows, 128 us for 2 M rows of 27 chars; now 119 us and 57 us).
-__device__ __attribute__((noinline)) void plain_chunk(const uint8_t* seg, uint32_t bytes_size, uint32_t dict_end,
-                                                     uint32_t flags, uint32_t ibo, uint32_t ibc, uint32_t row_begin,
-                                                     uint32_t rows, uint32_t col_row, uint32_t c, uint32_t n_chunks,
-                                                     FsstState* __restrict__ st, int32_t* __restrict__ offsets,
-                                                     uint8_t* __restrict__ chars, uint64_t chars_cap,
-                                                     uint32_t total_rows, uint32_t spin_limit, LdsPtr<FsstSmem> smp)
+// Bound by latency and instructions alike: a chunk takes a ticket, its
+// descriptors, the rows' indices, their entries and bytes, and the look-back,
+// each a round trip to memory that the next waits for.  So a thread owns RPT
+// rows, 512 apart (offsets are then stored whole lines at a time, and a chunk's
+// output leaves in row order however few rows a window holds), and its loads of
+// one kind are in flight together.  8 Mi label rows 119 -> 65 us, 2 M rows of 27
+// chars 57 -> 44 us (with the kernels' own register budgets, see k_plain).
+template <uint32_t RPT, class SM>
+__device__ __forceinline__ void plain_chunk(const PlainArgs& args, SM& sm)
 {
-  FsstSmem& sm        = *(FsstSmem*)smp;
+  const PlainArgs a   = uniform(args);
+  const uint32_t bytes_size = a.bytes_size, dict_end = a.dict_end, flags = a.flags, ibo = a.ibo, ibc = a.ibc;
+  const uint32_t row_begin = a.row_begin, rows = a.rows, col_row = a.col_row, c = a.c, n_chunks = a.n_chunks;
+  FsstState* const st = a.st;
+  const uint64_t chars_cap  = a.chars_cap;
+  const uint32_t spin_limit = a.spin_limit;
+  const uint8_t* seg        = a.seg;
   const uint32_t tid  = threadIdx.x;
-  const uint8_t* end  = seg + bytes_size;
   const bool dict     = flags & FI_DICT;
   const bool dfsst    = flags & FI_DFSST;
-  const uint32_t w    = flags & FI_WIDTH;
-  DictFsstSeg dd{};
+  uint32_t w          = flags & FI_WIDTH;
+  const uint8_t* bits = seg + 20;  // selection values or indices
+  const uint8_t* end  = seg + bytes_size;
+  const uint8_t* ent  = seg + (dict ? uint64_t{ibo} : 4ull);  // entry k is between words k - 1 and k
+  uint32_t n_ent      = dict ? ibc : 1u << 30;  // past every row of an UNCOMPRESSED segment
+  uint32_t size       = bytes_size;  // of the bytes the rows copy from
+  bool implied        = !dict;       // row r is entry r + 1
   if (dfsst) {  // seg is the segment's descriptor; rows copy from its entries
-    dd  = uniform(gload(reinterpret_cast<const DictFsstSeg*>(seg)));
-    seg = dd.src;
-    end = dd.src + dd.src_size;
+    const DictFsstSeg dd = uniform(gload(reinterpret_cast<const DictFsstSeg*>(seg)));
+    w       = dd.diw;
+    bits    = dd.bytes + dd.off_didx;
+    end     = dd.bytes + dd.bytes_size;
+    seg     = dd.src;
+    size    = dd.src_size < ~0u ? static_cast<uint32_t>(dd.src_size) : ~0u;
+    ent     = reinterpret_cast<const uint8_t*>(dd.e + 1);  // entry k is between e[k] and e[k + 1]
+    n_ent   = dd.dict_count;
+    implied = dd.mode == 2u;
   }
-  // the rows' entries [e0, e1): two loads, both rows' in flight together
-  uint32_t idx[ROWS_PER_THR], e0[ROWS_PER_THR] = {}, e1[ROWS_PER_THR] = {};
+  uint32_t idx[RPT];
+  if (implied) {
 #pragma unroll
-  for (uint32_t i = 0; i < ROWS_PER_THR; ++i) {
-    const uint32_t r = ROWS_PER_THR * tid + i, sr = row_begin + r;
-    idx[i]           = 0;
-    if (r < rows) {
-      if (dfsst) idx[i] = dfsst_index(dd, sr);
-      else if (dict) idx[i] = stream_bits32(seg + 20, end, uint64_t{sr} * w, w);
-      else idx[i] = sr + 1u;
+    for (uint32_t i = 0; i < RPT; ++i) idx[i] = row_begin + FSST_THREADS * i + tid + 1u;
+  } else if (w && bits + ((uint64_t{row_begin + rows} * w + 7u) >> 3) <= end) {
+    const uint64_t bit0          = uint64_t{row_begin} * w;
+    const uintptr_t at           = reinterpret_cast<uintptr_t>(bits) + (bit0 >> 3);
+    const uint32_t skew          = 8u * static_cast<uint32_t>(at & 3u) + static_cast<uint32_t>(bit0 & 7u);
+    const gptr<const uint32_t> p = gbl(reinterpret_cast<const uint32_t*>(at & ~uintptr_t{3}));
+#pragma unroll
+    for (uint32_t i = 0; i < RPT; ++i) {
+      const uint32_t r = FSST_THREADS * i + tid;
+      idx[i]           = bits32_inside(p, skew + (r < rows ? r : 0u) * w, w);
+    }
+  } else {
+#pragma unroll
+    for (uint32_t i = 0; i < RPT; ++i) {
+      const uint32_t r = FSST_THREADS * i + tid;
+      idx[i]           = r < rows ? stream_bits32(bits, end, uint64_t{row_begin + r} * w, w) : 0u;
     }
   }
+  uint32_t e0[RPT] = {}, e1[RPT] = {};
+  if (n_ent > 1u) {
+    uint32_t k[RPT];
 #pragma unroll
-  for (uint32_t i = 0; i < ROWS_PER_THR; ++i) {
-    const uint32_t k = idx[i];
-    if (dfsst) {
-      if (k != 0u && k < dd.dict_count) {
-        e0[i] = gbl(dd.e)[k];
-        e1[i] = gbl(dd.e)[k + 1u];
+    for (uint32_t i = 0; i < RPT; ++i)
+      k[i] = FSST_THREADS * i + tid < rows && idx[i] < n_ent && idx[i] ? idx[i] - 1u : 0u;
+    if ((reinterpret_cast<uintptr_t>(ent) & 3u) == 0 && n_ent <= 1u << 30) {  // uniform; offsets of 32 bits
+#pragma unroll
+      for (uint32_t i = 0; i < RPT; ++i) {
+        const u32x2_a4 e = *(gptr<const u32x2_a4>)(gbl(ent) + 4u * k[i]);
+        e0[i]            = e[0];
+        e1[i]            = e[1];
       }
-    } else if (dict) {
-      if (k != 0u && k < ibc) {
-        e1[i] = ld_u32_any(seg + ibo + 4ull * k);
-        e0[i] = ld_u32_any(seg + ibo + 4ull * (k - 1u));
+    } else {
+#pragma unroll
+      for (uint32_t i = 0; i < RPT; ++i) {
+        e0[i] = ld_u32_any(ent + 4ull * k[i]);
+        e1[i] = ld_u32_any(ent + 4ull * k[i] + 4u);
       }
-    } else if (k) {
-      const int32_t v1 = static_cast<int32_t>(ld_u32_any(seg + 8 + 4ull * (k - 1u)));
-      const int32_t v0 = k > 1u ? static_cast<int32_t>(ld_u32_any(seg + 8 + 4ull * (k - 2u))) : 0;
-      e1[i] = v1 < 0 ? 0u - static_cast<uint32_t>(v1) : static_cast<uint32_t>(v1);
+    }
+  }
+  uint32_t len[RPT], src[RPT], out[RPT];
+  uint32_t big = 0;
+  bool clip    = size > ~0u - 8u;  // the rows' bytes may end past the source's, or wrap
+#pragma unroll
+  for (uint32_t i = 0; i < RPT; ++i) {
+    const uint32_t r = FSST_THREADS * i + tid;
+    if (flags & FI_UNC) {  // |v|: the sign is a marker; word -1 is not an offset
+      const int32_t v0 = row_begin + r ? static_cast<int32_t>(e0[i]) : 0, v1 = static_cast<int32_t>(e1[i]);
       e0[i] = v0 < 0 ? 0u - static_cast<uint32_t>(v0) : static_cast<uint32_t>(v0);
+      e1[i] = v1 < 0 ? 0u - static_cast<uint32_t>(v1) : static_cast<uint32_t>(v1);
     }
-  }
-  uint32_t len[ROWS_PER_THR], src[ROWS_PER_THR];
-#pragma unroll
-  for (uint32_t i = 0; i < ROWS_PER_THR; ++i) {
     // a DICT_FSST segment's entries are front to back, the others' back to
     // front; a row whose end passes dict_end or falls below its start is empty
-    const bool sound = e1[i] >= e0[i] && (dfsst || e1[i] <= dict_end);
+    const bool sound = r < rows && idx[i] && idx[i] < n_ent && e1[i] >= e0[i] && (dfsst || e1[i] <= dict_end);
     len[i]           = sound ? e1[i] - e0[i] : 0u;
-    src[i]           = dfsst ? e0[i] : dict_end - e1[i];
+    src[i]           = !sound ? 0u : dfsst ? e0[i] : dict_end - e1[i];
+    big |= len[i] >> 18;
+    clip = clip || uint64_t{src[i]} + len[i] > size;
   }
-  // 64-bit prefixes as two scans of 16-bit halves: the rows are bounded by
-  // the segment, but a chunk of long rows can pass 2^31 chars
-  static_assert(ROWS_PER_THR == 2, "row arithmetic");
-  uint32_t plo, phi, tlo, thi;
-  block_excl_scan2((len[0] & 0xFFFFu) + (len[1] & 0xFFFFu), (len[0] >> 16) + (len[1] >> 16), sm.wave, plo, phi, tlo,
-                   thi);
-  const uint64_t T64 = tlo + (uint64_t{thi} << 16);
-  // publish a saturated total then, so the column reports overflow
+  // Output positions modulo 2^32: each wave's rows of step i, behind the waves
+  // and steps before them.  2^12 rows of less than 2^18 bytes can not overflow;
+  // a chunk with a longer one adds its total up in 64 bits as well.
+  uint32_t* const part = sm.plain_part();  // [i][wave]
+  uint64_t* const sum  = sm.plain_sum();   // [wave]
+  const uint32_t wv    = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(tid / WAVE)));
+  uint64_t wave_sum    = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < RPT; ++i) {
+    out[i] = wave_incl_sum_u32(len[i]);
+    if (lane_id() == WAVE - 1u) part[FSST_WAVES * i + wv] = out[i];
+    wave_sum += static_cast<uint32_t>(__builtin_amdgcn_readlane(out[i], WAVE - 1));
+    out[i] -= len[i];
+  }
+  if (ballot(big != 0u)) {
+    wave_sum = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < RPT; ++i) wave_sum += len[i];
+    wave_sum = readlane_u64(wave_incl_sum_u64(wave_sum), WAVE - 1) | 1ull << 63;
+  }
+  if (ballot(clip)) wave_sum |= 1ull << 62;
+  if (lane_id() == 0u) sum[wv] = wave_sum;
+  __syncthreads();
+  static_assert(FSST_WAVES * RPT <= WAVE, "a lane per step and wave");
+  const uint32_t mine = lane_id() < FSST_WAVES * RPT ? part[lane_id()] : 0u;
+  const uint32_t incl = wave_incl_sum_u32(mine);
+#pragma unroll
+  for (uint32_t i = 0; i < RPT; ++i) out[i] += __builtin_amdgcn_readlane(incl - mine, FSST_WAVES * i + wv);
+  uint64_t T64 = static_cast<uint32_t>(__builtin_amdgcn_readlane(incl, WAVE - 1));
+  const uint32_t marks = static_cast<uint32_t>(sum[lane_id() % FSST_WAVES] >> 62);
+  if (ballot(marks & 2u)) {  // the same in every wave
+    T64 = 0;
+    for (uint32_t v = 0; v < FSST_WAVES; ++v) T64 += sum[v] & ~(3ull << 62);
+  }
+  // publish a saturated total past 2^31, so the column reports overflow
   const uint64_t Tp = T64 > 0x7FFFFFFFull ? 0x80000000ull : T64;
   const uint32_t T  = static_cast<uint32_t>(Tp);
-  const uint32_t o0 = plo + (phi << 16), o1 = o0 + len[0];
   fsst_lookback_publish(c, Tp, st, spin_limit);
+  auto store_offsets = [&](uint64_t base) {
+    const gptr<int32_t> off = gbl(a.offsets) + col_row;
+#pragma unroll
+    for (uint32_t i = 0; i < RPT; ++i) {
+      const uint32_t r = FSST_THREADS * i + tid;
+      if (r < rows) off[r] = static_cast<int32_t>(static_cast<uint32_t>(base) + out[i]);
+    }
+    if (c == n_chunks - 1u && tid == 0)
+      gbl(a.offsets)[a.total_rows] = static_cast<int32_t>(static_cast<uint32_t>(base + Tp));
+  };
   if (Tp != T64) {  // nothing but the offsets can be written
-    const uint64_t base = fsst_lookback_wait(c, n_chunks, Tp, st, spin_limit, sm);
-    fsst_row_offsets(c, n_chunks, col_row, rows, Tp, base, o0, o1, offsets, total_rows);
+    store_offsets(fsst_lookback_wait(c, n_chunks, Tp, st, spin_limit, sm));
     return;
   }
-  uint64_t base = 0;
-#pragma unroll 1
-  for (uint32_t w0 = 0;;) {
-    const uint32_t nw = T - w0 < FSST_WINDOW ? T - w0 : FSST_WINDOW;
-    window_clear(sm, nw);
+  // Rows are copied B at a time, the arrays turned by B after each: one copy of
+  // the code, and only B rows' state in registers.
+  constexpr uint32_t B = 2;
+  auto turn = [&](uint32_t by) {
+    if (RPT == by) return;
+#pragma unroll
+    for (uint32_t j = 0; j < by; ++j) {
+      const uint32_t s0 = src[0], l0 = len[0], o0 = out[0];
+#pragma unroll
+      for (uint32_t i = 0; i + 1u < RPT; ++i) {
+        src[i] = src[i + 1u];
+        len[i] = len[i + 1u];
+        out[i] = out[i + 1u];
+      }
+      src[RPT - 1u] = s0;
+      len[RPT - 1u] = l0;
+      out[RPT - 1u] = o0;
+    }
+  };
+  if (T <= FSST_WINDOW && size && ballot(marks & 1u) == 0) {
+    window_clear(sm, T);
     __syncthreads();
 #pragma unroll 1
-    for (uint32_t i = 0; i < ROWS_PER_THR; ++i)
-      plain_copy_row(sm, seg + (i ? src[1] : src[0]), i ? len[1] : len[0], end, i ? o1 : o0, w0);
-    if (w0) {
-      __syncthreads();
-    } else {
-      base = fsst_lookback_wait(c, n_chunks, Tp, st, spin_limit, sm);  // synchronises the workgroup
-      fsst_row_offsets(c, n_chunks, col_row, rows, Tp, base, o0, o1, offsets, total_rows);
+    for (uint32_t i = 0; i < RPT; i += B) {
+      plain_copy_whole<B>(sm, seg, size, src, len, out);
+      turn(B);
     }
-    const uint64_t at = base + w0;
-    if (at >= chars_cap) return;
-    window_store(sm, reinterpret_cast<uintptr_t>(chars) + at,
-                 at + nw <= chars_cap ? nw : static_cast<uint32_t>(chars_cap - at));
-    w0 += nw;
-    if (w0 >= T) return;
-    __syncthreads();  // the stores have read the window
+    const uint64_t at = fsst_lookback_wait(c, n_chunks, Tp, st, spin_limit, sm);  // synchronises the workgroup
+    store_offsets(at);
+    if (at < chars_cap)
+      window_store(sm, reinterpret_cast<uintptr_t>(a.chars) + at,
+                   at + T <= chars_cap ? T : static_cast<uint32_t>(chars_cap - at));
+    return;
+  }
+  // A window or more for each step of 512 rows, output bytes [w0, hi)
+  const uint64_t base = fsst_lookback_wait(c, n_chunks, Tp, st, spin_limit, sm);
+  store_offsets(base);
+  uint32_t w0 = 0;
+#pragma unroll 1
+  for (uint32_t i = 0; i < RPT; ++i) {
+    const uint32_t hi =
+      i + 1u < RPT ? static_cast<uint32_t>(__builtin_amdgcn_readlane(incl - mine, FSST_WAVES * (i + 1u))) : T;
+    while (w0 < hi) {
+      const uint32_t nw = hi - w0 < FSST_WINDOW ? hi - w0 : FSST_WINDOW;
+      window_clear(sm, nw);
+      __syncthreads();
+      __asm__ volatile("" : "+v"(src[0]), "+v"(len[0]), "+v"(out[0]));  // keep no more of the row between windows
+      if (size) plain_copy_row(sm, seg, size, src[0], len[0], out[0], w0);
+      __syncthreads();
+      const uint64_t at = base + w0;
+      if (at >= chars_cap) return;
+      window_store(sm, reinterpret_cast<uintptr_t>(a.chars) + at,
+                   at + nw <= chars_cap ? nw : static_cast<uint32_t>(chars_cap - at));
+      w0 += nw;
+      __syncthreads();  // the stores have read the window
+    }
+    turn(1);
   }
 }
 
@@ -1324,9 +1550,9 @@ __device__ __forceinline__ void fsst_prep_segment(const FsstSeg sg, uint32_t si,
   const uint8_t* seg = sg.bytes;
   const uint8_t* end = seg + sg.bytes_size;
   const bool gap     = seg == nullptr;
-  for (uint32_t k = tid; k * FSST_CHUNK_ROWS < sg.row_count; k += NT) {
-    const uint32_t r0 = k * FSST_CHUNK_ROWS;
-    const uint32_t n  = sg.row_count - r0 < FSST_CHUNK_ROWS ? sg.row_count - r0 : FSST_CHUNK_ROWS;
+  for (uint32_t k = tid; uint64_t{k} * sg.chunk_rows < sg.row_count; k += NT) {
+    const uint32_t r0 = k * sg.chunk_rows;
+    const uint32_t n  = sg.row_count - r0 < sg.chunk_rows ? sg.row_count - r0 : sg.chunk_rows;
     const FsstChunk fc{gap ? FSST_GAP : si, gap ? 0u : r0, n, sg.col_row + r0};
     *gbl(reinterpret_cast<u32x4*>(chunks + sg.first_chunk + k)) = __builtin_bit_cast(u32x4, fc);
   }
@@ -1336,7 +1562,7 @@ __device__ __forceinline__ void fsst_prep_segment(const FsstSeg sg, uint32_t si,
     return;  // uniform per segment
   }
   if (sg.codec == SDR_CODEC_DICT_FSST) {  // bytes: the range's DictFsstSeg; pad: 1 if valid
-    for (uint32_t k = tid; k * FSST_CHUNK_ROWS < sg.row_count; k += NT) {
+    for (uint32_t k = tid; uint64_t{k} * sg.chunk_rows < sg.row_count; k += NT) {
       FsstChunkInfo ci{sg.bytes, 0u, 0u, 0u, FI_DFSST | (sg.pad ? FI_OK : 0u), 0u, 0u};
       const gptr<u32x4> dst = gbl(reinterpret_cast<u32x4*>(info + sg.first_chunk + k));
       const u32x8 cv        = __builtin_bit_cast(u32x8, ci);
@@ -1673,8 +1899,9 @@ __device__ __forceinline__ void fsst_chunk(const FsstChunk ch, const FsstChunkIn
   const bool ok       = ch.seg != FSST_GAP && (ci.flags & FI_OK);
   const uint32_t rows = ch.rows;
   if (ok && (ci.flags & (FI_DICT | FI_UNC | FI_DFSST))) {  // uniform per chunk
-    plain_chunk(ci.bytes, ci.bytes_size, ci.dict_end, ci.flags, ci.c_lo, ci.c_hi, ch.row_begin, rows, ch.col_row, c,
-                n_chunks, st, offsets, chars, chars_cap, total_rows, spin_limit, (LdsPtr<FsstSmem>)(&sm));
+    const PlainArgs args{ci.bytes,  ci.bytes_size, ci.dict_end, ci.flags, ci.c_lo, ci.c_hi, ch.row_begin, rows,
+                         ch.col_row, c, n_chunks, st, offsets, chars, chars_cap, total_rows, spin_limit};
+    plain_chunk<ROWS_PER_THR>(args, sm);
     return;
   }
   // Rows are stored back to front ending at dict_end: the chunk's bytes are

@@ -24,6 +24,39 @@ __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6)
                               chars, chars_cap, total_rows, spin_limit, sm);
 }
 
+// A column without FSST segments, in chunks of up to RPT * 512 rows.  A kernel
+// of its own: within k_fsst the decode was a call, which saved and restored
+// registers through scratch memory, the larger part of its time (8 Mi labels
+// 119 us, 2 M rows of 27 chars 57 us; here 65 us and 44 us).  Six wavefronts to a
+// SIMD are three workgroups to a CU; for four, rows' state spills (73 us, 70 us).
+template <uint32_t RPT>
+__global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_plain(const FsstChunk* __restrict__ chunks, uint32_t n_chunks,
+                                                        const FsstChunkInfo* __restrict__ info,
+                                                        FsstState* __restrict__ st, int32_t* __restrict__ offsets,
+                                                        uint8_t* __restrict__ chars, uint64_t chars_cap,
+                                                        uint32_t total_rows, uint32_t spin_limit)
+{
+  __shared__ PlainSmem sm;
+  __shared__ uint32_t s_ticket;
+  if (threadIdx.x == 0) s_ticket = atomicAdd(&st->ticket, 1u);
+  __syncthreads();
+  const uint32_t c = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(s_ticket)));
+  if (c >= n_chunks) return;  // grid size equals chunk count; never taken
+  const FsstChunk ch     = uniform(gload(chunks + c));
+  const FsstChunkInfo ci = uniform(gload(info + c));
+  if (ch.seg != FSST_GAP && (ci.flags & FI_OK)) {
+    plain_chunk<RPT>({ci.bytes, ci.bytes_size, ci.dict_end, ci.flags, ci.c_lo, ci.c_hi, ch.row_begin, ch.rows,
+                      ch.col_row, c, n_chunks, st, offsets, chars, chars_cap, total_rows, spin_limit}, sm);
+    return;
+  }
+  // rows of no segment, or of one with a bad header, are empty
+  const uint64_t base = fsst_lookback(c, n_chunks, 0u, st, spin_limit, sm);
+  for (uint32_t r = threadIdx.x; r < ch.rows; r += FSST_THREADS)
+    gbl(offsets)[ch.col_row + r] = static_cast<int32_t>(static_cast<uint32_t>(base));
+  if (c == n_chunks - 1u && threadIdx.x == 0)
+    gbl(offsets)[total_rows] = static_cast<int32_t>(static_cast<uint32_t>(base));
+}
+
 // Segment pre-pass: one workgroup per segment (grid-stride), which also clears
 // the look-back status of its chunks (a launch of its own for that, and a copy
 // of the ranges to the device before it, were 10 us of a 76 us call).
@@ -61,7 +94,7 @@ __global__ __launch_bounds__(Src::THREADS) void k_fsst_prep(Src src, uint32_t n_
   }
   for (uint32_t i = blockIdx.x; i < n_segs; i += gridDim.x) {
     const FsstSeg sg = src.at(i);
-    for (uint32_t k = threadIdx.x; k * FSST_CHUNK_ROWS < sg.row_count; k += Src::THREADS)
+    for (uint32_t k = threadIdx.x; uint64_t{k} * sg.chunk_rows < sg.row_count; k += Src::THREADS)
       gbl(st->status)[sg.first_chunk + k] = 0;
     fsst_prep_segment(sg, i, chunks, info, tabs + i, sm);
   }
@@ -200,7 +233,7 @@ hipError_t launch_fsst_prep(const FsstSeg* segs, uint32_t n_segs, FsstChunk* d_c
   return hipGetLastError();
 }
 
-hipError_t launch_fsst(const FsstChunk* d_chunks, uint32_t first, uint32_t n, uint32_t n_chunks_total,
+hipError_t launch_fsst(uint32_t chunk_rows, const FsstChunk* d_chunks, uint32_t first, uint32_t n, uint32_t n_chunks_total,
                        const FsstChunkInfo* d_info, const FsstSymTab* d_tabs, FsstState* d_state,
                        int32_t* d_offsets, uint8_t* d_chars, uint64_t chars_cap, uint32_t total_rows,
                        hipStream_t s)
@@ -209,8 +242,16 @@ hipError_t launch_fsst(const FsstChunk* d_chunks, uint32_t first, uint32_t n, ui
   // Tickets are global chunk numbers: a launch covering [first, first + n)
   // runs after every launch of lower chunks on the same stream.
   (void)first;
+  const uint32_t spin = tune(SDR_TUNE_FSST_SPIN_LIMIT);
+  if (chunk_rows) {
+    static_assert(FSST_CHUNK_ROWS == 2u * FSST_THREADS && WIDE_CHUNK_ROWS == 8u * FSST_THREADS, "one kernel a size");
+    auto* const k = chunk_rows <= FSST_CHUNK_ROWS ? k_plain<2> : chunk_rows < WIDE_CHUNK_ROWS ? k_plain<4> : k_plain<8>;
+    hipLaunchKernelGGL(k, dim3(n), dim3(FSST_THREADS), 0, s, d_chunks, n_chunks_total, d_info, d_state, d_offsets,
+                       d_chars, chars_cap, total_rows, spin);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(k_fsst, dim3(n), dim3(FSST_THREADS), 0, s, d_chunks, n_chunks_total, d_info, d_tabs, d_state,
-                     d_offsets, d_chars, chars_cap, total_rows, tune(SDR_TUNE_FSST_SPIN_LIMIT));
+                     d_offsets, d_chars, chars_cap, total_rows, spin);
   return hipGetLastError();
 }
 

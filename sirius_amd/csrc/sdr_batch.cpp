@@ -204,8 +204,8 @@ int batch_add_strings(sdr_batch* b, sdr_string_column* col)
   std::stable_sort(segs.begin(), segs.end(),
                    [](const auto& a, const auto& c) { return a.first->row_offset < c.first->row_offset; });
   auto add_range = [&](const uint8_t* bytes, uint32_t size, uint32_t col_row, uint32_t rows, uint32_t codec) {
-    bc.segs.push_back({bytes, size, rows, bc.n_chunks, col_row, codec, 0});
-    bc.n_chunks += fsst_chunk_count(rows);
+    bc.segs.push_back({bytes, size, rows, bc.n_chunks, col_row, static_cast<uint16_t>(codec), FSST_CHUNK_ROWS, 0});
+    bc.n_chunks += fsst_chunk_count(bc.segs.back());
   };
   uint32_t cursor = 0;
   for (const auto& sc : segs) {

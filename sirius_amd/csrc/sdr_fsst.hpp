@@ -9,6 +9,7 @@
 namespace sdr {
 
 constexpr uint32_t FSST_CHUNK_ROWS = 1024;        // rows per workgroup
+constexpr uint32_t WIDE_CHUNK_ROWS = 4096;        // ... at most, in columns of DICTIONARY segments
 constexpr uint32_t FSST_GAP        = 0xFFFFFFFFu;  // chunk of rows no segment covers
 constexpr uint32_t FSST_SPIN_LIMIT = 1u << 24;     // look-back wait bound (never reached)
 
@@ -23,13 +24,30 @@ struct FsstSeg {
   uint32_t row_count;
   uint32_t first_chunk;
   uint32_t col_row;
-  uint32_t codec;
+  uint16_t codec;
+  uint16_t chunk_rows;  // of its chunks but the last; FSST_CHUNK_ROWS but in columns of DICTIONARY segments
   uint32_t pad;
 };
 static_assert(sizeof(FsstSeg) == 32, "FsstSeg layout");
 
-// Chunks covering `rows` rows.
-inline uint32_t fsst_chunk_count(uint32_t rows) { return (rows + FSST_CHUNK_ROWS - 1u) / FSST_CHUNK_ROWS; }
+// Rows per chunk of a column of DICTIONARY segments alone: of 4096, 2048 and
+// 1024 the widest that still gives each of the 256 CUs a chunk.  A chunk's
+// ticket and look-back are steps that chunks take one after another (8 Mi
+// labels: 112 us in chunks of 1024 rows, 76 of 2048, 65 of 4096), but fewer
+// chunks than CUs leave some idle (a row group: 25, 26, 30 us; 512 Ki rows: 32,
+// 29, 33; 1 Mi: 42, 35, 36).
+inline uint32_t label_chunk_rows(uint32_t total_rows)
+{
+  uint32_t r = WIDE_CHUNK_ROWS;
+  while (r > FSST_CHUNK_ROWS && total_rows / r < 256u) r /= 2u;
+  return r;
+}
+
+// Chunks covering a range.
+inline uint32_t fsst_chunk_count(const FsstSeg& sg)
+{
+  return sg.row_count / sg.chunk_rows + (sg.row_count % sg.chunk_rows ? 1u : 0u);
+}
 
 // A chunk: `rows` rows starting at segment row `row_begin` (column row
 // `col_row`).  Chunks are listed in column row order.
@@ -131,7 +149,8 @@ constexpr uint32_t FSST_STATE_WORDS = 3;  // 8-byte words before status
 // travel in the kernel arguments, each of many is read by its block.
 hipError_t launch_fsst_prep(const FsstSeg* segs, uint32_t n_segs, FsstChunk* d_chunks, FsstChunkInfo* d_info,
                             FsstSymTab* d_tabs, FsstState* d_state, FsstResult* result, hipStream_t s, bool host);
-hipError_t launch_fsst(const FsstChunk* d_chunks, uint32_t first, uint32_t n, uint32_t n_chunks_total,
+// `chunk_rows`: 0 for a column with FSST segments, else the rows of its chunks.
+hipError_t launch_fsst(uint32_t chunk_rows, const FsstChunk* d_chunks, uint32_t first, uint32_t n, uint32_t n_chunks_total,
                        const FsstChunkInfo* d_info, const FsstSymTab* d_tabs, FsstState* d_state,
                        int32_t* d_offsets, uint8_t* d_chars, uint64_t chars_cap, uint32_t total_rows,
                        hipStream_t s);

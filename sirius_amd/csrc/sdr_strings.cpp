@@ -249,13 +249,23 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
   std::stable_sort(segs.begin(), segs.end(),
                    [](const auto& a, const auto& b) { return a.first->row_offset < b.first->row_offset; });
 
+  bool any_fsst = false, labels = true;
+  for (const auto& sc : segs) {
+    any_fsst = any_fsst || sc.second == SDR_CODEC_FSST;
+    labels   = labels && sc.second == SDR_CODEC_DICTIONARY;
+  }
+  const uint32_t chunk_rows = labels ? label_chunk_rows(n) : FSST_CHUNK_ROWS;
+  const uint32_t plain_rows = any_fsst ? 0u : chunk_rows;  // no chunk is FSST
   // row ranges: the segments and the gaps between them; the pre-pass
   // writes their chunk lists on the device
   std::vector<FsstSeg> hsegs;
   uint32_t n_chunks = 0;
+  size_t n_narrow   = 0;  // chunks there would be of FSST_CHUNK_ROWS rows
   auto add_range = [&](const uint8_t* bytes, uint32_t size, uint32_t col_row, uint32_t rows, uint32_t codec) {
-    hsegs.push_back({bytes, size, rows, n_chunks, col_row, codec, 0});
-    n_chunks += fsst_chunk_count(rows);
+    hsegs.push_back({bytes, size, rows, n_chunks, col_row, static_cast<uint16_t>(codec),
+                     static_cast<uint16_t>(chunk_rows), 0});
+    n_chunks += fsst_chunk_count(hsegs.back());
+    n_narrow += (size_t{rows} + FSST_CHUNK_ROWS - 1u) / FSST_CHUNK_ROWS;
   };
   uint32_t cursor = 0;
   for (const auto& sc : segs) {
@@ -283,8 +293,10 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
   void *h_slot = nullptr, *d_slot = nullptr, *slot = nullptr;
   const bool own = !scratch_mem && total_bytes > STRINGS_KEEP_BYTES;
   if (scratch_mem) {
-    // FsstState::result, unused here, does not count against the limit
-    const size_t counted = total_bytes - state_bytes + al(sizeof(FsstState) - sizeof(FsstResult*) + sizeof(uint64_t) * n_chunks);
+    // The limit is on columns, not on how they are cut: it counts chunks of
+    // FSST_CHUNK_ROWS rows, and not FsstState::result, unused here.
+    const size_t counted = seg_bytes + al(n_narrow * sizeof(FsstChunk)) + al(n_narrow * sizeof(FsstChunkInfo)) + tab_bytes +
+                           al(sizeof(FsstState) - sizeof(FsstResult*) + sizeof(uint64_t) * n_narrow) + sizeof(unsigned long long);
     if (counted > SDR_NOALLOC_SCRATCH_BYTES)
       return fail(SDR_E_CAPACITY, "string decode needs %llu bytes of descriptors; the no-allocation scratch holds %u",
                   static_cast<unsigned long long>(counted), SDR_NOALLOC_SCRATCH_BYTES);
@@ -348,10 +360,10 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
   if (e == hipSuccess) {
     if (mode == SDR_LAUNCH_PER_SEGMENT) {
       for (uint32_t i = 0; e == hipSuccess && i < n_ranges; ++i)
-        e = launch_fsst(d_chunks, hsegs[i].first_chunk, fsst_chunk_count(hsegs[i].row_count), n_chunks, d_info,
+        e = launch_fsst(plain_rows, d_chunks, hsegs[i].first_chunk, fsst_chunk_count(hsegs[i]), n_chunks, d_info,
                         d_tabs, d_state, col->d_offsets, col->d_chars, col->d_chars ? col->chars_capacity : 0, n, s);
     } else {
-      e = launch_fsst(d_chunks, 0, n_chunks, n_chunks, d_info, d_tabs, d_state, col->d_offsets, col->d_chars,
+      e = launch_fsst(plain_rows, d_chunks, 0, n_chunks, n_chunks, d_info, d_tabs, d_state, col->d_offsets, col->d_chars,
                       col->d_chars ? col->chars_capacity : 0, n, s);
     }
   }

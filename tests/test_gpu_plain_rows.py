@@ -86,3 +86,25 @@ def test_dict_fsst_rows(mode):
                                   A.LAUNCH_BATCHED, skew)
         np.testing.assert_array_equal(g_offs.astype(np.uint64), offs)
         np.testing.assert_array_equal(g_chars, chars)
+
+
+@pytest.mark.parametrize("longest", [9, 60], ids=["one_window", "windows"])
+@pytest.mark.parametrize("rows", [524_287, 524_289, 1_048_575, 1_049_601])
+def test_label_chunk_widths(rows, longest):
+    """Columns on either side of the sizes where a chunk of labels gets wider,
+    in segments that end inside chunks; rows past a window as well."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    rng = np.random.default_rng(rows + longest)
+    words = [None] + [rng.integers(0, 256, n, dtype=np.uint8).tobytes() for n in range(0, longest, 1 + longest // 12)]
+    b = StringBlob()
+    for lo, hi in ((0, 123_457), (123_457, rows)):
+        b.add(A.DICTIONARY, dictionary_string_segment([words[k] for k in rng.integers(0, len(words), hi - lo)]), lo, hi - lo)
+    table = np.array(b.table, np.int64)
+    o_offs, o_chars = oracle_string_runs(b.blob, table, rows)
+    for skew in (0, 3):
+        d = torch.zeros(b.blob.size + skew + 64, dtype=torch.uint8, device="cuda")
+        d[skew:skew + b.blob.size] = torch.from_numpy(b.blob)
+        offs, chars = _decode(duckdb_segments(table, d.data_ptr() + skew), rows, o_chars.size, A.LAUNCH_BATCHED, 4 * skew)
+        np.testing.assert_array_equal(offs, o_offs)
+        np.testing.assert_array_equal(chars, o_chars)
