@@ -954,33 +954,44 @@ __device__ __forceinline__ void plain_prep_segment(const FsstSeg& sg, FsstChunkI
 // DICTIONARY rows (:246-265, :324-360).  Bytes past the segment read as
 // zero; the byte a trailing escape counts is written as 0.
 
-// Dictionary index of segment row sr (row + 1 in mode 2).
-__device__ __forceinline__ uint32_t dfsst_index(const DictFsstSeg& d, uint32_t sr)
+// Calls f(byte) for the n bytes at p in order, read as aligned words, four in
+// flight (a byte at a time, each load waited for, was most of these passes).
+template <typename F>
+__device__ __forceinline__ void each_byte(const uint8_t* p, uint32_t n, F f)
 {
-  if (d.mode == 2u) return sr + 1u;
-  return stream_bits32(d.bytes + d.off_didx, d.bytes + d.bytes_size, uint64_t{sr} * d.diw, d.diw);
+  if (n == 0) return;
+  const uint32_t skew          = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p) & 3u);
+  const gptr<const uint32_t> w = gbl(reinterpret_cast<const uint32_t*>(p - skew));
+  const uint64_t stop          = uint64_t{skew} + n;
+  const uint32_t last          = static_cast<uint32_t>((stop - 1u) >> 2);
+  for (uint32_t k = 0; k <= last; k += 4) {
+    uint32_t v[4];
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) v[j] = w[k + j < last ? k + j : last];
+#pragma unroll
+    for (uint32_t b = 0; b < 16; ++b) {
+      const uint64_t y = 4ull * k + b;
+      if (y >= skew && y < stop) f(v[b / 4u] >> (8u * (b % 4u)) & 0xFFu);
+    }
+  }
 }
 
 // Decoded length of one compressed entry of n bytes at p (bytes at or past
 // `end` read as zero, i.e. as code 0): a code adds its symbol's length, an
-// escape adds one and skips the next byte, even past the entry's end.
+// escape adds one (len[255]) and skips the next byte, even past the entry's end.
 __device__ __forceinline__ uint32_t dfsst_entry_len(const uint8_t* p, uint32_t n, const uint8_t* end,
                                                     const uint8_t* len)
 {
   const uint64_t in = p < end ? static_cast<uint64_t>(end - p) : 0u;
   const uint32_t n_in = n < in ? n : static_cast<uint32_t>(in);
-  uint32_t pos = 0, dl = 0;
-  while (pos < n_in) {
-    const uint32_t code = *gbl(p + pos);
-    ++pos;
-    if (code < FSST_ESC) {
-      dl += len[code];
-    } else {
-      ++pos;
-      ++dl;
-    }
-  }
-  if (pos < n) dl += (n - pos) * len[0];  // the zero bytes past the segment
+  uint32_t dl = 0;
+  bool esc    = false;
+  each_byte(p, n_in, [&](uint32_t code) {
+    dl += esc ? 0u : len[code];
+    esc = !esc && code == FSST_ESC;
+  });
+  const uint32_t zeros = n - n_in;  // past the segment
+  if (zeros) dl += (zeros - (esc ? 1u : 0u)) * len[0];
   return dl;
 }
 
@@ -1457,7 +1468,7 @@ __device__ __forceinline__ void dfsst_prep_segment(const DictFsstSeg& d, uint32_
   const uint8_t* end  = seg + d.bytes_size;
   const bool fsst     = d.mode != 0u && d.dict_count > 1u;
   const uint32_t mylen = import_symtab(seg, d.bytes_size, d.off_symtab, fsst && d.off_symtab < d.bytes_size, tab, sm);
-  if (tid < 256u) sm.len[tid] = static_cast<uint8_t>(mylen);
+  if (tid < 256u) sm.len[tid] = static_cast<uint8_t>(tid == FSST_ESC ? 1u : mylen);
   __syncthreads();
   const uint8_t* slens = seg + d.off_slens;
   const uint8_t* dict  = seg + d.off_dict;
@@ -1500,6 +1511,48 @@ __device__ __forceinline__ void dfsst_prep_segment(const DictFsstSeg& d, uint32_
   }
 }
 
+// Bytes [o, lim) of `out`, appended up to eight at a time: whole words where
+// they are the writer's alone, single bytes at both ends.
+struct WordWriter {
+  uint8_t* at;   // word the next byte falls in
+  uint8_t* lim;
+  uint64_t acc = 0;     // bytes from `at` on
+  uint32_t fill, skip;  // of these, how many there are and how many are others'
+  __device__ __forceinline__ WordWriter(uint8_t* o, uint8_t* l) : lim(l)
+  {
+    skip = fill = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(o) & 3u);
+    at          = o - fill;
+  }
+  __device__ __forceinline__ bool room() const { return at + fill < lim; }
+  __device__ __forceinline__ void put_bytes(uint32_t n)
+  {
+    for (uint32_t b = skip; b < n; ++b)
+      if (at + b < lim) *gbl(at + b) = static_cast<uint8_t>(acc >> (8u * b));
+  }
+  __device__ __forceinline__ void append4(uint32_t v, uint32_t n)  // v is zero above its n <= 4 bytes
+  {
+    acc |= static_cast<uint64_t>(v) << (8u * fill);
+    fill += n;
+    if (fill < 4u) return;
+    if (skip == 0u && at + 4 <= lim) *gbl(reinterpret_cast<uint32_t*>(at)) = static_cast<uint32_t>(acc);
+    else put_bytes(4u);
+    skip = 0;
+    acc >>= 32;
+    fill -= 4u;
+    at += 4;
+  }
+  __device__ __forceinline__ void append(uint64_t v, uint32_t n)
+  {
+    append4(static_cast<uint32_t>(v), n < 4u ? n : 4u);
+    if (n > 4u) append4(static_cast<uint32_t>(v >> 32), n - 4u);
+  }
+  __device__ __forceinline__ void finish()
+  {
+    while (room()) append(0u, 8u);  // zeros up to the limit
+    put_bytes(fill);
+  }
+};
+
 // Predecode the FSST entries k >= 1 of one segment into d.src at d.e[k]
 // (exactly d.e[k + 1] - d.e[k] bytes; the byte of a trailing escape and
 // bytes past the decoded ones are 0), entries strided over `stride`
@@ -1515,23 +1568,62 @@ __device__ __forceinline__ void dfsst_predecode(const DictFsstSeg& d, const uint
     const uint32_t n  = c1 >= c0 ? c1 - c0 : 0u;
     uint64_t o        = gbl(d.e)[k];
     uint64_t lim      = gbl(d.e)[k + 1u];
-    if (lim < o) lim = o;
     if (lim > d.src_size) lim = d.src_size;
-    const uint8_t* p  = dict + c0;
-    uint32_t pos = 0;
-    while (pos < n && o < lim) {
-      const uint32_t code = p + pos < end ? *gbl(p + pos) : 0u;
-      ++pos;
-      if (code < FSST_ESC) {
-        const uint64_t v = sym[code];
-        for (uint32_t j = 0; j < len[code] && o < lim; ++j) *gbl(out + o++) = static_cast<uint8_t>(v >> (8u * j));
-      } else if (pos < n) {
-        *gbl(out + o++) = p + pos < end ? *gbl(p + pos) : 0u;
-        ++pos;
+    if (lim <= o) continue;
+    const uint8_t* p    = dict + c0;
+    const uint64_t in   = p < end ? static_cast<uint64_t>(end - p) : 0u;
+    const uint32_t n_in = n < in ? n : static_cast<uint32_t>(in);
+    WordWriter w(out + o, out + lim);
+    bool esc = false;
+    each_byte(p, n_in, [&](uint32_t code) {
+      if (!esc && code == FSST_ESC) {
+        esc = true;
+        return;
       }
+      if (w.room()) w.append(esc ? code : sym[code], esc ? 1u : len[code]);
+      esc = false;
+    });
+    // zeros past the segment: one may be an escape's byte, the others are code 0
+    for (uint32_t z = n_in; z < n && w.room(); ++z) {
+      w.append(esc ? 0u : sym[0], esc ? 1u : len[0]);
+      esc = false;
     }
-    while (o < lim) *gbl(out + o++) = 0u;
+    w.finish();
   }
+}
+
+// Clears the bits of null-mask byte `b` (value m0) of rows that are NULL in their
+// DICT_FSST range sg, whose descriptor is d: every row when the range is
+// invalid, outside mode 2 those that select entry 0 (dict_fsst.cu:426-446).
+__device__ __forceinline__ uint32_t dfsst_null_byte(uint32_t m, uint32_t row0, const FsstSeg& sg, const DictFsstSeg& d)
+{
+  if (d.valid && d.mode == 2u) return m;
+  // rows [j0, j1) of the byte's eight
+  const uint32_t j0 = sg.col_row > row0 ? sg.col_row - row0 : 0u;
+  const uint64_t e  = uint64_t{sg.col_row} + sg.row_count - row0;
+  const uint32_t j1 = e < 8u ? static_cast<uint32_t>(e) : 8u;
+  if (j0 >= j1) return m;
+  const uint32_t rows = (0xFFu >> (8u - (j1 - j0))) << j0;
+  if (!d.valid) return m & ~rows;
+  const uint8_t* bits = d.bytes + d.off_didx;
+  const uint8_t* end  = d.bytes + d.bytes_size;
+  const uint32_t w    = d.diw;
+  const uint32_t sr   = row0 + j0 - sg.col_row;
+  uint32_t null       = 0;
+  if (w && bits + ((uint64_t{sr + (j1 - j0)} * w + 7u) >> 3) <= end) {
+    const uint64_t bit0          = uint64_t{sr} * w;
+    const uintptr_t at           = reinterpret_cast<uintptr_t>(bits) + (bit0 >> 3);
+    const uint32_t skew          = 8u * static_cast<uint32_t>(at & 3u) + static_cast<uint32_t>(bit0 & 7u);
+    const gptr<const uint32_t> p = gbl(reinterpret_cast<const uint32_t*>(at & ~uintptr_t{3}));
+#pragma unroll
+    for (uint32_t j = 0; j < 8u; ++j)
+      null |= (bits32_inside(p, skew + (j < j1 - j0 ? j : 0u) * w, w) == 0u ? 1u : 0u) << j;
+    null <<= j0;
+  } else {
+    for (uint32_t j = j0; j < j1; ++j)
+      null |= (stream_bits32(bits, end, uint64_t{sr + j - j0} * w, w) == 0u ? 1u : 0u) << j;
+  }
+  return m & ~(null & rows);
 }
 
 // Range `si` with the calling NT-thread workgroup: its chunk descriptors
@@ -1561,9 +1653,14 @@ __device__ __forceinline__ void fsst_prep_segment(const FsstSeg sg, uint32_t si,
     plain_prep_segment<NT>(sg, info);
     return;  // uniform per segment
   }
-  if (sg.codec == SDR_CODEC_DICT_FSST) {  // bytes: the range's DictFsstSeg; pad: 1 if valid
+  if (sg.codec == SDR_CODEC_DICT_FSST) {  // bytes: the range's DictFsstSeg, pinned; pad: 1 if valid
+    // the chunks read it in device memory: the range's symbol table, whose
+    // entries are predecoded by now, gives way to it
+    static_assert(sizeof(DictFsstSeg) <= sizeof(FsstSymTab) && sizeof(DictFsstSeg) <= 4u * WAVE, "a word per lane");
+    if (tid < sizeof(DictFsstSeg) / 4u)
+      gbl(reinterpret_cast<uint32_t*>(tab))[tid] = gbl(reinterpret_cast<const uint32_t*>(sg.bytes))[tid];
     for (uint32_t k = tid; uint64_t{k} * sg.chunk_rows < sg.row_count; k += NT) {
-      FsstChunkInfo ci{sg.bytes, 0u, 0u, 0u, FI_DFSST | (sg.pad ? FI_OK : 0u), 0u, 0u};
+      FsstChunkInfo ci{reinterpret_cast<const uint8_t*>(tab), 0u, 0u, 0u, FI_DFSST | (sg.pad ? FI_OK : 0u), 0u, 0u};
       const gptr<u32x4> dst = gbl(reinterpret_cast<u32x4*>(info + sg.first_chunk + k));
       const u32x8 cv        = __builtin_bit_cast(u32x8, ci);
       dst[0]                = cv.lo;

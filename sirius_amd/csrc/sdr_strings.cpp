@@ -86,18 +86,58 @@ bool has_dict_fsst(const sdr_string_column* col)
 
 namespace {
 
-// Device memory of a column's DICT_FSST segments, released with the call's.
-struct DictFsstCall {
-  uint8_t* mem = nullptr;  // descriptors, range map, entry offsets, results
-  uint8_t* pre = nullptr;  // decoded FSST entries
-  DictFsstSeg* d_desc = nullptr;
-  uint32_t* d_range = nullptr;
-  bool any_inline = false;
-  void release(hipStream_t s)
+// A call's device memory past this size is its own, allocated and freed on the
+// stream; up to it, it is a slot's that later calls reuse.
+constexpr size_t STRINGS_KEEP_BYTES = 32u << 20;
+
+struct CallMemory {
+  uint8_t* p = nullptr;
+  void* slot = nullptr;  // null: p is the call's own
+  int get(size_t bytes, hipStream_t s)
   {
-    device_free(mem, s);
-    device_free(pre, s);
-    mem = pre = nullptr;
+    if (bytes > STRINGS_KEEP_BYTES) return device_alloc(reinterpret_cast<void**>(&p), bytes, s);
+    void *h = nullptr, *d = nullptr;
+    const int rc = slot_acquire(0, bytes, &h, &d, &slot);
+    p            = static_cast<uint8_t*>(d);
+    return rc;
+  }
+  // `synced`: nothing enqueued on it is pending
+  void release(hipStream_t s, bool synced)
+  {
+    if (!slot) device_free(p, s);
+    else if (synced) slot_release_idle(slot);
+    else (void)desc_release(slot, s);
+    p    = nullptr;
+    slot = nullptr;
+  }
+};
+
+// What the DICT_FSST segments of a column take: in pinned memory (part of the
+// call's slot) headers, descriptors, the dictionaries' totals and flags and the
+// counts of inline NULLs, which the passes read and write in place; in device
+// memory the entry offsets and the decoded FSST entries.
+struct DictFsstCall {
+  uint32_t* hdr     = nullptr;
+  DictFsstSeg* desc = nullptr;
+  uint32_t* out     = nullptr;
+  uint32_t* counts  = nullptr;
+  CallMemory offsets, pre;
+  bool any_inline = false;
+  static size_t pinned_bytes(size_t n_ranges)
+  {
+    return n_ranges * (16u + sizeof(DictFsstSeg) + 8u) + DFSST_NULL_COUNTS * sizeof(uint32_t);
+  }
+  void place(uint8_t* h, size_t n_ranges)
+  {
+    desc   = reinterpret_cast<DictFsstSeg*>(h);
+    hdr    = reinterpret_cast<uint32_t*>(desc + n_ranges);
+    out    = hdr + 4u * n_ranges;
+    counts = out + 2u * n_ranges;
+  }
+  void release(hipStream_t s, bool synced)
+  {
+    offsets.release(s, synced);
+    pre.release(s, synced);
   }
 };
 
@@ -107,30 +147,24 @@ uint32_t al8(uint32_t v) { return (v + 7u) & ~7u; }
 // host round trips as there): read the headers of the DICT_FSST ranges,
 // fill their descriptors (region offsets, validity, :516-525), run the
 // dictionary pre-pass, read back each segment's decoded total and inline-
-// NULL flag, predecode the FSST entries, then point the ranges at their
-// descriptors (bytes) with their validity (pad) and upload them again.
-int dict_fsst_phase(const sdr_string_column* col, std::vector<FsstSeg>& hsegs, FsstSeg* d_segs, FsstSymTab* d_tabs,
-                    hipStream_t s, DictFsstCall& dc)
+// NULL flag, predecode the FSST entries, then point the ranges (pinned, as all
+// that passes between host and passes here) at their descriptors (bytes) with
+// their validity (pad).
+int dict_fsst_phase(const sdr_string_column* col, FsstSeg* segs, uint32_t n_ranges, FsstSymTab* d_tabs, hipStream_t s,
+                    DictFsstCall& dc)
 {
-  const uint32_t n_ranges = static_cast<uint32_t>(hsegs.size());
   // 1. headers
-  uint32_t* d_hdr = nullptr;
-  int rc          = device_alloc(reinterpret_cast<void**>(&d_hdr), size_t{n_ranges} * 16u, s);
-  if (rc) return rc;
-  std::vector<uint32_t> hdr(size_t{n_ranges} * 4u);
-  hipError_t e = launch_dfsst_headers(d_segs, n_ranges, d_hdr, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(hdr.data(), d_hdr, hdr.size() * 4u, hipMemcpyDeviceToHost, s);
+  hipError_t e = launch_dfsst_headers(segs, n_ranges, dc.hdr, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  device_free(d_hdr, s);
   if (e != hipSuccess) return fail(SDR_E_HIP, "DICT_FSST headers: %s", hipGetErrorString(e));
   // 2. descriptors
-  std::vector<DictFsstSeg> ds;
   std::vector<uint32_t> range_d(n_ranges, ~0u);
   uint64_t n_e = 0;
+  uint32_t n_d = 0;
   for (uint32_t i = 0; i < n_ranges; ++i) {
-    const FsstSeg& sg = hsegs[i];
+    const FsstSeg& sg = segs[i];
     if (sg.codec != SDR_CODEC_DICT_FSST || !sg.bytes) continue;
-    const uint32_t* h = &hdr[4u * i];
+    const uint32_t* h = dc.hdr + 4u * i;
     DictFsstSeg d{};
     d.bytes      = sg.bytes;
     d.bytes_size = sg.bytes_size;
@@ -150,68 +184,56 @@ int dict_fsst_phase(const sdr_string_column* col, std::vector<FsstSeg>& hsegs, F
     d.e_byte     = static_cast<uint32_t>(n_e);
     if (d.valid) n_e += uint64_t{dict_count} + 1u;
     if (n_e > 0xFFFFFFFFull) return fail(SDR_E_CAPACITY, "DICT_FSST dictionaries hold more than 2^32 entries");
-    range_d[i] = static_cast<uint32_t>(ds.size());
-    ds.push_back(d);
+    range_d[i]      = n_d;
+    dc.desc[n_d++] = d;
   }
-  const uint32_t n_d = static_cast<uint32_t>(ds.size());
   if (n_d == 0) return SDR_OK;
-  auto al = [](size_t v) { return (v + 255u) & ~size_t{255}; };
-  const size_t b_desc = al(n_d * sizeof(DictFsstSeg)), b_range = al(size_t{n_ranges} * 4u);
-  const size_t b_e = al(std::max<uint64_t>(1, n_e) * 4u), b_out = al(size_t{n_d} * 8u);
-  rc = device_alloc(reinterpret_cast<void**>(&dc.mem), b_desc + b_range + 2u * b_e + b_out, s);
+  const size_t b_e = (std::max<uint64_t>(1, n_e) * 4u + 255u) & ~size_t{255};
+  int rc           = dc.offsets.get(2u * b_e, s);
   if (rc) return rc;
-  dc.d_desc       = reinterpret_cast<DictFsstSeg*>(dc.mem);
-  dc.d_range      = reinterpret_cast<uint32_t*>(dc.mem + b_desc);
-  auto* d_e_byte  = reinterpret_cast<uint32_t*>(dc.mem + b_desc + b_range);
-  auto* d_e_dec   = reinterpret_cast<uint32_t*>(dc.mem + b_desc + b_range + b_e);
-  auto* d_out     = reinterpret_cast<uint32_t*>(dc.mem + b_desc + b_range + 2u * b_e);
-  for (auto& d : ds) {
-    d.e = d_e_dec + d.e_byte;
+  auto* d_e_byte = reinterpret_cast<uint32_t*>(dc.offsets.p);
+  auto* d_e_dec  = reinterpret_cast<uint32_t*>(dc.offsets.p + b_e);
+  for (uint32_t j = 0; j < n_d; ++j) {
+    DictFsstSeg& d = dc.desc[j];
+    d.e            = d_e_dec + d.e_byte;
     if (d.mode == 0u || d.dict_count <= 1u) {  // rows copy raw dict bytes
       d.src      = d.bytes + d.off_dict;
       d.src_size = d.bytes_size > d.off_dict ? d.bytes_size - d.off_dict : 0u;
     }
   }
-  rc = upload_async(dc.d_desc, ds.data(), n_d * sizeof(DictFsstSeg), s);
-  if (!rc) rc = upload_async(dc.d_range, range_d.data(), size_t{n_ranges} * 4u, s);
-  if (rc) return rc;
   // 3. dictionary pre-pass, per-segment totals and inline-NULL flags
-  std::vector<uint32_t> out(size_t{n_d} * 2u);
-  e = launch_dfsst_prep(dc.d_desc, n_d, d_e_byte, d_e_dec, d_tabs, d_out, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(out.data(), d_out, out.size() * 4u, hipMemcpyDeviceToHost, s);
+  e = launch_dfsst_prep(dc.desc, n_d, d_e_byte, d_e_dec, d_tabs, dc.out, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return fail(SDR_E_HIP, "DICT_FSST dictionary pre-pass: %s", hipGetErrorString(e));
   uint64_t n_pre = 0;
   for (uint32_t j = 0; j < n_d; ++j) {
-    dc.any_inline = dc.any_inline || out[2u * j + 1u];
-    if (ds[j].valid && ds[j].mode != 0u && ds[j].dict_count > 1u) n_pre += out[2u * j];
+    dc.any_inline = dc.any_inline || dc.out[2u * j + 1u];
+    if (dc.desc[j].valid && dc.desc[j].mode != 0u && dc.desc[j].dict_count > 1u) n_pre += dc.out[2u * j];
   }
   if (dc.any_inline && col->total_rows && !col->d_null_mask)
     return fail(SDR_E_INVALID_ARG, "DICT_FSST segments hold inline NULLs (entry 0) and d_null_mask is NULL");
   // 4. predecode
   if (n_pre) {
-    rc = device_alloc(reinterpret_cast<void**>(&dc.pre), n_pre, s);
+    rc = dc.pre.get(n_pre, s);
     if (rc) return rc;
     uint64_t at = 0;
     for (uint32_t j = 0; j < n_d; ++j) {
-      auto& d = ds[j];
+      DictFsstSeg& d = dc.desc[j];
       if (!d.valid || d.mode == 0u || d.dict_count <= 1u) continue;
-      d.src      = dc.pre + at;
-      d.src_size = out[2u * j];
-      at += out[2u * j];
+      d.src      = dc.pre.p + at;
+      d.src_size = dc.out[2u * j];
+      at += dc.out[2u * j];
     }
-    rc = upload_async(dc.d_desc, ds.data(), n_d * sizeof(DictFsstSeg), s);
-    if (rc) return rc;
-    e = launch_dfsst_predecode(dc.d_desc, n_d, d_e_byte, d_tabs, s);
+    e = launch_dfsst_predecode(dc.desc, n_d, d_e_byte, d_tabs, s);
     if (e != hipSuccess) return fail(SDR_E_HIP, "DICT_FSST predecode: %s", hipGetErrorString(e));
   }
   // 5. the ranges now name their descriptors
   for (uint32_t i = 0; i < n_ranges; ++i)
     if (range_d[i] != ~0u) {
-      hsegs[i].bytes = reinterpret_cast<const uint8_t*>(dc.d_desc + range_d[i]);
-      hsegs[i].pad   = ds[range_d[i]].valid;
+      segs[i].bytes = reinterpret_cast<const uint8_t*>(dc.desc + range_d[i]);
+      segs[i].pad   = dc.desc[range_d[i]].valid;
     }
-  return upload_async(d_segs, hsegs.data(), hsegs.size() * sizeof(FsstSeg), s);
+  return SDR_OK;
 }
 
 }  // namespace
@@ -288,7 +310,6 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
   // pre-pass reads in place, and the result, which the kernels write: both in
   // a slot that later calls reuse (device memory past STRINGS_KEEP_BYTES, or
   // none when nothing may be allocated, is not the slot's).
-  constexpr size_t STRINGS_KEEP_BYTES = 32u << 20;
   uint8_t* d = scratch_mem;
   void *h_slot = nullptr, *d_slot = nullptr, *slot = nullptr;
   const bool own = !scratch_mem && total_bytes > STRINGS_KEEP_BYTES;
@@ -301,7 +322,9 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
       return fail(SDR_E_CAPACITY, "string decode needs %llu bytes of descriptors; the no-allocation scratch holds %u",
                   static_cast<unsigned long long>(counted), SDR_NOALLOC_SCRATCH_BYTES);
   } else {
-    rc = slot_acquire(sizeof(FsstResult) + hsegs.size() * sizeof(FsstSeg), own ? 0 : total_bytes, &h_slot, &d_slot, &slot);
+    const size_t b_pinned =
+      sizeof(FsstResult) + hsegs.size() * sizeof(FsstSeg) + (dfsst ? DictFsstCall::pinned_bytes(n_ranges) : 0u);
+    rc = slot_acquire(b_pinned, own ? 0 : total_bytes, &h_slot, &d_slot, &slot);
     if (!rc && own) rc = device_alloc(reinterpret_cast<void**>(&d), total_bytes, s);
     if (rc) {
       slot_release_idle(slot);
@@ -331,32 +354,27 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
     if (e != hipSuccess) return fail(SDR_E_HIP, "string decode: %s", hipGetErrorString(e));
   } else {
     *result = FsstResult{0, 0};
-    if (dfsst) {  // its passes read the ranges many times
-      rc = upload_async(d_segs, hsegs.data(), hsegs.size() * sizeof(FsstSeg), s);
-      if (rc) {
-        release();
-        return rc;
-      }
-    } else {
-      auto* hs = reinterpret_cast<FsstSeg*>(result + 1);
-      std::memcpy(hs, hsegs.data(), hsegs.size() * sizeof(FsstSeg));
-      prep_segs = hs;
-    }
+    auto* hs = reinterpret_cast<FsstSeg*>(result + 1);
+    std::memcpy(hs, hsegs.data(), hsegs.size() * sizeof(FsstSeg));
+    prep_segs = hs;
   }
   DictFsstCall dc;
   if (dfsst) {
-    rc = dict_fsst_phase(col, hsegs, d_segs, d_tabs, s, dc);
+    auto* hs = reinterpret_cast<FsstSeg*>(result + 1);
+    dc.place(reinterpret_cast<uint8_t*>(hs + n_ranges), n_ranges);
+    rc = dict_fsst_phase(col, hs, n_ranges, d_tabs, s, dc);
     if (rc) {
-      dc.release(s);  // stream-ordered: after every pass of the phase already enqueued
+      dc.release(s, false);  // after every pass of the phase already enqueued
       release();
       return rc;
     }
   }
   auto release_all = [&]() {
-    dc.release(s);
+    dc.release(s, synced);
     release();
   };
-  e = launch_fsst_prep(prep_segs, n_ranges, d_chunks, d_info, d_tabs, d_state, result, s, prep_segs != d_segs);
+  e = launch_fsst_prep(prep_segs, n_ranges, d_chunks, d_info, d_tabs, d_state, result, s, prep_segs != d_segs,
+                       dc.any_inline ? d_segs : nullptr);
   if (e == hipSuccess) {
     if (mode == SDR_LAUNCH_PER_SEGMENT) {
       for (uint32_t i = 0; e == hipSuccess && i < n_ranges; ++i)
@@ -371,9 +389,7 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
   std::vector<MaskUnit> units;
   const uint32_t* counts = nullptr;  // null count of each piece of the mask
   void* counts_token     = nullptr;
-  // nulls counted on the device: DICT_FSST's inline ones (or every one, when
-  // nothing may be allocated for the pieces' counts)
-  const bool device_nulls = masked && (dc.any_inline || scratch_mem);
+  const bool device_nulls = masked && scratch_mem;  // nothing may be allocated for the pieces' counts
   if (e == hipSuccess && masked) {
     add_mask_units(col->validity, col->has_nulls ? col->n_validity : 0u, n, col->d_null_mask, units);
     if (device_nulls) e = launch_fill_u8(reinterpret_cast<uint8_t*>(d_nulls), 0, sizeof(unsigned long long), s);
@@ -388,7 +404,7 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
     }
     // DICT_FSST inline NULLs (dict_fsst.cu:426-446) on top of the validity
     if (e == hipSuccess && dc.any_inline)
-      e = launch_dfsst_nulls(d_segs, n_ranges, dc.d_desc, dc.d_range, col->d_null_mask, n, d_nulls, s);
+      e = launch_dfsst_nulls(d_segs, n_ranges, d_tabs, col->d_null_mask, n, dc.counts, s);
   }
   struct {
     uint32_t ticket, error;
@@ -404,6 +420,7 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
     h.error = static_cast<uint32_t>(result->error);
   }
   for (size_t u = 0; synced && counts && u < units.size(); ++u) h_nulls += counts[u];
+  for (uint32_t u = 0; synced && dc.any_inline && u < dfsst_null_counts(n); ++u) h_nulls += dc.counts[u];
   if (synced) slot_release_idle(counts_token);
   else (void)desc_release(counts_token, s);
   release_all();
