@@ -16,11 +16,11 @@
 //      entries cost one pass, i.e. one memory round trip.
 //   2. expansion: the slice is split over the 4 wavefronts; each finds its
 //      first run from the LDS chunk bases, then walks windows of 64 runs:
-//      a DPP scan gives each run's end row.  A window of at most 4096 rows
+//      a DPP scan gives each run's end row.  A window with at most 4096 rows to write
 //      marks its run ends in a per-wave LDS bitmap, and each 64-row step
 //      reads its 64 bits, so a row's run index is the ballot count of ends
-//      at or before the step plus a popcount of those bits.  Longer windows
-//      build the step's mask with scalar readlanes; windows holding a
+//      at or before the step plus a popcount of those bits.  More rows
+//      build each step's mask with scalar readlanes; windows holding a
 //      zero-length run take an exact per-lane count.
 #pragma once
 
@@ -39,9 +39,10 @@ constexpr uint32_t RLE_SUPER       = RLE_THREADS * RLE_PER_THREAD;  // 8192 entr
 constexpr uint32_t RLE_MAX_SUPERS  = (RLE_MAX_ENTRIES + RLE_SUPER - 1) / RLE_SUPER;
 constexpr uint32_t RLE_STAGE_WORDS = (RLE_SUPER * 2 + 48) / 4;
 static_assert(RLE_SUPER % RLE_TILE == 0, "passes hold whole tiles");
+static_assert(RLE_SUPER / (2u * WAVE) % (4u * RLE_WAVES) == 0, "steps taken four at a time stay in the stage");
 
 // Per-wave bitmap of run ends over a window's 64-row steps, one 64-bit word
-// per step: RLE_BM_ROWS window rows, the up to 63 rows the first step starts
+// per step: RLE_BM_ROWS rows of it, the up to 63 rows the first step starts
 // before the window, and the step a pair may overrun.
 constexpr uint32_t RLE_BM_ROWS   = 4096;
 constexpr uint32_t RLE_BM_QWORDS = (RLE_BM_ROWS + 63u) / 64u + 3u;
@@ -66,10 +67,11 @@ __device__ __forceinline__ uint32_t lds_u16(const uint32_t* lds, uint32_t byte)
 // zero/overshoot entry of the pass in sm.match / sm.bad (UINT32_MAX: none).
 // Returns the pass's count total.  Called by all threads of the block.
 //
-// Wave w reads words [1024 w, 1024 w + 1024) of the staged counts (two
-// counts a word), 64 consecutive words per step, so the LDS reads are
-// conflict-free; a 16-lane row of a step is one 32-entry chunk, summed by a
-// DPP row scan.
+// A step reads 64 consecutive words of the staged counts (two counts a word),
+// so the LDS reads are conflict-free; a 16-lane row of it is one 32-entry chunk,
+// summed by a DPP row scan.  The waves take steps in turn, and none past the
+// last entry: segments of long runs hold few (600 entries for a row group in
+// runs of 200, five steps of 64 here).
 __device__ __forceinline__ uint32_t rle_pass(const uint8_t* counts, uint32_t t0, uint32_t n, uint32_t base,
                                              uint32_t rows, bool detect, uint32_t& head, RleSmem& sm)
 {
@@ -84,6 +86,7 @@ __device__ __forceinline__ uint32_t rle_pass(const uint8_t* counts, uint32_t t0,
   const uint32_t t    = threadIdx.x;
   const uint32_t lane = lane_id();
   const uint32_t wv   = t / WAVE;
+  const uint32_t wvs  = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(wv)));
   const uint32_t row  = lane >> 4;
   const uint32_t hq   = head >> 2;
   const uint32_t sh   = (head & 3u) * 8u;
@@ -92,14 +95,19 @@ __device__ __forceinline__ uint32_t rle_pass(const uint8_t* counts, uint32_t t0,
     const uint32_t w = __builtin_amdgcn_alignbit(sm.stage[hq + i + 1u], sm.stage[hq + i], sh);
     return w & ((2u * i + 1u < n ? 0xFFFF0000u : 0u) | (2u * i < n ? 0xFFFFu : 0u));
   };
-#pragma unroll 4
-  for (uint32_t k = 0; k < RLE_PER_THREAD / 2; ++k) {
-    const uint32_t w  = word(1024u * wv + 64u * k + lane);
-    const uint32_t rs = row_incl_sum_u32((w & 0xFFFFu) + (w >> 16));
-    if ((lane & 15u) == 15u) sm.chunk_base[64u * wv + 4u * k + row] = rs;  // the chunk's sum
+  const uint32_t steps = (n + 2u * WAVE - 1u) / (2u * WAVE);
+  // four of a wave's steps at a time, entries past the last reading as zero
+#pragma unroll 1
+  for (uint32_t k4 = wvs; k4 < steps; k4 += 4u * RLE_WAVES) {
+#pragma unroll
+    for (uint32_t k = k4; k < k4 + 4u * RLE_WAVES; k += RLE_WAVES) {
+      const uint32_t w  = word(64u * k + lane);
+      const uint32_t rs = row_incl_sum_u32((w & 0xFFFFu) + (w >> 16));
+      if ((lane & 15u) == 15u) sm.chunk_base[4u * k + row] = rs;  // the chunk's sum
+    }
   }
   __syncthreads();
-  const uint32_t s    = sm.chunk_base[t];  // chunk t's sum
+  const uint32_t s    = t < 4u * steps ? sm.chunk_base[t] : 0u;  // chunk t's sum
   const uint32_t incl = wave_incl_sum_u32(s);
   if (lane == WAVE - 1) sm.wave_sum[wv] = incl;
   __syncthreads();
@@ -114,20 +122,23 @@ __device__ __forceinline__ uint32_t rle_pass(const uint8_t* counts, uint32_t t0,
   if (detect) {
     __syncthreads();  // chunk bases visible
     uint32_t m = UINT32_MAX, bad = UINT32_MAX;  // this lane's first entries (they rise with k)
-#pragma unroll 4
-    for (uint32_t k = 0; k < RLE_PER_THREAD / 2; ++k) {
-      const uint32_t i  = 1024u * wv + 64u * k + lane;
-      const uint32_t w  = word(i);
-      const uint32_t c0 = w & 0xFFFFu, c1 = w >> 16;
-      const uint32_t rs = row_incl_sum_u32(c0 + c1);
-      const uint32_t r0 = sm.chunk_base[64u * wv + 4u * k + row] + rs - (c0 + c1) + c0;
-      const uint32_t r1 = r0 + c1;
-      const bool l0 = 2u * i < n, l1 = 2u * i + 1u < n;
-      const uint32_t e  = t0 + 2u * i;
-      const uint32_t hm = (l0 && r0 == rows) ? e : ((l1 && r1 == rows) ? e + 1u : UINT32_MAX);
-      const uint32_t hb = (l0 && (c0 == 0u || r0 > rows)) ? e : ((l1 && (c1 == 0u || r1 > rows)) ? e + 1u : UINT32_MAX);
-      m   = m < hm ? m : hm;
-      bad = bad < hb ? bad : hb;
+#pragma unroll 1
+    for (uint32_t k4 = wvs; k4 < steps; k4 += 4u * RLE_WAVES) {
+#pragma unroll
+      for (uint32_t k = k4; k < k4 + 4u * RLE_WAVES; k += RLE_WAVES) {
+        const uint32_t i  = 64u * k + lane;
+        const uint32_t w  = word(i);
+        const uint32_t c0 = w & 0xFFFFu, c1 = w >> 16;
+        const uint32_t rs = row_incl_sum_u32(c0 + c1);
+        const uint32_t r0 = sm.chunk_base[4u * k + row] + rs - (c0 + c1) + c0;
+        const uint32_t r1 = r0 + c1;
+        const bool l0 = 2u * i < n, l1 = 2u * i + 1u < n;
+        const uint32_t e  = t0 + 2u * i;
+        const uint32_t hm = (l0 && r0 == rows) ? e : ((l1 && r1 == rows) ? e + 1u : UINT32_MAX);
+        const uint32_t hb = (l0 && (c0 == 0u || r0 > rows)) ? e : ((l1 && (c1 == 0u || r1 > rows)) ? e + 1u : UINT32_MAX);
+        m   = m < hm ? m : hm;
+        bad = bad < hb ? bad : hb;
+      }
     }
     if (ballot(m != UINT32_MAX) != 0ull && m != UINT32_MAX) atomicMin(&sm.match, m);
     if (ballot(bad != UINT32_MAX) != 0ull && bad != UINT32_MAX) atomicMin(&sm.bad, bad);
@@ -214,11 +225,13 @@ __device__ __forceinline__ void rle_expand(const uint8_t* values, uint32_t t0, u
     const bool dup      = ballot(live && cnt1 == 0u) != 0;
     const uint32_t a    = __builtin_amdgcn_readfirstlane(wstart > lo ? wstart : lo);
     const uint32_t b    = __builtin_amdgcn_readfirstlane(wend < hi ? wend : hi);
-    // A window of at most RLE_BM_ROWS rows marks its run ends in the wave's
-    // bitmap once; a step then reads its 64 bits instead of collecting the
-    // ends one readlane at a time.
-    const bool use_bm = !dup && wend - wstart <= RLE_BM_ROWS && a < b;
     const uint32_t first = __builtin_amdgcn_readfirstlane(lo + ((a - lo) & ~(WAVE - 1u)));
+    // Of at most RLE_BM_ROWS rows to write, the window marks its run ends in the
+    // wave's bitmap once; a step then reads its 64 bits instead of collecting the
+    // ends one readlane at a time (asked of the whole window's rows, as it was,
+    // that held for no run longer than 64 rows on average: 10 M rows in runs of
+    // 200 took 22 us, now 12 us).
+    const bool use_bm = !dup && a < b && b - first <= RLE_BM_ROWS;
     if (use_bm) {
       // word k holds the ends in rows [first + 64 k, first + 64 k + 64):
       // bit l of a step's word is an end at row r0 + l, so a step reads one

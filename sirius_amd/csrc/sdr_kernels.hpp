@@ -16,7 +16,8 @@ struct FixedSeg {
 };
 static_assert(sizeof(FixedSeg) == 24, "FixedSeg layout");
 
-// Rows of one RLE slice (one 256-thread block decodes a slice).
+// Rows of one RLE slice (one 256-thread block decodes a slice): the knob's
+// default, at which a launch chooses by its size.
 constexpr uint32_t RLE_SLICE_ROWS = 16384;
 
 // Descriptors a launch can carry in its kernel arguments.
