@@ -446,25 +446,42 @@ void add_mask_units(const sdr_run* runs, uint32_t n, uint32_t total_rows, uint8_
   add(at, end, nullptr);
 }
 
+namespace {
+
+// Pieces and their counts in pinned memory: the kernel writes the counts and
+// reads a long list of pieces there, with no copy and no clear on the stream.
+int masks_prepare(const std::vector<MaskUnit>& units, MaskLaunch* m, void** token)
+{
+  const size_t n = units.size(), b_counts = (n * sizeof(uint32_t) + 15u) & ~size_t{15};
+  void *h = nullptr, *d = nullptr;
+  const int rc = slot_acquire(b_counts + n * sizeof(MaskUnit), 0, &h, &d, token);
+  if (rc) return rc;
+  auto* hu = reinterpret_cast<MaskUnit*>(static_cast<uint8_t*>(h) + b_counts);
+  std::memcpy(hu, units.data(), n * sizeof(MaskUnit));
+  *m = MaskLaunch{units.data(), hu, static_cast<uint32_t*>(h), static_cast<uint32_t>(n)};
+  return SDR_OK;
+}
+
+// The pieces in launches of their own.
+hipError_t launch_masks(const MaskLaunch& m, hipStream_t s)
+{
+  const bool host = m.host && m.n <= MASKS_INLINE;
+  return launch_null_mask(host ? m.host : m.units, m.n, m.counts, nullptr, s, host);
+}
+
+}  // namespace
+
 int masks_launch(const std::vector<MaskUnit>& units, hipStream_t s, const uint32_t** counts, void** token)
 {
-  // the counts are written to pinned memory by the kernel, and a long list of
-  // pieces is read from it: no copy and no clear on the stream
-  const size_t n = units.size(), b_counts = (n * sizeof(uint32_t) + 15u) & ~size_t{15};
-  const bool host = n <= MASKS_INLINE;
-  void *h = nullptr, *d = nullptr;
-  const int rc = slot_acquire(b_counts + (host ? 0u : n * sizeof(MaskUnit)), 0, &h, &d, token);
+  MaskLaunch m;
+  const int rc = masks_prepare(units, &m, token);
   if (rc) return rc;
-  auto* hc = static_cast<uint32_t*>(h);
-  auto* hu = reinterpret_cast<MaskUnit*>(static_cast<uint8_t*>(h) + b_counts);
-  if (!host) std::memcpy(hu, units.data(), n * sizeof(MaskUnit));
-  const hipError_t e =
-    launch_null_mask(host ? units.data() : hu, static_cast<uint32_t>(n), hc, nullptr, s, host);
+  const hipError_t e = launch_masks(m, s);
   if (e != hipSuccess) {
     (void)desc_release(*token, s);
     return fail(SDR_E_HIP, "null mask launch: %s", hipGetErrorString(e));
   }
-  *counts = hc;
+  *counts = m.counts;
   return SDR_OK;
 }
 
@@ -561,24 +578,32 @@ int build_batches(const std::vector<RunTarget>& targets, std::vector<Batch>& bat
 // `d`: the descriptors on the device, or null to carry them in the kernel
 // arguments from `all`.
 hipError_t launch_batches(const std::vector<Batch>& batches, const std::vector<FixedSeg>& all, const FixedSeg* d,
-                          uint32_t mode, uint32_t codec_filter, hipStream_t s, int* n_launches)
+                          uint32_t mode, uint32_t codec_filter, hipStream_t s, const MaskLaunch& masks)
 {
   hipError_t e = hipSuccess;
-  int n = 0;
   const bool host      = d == nullptr;
   const FixedSeg* segs = host ? all.data() : d;
+  if (mode != SDR_LAUNCH_PER_SEGMENT && !codec_filter) {
+    std::vector<FixedGroup> groups;
+    if (masks.n) groups.push_back({MASK_GROUP, 0, 0, masks.n, 0});
+    for (const Batch& b : batches)
+      if (b.count) groups.push_back({b.codec, b.ts, b.first, b.count, b.max_rows});
+    bool done = false;
+    e = launch_groups(groups.data(), static_cast<uint32_t>(groups.size()), segs, masks.units, masks.host,
+                      masks.counts, s, host, &done);
+    if (done || e != hipSuccess) return e;
+  }
   for (size_t i = 0; e == hipSuccess && i < batches.size(); ++i) {
     const Batch& b = batches[i];
     if (!b.count || (codec_filter && b.codec != codec_filter)) continue;
     if (mode == SDR_LAUNCH_PER_SEGMENT) {
-      for (uint32_t k = 0; k < b.count && e == hipSuccess; ++k, ++n)
+      for (uint32_t k = 0; k < b.count && e == hipSuccess; ++k)
         e = launch_batch(b, segs, b.first + k, 1, all[b.first + k].row_count, s, host);
     } else {
       e = launch_batch(b, segs, b.first, b.count, b.max_rows, s, host);
-      ++n;
     }
   }
-  if (n_launches) *n_launches = n;
+  if (e == hipSuccess && masks.n && !codec_filter) e = launch_masks(masks, s);
   return e;
 }
 
@@ -593,14 +618,14 @@ bool inline_descriptors(const std::vector<Batch>& batches, uint32_t mode)
   return true;
 }
 
-int decode_runs(const std::vector<RunTarget>& targets, hipStream_t s, uint32_t mode)
+int decode_runs(const std::vector<RunTarget>& targets, hipStream_t s, uint32_t mode, const MaskLaunch& masks)
 {
   std::vector<Batch> batches;
   std::vector<FixedSeg> all;
   build_batches(targets, batches, all);
-  if (all.empty()) return SDR_OK;
+  if (all.empty() && !masks.n) return SDR_OK;
   if (inline_descriptors(batches, mode)) {
-    const hipError_t e = launch_batches(batches, all, nullptr, mode, 0, s, nullptr);
+    const hipError_t e = launch_batches(batches, all, nullptr, mode, 0, s, masks);
     if (e != hipSuccess) return fail(SDR_E_HIP, "kernel launch failed: %s", hipGetErrorString(e));
     return SDR_OK;
   }
@@ -608,7 +633,7 @@ int decode_runs(const std::vector<RunTarget>& targets, hipStream_t s, uint32_t m
   void* token = nullptr;
   int rc = desc_acquire(all.data(), all.size() * sizeof(FixedSeg), s, &d, &token);
   if (rc) return rc;
-  const hipError_t e = launch_batches(batches, all, static_cast<FixedSeg*>(d), mode, 0, s, nullptr);
+  const hipError_t e = launch_batches(batches, all, static_cast<FixedSeg*>(d), mode, 0, s, masks);
   rc                 = desc_release(token, s);
   if (e != hipSuccess) return fail(SDR_E_HIP, "kernel launch failed: %s", hipGetErrorString(e));
   return rc;
@@ -628,32 +653,31 @@ int decode_table(sdr_column* cols, uint32_t n_cols, hipStream_t s, uint32_t mode
     cols[c].null_count = 0;
     for (uint32_t r = 0; r < cols[c].n_data; ++r) targets.push_back({&cols[c].data[r], cols[c].d_out, cols[c].type_size});
   }
-  rc = decode_runs(targets, s, mode);
-  if (rc) return rc;
-  // validity: one launch and one synchronisation for all columns
+  // validity: beside the data's blocks, with one synchronisation for all columns
   std::vector<uint32_t> masked;
   for (uint32_t c = 0; c < n_cols; ++c)
     if (cols[c].has_nulls && cols[c].n_validity && cols[c].total_rows) masked.push_back(c);
+  std::vector<MaskUnit> units;
+  std::vector<size_t> ends;
+  for (uint32_t c : masked) {
+    add_mask_units(cols[c].validity, cols[c].n_validity, cols[c].total_rows, cols[c].d_null_mask, units);
+    ends.push_back(units.size());
+  }
+  MaskLaunch masks;
+  void* token = nullptr;
+  if (!masked.empty()) rc = masks_prepare(units, &masks, &token);
+  if (!rc) rc = decode_runs(targets, s, mode, masks);
   if (!masked.empty()) {
-    std::vector<MaskUnit> units;
-    std::vector<size_t> ends;
-    for (uint32_t c : masked) {
-      add_mask_units(cols[c].validity, cols[c].n_validity, cols[c].total_rows, cols[c].d_null_mask, units);
-      ends.push_back(units.size());
-    }
-    const uint32_t* counts = nullptr;
-    void* token            = nullptr;
-    rc                     = masks_launch(units, s, &counts, &token);
-    if (rc) return rc;
-    const hipError_t e = hipStreamSynchronize(s);
+    const hipError_t e = rc ? hipErrorUnknown : hipStreamSynchronize(s);
     for (size_t i = 0, u = 0; e == hipSuccess && i < masked.size(); ++i)
-      for (; u < ends[i]; ++u) cols[masked[i]].null_count += counts[u];
+      for (; u < ends[i]; ++u) cols[masked[i]].null_count += masks.counts[u];
     if (e != hipSuccess) {
       (void)desc_release(token, s);
-      return fail(SDR_E_HIP, "null count: %s", hipGetErrorString(e));
+      return rc ? rc : fail(SDR_E_HIP, "null count: %s", hipGetErrorString(e));
     }
     slot_release_idle(token);
   }
+  if (rc) return rc;
   hipError_t e = hipPeekAtLastError();
   if (e != hipSuccess) return fail(SDR_E_HIP, "sticky launch error: %s", hipGetErrorString(e));
   return SDR_OK;
@@ -727,12 +751,10 @@ int plan_launch(sdr_plan* p, uint32_t codec, hipStream_t s)
 {
   clear_error();
   if (!p) return fail(SDR_E_INVALID_ARG, "plan is NULL");
-  hipError_t e = launch_batches(p->batches, p->all, p->d_segs, p->mode, codec, s, nullptr);
+  MaskLaunch masks;
+  if (!p->masked.empty()) masks = MaskLaunch{nullptr, p->d_units, p->d_counts, p->mask_ends.back()};
+  const hipError_t e = launch_batches(p->batches, p->all, p->d_segs, p->mode, codec, s, masks);
   if (e != hipSuccess) return fail(SDR_E_HIP, "kernel launch failed: %s", hipGetErrorString(e));
-  if (codec == 0 && !p->masked.empty()) {
-    e = launch_null_mask(p->d_units, p->mask_ends.back(), p->d_counts, nullptr, s, false);
-    if (e != hipSuccess) return fail(SDR_E_HIP, "null mask launch: %s", hipGetErrorString(e));
-  }
   return SDR_OK;
 }
 

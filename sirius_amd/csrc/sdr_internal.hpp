@@ -48,13 +48,23 @@ void add_mask_units(const sdr_run* runs, uint32_t n, uint32_t total_rows, uint8_
 // has been synchronised; desc_release(token, s) then ends the use of counts.
 int masks_launch(const std::vector<MaskUnit>& units, hipStream_t s, const uint32_t** counts, void** token);
 
+// A call's null-mask pieces: `units` in memory the device reads, and (null for a
+// plan) `host`, from which they may travel in kernel arguments; piece i's null
+// count goes to counts[i].
+struct MaskLaunch {
+  const MaskUnit* host  = nullptr;
+  const MaskUnit* units = nullptr;
+  uint32_t* counts      = nullptr;
+  uint32_t n            = 0;
+};
+
 // One fixed-width run and where its rows go.
 struct RunTarget {
   const sdr_run* run;
   void* d_out;
   uint32_t type_size;
 };
-int decode_runs(const std::vector<RunTarget>& targets, hipStream_t s, uint32_t mode);
+int decode_runs(const std::vector<RunTarget>& targets, hipStream_t s, uint32_t mode, const MaskLaunch& masks = {});
 int validate_fixed_columns(const sdr_column* cols, uint32_t n_cols);
 int validate_string_column(const sdr_string_column* col);
 // The column has DICT_FSST segments (decoded only by the per-column passes).

@@ -67,4 +67,20 @@ constexpr uint32_t MASKS_INLINE    = 120;   // pieces a launch can carry in its 
 hipError_t launch_null_mask(const MaskUnit* units, uint32_t n, uint32_t* counts, unsigned long long* total,
                             hipStream_t s, bool host);
 
+// Descriptors [first, first + count) of one codec and value width, or a call's
+// mask pieces (codec MASK_GROUP, counted from 0).
+constexpr uint32_t MASK_GROUP = 0xFFFFFFFFu;
+struct FixedGroup {
+  uint32_t codec, ts;
+  uint32_t first, count;
+  uint32_t max_rows;
+};
+// The groups in one launch (or as few as carry their descriptors in the kernel
+// arguments, with `host`), *done set; or nothing, where a single group or the
+// number of blocks asks for the codecs' own launches.  Null counts of `units` go
+// to counts[i]; units and, without `host`, segs are memory the device reads,
+// host_units (may be null) the pieces in host memory.
+hipError_t launch_groups(const FixedGroup* groups, uint32_t n_groups, const FixedSeg* segs, const MaskUnit* units,
+                         const MaskUnit* host_units, uint32_t* counts, hipStream_t s, bool host, bool* done);
+
 }  // namespace sdr
