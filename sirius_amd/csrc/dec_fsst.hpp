@@ -832,7 +832,7 @@ struct FsstPrepSmem {
   __attribute__((aligned(16))) uint32_t fields[(PREP_STAGE + 128) / 4];
   uint8_t len[256];  // code lengths of a DICT_FSST dictionary's table
   uint32_t sum[NT];
-  uint32_t huge[NT];
+  uint8_t huge[NT];
   uint32_t wave[NT / WAVE];
 };
 
@@ -1729,7 +1729,7 @@ __device__ __forceinline__ void fsst_prep_segment(const FsstSeg sg, uint32_t si,
         const bool any_hg = ballot(hg) != 0;
         if (lane == 0) {
           sm.sum[k - k0]  = tt;
-          sm.huge[k - k0] = any_hg;
+          sm.huge[k - k0] = any_hg ? 1u : 0u;
         }
       }
     __syncthreads();

@@ -16,10 +16,11 @@
 // claimed earlier by a block that started earlier.  The group kernels run as
 // parallel branches (graph nodes) or in stream order, sharing the GPU as
 // their queues drain.
-#include "dec_fixed.hpp"
 #include "dec_fsst.hpp"
-#include "dec_rle.hpp"
+#include "dec_groups.hpp"
 #include "sdr_batch.hpp"
+
+#include <algorithm>
 
 namespace sdr {
 
@@ -137,20 +138,51 @@ __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6)
                              col.state, col.offsets, col.chars, col.chars_cap, col.total_rows, spin, sm);
 }
 
-__global__ void k_batch_reset(BatchQueue* q)
+// The FSST segment pre-pass over the queue's segments with `blocks` workgroups, of
+// which this is the `block`-th; the first tells each column where its result goes.
+template <uint32_t NT>
+__device__ __forceinline__ void batch_prep(const BatchQueue* __restrict__ q, uint32_t block, uint32_t blocks,
+                                           FsstPrepSmem<NT>& sm)
 {
-  const uint32_t n = q->n_fsst_status;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) gbl(q->fsst_status)[i] = 0;
-  if (blockIdx.x == 0 && threadIdx.x < BG_COUNT) q->claimed[threadIdx.x].v = 0;
-  if (blockIdx.x == 0 && threadIdx.x == 0) q->error = 0;
+  if (block == 0)
+    for (uint32_t i = threadIdx.x; i < q->n_cols; i += NT) gbl(gload(q->fsst_cols + i).state)->result = q->results + i;
+  const uint32_t n = q->n_fsst_segs;
+  for (uint32_t i = block; i < n; i += blocks)
+    fsst_prep_segment(gload(q->fsst_segs + i), i, q->fsst_chunks, q->fsst_info, q->fsst_tabs + i, sm);
 }
 
 __global__ __launch_bounds__(BATCH_PREP_THREADS) void k_batch_fsst_prep(const BatchQueue* __restrict__ q)
 {
   __shared__ FsstPrepSmem<BATCH_PREP_THREADS> sm;
-  const uint32_t n = q->n_fsst_segs;
-  for (uint32_t i = blockIdx.x; i < n; i += gridDim.x)
-    fsst_prep_segment(gload(q->fsst_segs + i), i, q->fsst_chunks, q->fsst_info, q->fsst_tabs + i, sm);
+  batch_prep(q, blockIdx.x, gridDim.x, sm);
+}
+
+// A launch's first kernel: the arena's upload, read where the host laid it out,
+// the look-back states and the columns' results cleared.  (A copy to the device,
+// and a reset after it, took 12 us and a gap of 20 us between them.)
+__global__ __launch_bounds__(256) void k_batch_setup(u32x4* __restrict__ dst, const u32x4* __restrict__ src, uint32_t n,
+                                                     uint64_t* __restrict__ words, uint32_t n_words,
+                                                     uint64_t* __restrict__ results, uint32_t n_results)
+{
+  const uint32_t t = blockIdx.x * 256u + threadIdx.x, stride = gridDim.x * 256u;
+  for (uint32_t i = t; i < n; i += stride) gbl(dst)[i] = gbl(src)[i];
+  for (uint32_t i = t; i < n_words; i += stride) gbl(words)[i] = 0;
+  for (uint32_t i = t; i < n_results; i += stride) gbl(results)[i] = 0;
+}
+
+// The FSST pre-pass (its first `prep` workgroups), the fixed-width segments and
+// the null masks: the pre-pass waits on memory for most of its time and fills
+// half the chip, so the others run beside it.
+__global__ __launch_bounds__(BLOCK_THREADS) __attribute__((amdgpu_waves_per_eu(8))) void k_batch_front(
+  const BatchQueue* __restrict__ q, uint32_t prep, DevSegs src, GroupTable t)
+{
+  __shared__ union Smem {
+    FsstPrepSmem<BLOCK_THREADS> prep;
+    GroupSmem groups;
+    __device__ Smem() {}
+  } sm;
+  if (blockIdx.x < prep) batch_prep(q, blockIdx.x, prep, sm.prep);
+  else groups_block(src, t, blockIdx.x - prep, sm.groups);
 }
 
 namespace {
@@ -188,6 +220,31 @@ hipError_t batch_group_launch_params(uint32_t g, const void** func, uint32_t* bl
   return e;
 }
 
+hipError_t launch_batch_setup(void* dst, const void* src, size_t bytes, uint64_t* words, uint32_t n_words,
+                              FsstResult* results, uint32_t n_results, hipStream_t s)
+{
+  static_assert(sizeof(FsstResult) % sizeof(uint64_t) == 0, "cleared by words");
+  const uint32_t n = static_cast<uint32_t>(bytes / 16u), nr = n_results * static_cast<uint32_t>(sizeof(FsstResult) / 8u);
+  const uint32_t most = std::max(n, std::max(n_words, nr));
+  hipLaunchKernelGGL(k_batch_setup, dim3(std::min(512u, most / 256u + 1u)), dim3(256), 0, s, static_cast<u32x4*>(dst),
+                     static_cast<const u32x4*>(src), n, words, n_words, reinterpret_cast<uint64_t*>(results), nr);
+  return hipGetLastError();
+}
+
+hipError_t launch_batch_front(BatchQueue* q, uint32_t n_fsst_segs, const FixedGroup* groups, uint32_t n_groups,
+                              const FixedSeg* segs, const MaskUnit* units, uint32_t* counts, hipStream_t s, bool* done)
+{
+  GroupTable t{};
+  uint32_t blocks = 0;
+  *done           = n_groups == 0 || device_groups(groups, n_groups, units, counts, &t, &blocks);
+  if (!*done) return hipSuccess;
+  // a multiple of 8 blocks ahead of the groups': a block's XCD stays its own
+  const uint32_t prep = (std::min(n_fsst_segs, BATCH_PREP_GRID) + BATCH_XCDS - 1u) / BATCH_XCDS * BATCH_XCDS;
+  if (prep + blocks == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_batch_front, dim3(prep + blocks), dim3(BLOCK_THREADS), 0, s, q, prep, DevSegs{segs, 0}, t);
+  return hipGetLastError();
+}
+
 hipError_t launch_batch_fsst_prep(BatchQueue* q, hipStream_t s)
 {
   hipLaunchKernelGGL(k_batch_fsst_prep, dim3(BATCH_PREP_GRID), dim3(BATCH_PREP_THREADS), 0, s, q);
@@ -195,13 +252,6 @@ hipError_t launch_batch_fsst_prep(BatchQueue* q, hipStream_t s)
 }
 
 const void* batch_fsst_prep_kernel() { return reinterpret_cast<const void*>(k_batch_fsst_prep); }
-const void* batch_reset_kernel() { return reinterpret_cast<const void*>(k_batch_reset); }
-
-hipError_t launch_batch_reset(BatchQueue* q, hipStream_t s)
-{
-  hipLaunchKernelGGL(k_batch_reset, dim3(BATCH_RESET_GRID), dim3(256), 0, s, q);
-  return hipGetLastError();
-}
 
 hipError_t launch_batch_group(const BatchItem* items, BatchQueue* q, uint32_t g, uint32_t grid, hipStream_t s)
 {

@@ -43,11 +43,12 @@ struct sdr_batch {
   size_t stage_bytes   = 0;
   hipEvent_t upload_done = nullptr;
   bool upload_pending  = false;
-  uint8_t* h_readback  = nullptr;  // pinned copy of the look-back state and null counters
+  uint8_t* h_readback  = nullptr;  // pinned: what the columns report, then the mask pieces' null counts
   size_t readback_cap  = 0;
-  size_t readback_bytes = 0;
   size_t used_bytes    = 0;
-  size_t off_items = 0, off_cols = 0, off_chunks = 0, off_segs = 0, off_state = 0, off_nulls = 0, off_units = 0;
+  uint32_t n_fsst_segs = 0;  // row ranges of the last upload's string columns
+  size_t n_results     = 0;  // ... and these
+  size_t off_items = 0, off_cols = 0, off_chunks = 0, off_segs = 0, off_state = 0, off_units = 0;
   uint32_t n_status    = 0;
   hipEvent_t launch_done = nullptr;
   size_t n_entries     = 0;                         // queue entries of the last upload
@@ -360,7 +361,7 @@ int batch_upload(sdr_batch* b, hipStream_t s)
     n_chunks += c.n_chunks;
     n_segs += c.segs.size();
   }
-  // FsstState: FSST_STATE_WORDS + n words per column (its result is cleared to null: totals are read back)
+  // FsstState: FSST_STATE_WORDS + n words per column
   size_t state_words = 0;
   for (auto& c : b->cols) state_words += FSST_STATE_WORDS + c.n_chunks;
   size_t off                  = al(sizeof(BatchQueue));
@@ -385,9 +386,6 @@ int batch_upload(sdr_batch* b, hipStream_t s)
   off                         = al(off + b->mask_units.size() * sizeof(MaskUnit));
   b->off_state                = off;
   off                         = al(off + state_words * sizeof(uint64_t));
-  b->off_nulls                = off;
-  off                         = al(off + b->mask_units.size() * sizeof(uint32_t));
-  const size_t readback_end   = off;
   // written on the device by the FSST segment pre-pass: neither uploaded nor read back
   b->off_chunks               = off;
   off                         = al(off + n_chunks * sizeof(FsstChunk));
@@ -395,7 +393,7 @@ int batch_upload(sdr_batch* b, hipStream_t s)
   off                         = al(off + n_chunks * sizeof(FsstChunkInfo));
   const size_t off_tabs       = off;
   off                         = al(off + n_segs * sizeof(FsstSymTab));
-  const size_t upload_bytes   = b->off_state;  // the state is cleared on the device, the null counts are written there
+  const size_t upload_bytes   = b->off_state;  // the state is cleared on the device
   b->used_bytes               = off;
   if (off > b->arena_bytes) {
     if (b->d_arena) HIP_TRY(hipFree(b->d_arena));
@@ -413,13 +411,15 @@ int batch_upload(sdr_batch* b, hipStream_t s)
     HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&b->h_stage), upload_bytes + upload_bytes / 4, hipHostMallocDefault));
     b->stage_bytes = upload_bytes + upload_bytes / 4;
   }
-  b->readback_bytes = readback_end - b->off_state;  // state words and null counters
-  if (b->readback_bytes > b->readback_cap) {
+  const size_t readback_bytes = b->cols.size() * sizeof(FsstResult) + b->mask_units.size() * sizeof(uint32_t);
+  b->n_results = b->cols.size();
+  if (readback_bytes > b->readback_cap) {
+    if (b->launch_done) HIP_TRY(hipEventSynchronize(b->launch_done));  // its kernels write there
     if (b->h_readback) HIP_TRY(hipHostFree(b->h_readback));
     b->h_readback   = nullptr;
     b->readback_cap = 0;
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&b->h_readback), b->readback_bytes, hipHostMallocDefault));
-    b->readback_cap = b->readback_bytes;
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&b->h_readback), readback_bytes, hipHostMallocDefault));
+    b->readback_cap = readback_bytes;
   }
   uint8_t* h = b->h_stage;
   uint8_t* d = b->d_arena;
@@ -440,11 +440,14 @@ int batch_upload(sdr_batch* b, hipStream_t s)
   q.n_fsst_status = static_cast<uint32_t>(state_words);
   q.fsst_status   = reinterpret_cast<uint64_t*>(d + b->off_state);
   q.n_fsst_segs   = static_cast<uint32_t>(n_segs);
+  b->n_fsst_segs  = q.n_fsst_segs;
   q.spin_limit    = tune(SDR_TUNE_FSST_SPIN_LIMIT);
   q.fsst_segs     = reinterpret_cast<const FsstSeg*>(d + b->off_segs);
   q.fsst_chunks   = reinterpret_cast<FsstChunk*>(d + b->off_chunks);
   q.fsst_info     = reinterpret_cast<FsstChunkInfo*>(d + off_info);
   q.fsst_tabs     = reinterpret_cast<FsstSymTab*>(d + off_tabs);
+  q.results       = reinterpret_cast<FsstResult*>(b->h_readback);
+  q.n_cols        = static_cast<uint32_t>(b->cols.size());
   std::memcpy(h, &q, sizeof(q));
   // FSST columns, chunks, segments, state
   size_t ck = 0, sg = 0, st = 0;
@@ -494,15 +497,33 @@ int batch_upload(sdr_batch* b, hipStream_t s)
       dst.n_units    = std::min(per[g], it.n_units - u);
     }
   }
-  HIP_TRY(hipMemcpyAsync(d, h, upload_bytes, hipMemcpyHostToDevice, s));
+  HIP_TRY(launch_batch_setup(d, h, upload_bytes, q.fsst_status, q.n_fsst_status, q.results, q.n_cols, s));
   if (!b->upload_done) HIP_TRY(hipEventCreateWithFlags(&b->upload_done, hipEventDisableTiming));
   HIP_TRY(hipEventRecord(b->upload_done, s));
   b->upload_pending = true;
   return SDR_OK;
 }
 
-// The per-codec grids of the batch's fixed-width segments, one launch per
-// codec kind and value width: descriptors in the arena, in the kernel
+std::vector<FixedGroup> fixed_groups(const sdr_batch* b)
+{
+  std::vector<FixedGroup> g;
+  for (const auto& fl : b->fixed) {
+    uint32_t codec = SDR_CODEC_CONSTANT;
+    switch (fl.kind) {
+      case BK_BITPACKING: codec = SDR_CODEC_BITPACKING; break;
+      case BK_RLE: codec = SDR_CODEC_RLE; break;
+      case BK_ALP: codec = SDR_CODEC_ALP; break;
+      case BK_ALPRD: codec = SDR_CODEC_ALPRD; break;
+      case BK_COPY: codec = SDR_CODEC_UNCOMPRESSED; break;
+      default: break;
+    }
+    g.push_back({codec, fl.ts, fl.base, fl.n, fl.max_rows});
+  }
+  return g;
+}
+
+// The per-codec grids of the batch's fixed-width segments, in one launch or one
+// per codec kind and value width: descriptors in the arena, in the kernel
 // arguments (FS_INLINE) or at `slot` (FS_SLOT).
 hipError_t launch_fixed_grids(const sdr_batch* b, hipStream_t s, const FixedSeg* slot = nullptr)
 {
@@ -510,8 +531,12 @@ hipError_t launch_fixed_grids(const sdr_batch* b, hipStream_t s, const FixedSeg*
   const auto* segs = host                                 ? b->h_fsegs.data()
                      : b->fixed_src == sdr_batch::FS_SLOT ? slot
                                                           : reinterpret_cast<const FixedSeg*>(b->d_arena + b->off_fsegs);
+  const std::vector<FixedGroup> groups = fixed_groups(b);
+  bool done    = false;
+  hipError_t e = launch_groups(groups.data(), static_cast<uint32_t>(groups.size()), segs, nullptr, nullptr, nullptr, s,
+                               host, &done);
+  if (done || e != hipSuccess) return e;
   for (const auto& fl : b->fixed) {
-    hipError_t e = hipSuccess;
     switch (fl.kind) {
       case BK_BITPACKING: e = launch_bitpacking(segs, fl.base, fl.n, fl.max_rows, fl.ts, s, host); break;
       case BK_RLE: e = launch_rle(segs, fl.base, fl.n, fl.max_rows, fl.ts, s, host); break;
@@ -525,18 +550,51 @@ hipError_t launch_fixed_grids(const sdr_batch* b, hipStream_t s, const FixedSeg*
   return hipSuccess;
 }
 
-// Every kernel of a launch in stream order: the reset (when the batch holds
-// string columns or queue entries), the FSST pre-pass, the group kernels,
-// then the per-codec grids.
+// The null counts of the mask pieces, behind the columns' results.
+uint32_t* mask_counts(const sdr_batch* b)
+{
+  return reinterpret_cast<uint32_t*>(b->h_readback + b->n_results * sizeof(FsstResult));
+}
+
+// The validity masks (UNCOMPRESSED overlays) in a launch of their own.
+hipError_t launch_masks(const sdr_batch* b, hipStream_t s)
+{
+  return launch_null_mask(reinterpret_cast<const MaskUnit*>(b->d_arena + b->off_units),
+                          static_cast<uint32_t>(b->mask_units.size()), mask_counts(b), nullptr, s, false);
+}
+
+// Every kernel of a recorded launch in stream order: the FSST pre-pass, the group
+// kernels, then the per-codec grids.
 hipError_t enqueue_launch(const sdr_batch* b, BatchQueue* q, const BatchItem* items, uint32_t mask,
                           const uint32_t* grid, const uint32_t* cnt, hipStream_t s)
 {
   hipError_t e = hipSuccess;
-  if (mask || !b->cols.empty()) e = launch_batch_reset(q, s);
-  if (e == hipSuccess && (mask & (1u << BG_FSST))) e = launch_batch_fsst_prep(q, s);
+  if (mask & (1u << BG_FSST)) e = launch_batch_fsst_prep(q, s);
   for (uint32_t g = 0; e == hipSuccess && g < BG_COUNT; ++g)
     if (mask >> g & 1u) e = launch_batch_group(items, q, g, std::min(grid[g], cnt[g]), s);
   if (e == hipSuccess) e = launch_fixed_grids(b, s);
+  return e;
+}
+
+// The same without a recording, and the masks: all that does not wait for the
+// FSST pre-pass goes beside it.
+hipError_t enqueue_direct(const sdr_batch* b, BatchQueue* q, const BatchItem* items, uint32_t mask,
+                          const uint32_t* grid, const uint32_t* cnt, uint32_t n_fsst_segs, hipStream_t s)
+{
+  std::vector<FixedGroup> groups;
+  if (!b->mask_units.empty()) groups.push_back({MASK_GROUP, 0, 0, static_cast<uint32_t>(b->mask_units.size()), 0});
+  for (const FixedGroup& g : fixed_groups(b)) groups.push_back(g);
+  const uint32_t n_segs = mask & (1u << BG_FSST) ? n_fsst_segs : 0u;
+  bool done             = false;
+  hipError_t e          = launch_batch_front(q, n_segs, groups.data(), static_cast<uint32_t>(groups.size()),
+                                             reinterpret_cast<const FixedSeg*>(b->d_arena + b->off_fsegs),
+                                             reinterpret_cast<const MaskUnit*>(b->d_arena + b->off_units),
+                                             mask_counts(b), s, &done);
+  if (e == hipSuccess && !done && n_segs) e = launch_batch_fsst_prep(q, s);
+  for (uint32_t g = 0; e == hipSuccess && g < BG_COUNT; ++g)
+    if (mask >> g & 1u) e = launch_batch_group(items, q, g, std::min(grid[g], cnt[g]), s);
+  if (e == hipSuccess && !done) e = launch_fixed_grids(b, s);
+  if (e == hipSuccess && !done) e = launch_masks(b, s);
   return e;
 }
 
@@ -608,8 +666,8 @@ int batch_launch(sdr_batch* b, hipStream_t s)
     }
     HIP_TRY(hipGraphLaunch(b->gexec, s));
   } else if (b->use_graph && mask) {
-    // nodes: reset -> [FSST pre-pass] -> one persistent kernel per group, the
-    // group kernels parallel branches; node arguments are the arena
+    // nodes: [FSST pre-pass ->] one persistent kernel per group, the group
+    // kernels parallel branches; node arguments are the arena
     // addresses, entries change through the upload above, so one
     // instantiation replays every batch with the same groups
     if (!b->gexec || b->graph_arena != b->d_arena || b->graph_mask != mask || b->graph_gridopt != b->grid ||
@@ -623,19 +681,15 @@ int batch_launch(sdr_batch* b, hipStream_t s)
       b->graph = gr;
       BatchQueue* qa = q;
       const BatchItem* ia = items;
-      void* reset_args[] = {&qa};
+      void* prep_args[] = {&qa};
       hipKernelNodeParams kp{};
-      kp.func           = const_cast<void*>(batch_reset_kernel());
-      kp.gridDim        = dim3(BATCH_RESET_GRID);
-      kp.blockDim       = dim3(256);
-      kp.kernelParams   = reset_args;
-      hipGraphNode_t n_reset = nullptr, n_prep = nullptr;
-      HIP_TRY(hipGraphAddKernelNode(&n_reset, gr, nullptr, 0, &kp));
+      hipGraphNode_t n_prep = nullptr;
       if (strings) {
         kp.func     = const_cast<void*>(batch_fsst_prep_kernel());
         kp.gridDim  = dim3(BATCH_PREP_GRID);
         kp.blockDim = dim3(BATCH_PREP_THREADS);
-        HIP_TRY(hipGraphAddKernelNode(&n_prep, gr, &n_reset, 1, &kp));
+        kp.kernelParams = prep_args;
+        HIP_TRY(hipGraphAddKernelNode(&n_prep, gr, nullptr, 0, &kp));
       }
       uint32_t gids[BG_COUNT];
       for (uint32_t g = 0; g < BG_COUNT; ++g) {
@@ -650,8 +704,7 @@ int batch_launch(sdr_batch* b, hipStream_t s)
         kp.blockDim     = dim3(block);
         kp.kernelParams = args;
         hipGraphNode_t n = nullptr;
-        hipGraphNode_t dep = g == BG_FSST ? n_prep : n_reset;
-        HIP_TRY(hipGraphAddKernelNode(&n, gr, &dep, 1, &kp));
+        HIP_TRY(hipGraphAddKernelNode(&n, gr, g == BG_FSST ? &n_prep : nullptr, g == BG_FSST ? 1 : 0, &kp));
       }
       HIP_TRY(hipGraphInstantiate(&b->gexec, gr, nullptr, nullptr, 0));
       b->graph_arena   = b->d_arena;
@@ -661,20 +714,13 @@ int batch_launch(sdr_batch* b, hipStream_t s)
       b->graph_fsst    = cnt[BG_FSST];
     }
     HIP_TRY(hipGraphLaunch(b->gexec, s));
-  } else {  // also a batch with no entries: its columns' look-back state is cleared
-    HIP_TRY(enqueue_launch(b, q, items, mask, grid, cnt, s));
+  } else {
+    HIP_TRY(enqueue_direct(b, q, items, mask, grid, cnt, b->n_fsst_segs, s));
   }
+  if (b->use_graph && (mask || !b->fixed.empty())) HIP_TRY(launch_masks(b, s));
   // a column of no rows has no chunk to write its closing offset
   for (const auto& c : b->cols)
     if (c.total_rows == 0 && c.offsets) HIP_TRY(launch_fill_u8(reinterpret_cast<uint8_t*>(c.offsets), 0, sizeof(int32_t), s));
-  // validity masks (UNCOMPRESSED overlays) after the data decode
-  HIP_TRY(launch_null_mask(reinterpret_cast<const MaskUnit*>(b->d_arena + b->off_units),
-                           static_cast<uint32_t>(b->mask_units.size()),
-                           reinterpret_cast<uint32_t*>(b->d_arena + b->off_nulls), nullptr, s, false));
-  // the host reads string totals and null counts from a pinned copy once
-  // the launch has finished (batch_collect)
-  if (!b->cols.empty() || !b->masks.empty())  // otherwise there is nothing to write back
-    HIP_TRY(hipMemcpyAsync(b->h_readback, b->d_arena + b->off_state, b->readback_bytes, hipMemcpyDeviceToHost, s));
   if (!b->launch_done) HIP_TRY(hipEventCreateWithFlags(&b->launch_done, hipEventDisableTiming));
   HIP_TRY(hipEventRecord(b->launch_done, s));
   b->last_stream = s;
@@ -698,14 +744,14 @@ int batch_collect(sdr_batch* b)
 {
   if (!b->launched) return SDR_OK;
   b->launched = false;
-  const auto* st = reinterpret_cast<const uint64_t*>(b->h_readback);
-  const auto* nulls = reinterpret_cast<const uint32_t*>(b->h_readback + (b->off_nulls - b->off_state));
+  const auto* res       = reinterpret_cast<const FsstResult*>(b->h_readback);
+  const uint32_t* nulls = mask_counts(b);
   int rc = SDR_OK;
-  size_t w = 0;
   for (auto& c : b->cols) {
-    const uint32_t err   = static_cast<uint32_t>(st[w] >> 32);
-    const uint64_t total = st[w + 1];
-    w += FSST_STATE_WORDS + c.n_chunks;
+    if (res == reinterpret_cast<const FsstResult*>(b->h_readback) + b->n_results) break;  // added after the launch
+    const uint64_t err   = res->error;
+    const uint64_t total = res->total;
+    ++res;
     c.user->chars_used = total;
     c.status           = err ? SDR_E_HIP : (total > 0x7FFFFFFFull || total > c.cap) ? SDR_E_OVERFLOW : SDR_OK;
     if (c.status && !rc)

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "sdr_fsst.hpp"
+#include "sdr_kernels.hpp"
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -78,12 +79,12 @@ struct alignas(128) BatchCounter {
 
 // Queue header read by the kernels.
 struct BatchQueue {
-  BatchCounter claimed[BG_COUNT];  // next unclaimed entry of each group (reset per launch)
+  BatchCounter claimed[BG_COUNT];  // next unclaimed entry of each group (uploaded as 0)
   uint32_t first[BG_COUNT];        // each group's entries: [first, first + count)
   uint32_t count[BG_COUNT];
   uint32_t n_items;
   uint32_t error;
-  uint32_t n_fsst_status;  // status words to clear in `fsst_status`
+  uint32_t n_fsst_status;  // words of `fsst_status`, cleared by a launch's first kernel
   uint32_t spin_limit;     // look-back wait bound of the FSST chunks
   uint32_t n_fsst_segs;    // row ranges of all FSST columns, for the pre-pass
   uint32_t bp_chunk_rows[4];  // most rows a bitpacking wavefront stages at once, per width 1/2/4/8
@@ -94,11 +95,12 @@ struct BatchQueue {
   FsstSymTab* fsst_tabs;
   const FsstEntry* fsst_entries;  // the FSST group's entries (first[BG_FSST] is 0)
   const FsstColumn* fsst_cols;    // the string columns they index
+  FsstResult* results;            // what they report, in pinned memory
+  uint32_t n_cols;
 };
 
-// Fixed grids of the reset and FSST pre-pass kernels (both loop), so one
-// recorded launch serves every batch.
-constexpr uint32_t BATCH_RESET_GRID    = 64;
+// Fixed grid of the FSST pre-pass kernel (it loops), so one recorded launch
+// serves every batch.
 constexpr uint32_t BATCH_PREP_GRID     = 512;
 constexpr uint32_t BATCH_PREP_THREADS  = 512;  // the FSST pre-pass workgroup
 constexpr uint32_t BATCH_WAVES         = 4;    // wavefronts of a fixed-width group block
@@ -116,7 +118,14 @@ struct FixedLaunch {
   }
 };
 
-hipError_t launch_batch_reset(BatchQueue* q, hipStream_t s);
+// `bytes` (a multiple of 16) from pinned memory into the arena; the words and the
+// results cleared.
+hipError_t launch_batch_setup(void* dst, const void* src, size_t bytes, uint64_t* words, uint32_t n_words,
+                              FsstResult* results, uint32_t n_results, hipStream_t s);
+// The FSST pre-pass (unless n_fsst_segs is 0), the per-codec segments and the
+// masks in one launch, *done set; or nothing, where that takes too many blocks.
+hipError_t launch_batch_front(BatchQueue* q, uint32_t n_fsst_segs, const FixedGroup* groups, uint32_t n_groups,
+                              const FixedSeg* segs, const MaskUnit* units, uint32_t* counts, hipStream_t s, bool* done);
 // FSST segment pre-pass over the queue's segments.
 hipError_t launch_batch_fsst_prep(BatchQueue* q, hipStream_t s);
 // The persistent kernel of group g over `grid` blocks.
@@ -125,6 +134,5 @@ hipError_t launch_batch_group(const BatchItem* items, BatchQueue* q, uint32_t g,
 // and grid sizing).
 hipError_t batch_group_launch_params(uint32_t g, const void** func, uint32_t* block, uint32_t* blocks_per_cu);
 const void* batch_fsst_prep_kernel();
-const void* batch_reset_kernel();
 
 }  // namespace sdr
