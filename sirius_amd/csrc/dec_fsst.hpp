@@ -10,9 +10,8 @@
 // literally, a trailing escape is dropped (fsst.cu:273-281).
 //
 // One 512-thread workgroup decodes one chunk of up to FSST_CHUNK_ROWS rows.
-// Chunks are numbered in column row order and claimed in that order (an
-// atomic ticket or the position in a claimed work queue), so a chunk only
-// ever waits on chunks already running: each chunk publishes its
+// Chunks are numbered in column row order and taken in that order (by workgroup
+// number or by ticket, see FSST_UNORDERED_SHARE): each chunk publishes its
 // decoded byte count, looks back over its predecessors for the column-wide
 // exclusive prefix (a decoupled look-back), writes its rows' int32 offsets
 // and then its chars.
@@ -1176,13 +1175,13 @@ struct PlainArgs {
 // look-back for its chars offset, offsets, and the bytes (dictionary.cu:
 // 117-140, uncompressed.cu:88-120).  Every thread must call it.
 //
-// Bound by latency and instructions alike: a chunk takes a ticket, its
-// descriptors, the rows' indices, their entries and bytes, and the look-back,
+// Bound by latency and instructions alike: a chunk takes its descriptors, the
+// rows' indices, their entries and bytes, and the look-back,
 // each a round trip to memory that the next waits for.  So a thread owns RPT
 // rows, 512 apart (offsets are then stored whole lines at a time, and a chunk's
 // output leaves in row order however few rows a window holds), and its loads of
-// one kind are in flight together.  8 Mi label rows 119 -> 65 us, 2 M rows of 27
-// chars 57 -> 44 us (with the kernels' own register budgets, see k_plain).
+// one kind are in flight together.  8 Mi label rows 119 -> 57 us, 2 M rows of 27
+// chars 57 -> 35 us (with a kernel of its own and without tickets, see k_plain).
 template <uint32_t RPT, class SM>
 __device__ __forceinline__ void plain_chunk(const PlainArgs& args, SM& sm)
 {

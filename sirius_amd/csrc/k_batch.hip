@@ -10,10 +10,8 @@
 // A fixed-width group kernel's grid is its resident capacity.  Fixed-width
 // entries are independent, so block b takes entries b, b + grid, ... with no
 // claim at all; its four wavefronts decode an entry's units (an RLE slice is
-// decoded by the whole block).  The FSST kernel runs one block per chunk,
-// claimed in queue order with one atomic on the group's counter, which is
-// what lets a chunk wait on its predecessors' offsets: a predecessor was
-// claimed earlier by a block that started earlier.  The group kernels run as
+// decoded by the whole block).  The FSST kernel runs one block per chunk, in
+// queue order, which is what lets a chunk wait on its predecessors' offsets.  The group kernels run as
 // parallel branches (graph nodes) or in stream order, sharing the GPU as
 // their queues drain.
 #include "dec_fsst.hpp"
@@ -103,24 +101,26 @@ __global__ __launch_bounds__(BLOCK_THREADS) void k_bgroup_copy(const BatchItem* 
   }
 }
 
-// One block per FSST entry (the grid is the group's entry count).  The block
-// claims the next entry in queue order with one atomic, so a chunk's
-// predecessors in its column are held by blocks that started earlier, which
-// the look-back's progress needs (the per-column kernel's ticket does the
-// same).  One chunk per block, with no loop around it, keeps the kernel at
-// 80 VGPRs: three workgroups of eight waves per CU.
+// One block per FSST entry (the grid is the group's entry count): the entry of
+// its own number, or the next in queue order, claimed with one atomic, so that a
+// chunk's predecessors in its column are held by blocks that started earlier,
+// which the look-back's progress needs (as the per-column kernels do).  One chunk
+// per block, with no loop around it, keeps the kernel at 80 VGPRs: three
+// workgroups of eight waves per CU.
 __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_bgroup_fsst(
   const BatchItem* __restrict__ items, BatchQueue* __restrict__ q, uint32_t g)
 {
   __shared__ FsstSmem sm;
   __shared__ uint32_t s_idx;
   (void)items;  // the FSST group's entries are q->fsst_entries
-  // read before the claim, so they arrive while it does
   const uint32_t first = q->first[g], count = q->count[g];
   const uint32_t spin  = q->spin_limit;
-  if (threadIdx.x == 0) s_idx = atomicAdd(&q->claimed[g].v, 1u);
-  __syncthreads();
-  const uint32_t i = s_idx;
+  uint32_t i           = blockIdx.x;
+  if (q->ordered) {  // uniform
+    if (threadIdx.x == 0) s_idx = atomicAdd(&q->claimed[g].v, 1u);
+    __syncthreads();
+    i = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(s_idx)));
+  }
   if (i >= count) return;  // the grid is the entry count: never taken
   const uint32_t idx = first + i;
   // the entries list every column's chunks column by column, as the batch's

@@ -7,18 +7,27 @@
 
 namespace sdr {
 
+// The chunk of this workgroup of a launch over chunks [first, first + grid), of
+// which all before `first` are done: by its own number, or by ticket.
+__device__ __forceinline__ uint32_t chunk_number(FsstState* st, uint32_t first, uint32_t ordered)
+{
+  __shared__ uint32_t s_ticket;
+  if (!ordered) return first + blockIdx.x;
+  if (threadIdx.x == 0) s_ticket = atomicAdd(&st->ticket, 1u);
+  __syncthreads();
+  return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(s_ticket)));
+}
+
 __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_fsst(const FsstChunk* __restrict__ chunks, uint32_t n_chunks,
                                                        const FsstChunkInfo* __restrict__ info,
                                                        const FsstSymTab* __restrict__ tabs, FsstState* __restrict__ st,
                                                        int32_t* __restrict__ offsets, uint8_t* __restrict__ chars,
-                                                       uint64_t chars_cap, uint32_t total_rows, uint32_t spin_limit)
+                                                       uint64_t chars_cap, uint32_t total_rows, uint32_t spin_limit,
+                                                       uint32_t first, uint32_t ordered)
 {
   __shared__ FsstSmem sm;
-  __shared__ uint32_t s_ticket;
-  if (threadIdx.x == 0) s_ticket = atomicAdd(&st->ticket, 1u);
-  __syncthreads();
-  const uint32_t c = s_ticket;
-  if (c >= n_chunks) return;  // grid size equals chunk count; never taken
+  const uint32_t c = chunk_number(st, first, ordered);
+  if (c >= n_chunks) return;  // never taken: the grids are the chunk count
   const FsstChunk ch = chunks[c];
   fsst_chunk(ch, info[c], tabs + (ch.seg == FSST_GAP ? 0u : ch.seg), c, n_chunks, st, offsets,
                               chars, chars_cap, total_rows, spin_limit, sm);
@@ -27,21 +36,20 @@ __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6)
 // A column without FSST segments, in chunks of up to RPT * 512 rows.  A kernel
 // of its own: within k_fsst the decode was a call, which saved and restored
 // registers through scratch memory, the larger part of its time (8 Mi labels
-// 119 us, 2 M rows of 27 chars 57 us; here 65 us and 44 us).  Six wavefronts to a
+// 119 us, 2 M rows of 27 chars 57 us; here 57 us and 35 us, of which 8 us and 9 us
+// are the tickets it no longer draws).  Six wavefronts to a
 // SIMD are three workgroups to a CU; for four, rows' state spills (73 us, 70 us).
 template <uint32_t RPT>
 __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_plain(const FsstChunk* __restrict__ chunks, uint32_t n_chunks,
                                                         const FsstChunkInfo* __restrict__ info,
                                                         FsstState* __restrict__ st, int32_t* __restrict__ offsets,
                                                         uint8_t* __restrict__ chars, uint64_t chars_cap,
-                                                        uint32_t total_rows, uint32_t spin_limit)
+                                                        uint32_t total_rows, uint32_t spin_limit, uint32_t first,
+                                                        uint32_t ordered)
 {
   __shared__ PlainSmem sm;
-  __shared__ uint32_t s_ticket;
-  if (threadIdx.x == 0) s_ticket = atomicAdd(&st->ticket, 1u);
-  __syncthreads();
-  const uint32_t c = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(s_ticket)));
-  if (c >= n_chunks) return;  // grid size equals chunk count; never taken
+  const uint32_t c = chunk_number(st, first, ordered);
+  if (c >= n_chunks) return;  // never taken: the grids are the chunk count
   const FsstChunk ch     = uniform(gload(chunks + c));
   const FsstChunkInfo ci = uniform(gload(info + c));
   if (ch.seg != FSST_GAP && (ci.flags & FI_OK)) {
@@ -239,7 +247,7 @@ hipError_t launch_fsst_prep(const FsstSeg* segs, uint32_t n_segs, FsstChunk* d_c
   return hipGetLastError();
 }
 
-hipError_t launch_fsst(uint32_t chunk_rows, const FsstChunk* d_chunks, uint32_t first, uint32_t n, uint32_t n_chunks_total,
+hipError_t launch_fsst(bool ordered, uint32_t chunk_rows, const FsstChunk* d_chunks, uint32_t first, uint32_t n, uint32_t n_chunks_total,
                        const FsstChunkInfo* d_info, const FsstSymTab* d_tabs, FsstState* d_state,
                        int32_t* d_offsets, uint8_t* d_chars, uint64_t chars_cap, uint32_t total_rows,
                        hipStream_t s)
@@ -247,17 +255,16 @@ hipError_t launch_fsst(uint32_t chunk_rows, const FsstChunk* d_chunks, uint32_t 
   if (n == 0) return hipSuccess;
   // Tickets are global chunk numbers: a launch covering [first, first + n)
   // runs after every launch of lower chunks on the same stream.
-  (void)first;
-  const uint32_t spin = tune(SDR_TUNE_FSST_SPIN_LIMIT);
+  const uint32_t bound = tune(SDR_TUNE_FSST_SPIN_LIMIT), spin = ordered ? bound : bound / FSST_UNORDERED_SHARE;
   if (chunk_rows) {
     static_assert(FSST_CHUNK_ROWS == 2u * FSST_THREADS && WIDE_CHUNK_ROWS == 8u * FSST_THREADS, "one kernel a size");
     auto* const k = chunk_rows <= FSST_CHUNK_ROWS ? k_plain<2> : chunk_rows < WIDE_CHUNK_ROWS ? k_plain<4> : k_plain<8>;
     hipLaunchKernelGGL(k, dim3(n), dim3(FSST_THREADS), 0, s, d_chunks, n_chunks_total, d_info, d_state, d_offsets,
-                       d_chars, chars_cap, total_rows, spin);
+                       d_chars, chars_cap, total_rows, spin, first, ordered ? 1u : 0u);
     return hipGetLastError();
   }
   hipLaunchKernelGGL(k_fsst, dim3(n), dim3(FSST_THREADS), 0, s, d_chunks, n_chunks_total, d_info, d_tabs, d_state,
-                     d_offsets, d_chars, chars_cap, total_rows, spin);
+                     d_offsets, d_chars, chars_cap, total_rows, spin, first, ordered ? 1u : 0u);
   return hipGetLastError();
 }
 

@@ -48,6 +48,8 @@ struct sdr_batch {
   size_t used_bytes    = 0;
   uint32_t n_fsst_segs = 0;  // row ranges of the last upload's string columns
   size_t n_results     = 0;  // ... and these
+  size_t upload_bytes  = 0;  // of it, in h_stage
+  uint32_t spin_limit  = 0;  // the whole bound at the time
   size_t off_items = 0, off_cols = 0, off_chunks = 0, off_segs = 0, off_state = 0, off_units = 0;
   uint32_t n_status    = 0;
   hipEvent_t launch_done = nullptr;
@@ -353,6 +355,7 @@ int batch_upload(sdr_batch* b, hipStream_t s)
     const bool fits = std::all_of(b->fixed.begin(), b->fixed.end(),
                                   [](const FixedLaunch& fl) { return fl.n <= 2u * SEGS_INLINE; });
     b->fixed_src = fits ? sdr_batch::FS_INLINE : sdr_batch::FS_SLOT;
+    b->n_results = 0;
     return SDR_OK;
   }
   auto al = [](size_t v) { return (v + 255u) & ~size_t{255}; };
@@ -441,7 +444,10 @@ int batch_upload(sdr_batch* b, hipStream_t s)
   q.fsst_status   = reinterpret_cast<uint64_t*>(d + b->off_state);
   q.n_fsst_segs   = static_cast<uint32_t>(n_segs);
   b->n_fsst_segs  = q.n_fsst_segs;
-  q.spin_limit    = tune(SDR_TUNE_FSST_SPIN_LIMIT);
+  const uint32_t bound = tune(SDR_TUNE_FSST_SPIN_LIMIT);
+  q.ordered       = fsst_unordered(bound) ? 0u : 1u;
+  q.spin_limit    = q.ordered ? bound : bound / FSST_UNORDERED_SHARE;
+  b->spin_limit   = bound;
   q.fsst_segs     = reinterpret_cast<const FsstSeg*>(d + b->off_segs);
   q.fsst_chunks   = reinterpret_cast<FsstChunk*>(d + b->off_chunks);
   q.fsst_info     = reinterpret_cast<FsstChunkInfo*>(d + off_info);
@@ -497,6 +503,7 @@ int batch_upload(sdr_batch* b, hipStream_t s)
       dst.n_units    = std::min(per[g], it.n_units - u);
     }
   }
+  b->upload_bytes = upload_bytes;
   HIP_TRY(launch_batch_setup(d, h, upload_bytes, q.fsst_status, q.n_fsst_status, q.results, q.n_cols, s));
   if (!b->upload_done) HIP_TRY(hipEventCreateWithFlags(&b->upload_done, hipEventDisableTiming));
   HIP_TRY(hipEventRecord(b->upload_done, s));
@@ -738,13 +745,39 @@ int batch_ready(sdr_batch* b)
   return fail(SDR_E_HIP, "batch launch: %s", hipGetErrorString(e));
 }
 
+// The string columns of the finished launch once more, their chunks by ticket,
+// from the upload as it still is in the staging copy.
+int batch_strings_ordered(sdr_batch* b)
+{
+  hipStream_t s = b->last_stream;
+  auto* hq      = reinterpret_cast<BatchQueue*>(b->h_stage);
+  auto* q       = reinterpret_cast<BatchQueue*>(b->d_arena);
+  hq->ordered    = 1u;
+  hq->spin_limit = b->spin_limit;
+  HIP_TRY(launch_batch_setup(b->d_arena, b->h_stage, b->upload_bytes, hq->fsst_status, hq->n_fsst_status, hq->results,
+                             hq->n_cols, s));
+  HIP_TRY(launch_batch_fsst_prep(q, s));
+  HIP_TRY(launch_batch_group(reinterpret_cast<const BatchItem*>(b->d_arena + b->off_items), q, BG_FSST,
+                             b->entry_count[BG_FSST], s));
+  HIP_TRY(hipStreamSynchronize(s));
+  return SDR_OK;
+}
+
 // After the last launch finished: write string totals and null counts back
 // into the added columns and report look-back failures and overflow.
 int batch_collect(sdr_batch* b)
 {
   if (!b->launched) return SDR_OK;
   b->launched = false;
-  const auto* res       = reinterpret_cast<const FsstResult*>(b->h_readback);
+  const auto* res = reinterpret_cast<const FsstResult*>(b->h_readback);
+  if (b->n_results && !reinterpret_cast<const BatchQueue*>(b->h_stage)->ordered) {
+    bool again = false;  // chunks were not started in order
+    for (size_t i = 0; i < b->n_results; ++i) again = again || res[i].error;
+    if (again) {
+      const int rc = batch_strings_ordered(b);
+      if (rc) return rc;
+    }
+  }
   const uint32_t* nulls = mask_counts(b);
   int rc = SDR_OK;
   for (auto& c : b->cols) {

@@ -86,6 +86,7 @@ struct BatchQueue {
   uint32_t error;
   uint32_t n_fsst_status;  // words of `fsst_status`, cleared by a launch's first kernel
   uint32_t spin_limit;     // look-back wait bound of the FSST chunks
+  uint32_t ordered;        // their entries by ticket, see FSST_UNORDERED_SHARE
   uint32_t n_fsst_segs;    // row ranges of all FSST columns, for the pre-pass
   uint32_t bp_chunk_rows[4];  // most rows a bitpacking wavefront stages at once, per width 1/2/4/8
   uint64_t* fsst_status;   // contiguous FsstState storage of all FSST columns

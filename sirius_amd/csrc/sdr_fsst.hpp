@@ -12,6 +12,16 @@ constexpr uint32_t FSST_CHUNK_ROWS = 1024;        // rows per workgroup
 constexpr uint32_t WIDE_CHUNK_ROWS = 4096;        // ... at most, in columns of DICTIONARY segments
 constexpr uint32_t FSST_GAP        = 0xFFFFFFFFu;  // chunk of rows no segment covers
 constexpr uint32_t FSST_SPIN_LIMIT = 1u << 24;     // look-back wait bound (never reached)
+// A chunk waits on the chunks before it, so these must be running or done.  A
+// decode first takes each workgroup's number for its chunk's, the order in which
+// workgroups are in fact started, and waits a 1024th of the bound; if that was not
+// enough the decode is done again with chunks in the order of a ticket that
+// workgroups draw as they start, which needs no assumption but costs each of
+// them one of a queue of atomics on one word, 13 ns apart (16 Mi rows 293 us,
+// without 274; 2 M rows of 27 chars 44 us, 35 us; a batch's strings 182 us, 168 us).
+// A bound below 1024 (tests) goes to the tickets at once.
+constexpr uint32_t FSST_UNORDERED_SHARE = 1024;
+inline bool fsst_unordered(uint32_t spin_limit) { return spin_limit >= FSST_UNORDERED_SHARE; }
 
 // A row range of a column: a segment, or (bytes == nullptr) rows no
 // segment covers, which decode to empty strings.  Its rows are chunks
@@ -31,15 +41,15 @@ struct FsstSeg {
 static_assert(sizeof(FsstSeg) == 32, "FsstSeg layout");
 
 // Rows per chunk of a column of DICTIONARY segments alone: of 4096, 2048 and
-// 1024 the widest that still gives each of the 256 CUs a chunk.  A chunk's
-// ticket and look-back are steps that chunks take one after another (8 Mi
-// labels: 112 us in chunks of 1024 rows, 76 of 2048, 65 of 4096), but fewer
-// chunks than CUs leave some idle (a row group: 25, 26, 30 us; 512 Ki rows: 32,
-// 29, 33; 1 Mi: 42, 35, 36).
+// 1024 the widest that still gives each of the 256 CUs two chunks.  A chunk's
+// descriptors and look-back are round trips that more rows share (8 Mi labels: a
+// call of 110 us in chunks of 1024 rows, 79 of 2048, 73 of 4096), but fewer chunks
+// leave CUs idle (a row group: 24, 24, 29 us; 512 Ki rows: 28, 27, 32; 1 Mi: 35,
+// 31, 34; 2 Mi: 45, 40, 38).
 inline uint32_t label_chunk_rows(uint32_t total_rows)
 {
   uint32_t r = WIDE_CHUNK_ROWS;
-  while (r > FSST_CHUNK_ROWS && total_rows / r < 256u) r /= 2u;
+  while (r > FSST_CHUNK_ROWS && total_rows / r < 512u) r /= 2u;
   return r;
 }
 
@@ -160,7 +170,8 @@ hipError_t launch_fsst_prep(const FsstSeg* segs, uint32_t n_segs, FsstChunk* d_c
                             FsstSymTab* d_tabs, FsstState* d_state, FsstResult* result, hipStream_t s, bool host,
                             FsstSeg* copy);
 // `chunk_rows`: 0 for a column with FSST segments, else the rows of its chunks.
-hipError_t launch_fsst(uint32_t chunk_rows, const FsstChunk* d_chunks, uint32_t first, uint32_t n, uint32_t n_chunks_total,
+// `ordered`: by ticket, see FSST_UNORDERED_SHARE.
+hipError_t launch_fsst(bool ordered, uint32_t chunk_rows, const FsstChunk* d_chunks, uint32_t first, uint32_t n, uint32_t n_chunks_total,
                        const FsstChunkInfo* d_info, const FsstSymTab* d_tabs, FsstState* d_state,
                        int32_t* d_offsets, uint8_t* d_chars, uint64_t chars_cap, uint32_t total_rows,
                        hipStream_t s);

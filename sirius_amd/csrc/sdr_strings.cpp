@@ -8,6 +8,7 @@
 // pre-pass that imports symbol tables and bounds every chunk.
 #include "sdr_fsst.hpp"
 #include "sdr_internal.hpp"
+#include "sdr_tune.hpp"
 
 #include <algorithm>
 #include <cstdint>
@@ -373,18 +374,22 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
     dc.release(s, synced);
     release();
   };
-  e = launch_fsst_prep(prep_segs, n_ranges, d_chunks, d_info, d_tabs, d_state, result, s, prep_segs != d_segs,
-                       dc.any_inline ? d_segs : nullptr);
-  if (e == hipSuccess) {
-    if (mode == SDR_LAUNCH_PER_SEGMENT) {
-      for (uint32_t i = 0; e == hipSuccess && i < n_ranges; ++i)
-        e = launch_fsst(plain_rows, d_chunks, hsegs[i].first_chunk, fsst_chunk_count(hsegs[i]), n_chunks, d_info,
-                        d_tabs, d_state, col->d_offsets, col->d_chars, col->d_chars ? col->chars_capacity : 0, n, s);
-    } else {
-      e = launch_fsst(plain_rows, d_chunks, 0, n_chunks, n_chunks, d_info, d_tabs, d_state, col->d_offsets, col->d_chars,
-                      col->d_chars ? col->chars_capacity : 0, n, s);
+  auto decode = [&](bool ordered) {
+    hipError_t r = launch_fsst_prep(prep_segs, n_ranges, d_chunks, d_info, d_tabs, d_state, result, s,
+                                    prep_segs != d_segs, dc.any_inline ? d_segs : nullptr);
+    const uint64_t cap = col->d_chars ? col->chars_capacity : 0;
+    if (r == hipSuccess && mode == SDR_LAUNCH_PER_SEGMENT) {
+      for (uint32_t i = 0; r == hipSuccess && i < n_ranges; ++i)
+        r = launch_fsst(ordered, plain_rows, d_chunks, hsegs[i].first_chunk, fsst_chunk_count(hsegs[i]), n_chunks,
+                        d_info, d_tabs, d_state, col->d_offsets, col->d_chars, cap, n, s);
+    } else if (r == hipSuccess) {
+      r = launch_fsst(ordered, plain_rows, d_chunks, 0, n_chunks, n_chunks, d_info, d_tabs, d_state, col->d_offsets,
+                      col->d_chars, cap, n, s);
     }
-  }
+    return r;
+  };
+  const bool unordered = fsst_unordered(tune(SDR_TUNE_FSST_SPIN_LIMIT));
+  e                    = decode(!unordered);
   const bool masked = (col->has_nulls && col->d_null_mask) || dc.any_inline;
   std::vector<MaskUnit> units;
   const uint32_t* counts = nullptr;  // null count of each piece of the mask
@@ -411,13 +416,22 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
     uint64_t total;
   } h{};
   unsigned long long h_nulls = 0;
-  if (e == hipSuccess && scratch_mem) e = hipMemcpyAsync(&h, d_state, sizeof(h), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess && device_nulls) e = hipMemcpyAsync(&h_nulls, d_nulls, sizeof(h_nulls), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  synced = e == hipSuccess;
-  if (synced && result) {
-    h.total = result->total;
-    h.error = static_cast<uint32_t>(result->error);
+  auto finish = [&]() {
+    if (e == hipSuccess && scratch_mem) e = hipMemcpyAsync(&h, d_state, sizeof(h), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    synced = e == hipSuccess;
+    if (synced && result) {
+      h.total = result->total;
+      h.error = static_cast<uint32_t>(result->error);
+    }
+  };
+  finish();
+  if (synced && h.error && unordered) {  // chunks were not started in order: again, by ticket
+    synced = false;
+    if (result) *result = FsstResult{0, 0};
+    e = decode(true);
+    finish();
   }
   for (size_t u = 0; synced && counts && u < units.size(); ++u) h_nulls += counts[u];
   for (uint32_t u = 0; synced && dc.any_inline && u < dfsst_null_counts(n); ++u) h_nulls += dc.counts[u];

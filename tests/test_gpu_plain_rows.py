@@ -88,8 +88,19 @@ def test_dict_fsst_rows(mode):
         np.testing.assert_array_equal(g_chars, chars)
 
 
+def _label_segment(words, sel):
+    """A DICTIONARY segment of the rows words[sel] (entry 0 is NULL)."""
+    width = len(words).bit_length()
+    bits = np.packbits(((sel[:, None] >> np.arange(width)) & 1).astype(np.uint8).reshape(-1), bitorder="little")
+    ends = np.cumsum([0] + [len(x) for x in words[1:]]).astype("<u4")
+    ibo = 20 + bits.size + (-bits.size) % 4
+    body = b"".join(reversed(words[1:]))
+    head = np.array([len(body), ibo + ends.nbytes + len(body), ibo, ends.size, width], "<u4")
+    return head.tobytes() + bits.tobytes() + bytes(ibo - 20 - bits.size) + ends.tobytes() + body
+
+
 @pytest.mark.parametrize("longest", [9, 60], ids=["one_window", "windows"])
-@pytest.mark.parametrize("rows", [524_287, 524_289, 1_048_575, 1_049_601])
+@pytest.mark.parametrize("rows", [1_048_575, 1_049_601, 2_097_151, 2_097_153])
 def test_label_chunk_widths(rows, longest):
     """Columns on either side of the sizes where a chunk of labels gets wider,
     in segments that end inside chunks; rows past a window as well."""
@@ -99,7 +110,7 @@ def test_label_chunk_widths(rows, longest):
     words = [None] + [rng.integers(0, 256, n, dtype=np.uint8).tobytes() for n in range(0, longest, 1 + longest // 12)]
     b = StringBlob()
     for lo, hi in ((0, 123_457), (123_457, rows)):
-        b.add(A.DICTIONARY, dictionary_string_segment([words[k] for k in rng.integers(0, len(words), hi - lo)]), lo, hi - lo)
+        b.add(A.DICTIONARY, _label_segment(words, rng.integers(0, len(words), hi - lo)), lo, hi - lo)
     table = np.array(b.table, np.int64)
     o_offs, o_chars = oracle_string_runs(b.blob, table, rows)
     for skew in (0, 3):
