@@ -154,21 +154,23 @@ __device__ __forceinline__ void bp_group(const uint8_t* seg, uint32_t bytes, uin
     wave_lds_sync();
     const uint32_t head = stage_to_lds(lds, stream + (c0 * width) / 8u, (rows * width + 7u) / 8u);
     wave_lds_sync();
-    for (uint32_t s0 = 0; s0 < rows; s0 += WAVE * VPL) {
+    // A lane's VPL rows of the step at s0: read without a branch, which would
+    // hold each LDS read back until the one before it is done (a row group of
+    // dates, where latency is all: 5.8 -> 5.0 us); rows past the chunk read its
+    // last row again.
+    auto step = [&](uint32_t s0, auto full) {
       const uint32_t r = s0 + lane_id() * VPL;
       T v[VPL];
 #pragma unroll
       for (uint32_t i = 0; i < VPL; ++i) {
-        const uint32_t row = r + i;
-        T u                = 0;
-        if (row < rows) {
-          const uint32_t bp = head + row * width;
-          if constexpr (TS == 8) u = static_cast<T>(lds_bits64(lds, bp, width));
-          else u = static_cast<T>(lds_bits32(lds, bp, width));
-        }
-        v[i] = row < rows ? static_cast<T>(static_cast<A>(tframe) + static_cast<A>(u)) : T(0);
+        const uint32_t row = decltype(full)::value || r + i < rows ? r + i : rows - 1u;
+        const uint32_t bp  = head + row * width;
+        T u;
+        if constexpr (TS == 8) u = static_cast<T>(lds_bits64(lds, bp, width));
+        else u = static_cast<T>(lds_bits32(lds, bp, width));
+        v[i] = static_cast<T>(static_cast<A>(tframe) + static_cast<A>(u));
       }
-      if (mode == BP_DELTA_FOR) {
+      if (mode == BP_DELTA_FOR) {  // rows past the chunk come last: nothing that is stored adds them
         A loc[VPL];
         loc[0] = v[0];
 #pragma unroll
@@ -181,7 +183,10 @@ __device__ __forceinline__ void bp_group(const uint8_t* seg, uint32_t bytes, uin
         carry += readlane_acc<T>(incl, 63);
       }
       if (r < rows) store_vec<T>(out + c0 + r, v, rows - r, al);
-    }
+    };
+    uint32_t s0 = 0;
+    for (; s0 + WAVE * VPL <= rows; s0 += WAVE * VPL) step(s0, std::true_type{});
+    if (s0 < rows) step(s0, std::false_type{});
   }
 }
 
