@@ -202,8 +202,8 @@ __device__ __forceinline__ void mask_block(const MaskUnit& u, uint32_t index, ui
 // kernels, one after another, each end in a tail of few blocks and begin with
 // the latency of their first loads; a small call is nothing else: ten row groups
 // of five nullable columns took 48 us for the call, now 30 us (one launch in place
-// of five of 4 to 11 us); 10 M rows of six other widths 111 and 90 us; 16 Mi rows
-// of ALP and ALP-RD 123 and 116 us; 32 Mi nullable rows 118 and 97 us.  Eight
+// of five of 4 to 11 us); 10 M rows of six other widths 111 and 78 us; 16 Mi rows
+// of ALP and ALP-RD 123 and 112 us; 32 Mi nullable rows 118 and 97 us.  Eight
 // wavefronts a SIMD, as most of the codecs' own kernels.
 //
 // A group's blocks are consecutive and begin at a multiple of 8, so that a block

@@ -583,7 +583,9 @@ hipError_t launch_batches(const std::vector<Batch>& batches, const std::vector<F
   hipError_t e = hipSuccess;
   const bool host      = d == nullptr;
   const FixedSeg* segs = host ? all.data() : d;
-  if (mode != SDR_LAUNCH_PER_SEGMENT && !codec_filter) {
+  size_t live = masks.n ? 1 : 0;
+  for (const Batch& b : batches) live += b.count != 0;
+  if (live > 1 && mode != SDR_LAUNCH_PER_SEGMENT && !codec_filter) {
     std::vector<FixedGroup> groups;
     if (masks.n) groups.push_back({MASK_GROUP, 0, 0, masks.n, 0});
     for (const Batch& b : batches)
