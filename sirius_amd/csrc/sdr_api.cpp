@@ -68,71 +68,6 @@ void device_free(void* p, hipStream_t s)
 }
 
 namespace {
-// Pinned staging slots for descriptor uploads, kept for the process.  The
-// list's lock only guards choosing a slot (a non-blocking event query per
-// slot); allocation, the host copy and the enqueue run outside it on a slot
-// the caller holds.
-struct StageSlot {
-  void* h          = nullptr;
-  size_t cap       = 0;
-  hipEvent_t done  = nullptr;  // recorded after the slot's last copy
-  int dev          = -1;
-  bool busy        = false;    // held by a caller between choice and enqueue
-};
-std::mutex g_stage_mu;
-std::vector<StageSlot*> g_stage;  // never shrinks: held pointers stay valid
-constexpr size_t STAGE_SLOTS_MAX = 64;
-constexpr size_t STAGE_MIN_BYTES = 64u << 10;
-}  // namespace
-
-int upload_async(void* d_dst, const void* h_src, size_t bytes, hipStream_t s)
-{
-  if (bytes == 0) return SDR_OK;
-  int dev = 0;
-  HIP_TRY(hipGetDevice(&dev));
-  StageSlot* slot = nullptr;
-  bool fresh      = false;
-  {
-    std::lock_guard<std::mutex> lk(g_stage_mu);
-    for (StageSlot* sl : g_stage)
-      if (sl->dev == dev && !sl->busy && sl->cap >= bytes && hipEventQuery(sl->done) == hipSuccess) {
-        slot = sl;
-        break;
-      }
-    if (!slot && g_stage.size() < STAGE_SLOTS_MAX) {
-      slot      = new StageSlot;
-      slot->dev = dev;
-      g_stage.push_back(slot);
-      fresh = true;
-    }
-    if (slot) slot->busy = true;
-  }
-  if (!slot) {  // every slot busy: a copy from the caller's memory (the runtime stages it)
-    HIP_TRY(hipMemcpyAsync(d_dst, h_src, bytes, hipMemcpyHostToDevice, s));
-    return SDR_OK;
-  }
-  hipError_t e = hipSuccess;
-  if (fresh) {
-    size_t cap = STAGE_MIN_BYTES;
-    while (cap < bytes) cap *= 2;
-    e = hipHostMalloc(&slot->h, cap, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&slot->done, hipEventDisableTiming);
-    if (e == hipSuccess) slot->cap = cap;
-  }
-  if (e == hipSuccess) {
-    std::memcpy(slot->h, h_src, bytes);
-    e = hipMemcpyAsync(d_dst, slot->h, bytes, hipMemcpyHostToDevice, s);
-  }
-  if (e == hipSuccess) e = hipEventRecord(slot->done, s);
-  {
-    std::lock_guard<std::mutex> lk(g_stage_mu);
-    slot->busy = false;  // a slot whose set-up failed keeps cap 0 and is never chosen
-  }
-  if (e != hipSuccess) return fail(SDR_E_HIP, "descriptor upload: %s", hipGetErrorString(e));
-  return SDR_OK;
-}
-
-namespace {
 // Descriptor slots for the per-call decode: a pinned host buffer and a
 // device buffer, reused once the event recorded after the last launch that
 // read them has completed.  At most DESC_SLOTS_PER_DEV are in flight per
@@ -282,6 +217,14 @@ int slot_acquire(size_t h_bytes, size_t d_bytes, void** h_out, void** d_out, voi
 void slot_release_idle(void* token)
 {
   if (token) (void)slot_unhold(static_cast<DescSlot*>(token), SDR_OK);
+}
+
+int desc_pinned(const void* h_src, size_t bytes, void** p, void** token)
+{
+  void* d      = nullptr;
+  const int rc = slot_acquire(bytes, 0, p, &d, token);
+  if (!rc) std::memcpy(*p, h_src, bytes);
+  return rc;
 }
 
 int desc_acquire(const void* h_src, size_t bytes, hipStream_t s, void** d_out, void** token)
@@ -633,7 +576,7 @@ int decode_runs(const std::vector<RunTarget>& targets, hipStream_t s, uint32_t m
   }
   void* d     = nullptr;
   void* token = nullptr;
-  int rc = desc_acquire(all.data(), all.size() * sizeof(FixedSeg), s, &d, &token);
+  int rc = desc_pinned(all.data(), all.size() * sizeof(FixedSeg), &d, &token);
   if (rc) return rc;
   const hipError_t e = launch_batches(batches, all, static_cast<FixedSeg*>(d), mode, 0, s, masks);
   rc                 = desc_release(token, s);

@@ -351,7 +351,7 @@ int batch_upload(sdr_batch* b, hipStream_t s)
   if (b->fixed_grids && mask == 0 && b->cols.empty() && b->masks.empty() && !b->fixed.empty()) {
     // nothing on the device reads the arena: up to two launches of
     // SEGS_INLINE descriptors per grid travel in the kernel arguments,
-    // larger grids read a descriptor slot uploaded at launch
+    // larger grids read a descriptor slot in pinned memory
     const bool fits = std::all_of(b->fixed.begin(), b->fixed.end(),
                                   [](const FixedLaunch& fl) { return fl.n <= 2u * SEGS_INLINE; });
     b->fixed_src = fits ? sdr_batch::FS_INLINE : sdr_batch::FS_SLOT;
@@ -616,7 +616,7 @@ int batch_launch(sdr_batch* b, hipStream_t s)
     void* d     = nullptr;
     void* token = nullptr;
     if (b->fixed_src == sdr_batch::FS_SLOT) {
-      rc = desc_acquire(b->h_fsegs.data(), b->h_fsegs.size() * sizeof(FixedSeg), s, &d, &token);
+      rc = desc_pinned(b->h_fsegs.data(), b->h_fsegs.size() * sizeof(FixedSeg), &d, &token);
       if (rc) return rc;
     }
     const hipError_t e = launch_fixed_grids(b, s, static_cast<const FixedSeg*>(d));
