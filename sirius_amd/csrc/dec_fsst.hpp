@@ -953,20 +953,19 @@ __device__ __forceinline__ void plain_prep_segment(const FsstSeg& sg, FsstChunkI
 // DICTIONARY rows (:246-265, :324-360).  Bytes past the segment read as
 // zero; the byte a trailing escape counts is written as 0.
 
-// Calls f(byte) for the n bytes at p in order, read as aligned words, four in
-// flight (a byte at a time, each load waited for, was most of these passes).
-template <typename F>
-__device__ __forceinline__ void each_byte(const uint8_t* p, uint32_t n, F f)
+// Calls f(byte) for n bytes in order, the first of them byte `skew` (0..3) of word
+// 0 of those that w(k) reads, four words in flight (a byte at a time, each load
+// waited for, was most of the DICT_FSST passes).
+template <typename W, typename F>
+__device__ __forceinline__ void each_byte(W w, uint32_t skew, uint32_t n, F f)
 {
   if (n == 0) return;
-  const uint32_t skew          = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p) & 3u);
-  const gptr<const uint32_t> w = gbl(reinterpret_cast<const uint32_t*>(p - skew));
-  const uint64_t stop          = uint64_t{skew} + n;
-  const uint32_t last          = static_cast<uint32_t>((stop - 1u) >> 2);
+  const uint64_t stop = uint64_t{skew} + n;
+  const uint32_t last = static_cast<uint32_t>((stop - 1u) >> 2);
   for (uint32_t k = 0; k <= last; k += 4) {
     uint32_t v[4];
 #pragma unroll
-    for (uint32_t j = 0; j < 4; ++j) v[j] = w[k + j < last ? k + j : last];
+    for (uint32_t j = 0; j < 4; ++j) v[j] = w(k + j < last ? k + j : last);
 #pragma unroll
     for (uint32_t b = 0; b < 16; ++b) {
       const uint64_t y = 4ull * k + b;
@@ -975,17 +974,28 @@ __device__ __forceinline__ void each_byte(const uint8_t* p, uint32_t n, F f)
   }
 }
 
-// Decoded length of one compressed entry of n bytes at p (bytes at or past
-// `end` read as zero, i.e. as code 0): a code adds its symbol's length, an
-// escape adds one (len[255]) and skips the next byte, even past the entry's end.
-__device__ __forceinline__ uint32_t dfsst_entry_len(const uint8_t* p, uint32_t n, const uint8_t* end,
-                                                    const uint8_t* len)
+// The words at p rounded down, in memory.
+struct GlobalWords {
+  gptr<const uint32_t> w;
+  uint32_t skew;
+  __device__ __forceinline__ explicit GlobalWords(const uint8_t* p)
+    : skew(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p) & 3u))
+  {
+    w = gbl(reinterpret_cast<const uint32_t*>(p - skew));
+  }
+  __device__ __forceinline__ uint32_t operator()(uint32_t k) const { return w[k]; }
+};
+
+// Decoded length of one compressed entry of n bytes, of which those past the first
+// `in` read as zero, i.e. as code 0: a code adds its symbol's length, an escape
+// adds one (len[255]) and skips the next byte, even past the entry's end.
+template <typename W>
+__device__ __forceinline__ uint32_t dfsst_entry_len(W w, uint32_t skew, uint32_t n, uint64_t in, const uint8_t* len)
 {
-  const uint64_t in = p < end ? static_cast<uint64_t>(end - p) : 0u;
   const uint32_t n_in = n < in ? n : static_cast<uint32_t>(in);
   uint32_t dl = 0;
   bool esc    = false;
-  each_byte(p, n_in, [&](uint32_t code) {
+  each_byte(w, skew, n_in, [&](uint32_t code) {
     dl += esc ? 0u : len[code];
     esc = !esc && code == FSST_ESC;
   });
@@ -1447,46 +1457,83 @@ __device__ __forceinline__ uint32_t import_symtab(const uint8_t* seg, uint32_t b
   return len;
 }
 
+// LDS of a dictionary pre-pass: what fits of the dictionary is staged.
+constexpr uint32_t DICT_STAGE = 32768;
+template <uint32_t NT>
+struct DfsstPrepSmem {
+  FsstPrepSmem<NT> tab;
+  __attribute__((aligned(16))) uint32_t dict[(DICT_STAGE + 64) / 4];
+};
+
 // Dictionary pre-pass of one DICT_FSST segment with the calling block: the
 // entry byte offsets e_byte[0..dict_count] (scanned bit-packed lengths), for
 // the FSST modes with more than one entry the symbol table and the decoded
 // entry offsets (entry 0 empty), otherwise the byte offsets again, into
-// e_dec; out = {decoded total, inline-NULL flag}.  32-bit sums, as the
-// reference's scans.
+// e_dec; out = {decoded total, inline-NULL flag} and *pre = the bytes its
+// predecoded entries take.  32-bit sums, as the reference's scans.
+//
+// Bound by latency, there being few dictionaries: the entries go to LDS beside
+// the symbol table, two to a thread (66 dictionaries of 2000 entries: 22 us with
+// four to a thread, each walked in memory; now 17 us).
 template <uint32_t NT>
 __device__ __forceinline__ void dfsst_prep_segment(const DictFsstSeg& d, uint32_t* __restrict__ e_byte,
                                                    uint32_t* __restrict__ e_dec, FsstSymTab* __restrict__ tab,
-                                                   uint32_t* __restrict__ out, FsstPrepSmem<NT>& sm)
+                                                   uint32_t* __restrict__ out, uint32_t* __restrict__ pre,
+                                                   DfsstPrepSmem<NT>& dsm)
 {
-  const uint32_t tid = threadIdx.x;
+  constexpr uint32_t EPT = 2;  // entries of a thread
+  FsstPrepSmem<NT>& sm   = dsm.tab;
+  const uint32_t tid     = threadIdx.x;
   if (!d.valid) {  // uniform per block
-    if (tid == 0) out[0] = out[1] = 0;
+    if (tid == 0) out[0] = out[1] = *pre = 0;
     return;
   }
   const uint8_t* seg  = d.bytes;
   const uint8_t* end  = seg + d.bytes_size;
   const bool fsst     = d.mode != 0u && d.dict_count > 1u;
+  const uint8_t* dict = seg + d.off_dict;
+  const uint32_t left = d.bytes_size > d.off_dict ? d.bytes_size - d.off_dict : 0u;
+  const uint32_t bn   = !fsst ? 0u : left < DICT_STAGE ? left : DICT_STAGE;
+  const uint32_t head = block_issue<NT>(dsm.dict, dict, bn);
   const uint32_t mylen = import_symtab(seg, d.bytes_size, d.off_symtab, fsst && d.off_symtab < d.bytes_size, tab, sm);
   if (tid < 256u) sm.len[tid] = static_cast<uint8_t>(tid == FSST_ESC ? 1u : mylen);
   __syncthreads();
   const uint8_t* slens = seg + d.off_slens;
-  const uint8_t* dict  = seg + d.off_dict;
+  const uint32_t w     = d.slw;
+  const bool inside    = w && uint64_t{d.off_slens} + ((uint64_t{d.dict_count} * w + 7u) >> 3) <= d.bytes_size;
   uint32_t carry_b = 0, carry_d = 0, first_len = 0;
-  for (uint32_t k0 = 0; k0 < d.dict_count; k0 += 4u * NT) {
-    uint32_t v[4], dl[4], sb = 0, sd = 0;
+  for (uint32_t k0 = 0; k0 < d.dict_count; k0 += EPT * NT) {
+    uint32_t v[EPT], dl[EPT], sb = 0, sd = 0;
+    const uint64_t bit0          = uint64_t{k0} * w;
+    const uintptr_t at           = reinterpret_cast<uintptr_t>(slens) + (bit0 >> 3);
+    const uint32_t skew          = 8u * static_cast<uint32_t>(at & 3u) + static_cast<uint32_t>(bit0 & 7u);
+    const gptr<const uint32_t> p = gbl(reinterpret_cast<const uint32_t*>(at & ~uintptr_t{3}));
 #pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-      const uint32_t k = k0 + 4u * tid + i;
-      v[i] = k < d.dict_count ? stream_bits32(slens, end, uint64_t{k} * d.slw, d.slw) : 0u;
+    for (uint32_t i = 0; i < EPT; ++i) {
+      const uint32_t k = k0 + EPT * tid + i;
+      if (inside) v[i] = bits32_inside(p, skew + (k < d.dict_count ? k - k0 : 0u) * w, w);  // uniform
+      else v[i] = k < d.dict_count ? stream_bits32(slens, end, uint64_t{k} * w, w) : 0u;
+      v[i] = k < d.dict_count ? v[i] : 0u;
       sb += v[i];
     }
     uint32_t tb = 0;
     uint32_t run = carry_b + block_excl_scan<NT / WAVE>(sb, sm.wave, &tb);
+    const bool staged = ballot(uint64_t{run} + sb > bn) == 0;  // the wave's entries
 #pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-      const uint32_t k = k0 + 4u * tid + i;
+    for (uint32_t i = 0; i < EPT; ++i) {
+      const uint32_t k = k0 + EPT * tid + i;
       if (k < d.dict_count) e_byte[d.e_byte + k] = run;
-      dl[i] = !fsst ? v[i] : (k == 0u || k >= d.dict_count) ? 0u : dfsst_entry_len(dict + run, v[i], end, sm.len);
+      if (!fsst) {
+        dl[i] = v[i];
+      } else if (staged) {
+        const uint32_t* ew = dsm.dict + ((head + run) >> 2);
+        dl[i] = dfsst_entry_len([&](uint32_t j) { return ew[j]; }, (head + run) & 3u, v[i], v[i], sm.len);
+      } else {
+        const uint8_t* ep = dict + run;
+        const GlobalWords gw(ep);
+        dl[i] = dfsst_entry_len(gw, gw.skew, v[i], ep < end ? static_cast<uint64_t>(end - ep) : 0u, sm.len);
+      }
+      if (fsst && k == 0u) dl[i] = 0u;
       if (k == 0u) first_len = v[i];
       run += v[i];
       sd += dl[i];
@@ -1494,8 +1541,8 @@ __device__ __forceinline__ void dfsst_prep_segment(const DictFsstSeg& d, uint32_
     uint32_t td = 0;
     uint32_t rd = carry_d + block_excl_scan<NT / WAVE>(sd, sm.wave, &td);
 #pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-      const uint32_t k = k0 + 4u * tid + i;
+    for (uint32_t i = 0; i < EPT; ++i) {
+      const uint32_t k = k0 + EPT * tid + i;
       if (k < d.dict_count) e_dec[d.e_byte + k] = rd;
       rd += dl[i];
     }
@@ -1507,6 +1554,7 @@ __device__ __forceinline__ void dfsst_prep_segment(const DictFsstSeg& d, uint32_
     e_dec[d.e_byte + d.dict_count]  = carry_d;
     out[0] = carry_d;
     out[1] = d.mode != 2u && d.dict_count > 1u && first_len == 0u;
+    *pre   = fsst ? carry_d : 0u;
   }
 }
 
@@ -1573,8 +1621,9 @@ __device__ __forceinline__ void dfsst_predecode(const DictFsstSeg& d, const uint
     const uint64_t in   = p < end ? static_cast<uint64_t>(end - p) : 0u;
     const uint32_t n_in = n < in ? n : static_cast<uint32_t>(in);
     WordWriter w(out + o, out + lim);
+    const GlobalWords gw(p);
     bool esc = false;
-    each_byte(p, n_in, [&](uint32_t code) {
+    each_byte(gw, gw.skew, n_in, [&](uint32_t code) {
       if (!esc && code == FSST_ESC) {
         esc = true;
         return;
@@ -1652,14 +1701,9 @@ __device__ __forceinline__ void fsst_prep_segment(const FsstSeg sg, uint32_t si,
     plain_prep_segment<NT>(sg, info);
     return;  // uniform per segment
   }
-  if (sg.codec == SDR_CODEC_DICT_FSST) {  // bytes: the range's DictFsstSeg, pinned; pad: 1 if valid
-    // the chunks read it in device memory: the range's symbol table, whose
-    // entries are predecoded by now, gives way to it
-    static_assert(sizeof(DictFsstSeg) <= sizeof(FsstSymTab) && sizeof(DictFsstSeg) <= 4u * WAVE, "a word per lane");
-    if (tid < sizeof(DictFsstSeg) / 4u)
-      gbl(reinterpret_cast<uint32_t*>(tab))[tid] = gbl(reinterpret_cast<const uint32_t*>(sg.bytes))[tid];
+  if (sg.codec == SDR_CODEC_DICT_FSST) {  // bytes: the range's DictFsstSeg; pad: 1 if valid
     for (uint32_t k = tid; uint64_t{k} * sg.chunk_rows < sg.row_count; k += NT) {
-      FsstChunkInfo ci{reinterpret_cast<const uint8_t*>(tab), 0u, 0u, 0u, FI_DFSST | (sg.pad ? FI_OK : 0u), 0u, 0u};
+      FsstChunkInfo ci{sg.bytes, 0u, 0u, 0u, FI_DFSST | (sg.pad ? FI_OK : 0u), 0u, 0u};
       const gptr<u32x4> dst = gbl(reinterpret_cast<u32x4*>(info + sg.first_chunk + k));
       const u32x8 cv        = __builtin_bit_cast(u32x8, ci);
       dst[0]                = cv.lo;

@@ -87,32 +87,41 @@ struct RangesInline {
   __device__ __forceinline__ FsstSeg at(uint32_t i) const { return uniform(seg[i]); }
 };
 
-template <class Src>
-__global__ __launch_bounds__(Src::THREADS) void k_fsst_prep(Src src, uint32_t n_segs, FsstChunk* __restrict__ chunks,
-                                                            FsstChunkInfo* __restrict__ info,
-                                                            FsstSymTab* __restrict__ tabs, FsstState* __restrict__ st,
-                                                            FsstResult* __restrict__ result,
-                                                            FsstSeg* __restrict__ copy)
+template <uint32_t NT, class Src>
+__device__ __forceinline__ void fsst_prep_block(const Src& src, uint32_t n_segs, uint32_t block, uint32_t blocks,
+                                                FsstChunk* __restrict__ chunks, FsstChunkInfo* __restrict__ info,
+                                                FsstSymTab* __restrict__ tabs, FsstState* __restrict__ st,
+                                                FsstResult* __restrict__ result, FsstSeg* __restrict__ copy,
+                                                FsstPrepSmem<NT>& sm)
 {
-  __shared__ FsstPrepSmem<Src::THREADS> sm;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  if (block == 0 && threadIdx.x == 0) {
     st->ticket = 0;
     st->error  = 0;
     st->total  = 0;
     st->result = result;
   }
-  for (uint32_t i = blockIdx.x; i < n_segs; i += gridDim.x) {
+  for (uint32_t i = block; i < n_segs; i += blocks) {
     const FsstSeg sg = src.at(i);
-    for (uint32_t k = threadIdx.x; uint64_t{k} * sg.chunk_rows < sg.row_count; k += Src::THREADS)
+    for (uint32_t k = threadIdx.x; uint64_t{k} * sg.chunk_rows < sg.row_count; k += NT)
       gbl(st->status)[sg.first_chunk + k] = 0;
     if (copy && threadIdx.x == 0) copy[i] = sg;
     fsst_prep_segment(sg, i, chunks, info, tabs + i, sm);
   }
 }
 
+template <class Src>
+__global__ __launch_bounds__(Src::THREADS) void k_fsst_prep(Src src, uint32_t n_segs, FsstChunk* __restrict__ chunks,
+                                                            FsstChunkInfo* __restrict__ info,
+                                                            FsstSymTab* __restrict__ tabs, FsstState* __restrict__ st,
+                                                            FsstResult* __restrict__ result)
+{
+  __shared__ FsstPrepSmem<Src::THREADS> sm;
+  fsst_prep_block(src, n_segs, blockIdx.x, gridDim.x, chunks, info, tabs, st, result, nullptr, sm);
+}
+
 // ---- DICT_FSST passes ----
 
-constexpr uint32_t DFSST_PREP_THREADS = 512;  // 66 dictionaries: 256 threads 38 us, 512 24 us
+constexpr uint32_t DFSST_PREP_THREADS = 1024;
 
 __global__ void k_dfsst_headers(const FsstSeg* __restrict__ segs, uint32_t n, uint32_t* __restrict__ hdr)
 {
@@ -124,43 +133,81 @@ __global__ void k_dfsst_headers(const FsstSeg* __restrict__ segs, uint32_t n, ui
   }
 }
 
+// The descriptors come in pinned memory and go to d_desc as well, which the passes
+// after this one read.
 __global__ __launch_bounds__(DFSST_PREP_THREADS) void k_dfsst_prep(const DictFsstSeg* __restrict__ dseg, uint32_t n,
-                                                             uint32_t* __restrict__ e_byte,
-                                                             uint32_t* __restrict__ e_dec,
-                                                             FsstSymTab* __restrict__ tabs, uint32_t* __restrict__ out)
+                                                                   DfsstWork wk, FsstSymTab* __restrict__ tabs,
+                                                                   uint32_t* __restrict__ out)
 {
-  __shared__ FsstPrepSmem<DFSST_PREP_THREADS> sm;
+  __shared__ DfsstPrepSmem<DFSST_PREP_THREADS> sm;
   for (uint32_t j = blockIdx.x; j < n; j += gridDim.x) {
-    const DictFsstSeg d = gload(dseg + j);
-    dfsst_prep_segment(d, e_byte, e_dec, tabs + d.range, out + 2u * j, sm);
+    const DictFsstSeg d = uniform(gload(dseg + j));
+    if (threadIdx.x == 0) wk.desc[j] = d;
+    dfsst_prep_segment(d, wk.e_byte, wk.e_dec, tabs + d.range, out + 2u * j, wk.pre_size + j, sm);
     __syncthreads();  // sm is reused by the next segment
   }
 }
 
+// Eight workgroups share a segment's entries, predecoded to `pre` behind those of
+// the segments before it; beside them the column's segment pre-pass, which needs
+// nothing of theirs.
 constexpr uint32_t PREDECODE_THREADS = 256;  // one code of the table per thread
-
-// grid.y: segments; grid.x blocks share a segment's entries
-__global__ __launch_bounds__(PREDECODE_THREADS) void k_dfsst_predecode(const DictFsstSeg* __restrict__ dseg,
-                                                                       const uint32_t* __restrict__ e_byte,
-                                                                       const FsstSymTab* __restrict__ tabs)
+constexpr uint32_t PREDECODE_SHARE   = 8;
+struct PredecodeSmem {
+  uint64_t sym[256];
+  uint8_t len[256];
+};
+__device__ __forceinline__ void dfsst_predecode_block(const DfsstWork& wk, uint32_t j, uint32_t part,
+                                                      const FsstSymTab* __restrict__ tabs, PredecodeSmem& sm)
 {
-  __shared__ uint64_t sym[256];
-  __shared__ uint8_t len[256];
-  const DictFsstSeg d = gload(dseg + blockIdx.y);
+  DictFsstSeg d = uniform(gload(wk.desc + j));
   if (!d.valid || d.mode == 0u || d.dict_count <= 1u) return;  // uniform per block
-  sym[threadIdx.x] = gbl(tabs[d.range].sym)[threadIdx.x];
-  len[threadIdx.x] = gbl(tabs[d.range].len)[threadIdx.x];
+  uint64_t at = 0;
+  for (uint32_t i = lane_id(); i < j; i += WAVE) at += gbl(wk.pre_size)[i];
+  at         = readlane_u64(wave_incl_sum_u64(at), WAVE - 1);
+  d.src      = wk.pre + at;
+  d.src_size = gbl(wk.pre_size)[j];
+  if (part == 0 && threadIdx.x == 0) {
+    wk.desc[j].src      = d.src;
+    wk.desc[j].src_size = d.src_size;
+  }
+  sm.sym[threadIdx.x] = gbl(tabs[d.range].sym)[threadIdx.x];
+  sm.len[threadIdx.x] = gbl(tabs[d.range].len)[threadIdx.x];
   __syncthreads();
-  dfsst_predecode(d, e_byte, sym, len, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+  dfsst_predecode(d, wk.e_byte, sm.sym, sm.len, part * PREDECODE_THREADS + threadIdx.x,
+                  PREDECODE_SHARE * PREDECODE_THREADS);
+}
+
+template <class Src>
+__global__ __launch_bounds__(PREDECODE_THREADS) void k_dfsst_front(Src src, uint32_t n_segs, uint32_t prep, DfsstWork wk,
+                                                                   FsstChunk* __restrict__ chunks,
+                                                                   FsstChunkInfo* __restrict__ info,
+                                                                   FsstSymTab* __restrict__ tabs,
+                                                                   FsstState* __restrict__ st,
+                                                                   FsstResult* __restrict__ result,
+                                                                   FsstSeg* __restrict__ copy)
+{
+  __shared__ union Smem {
+    FsstPrepSmem<PREDECODE_THREADS> prep;
+    PredecodeSmem pre;
+    __device__ Smem() {}
+  } sm;
+  if (blockIdx.x < prep) {
+    fsst_prep_block(src, n_segs, blockIdx.x, prep, chunks, info, tabs, st, result, copy, sm.prep);
+  } else {
+    const uint32_t b = blockIdx.x - prep;
+    dfsst_predecode_block(wk, b / PREDECODE_SHARE, b % PREDECODE_SHARE, tabs, sm.pre);
+  }
 }
 
 // DICT_FSST's inline NULLs: a thread per byte of the null mask, a tile of 256
 // bytes at a time, whose ranges the workgroup finds once (a search by every row,
 // and each row's index in turn, took 15 us for 2 M rows; now 7 us).  The rows
-// cleared are counted per workgroup, into pinned memory.
+// cleared are counted per workgroup, into pinned memory.  `fresh`: the mask is all
+// valid and not written yet.
 __global__ __launch_bounds__(256) void k_dfsst_nulls(const FsstSeg* __restrict__ segs, uint32_t n_ranges,
-                                                     const FsstSymTab* __restrict__ tabs, uint8_t* __restrict__ mask,
-                                                     uint32_t total_rows, uint32_t* __restrict__ counts)
+                                                     uint8_t* __restrict__ mask, uint32_t total_rows, uint32_t fresh,
+                                                     uint32_t* __restrict__ counts)
 {
   __shared__ uint32_t s_sum[4];
   uint32_t cleared = 0;
@@ -173,18 +220,18 @@ __global__ __launch_bounds__(256) void k_dfsst_nulls(const FsstSeg* __restrict__
       else hi = mid;
     }
     const bool mine   = row0 < total_rows;
-    const uint32_t m0 = mine ? mask[row0 / 8u] : 0u;
+    const uint32_t m0 = !mine ? 0u : fresh ? 0xFFu : mask[row0 / 8u];
     uint32_t m        = total_rows - row0 < 8u && mine ? m0 & ((1u << (total_rows - row0)) - 1u) : m0;
     const uint32_t in = m;
     for (uint32_t k = lo; k < n_ranges; ++k) {
       const FsstSeg sg = uniform(gload(segs + k));
       if (sg.col_row >= t0 + 2048u) break;
       if (sg.codec != SDR_CODEC_DICT_FSST || !sg.bytes) continue;
-      const DictFsstSeg d = uniform(gload(reinterpret_cast<const DictFsstSeg*>(tabs + k)));
+      const DictFsstSeg d = uniform(gload(reinterpret_cast<const DictFsstSeg*>(sg.bytes)));
       if (m && uint64_t{sg.col_row} + sg.row_count > row0 && sg.col_row < uint64_t{row0} + 8u)
         m = dfsst_null_byte(m, row0, sg, d);
     }
-    if (m != in) {
+    if (m != in || (fresh && mine)) {
       mask[row0 / 8u] = static_cast<uint8_t>(m0 & ~(in & ~m));
       cleared += static_cast<uint32_t>(__builtin_popcount(in & ~m));
     }
@@ -203,46 +250,47 @@ hipError_t launch_dfsst_headers(const FsstSeg* d_segs, uint32_t n_ranges, uint32
   return hipGetLastError();
 }
 
-hipError_t launch_dfsst_prep(const DictFsstSeg* d_dseg, uint32_t n_dseg, uint32_t* d_e_byte, uint32_t* d_e_dec,
-                             FsstSymTab* d_tabs, uint32_t* d_out, hipStream_t s)
+hipError_t launch_dfsst_prep(const DictFsstSeg* dseg, uint32_t n_dseg, const DfsstWork& wk, FsstSymTab* d_tabs,
+                             uint32_t* out, hipStream_t s)
 {
   if (n_dseg == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_dfsst_prep, dim3(n_dseg < 4096u ? n_dseg : 4096u), dim3(DFSST_PREP_THREADS), 0, s, d_dseg, n_dseg,
-                     d_e_byte, d_e_dec, d_tabs, d_out);
+  hipLaunchKernelGGL(k_dfsst_prep, dim3(n_dseg < 4096u ? n_dseg : 4096u), dim3(DFSST_PREP_THREADS), 0, s, dseg, n_dseg,
+                     wk, d_tabs, out);
   return hipGetLastError();
 }
 
-hipError_t launch_dfsst_predecode(const DictFsstSeg* d_dseg, uint32_t n_dseg, const uint32_t* d_e_byte,
-                                  const FsstSymTab* d_tabs, hipStream_t s)
-{
-  if (n_dseg == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_dfsst_predecode, dim3(8, n_dseg), dim3(PREDECODE_THREADS), 0, s, d_dseg, d_e_byte, d_tabs);
-  return hipGetLastError();
-}
-
-hipError_t launch_dfsst_nulls(const FsstSeg* d_segs, uint32_t n_ranges, const FsstSymTab* d_tabs, uint8_t* d_mask,
-                              uint32_t total_rows, uint32_t* counts, hipStream_t s)
+hipError_t launch_dfsst_nulls(const FsstSeg* d_segs, uint32_t n_ranges, uint8_t* d_mask, uint32_t total_rows,
+                              bool fresh, uint32_t* counts, hipStream_t s)
 {
   if (total_rows == 0 || n_ranges == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_dfsst_nulls, dim3(dfsst_null_counts(total_rows)), dim3(256), 0, s, d_segs, n_ranges, d_tabs,
-                     d_mask, total_rows, counts);
+  hipLaunchKernelGGL(k_dfsst_nulls, dim3(dfsst_null_counts(total_rows)), dim3(256), 0, s, d_segs, n_ranges, d_mask,
+                     total_rows, fresh ? 1u : 0u, counts);
   return hipGetLastError();
 }
 
 hipError_t launch_fsst_prep(const FsstSeg* segs, uint32_t n_segs, FsstChunk* d_chunks, FsstChunkInfo* d_info,
                             FsstSymTab* d_tabs, FsstState* d_state, FsstResult* result, hipStream_t s, bool host,
-                            FsstSeg* copy)
+                            const DfsstWork* wk, uint32_t n_dseg, FsstSeg* copy)
 {
   if (n_segs == 0) return hipSuccess;
-  const dim3 grid(n_segs < 4096u ? n_segs : 4096u);
+  const uint32_t blocks = n_segs < 4096u ? n_segs : 4096u;
+  auto go = [&](auto src) {
+    using S = decltype(src);
+    if (wk) {
+      const uint32_t pre = wk->pre ? n_dseg * PREDECODE_SHARE : 0u;
+      hipLaunchKernelGGL((k_dfsst_front<S>), dim3(blocks + pre), dim3(PREDECODE_THREADS), 0, s, src, n_segs, blocks, *wk,
+                         d_chunks, d_info, d_tabs, d_state, result, copy);
+    } else {
+      hipLaunchKernelGGL((k_fsst_prep<S>), dim3(blocks), dim3(S::THREADS), 0, s, src, n_segs, d_chunks, d_info, d_tabs,
+                         d_state, result);
+    }
+  };
   if (host && n_segs <= RANGES_INLINE) {
     RangesInline ri{};
     std::memcpy(ri.seg, segs, size_t{n_segs} * sizeof(FsstSeg));
-    hipLaunchKernelGGL((k_fsst_prep<RangesInline>), grid, dim3(RangesInline::THREADS), 0, s, ri, n_segs, d_chunks, d_info, d_tabs, d_state,
-                       result, copy);
+    go(ri);
   } else {
-    hipLaunchKernelGGL((k_fsst_prep<DevRanges>), grid, dim3(DevRanges::THREADS), 0, s, DevRanges{segs}, n_segs, d_chunks, d_info, d_tabs,
-                       d_state, result, copy);
+    go(DevRanges{segs});
   }
   return hipGetLastError();
 }

@@ -120,15 +120,25 @@ struct DictFsstSeg {
 };
 static_assert(sizeof(DictFsstSeg) == 72, "DictFsstSeg layout");
 
+// Device memory of a column's DICT_FSST passes.
+struct DfsstWork {
+  DictFsstSeg* desc;   // the descriptors
+  uint32_t* pre_size;  // bytes of each segment's predecoded entries
+  uint32_t* e_byte;    // entry offsets: compressed ...
+  uint32_t* e_dec;     // ... and decoded
+  uint8_t* pre;        // the predecoded entries, segment by segment (null: none)
+};
+
 // DICT_FSST passes (k_fsst.hip): the 16-byte headers of the DICT_FSST
 // ranges into hdr[4 * i] (ranges of other codecs are skipped); the
 // per-segment dictionary pre-pass (byte and decoded entry offsets, symbol
 // table, per-segment decoded total and inline-NULL flag into out[2 * j]);
-// the predecode of FSST-mode entries; and the inline-NULL marking of a
-// column's mask, with the rows it clears in each of dfsst_null_counts()
-// counts.  Ranges, descriptors, headers, `out` and `counts` are pinned host
-// memory, which the passes read and write in place; the last pass takes ranges
-// and descriptors from where the segment pre-pass left them on the device.
+// the predecode of FSST-mode entries, beside the segment pre-pass
+// (launch_fsst_prep); and the inline-NULL marking of a column's mask (`fresh`: all
+// valid, not written yet), with the rows it clears in each of
+// dfsst_null_counts() counts.  Ranges, descriptors, headers, `out` and `counts`
+// are pinned host memory, which the passes read and write in place; the last pass
+// takes the ranges from the copy that the segment pre-pass left on the device.
 constexpr uint32_t DFSST_NULL_COUNTS = 2048;  // at most
 inline uint32_t dfsst_null_counts(uint32_t total_rows)
 {
@@ -136,12 +146,10 @@ inline uint32_t dfsst_null_counts(uint32_t total_rows)
   return tiles < DFSST_NULL_COUNTS ? tiles : DFSST_NULL_COUNTS;
 }
 hipError_t launch_dfsst_headers(const FsstSeg* segs, uint32_t n_ranges, uint32_t* hdr, hipStream_t s);
-hipError_t launch_dfsst_prep(const DictFsstSeg* dseg, uint32_t n_dseg, uint32_t* d_e_byte, uint32_t* d_e_dec,
-                             FsstSymTab* d_tabs, uint32_t* out, hipStream_t s);
-hipError_t launch_dfsst_predecode(const DictFsstSeg* dseg, uint32_t n_dseg, const uint32_t* d_e_byte,
-                                  const FsstSymTab* d_tabs, hipStream_t s);
-hipError_t launch_dfsst_nulls(const FsstSeg* d_segs, uint32_t n_ranges, const FsstSymTab* d_tabs, uint8_t* d_mask,
-                              uint32_t total_rows, uint32_t* counts, hipStream_t s);
+hipError_t launch_dfsst_prep(const DictFsstSeg* dseg, uint32_t n_dseg, const DfsstWork& wk, FsstSymTab* d_tabs,
+                             uint32_t* out, hipStream_t s);
+hipError_t launch_dfsst_nulls(const FsstSeg* d_segs, uint32_t n_ranges, uint8_t* d_mask, uint32_t total_rows,
+                              bool fresh, uint32_t* counts, hipStream_t s);
 
 // What a column decode reports to the host, in pinned memory.
 struct FsstResult {
@@ -164,11 +172,12 @@ constexpr uint32_t FSST_STATE_WORDS = 3;  // 8-byte words before status
 // Segment pre-pass over n_segs ranges: writes the chunk list, the chunks'
 // FsstChunkInfo and the segments' symbol tables, and sets up the state (its
 // result may be null).  With `host` the ranges are pinned host memory: a few
-// travel in the kernel arguments, each of many is read by its block.  `copy`, if
-// set, receives the ranges in device memory.
+// travel in the kernel arguments, each of many is read by its block.  With `wk` the
+// n_dseg DICT_FSST segments' entries are predecoded in the same launch, and
+// `copy`, if set, receives the ranges in device memory.
 hipError_t launch_fsst_prep(const FsstSeg* segs, uint32_t n_segs, FsstChunk* d_chunks, FsstChunkInfo* d_info,
                             FsstSymTab* d_tabs, FsstState* d_state, FsstResult* result, hipStream_t s, bool host,
-                            FsstSeg* copy);
+                            const DfsstWork* wk, uint32_t n_dseg, FsstSeg* copy);
 // `chunk_rows`: 0 for a column with FSST segments, else the rows of its chunks.
 // `ordered`: by ticket, see FSST_UNORDERED_SHARE.
 hipError_t launch_fsst(bool ordered, uint32_t chunk_rows, const FsstChunk* d_chunks, uint32_t first, uint32_t n, uint32_t n_chunks_total,

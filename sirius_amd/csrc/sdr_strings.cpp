@@ -123,6 +123,8 @@ struct DictFsstCall {
   uint32_t* out     = nullptr;
   uint32_t* counts  = nullptr;
   CallMemory offsets, pre;
+  DfsstWork work{};  // within the two
+  uint32_t n_d    = 0;
   bool any_inline = false;
   static size_t pinned_bytes(size_t n_ranges)
   {
@@ -148,9 +150,9 @@ uint32_t al8(uint32_t v) { return (v + 7u) & ~7u; }
 // host round trips as there): read the headers of the DICT_FSST ranges,
 // fill their descriptors (region offsets, validity, :516-525), run the
 // dictionary pre-pass, read back each segment's decoded total and inline-
-// NULL flag, predecode the FSST entries, then point the ranges (pinned, as all
-// that passes between host and passes here) at their descriptors (bytes) with
-// their validity (pad).
+// NULL flag and make room for the FSST entries, then point the ranges (pinned, as
+// all that passes between host and passes here) at their descriptors on the device
+// (bytes) with their validity (pad).
 int dict_fsst_phase(const sdr_string_column* col, FsstSeg* segs, uint32_t n_ranges, FsstSymTab* d_tabs, hipStream_t s,
                     DictFsstCall& dc)
 {
@@ -189,21 +191,25 @@ int dict_fsst_phase(const sdr_string_column* col, FsstSeg* segs, uint32_t n_rang
     dc.desc[n_d++] = d;
   }
   if (n_d == 0) return SDR_OK;
-  const size_t b_e = (std::max<uint64_t>(1, n_e) * 4u + 255u) & ~size_t{255};
-  int rc           = dc.offsets.get(2u * b_e, s);
+  auto al           = [](size_t v) { return (v + 255u) & ~size_t{255}; };
+  const size_t b_e  = al(std::max<uint64_t>(1, n_e) * 4u), b_desc = al(n_d * sizeof(DictFsstSeg));
+  int rc            = dc.offsets.get(2u * b_e + b_desc + n_d * sizeof(uint32_t), s);
   if (rc) return rc;
-  auto* d_e_byte = reinterpret_cast<uint32_t*>(dc.offsets.p);
-  auto* d_e_dec  = reinterpret_cast<uint32_t*>(dc.offsets.p + b_e);
+  dc.n_d           = n_d;
+  dc.work.e_byte   = reinterpret_cast<uint32_t*>(dc.offsets.p);
+  dc.work.e_dec    = reinterpret_cast<uint32_t*>(dc.offsets.p + b_e);
+  dc.work.desc     = reinterpret_cast<DictFsstSeg*>(dc.offsets.p + 2u * b_e);
+  dc.work.pre_size = reinterpret_cast<uint32_t*>(dc.offsets.p + 2u * b_e + b_desc);
   for (uint32_t j = 0; j < n_d; ++j) {
     DictFsstSeg& d = dc.desc[j];
-    d.e            = d_e_dec + d.e_byte;
+    d.e            = dc.work.e_dec + d.e_byte;
     if (d.mode == 0u || d.dict_count <= 1u) {  // rows copy raw dict bytes
       d.src      = d.bytes + d.off_dict;
       d.src_size = d.bytes_size > d.off_dict ? d.bytes_size - d.off_dict : 0u;
     }
   }
   // 3. dictionary pre-pass, per-segment totals and inline-NULL flags
-  e = launch_dfsst_prep(dc.desc, n_d, d_e_byte, d_e_dec, d_tabs, dc.out, s);
+  e = launch_dfsst_prep(dc.desc, n_d, dc.work, d_tabs, dc.out, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return fail(SDR_E_HIP, "DICT_FSST dictionary pre-pass: %s", hipGetErrorString(e));
   uint64_t n_pre = 0;
@@ -213,25 +219,16 @@ int dict_fsst_phase(const sdr_string_column* col, FsstSeg* segs, uint32_t n_rang
   }
   if (dc.any_inline && col->total_rows && !col->d_null_mask)
     return fail(SDR_E_INVALID_ARG, "DICT_FSST segments hold inline NULLs (entry 0) and d_null_mask is NULL");
-  // 4. predecode
+  // 4. room for the predecoded entries, which the segment pre-pass's launch fills
   if (n_pre) {
     rc = dc.pre.get(n_pre, s);
     if (rc) return rc;
-    uint64_t at = 0;
-    for (uint32_t j = 0; j < n_d; ++j) {
-      DictFsstSeg& d = dc.desc[j];
-      if (!d.valid || d.mode == 0u || d.dict_count <= 1u) continue;
-      d.src      = dc.pre.p + at;
-      d.src_size = dc.out[2u * j];
-      at += dc.out[2u * j];
-    }
-    e = launch_dfsst_predecode(dc.desc, n_d, d_e_byte, d_tabs, s);
-    if (e != hipSuccess) return fail(SDR_E_HIP, "DICT_FSST predecode: %s", hipGetErrorString(e));
+    dc.work.pre = dc.pre.p;
   }
   // 5. the ranges now name their descriptors
   for (uint32_t i = 0; i < n_ranges; ++i)
     if (range_d[i] != ~0u) {
-      segs[i].bytes = reinterpret_cast<const uint8_t*>(dc.desc + range_d[i]);
+      segs[i].bytes = reinterpret_cast<const uint8_t*>(dc.work.desc + range_d[i]);
       segs[i].pad   = dc.desc[range_d[i]].valid;
     }
   return SDR_OK;
@@ -376,7 +373,8 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
   };
   auto decode = [&](bool ordered) {
     hipError_t r = launch_fsst_prep(prep_segs, n_ranges, d_chunks, d_info, d_tabs, d_state, result, s,
-                                    prep_segs != d_segs, dc.any_inline ? d_segs : nullptr);
+                                    prep_segs != d_segs, dc.n_d ? &dc.work : nullptr, dc.n_d,
+                                    dc.any_inline ? d_segs : nullptr);
     const uint64_t cap = col->d_chars ? col->chars_capacity : 0;
     if (r == hipSuccess && mode == SDR_LAUNCH_PER_SEGMENT) {
       for (uint32_t i = 0; r == hipSuccess && i < n_ranges; ++i)
@@ -395,7 +393,8 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
   const uint32_t* counts = nullptr;  // null count of each piece of the mask
   void* counts_token     = nullptr;
   const bool device_nulls = masked && scratch_mem;  // nothing may be allocated for the pieces' counts
-  if (e == hipSuccess && masked) {
+  const bool runs = col->has_nulls && col->n_validity;
+  if (e == hipSuccess && masked && (runs || !dc.any_inline)) {
     add_mask_units(col->validity, col->has_nulls ? col->n_validity : 0u, n, col->d_null_mask, units);
     if (device_nulls) e = launch_fill_u8(reinterpret_cast<uint8_t*>(d_nulls), 0, sizeof(unsigned long long), s);
     if (e == hipSuccess && scratch_mem) {
@@ -407,10 +406,10 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
         return rc;
       }
     }
-    // DICT_FSST inline NULLs (dict_fsst.cu:426-446) on top of the validity
-    if (e == hipSuccess && dc.any_inline)
-      e = launch_dfsst_nulls(d_segs, n_ranges, d_tabs, col->d_null_mask, n, dc.counts, s);
   }
+  // DICT_FSST inline NULLs (dict_fsst.cu:426-446) on top of the validity
+  if (e == hipSuccess && dc.any_inline)
+    e = launch_dfsst_nulls(d_segs, n_ranges, col->d_null_mask, n, !runs, dc.counts, s);
   struct {
     uint32_t ticket, error;
     uint64_t total;
