@@ -32,6 +32,8 @@
 #include "sdr_device.hpp"
 #include "sdr_fsst.hpp"
 
+#include <cstddef>
+
 namespace sdr {
 
 constexpr uint32_t FSST_THREADS   = 512;  // a chunk's workgroup
@@ -1160,10 +1162,19 @@ __device__ __forceinline__ void plain_copy_whole(SM& sm, const uint8_t* seg, uin
   }
 }
 
+// A DICTIONARY segment's entries in LDS: as many and as long ones as there is room for.
+constexpr uint32_t LABEL_ENTRIES = 256;
+constexpr uint32_t LABEL_BYTES   = 32;
+
 // LDS of a workgroup that decodes no FSST chunk.
 struct PlainSmem {
+  __attribute__((aligned(16))) uint32_t lead[4];  // a row's first word may be ORed, with zeros, one before the window
   __attribute__((aligned(16))) uint8_t out[FSST_WINDOW + 48];
+  __attribute__((aligned(16))) uint32_t label[LABEL_ENTRIES][LABEL_BYTES / 4];  // zero past an entry's end
+  uint32_t label_src[LABEL_ENTRIES];  // where it lies in the segment
+  uint8_t label_len[LABEL_ENTRIES];
   uint32_t part[WAVE];
+  uint32_t flag[FSST_WAVES];
   uint64_t sum[FSST_WAVES];
   uint64_t base;
   __device__ __forceinline__ uint32_t* plain_part() { return part; }
@@ -1394,6 +1405,160 @@ __device__ __forceinline__ void plain_chunk(const PlainArgs& args, SM& sm)
     }
     turn(1);
   }
+}
+
+// ORs the bytes of label e into the window (cleared) at byte p.
+__device__ __forceinline__ void label_or(PlainSmem& sm, uint32_t e, uint32_t p)
+{
+  static_assert(offsetof(PlainSmem, out) == sizeof(PlainSmem::lead), "the lead is the word before the window");
+  const uint32_t sh = p & 3u;
+  const uint32_t f  = sh ? 0u : 1u;                       // then the first pair of words makes nothing
+  const uint32_t nb = sm.label_len[e] + sh + 4u * f;      // bytes from the first word ORed
+  const uint32_t ph = 0u - sh;                            // the funnel takes it modulo 4
+  uint32_t* const o = sm.lead + (4u + (p >> 2) - f);
+  uint32_t carry    = 0;
+#pragma unroll
+  for (uint32_t h = 0; h < LABEL_BYTES / 16u; ++h) {
+    if (h && !ballot(nb > 16u * h)) return;
+    const u32x4 n = *reinterpret_cast<const u32x4*>(&sm.label[e][4u * h]);
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+      const uint32_t v = __builtin_amdgcn_alignbyte(n[j], carry, ph);
+      carry            = n[j];
+      if (16u * h + 4u * j < nb)
+        __hip_atomic_fetch_or(o + 4u * h + j, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+  }
+  if (nb > LABEL_BYTES)
+    __hip_atomic_fetch_or(o + LABEL_BYTES / 4u, __builtin_amdgcn_alignbyte(0u, carry, ph), __ATOMIC_RELAXED,
+                          __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// plain_chunk for a DICTIONARY segment of at most LABEL_ENTRIES entries of at most
+// LABEL_BYTES bytes, and whether it was one: the entries go to LDS, whole words
+// and zero past their ends, so that a row costs an index, a length and an OR for
+// each word of its entry (8 Mi label rows: 57 us through memory, 189 vector
+// instructions for 64 rows; here 36 us).
+template <uint32_t RPT>
+__device__ __forceinline__ bool label_chunk(const PlainArgs& args, PlainSmem& sm)
+{
+  const PlainArgs a   = uniform(args);
+  const uint32_t tid  = threadIdx.x;
+  const uint32_t w    = a.flags & FI_WIDTH;
+  const uint32_t rows = a.rows;
+  const uint8_t* bits = a.seg + 20;
+  if (!w || bits + ((uint64_t{a.row_begin + rows} * w + 7u) >> 3) > a.seg + a.bytes_size) return false;
+  uint32_t idx[RPT];
+  {
+    const uint64_t bit0          = uint64_t{a.row_begin} * w;
+    const uintptr_t at           = reinterpret_cast<uintptr_t>(bits) + (bit0 >> 3);
+    const uint32_t skew          = 8u * static_cast<uint32_t>(at & 3u) + static_cast<uint32_t>(bit0 & 7u);
+    const gptr<const uint32_t> p = gbl(reinterpret_cast<const uint32_t*>(at & ~uintptr_t{3}));
+#pragma unroll
+    for (uint32_t i = 0; i < RPT; ++i) {
+      const uint32_t r = FSST_THREADS * i + tid;
+      idx[i]           = bits32_inside(p, skew + (r < rows ? r : 0u) * w, w);
+    }
+  }
+  // entry k is [dict_end - end[k], dict_end - end[k - 1]); 0 is NULL; one whose end
+  // passes dict_end or falls below its start is empty
+  uint32_t elen = 0, esrc = 0;
+  if (tid != 0u && tid < a.ibc) {
+    const uint8_t* e  = a.seg + a.ibo + 4ull * tid;
+    const uint32_t e1 = ld_u32_any(e), e0 = ld_u32_any(e - 4);
+    if (e1 >= e0 && e1 <= a.dict_end) {
+      elen = e1 - e0;
+      esrc = a.dict_end - e1;
+    }
+  }
+  if (tid < LABEL_ENTRIES) {
+    sm.label_len[tid] = static_cast<uint8_t>(elen);
+    sm.label_src[tid] = esrc;
+  }
+  const bool longer = ballot(elen > LABEL_BYTES) != 0;
+  if (lane_id() == 0u) sm.flag[tid / WAVE] = longer;
+  __syncthreads();
+  if (ballot(sm.flag[lane_id() % FSST_WAVES] != 0u)) return false;  // the same in every wave
+  {  // half an entry a thread
+    static_assert(LABEL_ENTRIES * 2u == FSST_THREADS && LABEL_BYTES == 32u, "16 bytes a thread");
+    const uint32_t e = tid / 2u, h = 16u * (tid & 1u), l = sm.label_len[e];
+    const uint32_t n = l > h ? (l - h < 16u ? l - h : 16u) : 0u;
+    u32x4 v          = {0u, 0u, 0u, 0u};
+    if (n) {
+      const uint8_t* p             = a.seg + sm.label_src[e] + h;
+      const uint32_t skew          = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p) & 3u);
+      const gptr<const uint32_t> g = gbl(reinterpret_cast<const uint32_t*>(p - skew));
+      const uint32_t last          = (skew + n - 1u) >> 2;
+      uint32_t x[5];
+#pragma unroll
+      for (uint32_t j = 0; j < 5; ++j) x[j] = g[j < last ? j : last];
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j) {
+        const uint32_t y = __builtin_amdgcn_alignbyte(x[j + 1], x[j], skew);
+        v[j] = n >= 4u * j + 4u ? y : n > 4u * j ? y & ((1u << (8u * (n - 4u * j))) - 1u) : 0u;
+      }
+    }
+    *reinterpret_cast<u32x4*>(&sm.label[e][h / 4u]) = v;
+  }
+  // output positions, as in plain_chunk
+  const uint32_t wv = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(tid / WAVE)));
+  uint32_t out[RPT];
+#pragma unroll
+  for (uint32_t i = 0; i < RPT; ++i) {
+    idx[i]             = FSST_THREADS * i + tid < rows && idx[i] < a.ibc ? idx[i] : 0u;
+    const uint32_t len = sm.label_len[idx[i]];
+    out[i]             = wave_incl_sum_u32(len);
+    if (lane_id() == WAVE - 1u) sm.part[FSST_WAVES * i + wv] = out[i];
+    out[i] -= len;
+  }
+  __syncthreads();
+  static_assert(FSST_WAVES * RPT <= WAVE, "a lane per step and wave");
+  const uint32_t mine = lane_id() < FSST_WAVES * RPT ? sm.part[lane_id()] : 0u;
+  const uint32_t incl = wave_incl_sum_u32(mine);
+#pragma unroll
+  for (uint32_t i = 0; i < RPT; ++i) out[i] += __builtin_amdgcn_readlane(incl - mine, FSST_WAVES * i + wv);
+  const uint32_t T = __builtin_amdgcn_readlane(incl, WAVE - 1);
+  fsst_lookback_publish(a.c, T, a.st, a.spin_limit);
+  // one window if the chunk fits it, else one for each step of 512 rows
+  static_assert(FSST_THREADS * LABEL_BYTES <= FSST_WINDOW, "a step fits the window");
+  const bool whole = T <= FSST_WINDOW;
+  if (whole) {
+    window_clear(sm, T);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < RPT; ++i) label_or(sm, idx[i], out[i]);
+  }
+  const uint64_t base     = fsst_lookback_wait(a.c, a.n_chunks, T, a.st, a.spin_limit, sm);  // synchronises the workgroup
+  const gptr<int32_t> off = gbl(a.offsets) + a.col_row;
+#pragma unroll
+  for (uint32_t i = 0; i < RPT; ++i) {
+    const uint32_t r = FSST_THREADS * i + tid;
+    if (r < rows) off[r] = static_cast<int32_t>(static_cast<uint32_t>(base) + out[i]);
+  }
+  if (a.c == a.n_chunks - 1u && tid == 0)
+    gbl(a.offsets)[a.total_rows] = static_cast<int32_t>(static_cast<uint32_t>(base + T));
+  auto store = [&](uint32_t w0, uint32_t n) {
+    const uint64_t at = base + w0;
+    if (at < a.chars_cap)
+      window_store(sm, reinterpret_cast<uintptr_t>(a.chars) + at,
+                   at + n <= a.chars_cap ? n : static_cast<uint32_t>(a.chars_cap - at));
+  };
+  if (whole) {
+    store(0u, T);
+    return true;
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < RPT; ++i) {
+    const uint32_t lo = __builtin_amdgcn_readlane(incl - mine, FSST_WAVES * i);
+    const uint32_t hi = i + 1u < RPT ? __builtin_amdgcn_readlane(incl - mine, FSST_WAVES * (i + 1u) % WAVE) : T;
+    window_clear(sm, hi - lo);
+    __syncthreads();
+    label_or(sm, idx[i], out[i] - lo);
+    __syncthreads();
+    store(lo, hi - lo);
+    __syncthreads();  // the stores have read the window
+  }
+  return true;
 }
 
 // Import the symbol table serialised at seg + symoff (at most

@@ -36,8 +36,8 @@ __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6)
 // A column without FSST segments, in chunks of up to RPT * 512 rows.  A kernel
 // of its own: within k_fsst the decode was a call, which saved and restored
 // registers through scratch memory, the larger part of its time (8 Mi labels
-// 119 us, 2 M rows of 27 chars 57 us; here 57 us and 35 us, of which 8 us and 9 us
-// are the tickets it no longer draws).  Six wavefronts to a
+// 119 us, 2 M rows of 27 chars 57 us; here 57 us, with the labels in LDS 36 us, and
+// 35 us, of which 8 us and 9 us are the tickets it no longer draws).  Six wavefronts to a
 // SIMD are three workgroups to a CU; for four, rows' state spills (73 us, 70 us).
 template <uint32_t RPT>
 __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_plain(const FsstChunk* __restrict__ chunks, uint32_t n_chunks,
@@ -53,8 +53,11 @@ __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6)
   const FsstChunk ch     = uniform(gload(chunks + c));
   const FsstChunkInfo ci = uniform(gload(info + c));
   if (ch.seg != FSST_GAP && (ci.flags & FI_OK)) {
-    plain_chunk<RPT>({ci.bytes, ci.bytes_size, ci.dict_end, ci.flags, ci.c_lo, ci.c_hi, ch.row_begin, ch.rows,
-                      ch.col_row, c, n_chunks, st, offsets, chars, chars_cap, total_rows, spin_limit}, sm);
+    const PlainArgs args{ci.bytes,   ci.bytes_size, ci.dict_end, ci.flags, ci.c_lo, ci.c_hi,   ch.row_begin, ch.rows,
+                         ch.col_row, c,             n_chunks,    st,       offsets, chars,     chars_cap,    total_rows,
+                         spin_limit};
+    if ((ci.flags & FI_DICT) && ci.c_hi <= LABEL_ENTRIES && label_chunk<RPT>(args, sm)) return;
+    plain_chunk<RPT>(args, sm);
     return;
   }
   // rows of no segment, or of one with a bad header, are empty

@@ -119,3 +119,32 @@ def test_label_chunk_widths(rows, longest):
         offs, chars = _decode(duckdb_segments(table, d.data_ptr() + skew), rows, o_chars.size, A.LAUNCH_BATCHED, 4 * skew)
         np.testing.assert_array_equal(offs, o_offs)
         np.testing.assert_array_equal(chars, o_chars)
+
+
+@pytest.mark.parametrize("rows", [1_500, 1_100_003, 2_200_001])
+@pytest.mark.parametrize("entries,longest", [(2, 32), (255, 31), (256, 32), (257, 32), (256, 33), (9, 0), (40, 17)])
+def test_labels_in_lds(entries, longest, rows):
+    """Dictionaries on either side of what a workgroup keeps in LDS, output of
+    less and of more than a window, entries with bad ends among them."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    rng = np.random.default_rng(entries * 64 + longest)
+    lens = [longest if k == 1 else int(rng.integers(0, longest + 1)) for k in range(1, entries)]
+    words = [None] + [rng.integers(0, 256, n, dtype=np.uint8).tobytes() for n in lens]
+    seg = bytearray(_label_segment(words, rng.integers(0, entries, rows)))
+    ibo = int.from_bytes(seg[8:12], "little")
+    for k in (2, entries // 2):  # an end below its start, and one past dict_end
+        if 1 < k < entries - 1:
+            at = ibo + 4 * k
+            seg[at:at + 4] = int(0 if k == 2 else 1 << 30).to_bytes(4, "little")
+    b = StringBlob()
+    b.add(A.DICTIONARY, bytes(seg), 0, rows)
+    table = np.array(b.table, np.int64)
+    o_offs, o_chars = oracle_string_runs(b.blob, table, rows)
+    for skew in (0, 1):
+        d = torch.zeros(b.blob.size + skew + 64, dtype=torch.uint8, device="cuda")
+        d[skew:skew + b.blob.size] = torch.from_numpy(b.blob)
+        print(f"[gpu] labels entries={entries} longest={longest} rows={rows} skew={skew}", flush=True)
+        offs, chars = _decode(duckdb_segments(table, d.data_ptr() + skew), rows, o_chars.size, A.LAUNCH_BATCHED, 7 * skew)
+        np.testing.assert_array_equal(offs, o_offs)
+        np.testing.assert_array_equal(chars, o_chars)
