@@ -135,11 +135,13 @@ struct MasksInline {
   __device__ __forceinline__ MaskUnit at(uint32_t i) const { return uniform(unit[i]); }
 };
 
+template <uint32_t NT = BLOCK_THREADS>
 struct MaskSmem {
-  uint32_t wave_nulls[WAVES_PER_BLOCK];
+  uint32_t wave_nulls[NT / WAVE];
 };
+template <uint32_t NT>
 __device__ __forceinline__ void mask_block(const MaskUnit& u, uint32_t index, uint32_t* __restrict__ counts,
-                                           unsigned long long* __restrict__ total, MaskSmem& sm)
+                                           unsigned long long* __restrict__ total, MaskSmem<NT>& sm)
 {
   const uint32_t t = threadIdx.x;
   const gptr<uint8_t> dst = gbl(u.dst);
@@ -151,7 +153,7 @@ __device__ __forceinline__ void mask_block(const MaskUnit& u, uint32_t index, ui
     const uint32_t nb   = (u.bytes - h) / 16u;
     if (t < h) dst[t] = 0xFFu;
     const gptr<u32x4> v = reinterpret_cast<gptr<u32x4>>(dst + h);
-    for (uint32_t i = t; i < nb; i += BLOCK_THREADS) v[i] = u32x4{~0u, ~0u, ~0u, ~0u};
+    for (uint32_t i = t; i < nb; i += NT) v[i] = u32x4{~0u, ~0u, ~0u, ~0u};
     const uint32_t e = h + nb * 16u + t;
     if (e < u.bytes && t < 16u) dst[e] = 0xFFu;
   } else {
@@ -167,16 +169,16 @@ __device__ __forceinline__ void mask_block(const MaskUnit& u, uint32_t index, ui
       nulls += 8u - static_cast<uint32_t>(__builtin_popcount(b));
     };
     if (t < h) one(t);
-    constexpr uint32_t K = MASK_UNIT_BYTES / 4u / BLOCK_THREADS;  // a thread's words, loaded together
+    constexpr uint32_t K = MASK_UNIT_BYTES / 4u / NT;  // a thread's words, loaded together
     uint32_t w[K];
 #pragma unroll
     for (uint32_t k = 0; k < K; ++k) {
-      const uint32_t i = k * BLOCK_THREADS + t;
+      const uint32_t i = k * NT + t;
       w[k]             = i < nw ? ld_u32_any(u.src + h + 4u * i) : ~0u;
     }
 #pragma unroll
     for (uint32_t k = 0; k < K; ++k) {
-      const uint32_t i = k * BLOCK_THREADS + t;
+      const uint32_t i = k * NT + t;
       if (i < nw) v[i] = w[k];
       nulls += 32u - static_cast<uint32_t>(__builtin_popcount(w[k]));
     }
@@ -191,7 +193,7 @@ __device__ __forceinline__ void mask_block(const MaskUnit& u, uint32_t index, ui
   if (t == 0) {
     uint32_t all = 0;
 #pragma unroll
-    for (uint32_t k = 0; k < WAVES_PER_BLOCK; ++k) all += sm.wave_nulls[k];
+    for (uint32_t k = 0; k < NT / WAVE; ++k) all += sm.wave_nulls[k];
     if (counts) gbl(counts)[index] = all;
     else if (all) atomicAdd(total, static_cast<unsigned long long>(all));
   }
@@ -247,7 +249,7 @@ union GroupSmem {
   AlpSmem<false> alp;
   AlpSmem<true> alprd;
   RleSmem rle;
-  MaskSmem mask;
+  MaskSmem<> mask;
   __device__ GroupSmem() {}
 };
 

@@ -54,7 +54,7 @@ template <class Src>
 __global__ __launch_bounds__(BLOCK_THREADS) void k_null_mask(Src src, uint32_t* __restrict__ counts,
                                                              unsigned long long* __restrict__ total)
 {
-  __shared__ MaskSmem sm;
+  __shared__ MaskSmem<> sm;
   mask_block(src.at(blockIdx.x), blockIdx.x, counts, total, sm);
 }
 

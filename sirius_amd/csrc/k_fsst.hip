@@ -1,6 +1,7 @@
 // k_fsst.hip — per-column FSST decode kernel (one launch decodes every chunk
 // of a VARCHAR column; see dec_fsst.hpp for the chunk decoder).
 #include "dec_fsst.hpp"
+#include "dec_groups.hpp"
 #include "sdr_tune.hpp"
 
 #include <cstring>
@@ -112,14 +113,28 @@ __device__ __forceinline__ void fsst_prep_block(const Src& src, uint32_t n_segs,
   }
 }
 
+// Its first `prep` workgroups; the others build the column's null mask, a piece
+// each (in a launch of its own after the decode that took 4 us of a call of 58).
 template <class Src>
-__global__ __launch_bounds__(Src::THREADS) void k_fsst_prep(Src src, uint32_t n_segs, FsstChunk* __restrict__ chunks,
+__global__ __launch_bounds__(Src::THREADS) void k_fsst_prep(Src src, uint32_t n_segs, uint32_t prep,
+                                                            FsstChunk* __restrict__ chunks,
                                                             FsstChunkInfo* __restrict__ info,
                                                             FsstSymTab* __restrict__ tabs, FsstState* __restrict__ st,
-                                                            FsstResult* __restrict__ result)
+                                                            FsstResult* __restrict__ result,
+                                                            const MaskUnit* __restrict__ units,
+                                                            uint32_t* __restrict__ counts)
 {
-  __shared__ FsstPrepSmem<Src::THREADS> sm;
-  fsst_prep_block(src, n_segs, blockIdx.x, gridDim.x, chunks, info, tabs, st, result, nullptr, sm);
+  __shared__ union Smem {
+    FsstPrepSmem<Src::THREADS> prep;
+    MaskSmem<Src::THREADS> mask;
+    __device__ Smem() {}
+  } sm;
+  if (blockIdx.x < prep) {
+    fsst_prep_block(src, n_segs, blockIdx.x, prep, chunks, info, tabs, st, result, nullptr, sm.prep);
+  } else {
+    const uint32_t u = blockIdx.x - prep;
+    mask_block(uniform(gload(units + u)), u, counts, nullptr, sm.mask);
+  }
 }
 
 // ---- DICT_FSST passes ----
@@ -273,7 +288,8 @@ hipError_t launch_dfsst_nulls(const FsstSeg* d_segs, uint32_t n_ranges, uint8_t*
 
 hipError_t launch_fsst_prep(const FsstSeg* segs, uint32_t n_segs, FsstChunk* d_chunks, FsstChunkInfo* d_info,
                             FsstSymTab* d_tabs, FsstState* d_state, FsstResult* result, hipStream_t s, bool host,
-                            const DfsstWork* wk, uint32_t n_dseg, FsstSeg* copy)
+                            const DfsstWork* wk, uint32_t n_dseg, FsstSeg* copy, const MaskUnit* units,
+                            uint32_t n_units, uint32_t* counts)
 {
   if (n_segs == 0) return hipSuccess;
   const uint32_t blocks = n_segs < 4096u ? n_segs : 4096u;
@@ -284,8 +300,8 @@ hipError_t launch_fsst_prep(const FsstSeg* segs, uint32_t n_segs, FsstChunk* d_c
       hipLaunchKernelGGL((k_dfsst_front<S>), dim3(blocks + pre), dim3(PREDECODE_THREADS), 0, s, src, n_segs, blocks, *wk,
                          d_chunks, d_info, d_tabs, d_state, result, copy);
     } else {
-      hipLaunchKernelGGL((k_fsst_prep<S>), dim3(blocks), dim3(S::THREADS), 0, s, src, n_segs, d_chunks, d_info, d_tabs,
-                         d_state, result);
+      hipLaunchKernelGGL((k_fsst_prep<S>), dim3(blocks + n_units), dim3(S::THREADS), 0, s, src, n_segs, blocks, d_chunks,
+                         d_info, d_tabs, d_state, result, units, counts);
     }
   };
   if (host && n_segs <= RANGES_INLINE) {

@@ -389,8 +389,6 @@ void add_mask_units(const sdr_run* runs, uint32_t n, uint32_t total_rows, uint8_
   add(at, end, nullptr);
 }
 
-namespace {
-
 // Pieces and their counts in pinned memory: the kernel writes the counts and
 // reads a long list of pieces there, with no copy and no clear on the stream.
 int masks_prepare(const std::vector<MaskUnit>& units, MaskLaunch* m, void** token)
@@ -404,6 +402,8 @@ int masks_prepare(const std::vector<MaskUnit>& units, MaskLaunch* m, void** toke
   *m = MaskLaunch{units.data(), hu, static_cast<uint32_t*>(h), static_cast<uint32_t>(n)};
   return SDR_OK;
 }
+
+namespace {
 
 // The pieces in launches of their own.
 hipError_t launch_masks(const MaskLaunch& m, hipStream_t s)

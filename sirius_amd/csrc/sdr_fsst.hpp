@@ -8,6 +8,8 @@
 
 namespace sdr {
 
+struct MaskUnit;
+
 constexpr uint32_t FSST_CHUNK_ROWS = 1024;        // rows per workgroup
 constexpr uint32_t WIDE_CHUNK_ROWS = 4096;        // ... at most, in columns of DICTIONARY segments
 constexpr uint32_t FSST_GAP        = 0xFFFFFFFFu;  // chunk of rows no segment covers
@@ -43,9 +45,9 @@ static_assert(sizeof(FsstSeg) == 32, "FsstSeg layout");
 // Rows per chunk of a column of DICTIONARY segments alone: of 4096, 2048 and
 // 1024 the widest that still gives each of the 256 CUs two chunks.  A chunk's
 // descriptors and look-back are round trips that more rows share (8 Mi labels: a
-// call of 110 us in chunks of 1024 rows, 79 of 2048, 73 of 4096), but fewer chunks
-// leave CUs idle (a row group: 24, 24, 29 us; 512 Ki rows: 28, 27, 32; 1 Mi: 35,
-// 31, 34; 2 Mi: 45, 40, 38).
+// call of 103 us in chunks of 1024 rows, 71 of 2048, 54 of 4096), but fewer chunks
+// leave CUs idle (a row group: 23, 23, 25 us; 512 Ki rows: 26, 26, 28; 1 Mi: 33,
+// 28, 29; 2 Mi: 43, 35, 32).
 inline uint32_t label_chunk_rows(uint32_t total_rows)
 {
   uint32_t r = WIDE_CHUNK_ROWS;
@@ -174,10 +176,13 @@ constexpr uint32_t FSST_STATE_WORDS = 3;  // 8-byte words before status
 // result may be null).  With `host` the ranges are pinned host memory: a few
 // travel in the kernel arguments, each of many is read by its block.  With `wk` the
 // n_dseg DICT_FSST segments' entries are predecoded in the same launch, and
-// `copy`, if set, receives the ranges in device memory.
+// `copy`, if set, receives the ranges in device memory; without it the column's
+// n_units mask pieces (memory the device reads) are built in the same launch, with
+// their null counts.
 hipError_t launch_fsst_prep(const FsstSeg* segs, uint32_t n_segs, FsstChunk* d_chunks, FsstChunkInfo* d_info,
                             FsstSymTab* d_tabs, FsstState* d_state, FsstResult* result, hipStream_t s, bool host,
-                            const DfsstWork* wk, uint32_t n_dseg, FsstSeg* copy);
+                            const DfsstWork* wk, uint32_t n_dseg, FsstSeg* copy, const MaskUnit* units,
+                            uint32_t n_units, uint32_t* counts);
 // `chunk_rows`: 0 for a column with FSST segments, else the rows of its chunks.
 // `ordered`: by ticket, see FSST_UNORDERED_SHARE.
 hipError_t launch_fsst(bool ordered, uint32_t chunk_rows, const FsstChunk* d_chunks, uint32_t first, uint32_t n, uint32_t n_chunks_total,

@@ -59,6 +59,8 @@ struct MaskLaunch {
   uint32_t* counts      = nullptr;
   uint32_t n            = 0;
 };
+// Pieces and counts in pinned memory, to be launched; `token` as for masks_launch.
+int masks_prepare(const std::vector<MaskUnit>& units, MaskLaunch* m, void** token);
 
 // One fixed-width run and where its rows go.
 struct RunTarget {

@@ -371,10 +371,26 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
     dc.release(s, synced);
     release();
   };
+  const bool masked = (col->has_nulls && col->d_null_mask) || dc.any_inline;
+  std::vector<MaskUnit> units;
+  const uint32_t* counts = nullptr;  // null count of each piece of the mask
+  void* counts_token     = nullptr;
+  const bool runs        = col->has_nulls && col->n_validity;
+  if (masked && (runs || !dc.any_inline))
+    add_mask_units(col->validity, col->has_nulls ? col->n_validity : 0u, n, col->d_null_mask, units);
+  MaskLaunch beside;  // the pieces built beside the pre-pass
+  if (!units.empty() && !scratch_mem && !dc.n_d) {
+    rc     = masks_prepare(units, &beside, &counts_token);
+    counts = beside.counts;
+    if (rc) {
+      release_all();
+      return rc;
+    }
+  }
   auto decode = [&](bool ordered) {
     hipError_t r = launch_fsst_prep(prep_segs, n_ranges, d_chunks, d_info, d_tabs, d_state, result, s,
                                     prep_segs != d_segs, dc.n_d ? &dc.work : nullptr, dc.n_d,
-                                    dc.any_inline ? d_segs : nullptr);
+                                    dc.any_inline ? d_segs : nullptr, beside.units, beside.n, beside.counts);
     const uint64_t cap = col->d_chars ? col->chars_capacity : 0;
     if (r == hipSuccess && mode == SDR_LAUNCH_PER_SEGMENT) {
       for (uint32_t i = 0; r == hipSuccess && i < n_ranges; ++i)
@@ -388,23 +404,17 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
   };
   const bool unordered = fsst_unordered(tune(SDR_TUNE_FSST_SPIN_LIMIT));
   e                    = decode(!unordered);
-  const bool masked = (col->has_nulls && col->d_null_mask) || dc.any_inline;
-  std::vector<MaskUnit> units;
-  const uint32_t* counts = nullptr;  // null count of each piece of the mask
-  void* counts_token     = nullptr;
-  const bool device_nulls = masked && scratch_mem;  // nothing may be allocated for the pieces' counts
-  const bool runs = col->has_nulls && col->n_validity;
-  if (e == hipSuccess && masked && (runs || !dc.any_inline)) {
-    add_mask_units(col->validity, col->has_nulls ? col->n_validity : 0u, n, col->d_null_mask, units);
-    if (device_nulls) e = launch_fill_u8(reinterpret_cast<uint8_t*>(d_nulls), 0, sizeof(unsigned long long), s);
-    if (e == hipSuccess && scratch_mem) {
+  // nulls counted on the device, when nothing may be allocated for the pieces' counts
+  const bool device_nulls = masked && scratch_mem;
+  if (e == hipSuccess && device_nulls) {
+    e = launch_fill_u8(reinterpret_cast<uint8_t*>(d_nulls), 0, sizeof(unsigned long long), s);
+    if (e == hipSuccess)
       e = launch_null_mask(units.data(), static_cast<uint32_t>(units.size()), nullptr, d_nulls, s, true);
-    } else if (e == hipSuccess) {
-      rc = masks_launch(units, s, &counts, &counts_token);
-      if (rc) {
-        release_all();
-        return rc;
-      }
+  } else if (e == hipSuccess && !units.empty() && !beside.n) {
+    rc = masks_launch(units, s, &counts, &counts_token);
+    if (rc) {
+      release_all();
+      return rc;
     }
   }
   // DICT_FSST inline NULLs (dict_fsst.cu:426-446) on top of the validity
