@@ -35,7 +35,7 @@ __device__ __forceinline__ FixedSeg uniform_seg(const FixedSeg& v)
 struct DevSegs {
   const FixedSeg* p;
   uint32_t base;
-  __device__ __forceinline__ FixedSeg at(uint32_t i) const { return uniform_seg(gload(p + base + i)); }
+  __device__ __forceinline__ FixedSeg at(uint32_t i) const { return sload(p + base + i); }
 };
 struct SegsInline {
   FixedSeg seg[SEGS_INLINE];
@@ -128,7 +128,7 @@ __device__ __forceinline__ void copy_block(const FixedSeg& sd, uint32_t x, uint3
 // segments, and 300 us beside 43 us for ten row groups of five columns.)
 struct DevMasks {
   const MaskUnit* p;
-  __device__ __forceinline__ MaskUnit at(uint32_t i) const { return uniform(gload(p + i)); }
+  __device__ __forceinline__ MaskUnit at(uint32_t i) const { return sload(p + i); }
 };
 struct MasksInline {
   MaskUnit unit[MASKS_INLINE];
@@ -235,13 +235,13 @@ struct GroupTable {
 };
 __device__ __forceinline__ MaskUnit mask_unit(const SegsInline& src, const GroupTable& t, uint32_t i)
 {
-  if (t.units) return uniform(gload(t.units + i));
+  if (t.units) return sload(t.units + i);
   const FixedSeg f = src.at(i);
   return MaskUnit{f.bytes, f.out, f.bytes_size, f.row_count};
 }
 __device__ __forceinline__ MaskUnit mask_unit(const DevSegs&, const GroupTable& t, uint32_t i)
 {
-  return uniform(gload(t.units + i));
+  return sload(t.units + i);
 }
 
 union GroupSmem {

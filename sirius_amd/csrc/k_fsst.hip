@@ -51,8 +51,8 @@ __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6)
   __shared__ PlainSmem sm;
   const uint32_t c = chunk_number(st, first, ordered);
   if (c >= n_chunks) return;  // never taken: the grids are the chunk count
-  const FsstChunk ch     = uniform(gload(chunks + c));
-  const FsstChunkInfo ci = uniform(gload(info + c));
+  const FsstChunk ch     = sload(chunks + c);
+  const FsstChunkInfo ci = sload(info + c);
   if (ch.seg != FSST_GAP && (ci.flags & FI_OK)) {
     const PlainArgs args{ci.bytes,   ci.bytes_size, ci.dict_end, ci.flags, ci.c_lo, ci.c_hi,   ch.row_begin, ch.rows,
                          ch.col_row, c,             n_chunks,    st,       offsets, chars,     chars_cap,    total_rows,
@@ -83,7 +83,7 @@ constexpr uint32_t RANGES_INLINE = 100;
 struct DevRanges {
   static constexpr uint32_t THREADS = 256;
   const FsstSeg* p;
-  __device__ __forceinline__ FsstSeg at(uint32_t i) const { return uniform(gload(p + i)); }
+  __device__ __forceinline__ FsstSeg at(uint32_t i) const { return sload(p + i); }
 };
 struct RangesInline {
   static constexpr uint32_t THREADS = 512;
@@ -133,7 +133,7 @@ __global__ __launch_bounds__(Src::THREADS) void k_fsst_prep(Src src, uint32_t n_
     fsst_prep_block(src, n_segs, blockIdx.x, prep, chunks, info, tabs, st, result, nullptr, sm.prep);
   } else {
     const uint32_t u = blockIdx.x - prep;
-    mask_block(uniform(gload(units + u)), u, counts, nullptr, sm.mask);
+    mask_block(sload(units + u), u, counts, nullptr, sm.mask);
   }
 }
 
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(DFSST_PREP_THREADS) void k_dfsst_prep(const DictFss
 {
   __shared__ DfsstPrepSmem<DFSST_PREP_THREADS> sm;
   for (uint32_t j = blockIdx.x; j < n; j += gridDim.x) {
-    const DictFsstSeg d = uniform(gload(dseg + j));
+    const DictFsstSeg d = sload(dseg + j);
     if (threadIdx.x == 0) wk.desc[j] = d;
     dfsst_prep_segment(d, wk.e_byte, wk.e_dec, tabs + d.range, out + 2u * j, wk.pre_size + j, sm);
     __syncthreads();  // sm is reused by the next segment
