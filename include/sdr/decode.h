@@ -213,16 +213,15 @@ int sdr_plan_destroy(sdr_plan* plan);
 /* ---- persistent batches ------------------------------------------------- */
 
 /* A batch collects the work of many columns (fixed-width and VARCHAR, any
- * codec mix) into one launch: the fixed-width segments of each codec and
- * value width decode in one per-codec grid over descriptors in the batch's
- * arena (or, with SDR_BATCH_FIXED_KERNELS = 1, in persistent group kernels
- * that drain a work queue), and the VARCHAR chunks in a kernel of one
- * block per chunk that claims them from the queue in order.  The arena is
- * uploaded from pinned memory with one copy ahead of the kernels.  A batch of fixed-width segments alone
- * (no string column, validity mask or queue entry) passes its descriptors as
- * sdr_decode_table does instead: up to 256 per per-codec grid in the kernel
- * arguments, more through a reused descriptor buffer; it is never replayed
- * from a graph.  It has no
+ * codec mix) into one launch: the fixed-width segments decode in one kernel,
+ * each codec and value width a part of its grid, over descriptors in the
+ * batch's arena (or, with SDR_BATCH_FIXED_KERNELS = 1, in persistent group
+ * kernels that drain a work queue), and the VARCHAR chunks in a kernel of one
+ * block per chunk.  The launch's first kernel copies the arena from pinned
+ * memory.  A batch of fixed-width segments alone (no string column, validity
+ * mask or queue entry) passes its descriptors as sdr_decode_table does
+ * instead: up to 256 per codec and width in the kernel arguments, more in a
+ * reused pinned buffer; it is never replayed from a graph.  It has no
  * counterpart in the reference, which launches one kernel per codec run
  * (src/cuda/scan/gpu_native_decode.cu:356-386, gpu_decode_strings.cu:257-366);
  * every output is identical to sdr_decode_table / sdr_decode_strings_column.
@@ -397,7 +396,8 @@ int sdr_server_destroy(sdr_server* server);
  * table that sdr_tune_load applies. */
 typedef enum sdr_tune_key {
   SDR_TUNE_RLE_SLICE_ROWS      = 1, /* rows one 256-thread block expands:
-                                       1024..1048576, multiple of 64 (16384) */
+                                       1024..1048576, multiple of 64 (16384:
+                                       each launch chooses by its size)      */
   SDR_TUNE_BP_GROUPS_PER_WAVE  = 2, /* 2048-row groups one wavefront decodes
                                        in turn, 1..16 (1)                    */
   SDR_TUNE_BP_CHUNK_ROWS       = 3, /* most rows a wavefront stages per LDS
@@ -407,7 +407,8 @@ typedef enum sdr_tune_key {
   SDR_TUNE_FSST_SPIN_LIMIT     = 5, /* sleeps a VARCHAR chunk waits for its
                                        predecessors' chars offsets before its
                                        decode reports SDR_E_HIP, 0..2^31
-                                       (2^24, never reached); 0 reports at
+                                       (2^24, never reached); a first attempt
+                                       waits a 1024th of it.  0 reports at
                                        once without waiting (for tests)      */
   /* work units per queue entry of a persistent batch, for every batch that
    * does not set SDR_BATCH_UNITS_* itself: 1..2^20 */

@@ -203,13 +203,14 @@ __device__ __forceinline__ void block_excl_scan2(uint32_t a, uint32_t b, uint32_
 // in 256-thread workgroups with an 11 KiB window: 70 VALU and 52 LDS cycles
 // per 64 bytes, 560 us for 16 Mi rows of 27 chars (12.9 compressed).  Row
 // starts as a bitmap, packed prefix sums and two lookups and two to three ORs
-// per byte take it to 32 VALU and 31 LDS cycles and 294 us, both busy 58% of
-// the time.  512 threads with two groups each keep a 16 KiB run in registers,
-// so nothing is read twice; three such workgroups share a CU (51 KB of LDS, 80
-// VGPRs), whose 38 KiB window builds most chunks in one piece.  Rows of 70 and
-// 200 chars, whose chunks take several runs, went from 945 to 221 and from 2956
-// to 324 us (137 and 197 MB of chars); the row-wise path is left to malformed
-// chunks and to rows that no run holds.
+// per byte take it to 32 VALU and 31 LDS cycles, both busy 60% of the time, and
+// 272 us (293 us when chunks were taken by ticket, see FSST_UNORDERED_SHARE).
+// 512 threads with two groups each keep a 16 KiB run in registers, so nothing is
+// read twice; three such workgroups share a CU (51 KB of LDS, 80 VGPRs), whose
+// 38 KiB window builds most chunks in one piece.  Rows of 70 and 200 chars,
+// whose chunks take several runs, went from 945 to 221 and from 2956 to 324 us
+// (137 and 197 MB of chars); the row-wise path is left to malformed chunks and to
+// rows that no run holds.
 constexpr uint32_t FSST_SYMSTAGE = 17u + 8u * FSST_NSYM;  // the largest symbol table (2057 bytes)
 // Compressed bytes that the staged path takes at a time, the head of up to
 // 15 bytes before them included: GROUPS_PER_THR 16-byte groups per thread.

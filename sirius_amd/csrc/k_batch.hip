@@ -11,9 +11,9 @@
 // entries are independent, so block b takes entries b, b + grid, ... with no
 // claim at all; its four wavefronts decode an entry's units (an RLE slice is
 // decoded by the whole block).  The FSST kernel runs one block per chunk, in
-// queue order, which is what lets a chunk wait on its predecessors' offsets.  The group kernels run as
-// parallel branches (graph nodes) or in stream order, sharing the GPU as
-// their queues drain.
+// queue order, which is what lets a chunk wait on its predecessors' offsets.  By
+// default fixed-width segments are not queued: the front kernel decodes them
+// beside the FSST pre-pass.
 #include "dec_fsst.hpp"
 #include "dec_groups.hpp"
 #include "sdr_batch.hpp"

@@ -19,19 +19,18 @@ __device__ __forceinline__ uint32_t chunk_number(FsstState* st, uint32_t first, 
   return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(s_ticket)));
 }
 
-__global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_fsst(const FsstChunk* __restrict__ chunks, uint32_t n_chunks,
-                                                       const FsstChunkInfo* __restrict__ info,
-                                                       const FsstSymTab* __restrict__ tabs, FsstState* __restrict__ st,
-                                                       int32_t* __restrict__ offsets, uint8_t* __restrict__ chars,
-                                                       uint64_t chars_cap, uint32_t total_rows, uint32_t spin_limit,
-                                                       uint32_t first, uint32_t ordered)
+__global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_fsst(
+  const FsstChunk* __restrict__ chunks, uint32_t n_chunks, const FsstChunkInfo* __restrict__ info,
+  const FsstSymTab* __restrict__ tabs, FsstState* __restrict__ st, int32_t* __restrict__ offsets,
+  uint8_t* __restrict__ chars, uint64_t chars_cap, uint32_t total_rows, uint32_t spin_limit, uint32_t first,
+  uint32_t ordered)
 {
   __shared__ FsstSmem sm;
   const uint32_t c = chunk_number(st, first, ordered);
   if (c >= n_chunks) return;  // never taken: the grids are the chunk count
   const FsstChunk ch = chunks[c];
-  fsst_chunk(ch, info[c], tabs + (ch.seg == FSST_GAP ? 0u : ch.seg), c, n_chunks, st, offsets,
-                              chars, chars_cap, total_rows, spin_limit, sm);
+  fsst_chunk(ch, info[c], tabs + (ch.seg == FSST_GAP ? 0u : ch.seg), c, n_chunks, st, offsets, chars, chars_cap,
+             total_rows, spin_limit, sm);
 }
 
 // A column without FSST segments, in chunks of up to RPT * 512 rows.  A kernel
@@ -41,12 +40,10 @@ __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6)
 // 35 us, of which 8 us and 9 us are the tickets it no longer draws).  Six wavefronts to a
 // SIMD are three workgroups to a CU; for four, rows' state spills (73 us, 70 us).
 template <uint32_t RPT>
-__global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_plain(const FsstChunk* __restrict__ chunks, uint32_t n_chunks,
-                                                        const FsstChunkInfo* __restrict__ info,
-                                                        FsstState* __restrict__ st, int32_t* __restrict__ offsets,
-                                                        uint8_t* __restrict__ chars, uint64_t chars_cap,
-                                                        uint32_t total_rows, uint32_t spin_limit, uint32_t first,
-                                                        uint32_t ordered)
+__global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_plain(
+  const FsstChunk* __restrict__ chunks, uint32_t n_chunks, const FsstChunkInfo* __restrict__ info,
+  FsstState* __restrict__ st, int32_t* __restrict__ offsets, uint8_t* __restrict__ chars, uint64_t chars_cap,
+  uint32_t total_rows, uint32_t spin_limit, uint32_t first, uint32_t ordered)
 {
   __shared__ PlainSmem sm;
   const uint32_t c = chunk_number(st, first, ordered);
@@ -314,10 +311,10 @@ hipError_t launch_fsst_prep(const FsstSeg* segs, uint32_t n_segs, FsstChunk* d_c
   return hipGetLastError();
 }
 
-hipError_t launch_fsst(bool ordered, uint32_t chunk_rows, const FsstChunk* d_chunks, uint32_t first, uint32_t n, uint32_t n_chunks_total,
-                       const FsstChunkInfo* d_info, const FsstSymTab* d_tabs, FsstState* d_state,
-                       int32_t* d_offsets, uint8_t* d_chars, uint64_t chars_cap, uint32_t total_rows,
-                       hipStream_t s)
+hipError_t launch_fsst(bool ordered, uint32_t chunk_rows, const FsstChunk* d_chunks, uint32_t first, uint32_t n,
+                       uint32_t n_chunks_total, const FsstChunkInfo* d_info, const FsstSymTab* d_tabs,
+                       FsstState* d_state, int32_t* d_offsets, uint8_t* d_chars, uint64_t chars_cap,
+                       uint32_t total_rows, hipStream_t s)
 {
   if (n == 0) return hipSuccess;
   // Tickets are global chunk numbers: a launch covering [first, first + n)

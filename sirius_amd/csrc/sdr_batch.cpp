@@ -1,9 +1,9 @@
 // sdr_batch.cpp — host side of the persistent mixed-codec decode: builds the
 // device work queue (one arena: header, entries grouped by decoder and
-// width, FSST columns, chunks, segments, look-back state), uploads it from
-// pinned memory with one copy, and launches the groups' persistent kernels,
-// optionally as a replayed hipGraph whose group kernels are parallel
-// branches.
+// width, FSST columns, chunks, segments, look-back state) in pinned memory, and
+// launches a kernel that copies it to the device, one for the string pre-pass,
+// the fixed-width segments and the null masks, and one for the string chunks;
+// optionally all but the first as a replayed hipGraph.
 #include "sdr_batch.hpp"
 #include "sdr_internal.hpp"
 #include "sdr_kernels.hpp"

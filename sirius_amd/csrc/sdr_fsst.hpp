@@ -185,9 +185,9 @@ hipError_t launch_fsst_prep(const FsstSeg* segs, uint32_t n_segs, FsstChunk* d_c
                             uint32_t n_units, uint32_t* counts);
 // `chunk_rows`: 0 for a column with FSST segments, else the rows of its chunks.
 // `ordered`: by ticket, see FSST_UNORDERED_SHARE.
-hipError_t launch_fsst(bool ordered, uint32_t chunk_rows, const FsstChunk* d_chunks, uint32_t first, uint32_t n, uint32_t n_chunks_total,
-                       const FsstChunkInfo* d_info, const FsstSymTab* d_tabs, FsstState* d_state,
-                       int32_t* d_offsets, uint8_t* d_chars, uint64_t chars_cap, uint32_t total_rows,
-                       hipStream_t s);
+hipError_t launch_fsst(bool ordered, uint32_t chunk_rows, const FsstChunk* d_chunks, uint32_t first, uint32_t n,
+                       uint32_t n_chunks_total, const FsstChunkInfo* d_info, const FsstSymTab* d_tabs,
+                       FsstState* d_state, int32_t* d_offsets, uint8_t* d_chars, uint64_t chars_cap,
+                       uint32_t total_rows, hipStream_t s);
 
 }  // namespace sdr
