@@ -78,20 +78,27 @@ __device__ __forceinline__ void alp_block(const FixedSeg& sd, uint32_t x, uint32
   }
 }
 
-// One block per (segment, slice of `slice_rows` rows) over a 1-D grid of
-// n_blocks (a multiple of 8).  Workgroups are dispatched to the 8 XCDs
-// round-robin, so block b runs on XCD b % 8; the remap below hands each XCD
-// a contiguous range of (segment, slice) pairs, so the slices of a segment
-// share one L2 and its counts are fetched from HBM about once.
-constexpr uint32_t N_XCD = 8;
+// One block per (segment, slice of `slice_rows` rows) over a 1-D grid.
+// Workgroups are dispatched to the 8 XCDs round-robin, each with an L2 of its
+// own, and every slice reads all of its segment's counts.  So an XCD takes eight
+// slices in a row, half a row group, and the next XCD the next eight: the chip
+// writes within 4 MiB at a time.  An eighth of the whole launch to each XCD, as it
+// was, reads the counts once but writes eight places far apart, and memory takes
+// that less well (32 Mi int64 rows in runs of 64: 56.0 us, so 54.0; runs of 16:
+// 65.0, 62.6; runs of 2, whose counts are as much as a quarter of what is moved:
+// 180.1, 181.0; int32 in runs of 300: 32.9, 31.6, of 2: 194.5, 197.0; 64 Mi integers and dates 230.9,
+// 227.5).
+constexpr uint32_t N_XCD          = 8;
+constexpr uint32_t RLE_XCD_BLOCKS = 8;
+constexpr uint32_t RLE_XCD_TURN   = N_XCD * RLE_XCD_BLOCKS;  // the grid is a multiple of it
 
-// Block `block` of `blocks` (a multiple of 8, the first of them on an XCD 0).
+// Block `block`, the first of which is on an XCD 0.
 template <uint32_t TS, class Src>
 __device__ __forceinline__ void rle_block(const Src& src, uint32_t seg0, uint32_t n_segs, uint32_t block,
-                                          uint32_t blocks, uint32_t slices, uint32_t slice_rows, RleSmem& sm)
+                                          uint32_t slices, uint32_t slice_rows, RleSmem& sm)
 {
-  const uint32_t per_xcd = blocks / N_XCD;
-  const uint32_t logical = (block % N_XCD) * per_xcd + block / N_XCD;
+  const uint32_t in_turn = block % RLE_XCD_TURN;
+  const uint32_t logical = block - in_turn + in_turn % N_XCD * RLE_XCD_BLOCKS + in_turn / N_XCD;
   const uint32_t sgi     = logical / slices;
   if (sgi >= n_segs) return;
   const FixedSeg sd = src.at(seg0 + sgi);
@@ -264,10 +271,10 @@ __device__ __forceinline__ void groups_block(const Src& src, const GroupTable& t
   if (block >= g.blocks) return;  // between two groups
   if (g.kind - GK_RLE < 4u) {
     switch (g.kind - GK_RLE) {
-      case 0: rle_block<1>(src, g.seg, g.n_segs, block, g.blocks, g.per_seg, g.a, sm.rle); break;
-      case 1: rle_block<2>(src, g.seg, g.n_segs, block, g.blocks, g.per_seg, g.a, sm.rle); break;
-      case 2: rle_block<4>(src, g.seg, g.n_segs, block, g.blocks, g.per_seg, g.a, sm.rle); break;
-      default: rle_block<8>(src, g.seg, g.n_segs, block, g.blocks, g.per_seg, g.a, sm.rle); break;
+      case 0: rle_block<1>(src, g.seg, g.n_segs, block, g.per_seg, g.a, sm.rle); break;
+      case 1: rle_block<2>(src, g.seg, g.n_segs, block, g.per_seg, g.a, sm.rle); break;
+      case 2: rle_block<4>(src, g.seg, g.n_segs, block, g.per_seg, g.a, sm.rle); break;
+      default: rle_block<8>(src, g.seg, g.n_segs, block, g.per_seg, g.a, sm.rle); break;
     }
     return;
   }

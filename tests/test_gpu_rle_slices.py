@@ -51,3 +51,10 @@ def test_long_runs(n_segs, entries, longest, dtype):
     got = out.cpu().numpy()
     np.testing.assert_array_equal(got[:want.nbytes].view("<" + dtype), want)
     assert (got[want.nbytes:] == 0xCC).all()
+
+
+@pytest.mark.parametrize("n_segs,rows", [(7, 16_000), (8, 16_384), (9, 16_385), (63, 100), (64, 2_048), (65, 2_048),
+                                         (32, 4_096), (43, 4_097), (129, 100)])
+def test_launch_edges(n_segs, rows):
+    """Launches of one slice less, as many and one more than whole turns of 64."""
+    test_long_runs(n_segs, rows // 10, 10, "u4")
