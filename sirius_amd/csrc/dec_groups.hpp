@@ -78,27 +78,33 @@ __device__ __forceinline__ void alp_block(const FixedSeg& sd, uint32_t x, uint32
   }
 }
 
-// One block per (segment, slice of `slice_rows` rows) over a 1-D grid.
-// Workgroups are dispatched to the 8 XCDs round-robin, each with an L2 of its
-// own, and every slice reads all of its segment's counts.  So an XCD takes eight
-// slices in a row, half a row group, and the next XCD the next eight: the chip
-// writes within 4 MiB at a time.  An eighth of the whole launch to each XCD, as it
-// was, reads the counts once but writes eight places far apart, and memory takes
-// that less well (32 Mi int64 rows in runs of 64: 56.0 us, so 54.0; runs of 16:
-// 65.0, 62.6; runs of 2, whose counts are as much as a quarter of what is moved:
-// 180.1, 181.0; int32 in runs of 300: 32.9, 31.6, of 2: 194.5, 197.0; 64 Mi integers and dates 230.9,
-// 227.5).
-constexpr uint32_t N_XCD          = 8;
-constexpr uint32_t RLE_XCD_BLOCKS = 8;
-constexpr uint32_t RLE_XCD_TURN   = N_XCD * RLE_XCD_BLOCKS;  // the grid is a multiple of it
+// Workgroups are dispatched to the 8 XCDs round-robin, each with an L2 and address
+// translations of its own.  The block of a grid of `blocks` that the `block`-th
+// workgroup takes, so that an XCD takes `run` in a row and the next XCD the next
+// `run`; what is left after whole turns of all XCDs is taken in plain order.
+constexpr uint32_t N_XCD = 8;
+__device__ __forceinline__ uint32_t xcd_order(uint32_t block, uint32_t blocks, uint32_t run)
+{
+  const uint32_t in_turn = block % (N_XCD * run), turn = block - in_turn;
+  return turn + N_XCD * run <= blocks ? turn + in_turn % N_XCD * run + in_turn / N_XCD : block;
+}
 
-// Block `block`, the first of which is on an XCD 0.
+// One block per (segment, slice of `slice_rows` rows) over a 1-D grid.  Every
+// slice reads all of its segment's counts, so an XCD takes eight in a row, half a
+// row group, and the chip writes within 4 MiB at a time.  An eighth of the whole
+// launch to each XCD, as it was, reads the counts once but writes eight places far
+// apart, and memory takes that less well (32 Mi int64 rows in runs of 64: 56.0 us,
+// so 54.0; runs of 16: 65.0, 62.6; runs of 2, whose counts are as much as a quarter
+// of what is moved: 180.1, 181.0; int32 in runs of 300: 32.9, 31.6, of 2: 194.5,
+// 197.0; 64 Mi integers and dates 230.9, 227.5).
+constexpr uint32_t RLE_XCD_RUN = 8;
+
+// Block `block` of `blocks`, the first of them on an XCD 0.
 template <uint32_t TS, class Src>
 __device__ __forceinline__ void rle_block(const Src& src, uint32_t seg0, uint32_t n_segs, uint32_t block,
-                                          uint32_t slices, uint32_t slice_rows, RleSmem& sm)
+                                          uint32_t blocks, uint32_t slices, uint32_t slice_rows, RleSmem& sm)
 {
-  const uint32_t in_turn = block % RLE_XCD_TURN;
-  const uint32_t logical = block - in_turn + in_turn % N_XCD * RLE_XCD_BLOCKS + in_turn / N_XCD;
+  const uint32_t logical = xcd_order(block, blocks, RLE_XCD_RUN);
   const uint32_t sgi     = logical / slices;
   if (sgi >= n_segs) return;
   const FixedSeg sd = src.at(seg0 + sgi);
@@ -216,7 +222,12 @@ __device__ __forceinline__ void mask_block(const MaskUnit& u, uint32_t index, ui
 // wavefronts a SIMD, as most of the codecs' own kernels.
 //
 // A group's blocks are consecutive and begin at a multiple of 8, so that a block
-// runs on the XCD its number within the group says.
+// runs on the XCD its number within the group says.  An XCD takes 32 of them in a
+// row, so that it translates the addresses of an eighth of the pages that are in
+// use (in plain order, and 32 in a row: 16 Mi rows of ALP and ALP-RD 107.4 and
+// 104.6 us, 64 Mi integers and dates 227.8 and 226.0, 10 M rows of six widths 76.2
+// and 75.0; 8 in a row 105.6, 228.4, 75.5; 128 in a row 104.5, 230.0, 76.9).
+constexpr uint32_t GROUP_XCD_RUN = 32;
 enum GroupKind : uint32_t {  // + log2 of the value width
   GK_BITPACKING = 0,
   GK_RLE        = 4,
@@ -271,10 +282,10 @@ __device__ __forceinline__ void groups_block(const Src& src, const GroupTable& t
   if (block >= g.blocks) return;  // between two groups
   if (g.kind - GK_RLE < 4u) {
     switch (g.kind - GK_RLE) {
-      case 0: rle_block<1>(src, g.seg, g.n_segs, block, g.per_seg, g.a, sm.rle); break;
-      case 1: rle_block<2>(src, g.seg, g.n_segs, block, g.per_seg, g.a, sm.rle); break;
-      case 2: rle_block<4>(src, g.seg, g.n_segs, block, g.per_seg, g.a, sm.rle); break;
-      default: rle_block<8>(src, g.seg, g.n_segs, block, g.per_seg, g.a, sm.rle); break;
+      case 0: rle_block<1>(src, g.seg, g.n_segs, block, g.blocks, g.per_seg, g.a, sm.rle); break;
+      case 1: rle_block<2>(src, g.seg, g.n_segs, block, g.blocks, g.per_seg, g.a, sm.rle); break;
+      case 2: rle_block<4>(src, g.seg, g.n_segs, block, g.blocks, g.per_seg, g.a, sm.rle); break;
+      default: rle_block<8>(src, g.seg, g.n_segs, block, g.blocks, g.per_seg, g.a, sm.rle); break;
     }
     return;
   }
@@ -282,7 +293,8 @@ __device__ __forceinline__ void groups_block(const Src& src, const GroupTable& t
     mask_block(mask_unit(src, t, g.seg + block), g.a + block, t.counts, nullptr, sm.mask);
     return;
   }
-  const uint32_t y  = block / g.per_seg, x = block - y * g.per_seg;
+  const uint32_t b  = xcd_order(block, g.blocks, GROUP_XCD_RUN);
+  const uint32_t y  = b / g.per_seg, x = b - y * g.per_seg;
   const FixedSeg sd = src.at(g.seg + y);
   switch (g.kind) {
     case GK_BITPACKING + 0: bp_block<uint8_t>(sd, x, g.a, g.b, sm.bp); break;

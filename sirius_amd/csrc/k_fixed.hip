@@ -29,7 +29,7 @@ template <uint32_t TS, class Src>
 __global__ __launch_bounds__(RLE_THREADS) void k_rle(Src src, uint32_t n_segs, uint32_t slices, uint32_t slice_rows)
 {
   __shared__ RleSmem sm;
-  rle_block<TS>(src, 0, n_segs, blockIdx.x, slices, slice_rows, sm);
+  rle_block<TS>(src, 0, n_segs, blockIdx.x, gridDim.x, slices, slice_rows, sm);
 }
 
 template <class Src>
@@ -135,11 +135,10 @@ hipError_t launch_rle(const FixedSeg* segs, uint32_t seg_base, uint32_t n, uint3
   const uint32_t sr     = rle_slice_rows(n, max_rows, ts);
   const uint32_t slices = (max_rows + sr - 1) / sr;
   // segments per launch so that the 1-D grid stays below 2^31 blocks
-  const uint32_t per = static_cast<uint32_t>(std::min<uint64_t>(MAX_GRID_Y, (0x7FFFFF00ull / slices)));
+  const uint32_t per = static_cast<uint32_t>(std::min<uint64_t>(MAX_GRID_Y, (0x7FFFFFF0ull / slices)));
   return for_segs(segs, seg_base, n, host, per, [&](auto src, uint32_t m) {
     using S = decltype(src);
-    const uint64_t blocks = (uint64_t{m} * slices + RLE_XCD_TURN - 1) / RLE_XCD_TURN * RLE_XCD_TURN;
-    const dim3 grid(static_cast<uint32_t>(blocks)), block(RLE_THREADS);
+    const dim3 grid(m * slices), block(RLE_THREADS);
     switch (ts) {
       case 1: hipLaunchKernelGGL((k_rle<1, S>), grid, block, 0, s, src, m, slices, sr); break;
       case 2: hipLaunchKernelGGL((k_rle<2, S>), grid, block, 0, s, src, m, slices, sr); break;
@@ -279,7 +278,6 @@ static Group group_of(const FixedGroup& f, uint32_t n)
       g.per_seg = static_cast<uint32_t>((uint64_t{f.max_rows} * f.ts + COPY_UNIT - 1) / COPY_UNIT);
   }
   blocks = uint64_t{n} * g.per_seg;
-  if (f.codec == SDR_CODEC_RLE) blocks = (blocks + RLE_XCD_TURN - 1) / RLE_XCD_TURN * RLE_XCD_TURN;
   g.blocks = blocks < 0x7FFFFFF0u ? static_cast<uint32_t>(blocks) : 0u;  // 0: too many for a launch
   return g;
 }
