@@ -73,3 +73,27 @@ def test_all_groups(mode, segs):
             np.testing.assert_array_equal(got[:bits.size], bits)
             assert (got[bits.size:] == 0xA5).all()
             assert arr[c].null_count == rows - int(np.unpackbits(bits, bitorder="little")[:rows].sum())
+
+
+@pytest.mark.parametrize("segs", [1023, 1024, 1025, 1300])
+@pytest.mark.parametrize("which", ["alp4", "alp8", "alprd8", "copy8"])
+def test_blocks_of_one_group(which, segs):
+    """One segment less, as many and one more than the blocks a launch takes in
+    the order of the dies, and some past its last whole turn."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    rng = np.random.default_rng(segs)
+    rows = segs * SEG - 5
+    i = {"alp4": 8, "alp8": 9, "alprd8": 11, "copy8": 12}[which]
+    codec, values, encode = _columns(rows, rng)[i]
+    ts = values.dtype.itemsize
+    enc = encode(values, rg_rows=SEG)
+    d = torch.from_numpy(np.concatenate([enc.blob, np.zeros(64, np.uint8)])).cuda()
+    out = torch.full((rows * ts + 64,), 0xCC, dtype=torch.uint8, device="cuda")
+    col, keep = fixed_column([(codec, enc.segments(d.data_ptr()))], ts, rows, out.data_ptr())
+    print(f"[gpu] one group {which} segs={segs}", flush=True)
+    L.check(L.load().sdr_decode_table(C.byref(col), 1, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    np.testing.assert_array_equal(got[:values.nbytes], values.view(np.uint8).reshape(-1))
+    assert (got[values.nbytes:] == 0xCC).all()
