@@ -205,7 +205,9 @@ int sdr_plan_create(const sdr_column* cols, uint32_t n_cols, uint32_t launch_mod
 int sdr_plan_launch(sdr_plan* plan, sdr_stream_t stream);
 /* Launch only the kernels of one codec (codec 0 = all). */
 int sdr_plan_launch_codec(sdr_plan* plan, uint32_t codec, sdr_stream_t stream);
-/* Number of kernel launches one sdr_plan_launch enqueues. */
+/* Number of decode launches of a plan, one for each codec and width (in the
+ * plain mode for each segment); sdr_plan_launch enqueues those of a batched
+ * plan as one kernel where it can. */
 int sdr_plan_num_launches(const sdr_plan* plan);
 int sdr_plan_null_counts(sdr_plan* plan, int64_t* counts, uint32_t n_cols, sdr_stream_t stream);
 int sdr_plan_destroy(sdr_plan* plan);
