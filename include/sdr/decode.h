@@ -226,7 +226,9 @@ int sdr_plan_destroy(sdr_plan* plan);
  * reused pinned buffer; it is never replayed from a graph.  It has no
  * counterpart in the reference, which launches one kernel per codec run
  * (src/cuda/scan/gpu_native_decode.cu:356-386, gpu_decode_strings.cu:257-366);
- * every output is identical to sdr_decode_table / sdr_decode_strings_column.
+ * every output is identical to sdr_decode_table / sdr_decode_strings_column
+ * and complete once the launch's stream has passed it; sdr_batch_finish
+ * reports what the columns took, null counts and errors.
  * Columns, segment bytes and outputs must stay valid until sdr_batch_finish.
  * A batch is used from one thread; its launches are ordered on the stream
  * of the previous launch. */

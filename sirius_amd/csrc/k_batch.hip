@@ -10,8 +10,8 @@
 // A fixed-width group kernel's grid is its resident capacity.  Fixed-width
 // entries are independent, so block b takes entries b, b + grid, ... with no
 // claim at all; its four wavefronts decode an entry's units (an RLE slice is
-// decoded by the whole block).  The FSST kernel runs one block per chunk, in
-// queue order, which is what lets a chunk wait on its predecessors' offsets.  By
+// decoded by the whole block).  The FSST kernel runs one block per chunk; a
+// chunk waits on its predecessors' offsets.  By
 // default fixed-width segments are not queued: the front kernel decodes them
 // beside the FSST pre-pass.
 #include "dec_fsst.hpp"
@@ -101,28 +101,10 @@ __global__ __launch_bounds__(BLOCK_THREADS) void k_bgroup_copy(const BatchItem* 
   }
 }
 
-// One block per FSST entry (the grid is the group's entry count): the entry of
-// its own number, or the next in queue order, claimed with one atomic, so that a
-// chunk's predecessors in its column are held by blocks that started earlier,
-// which the look-back's progress needs (as the per-column kernels do).  One chunk
-// per block, with no loop around it, keeps the kernel at 80 VGPRs: three
-// workgroups of eight waves per CU.
-__global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_bgroup_fsst(
-  const BatchItem* __restrict__ items, BatchQueue* __restrict__ q, uint32_t g)
+// Entry `idx` of the FSST group with the calling workgroup: on the columns' first
+// states, or on those of the second attempt.
+__device__ __forceinline__ void fsst_entry(const BatchQueue* __restrict__ q, uint32_t idx, bool again, FsstSmem& sm)
 {
-  __shared__ FsstSmem sm;
-  __shared__ uint32_t s_idx;
-  (void)items;  // the FSST group's entries are q->fsst_entries
-  const uint32_t first = q->first[g], count = q->count[g];
-  const uint32_t spin  = q->spin_limit;
-  uint32_t i           = blockIdx.x;
-  if (q->ordered) {  // uniform
-    if (threadIdx.x == 0) s_idx = atomicAdd(&q->claimed[g].v, 1u);
-    __syncthreads();
-    i = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(s_idx)));
-  }
-  if (i >= count) return;  // the grid is the entry count: never taken
-  const uint32_t idx = first + i;
   // the entries list every column's chunks column by column, as the batch's
   // chunk and chunk-info arrays do: entry idx describes chunk idx of those
   // arrays, so the chunk loads need not wait for the column's; every lane
@@ -135,7 +117,46 @@ __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6)
   // the compressed bytes
   const FsstColumn col = sload(q->fsst_cols + e.col);
   fsst_chunk(ch, ci, q->fsst_tabs + (ch.seg == FSST_GAP ? 0u : ch.seg), e.chunk, col.n_chunks,
-                             col.state, col.offsets, col.chars, col.chars_cap, col.total_rows, spin, sm);
+             again ? col.again : col.state, col.offsets, col.chars, col.chars_cap, col.total_rows,
+             again ? q->spin_limit : q->spin_limit / FSST_UNORDERED_SHARE, sm);
+}
+
+// One block per FSST entry (the grid is the group's entry count), that of its own
+// number.  One chunk per block, with no loop around it, keeps the kernel at 80
+// VGPRs: three workgroups of eight waves per CU.
+__global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_bgroup_fsst(
+  const BatchItem* __restrict__ items, BatchQueue* __restrict__ q, uint32_t g)
+{
+  __shared__ FsstSmem sm;
+  (void)items;  // the FSST group's entries are q->fsst_entries
+  if (blockIdx.x >= q->count[g]) return;  // the grid is the entry count: never taken
+  fsst_entry(q, q->first[g] + blockIdx.x, false, sm);
+}
+
+// The columns that k_bgroup_fsst reported incomplete, from the start: their chunks
+// in the order of tickets, so that a chunk's predecessors are done or held by
+// workgroups that run, in whatever order those are started.  Right behind it on the
+// stream: what follows a launch finds its columns complete.  Nearly always there are
+// none (a served batch of 128 requests 334 us without this kernel, 333 us with it, 355 us
+// with a ticket for each chunk at once).
+// (Its occupancy is that of k_bgroup_fsst, with which it shares a called function.)
+__global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_batch_again(BatchQueue* __restrict__ q, uint32_t n)
+{
+  __shared__ FsstSmem sm;
+  __shared__ uint32_t s_next;
+  bool failed = false;
+  for (uint32_t i = threadIdx.x; i < q->n_cols; i += FSST_THREADS)
+    failed = failed || *gbl(&gload(q->fsst_cols + i).state->error) != 0u;
+  if (!__syncthreads_or(failed)) return;
+  for (;;) {
+    if (threadIdx.x == 0) s_next = atomicAdd(&q->ticket, 1u);
+    __syncthreads();
+    const uint32_t i = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(s_next)));
+    if (i >= n) return;
+    const uint32_t idx = q->first[BG_FSST] + i;
+    if (*gbl(&gload(q->fsst_cols + gload(q->fsst_entries + idx).col).state->error) != 0u) fsst_entry(q, idx, true, sm);
+    __syncthreads();  // the next entry's use of sm and s_next
+  }
 }
 
 // The FSST segment pre-pass over the queue's segments with `blocks` workgroups, of
@@ -145,7 +166,11 @@ __device__ __forceinline__ void batch_prep(const BatchQueue* __restrict__ q, uin
                                            FsstPrepSmem<NT>& sm)
 {
   if (block == 0)
-    for (uint32_t i = threadIdx.x; i < q->n_cols; i += NT) gbl(gload(q->fsst_cols + i).state)->result = q->results + i;
+    for (uint32_t i = threadIdx.x; i < q->n_cols; i += NT) {
+      const FsstColumn col      = gload(q->fsst_cols + i);
+      gbl(col.state)->result = q->results + i;
+      gbl(col.again)->result = q->results + q->n_cols + i;
+    }
   const uint32_t n = q->n_fsst_segs;
   for (uint32_t i = block; i < n; i += blocks)
     fsst_prep_segment(gload(q->fsst_segs + i), i, q->fsst_chunks, q->fsst_info, q->fsst_tabs + i, sm);
@@ -252,6 +277,12 @@ hipError_t launch_batch_fsst_prep(BatchQueue* q, hipStream_t s)
 }
 
 const void* batch_fsst_prep_kernel() { return reinterpret_cast<const void*>(k_batch_fsst_prep); }
+
+hipError_t launch_batch_again(BatchQueue* q, uint32_t n_entries, hipStream_t s)
+{
+  hipLaunchKernelGGL(k_batch_again, dim3(std::min(n_entries, 256u)), dim3(FSST_THREADS), 0, s, q, n_entries);
+  return hipGetLastError();
+}
 
 hipError_t launch_batch_group(const BatchItem* items, BatchQueue* q, uint32_t g, uint32_t grid, hipStream_t s)
 {

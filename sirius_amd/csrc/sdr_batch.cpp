@@ -48,8 +48,6 @@ struct sdr_batch {
   size_t used_bytes    = 0;
   uint32_t n_fsst_segs = 0;  // row ranges of the last upload's string columns
   size_t n_results     = 0;  // ... and these
-  size_t upload_bytes  = 0;  // of it, in h_stage
-  uint32_t spin_limit  = 0;  // the whole bound at the time
   size_t off_items = 0, off_cols = 0, off_chunks = 0, off_segs = 0, off_state = 0, off_units = 0;
   uint32_t n_status    = 0;
   hipEvent_t launch_done = nullptr;
@@ -364,9 +362,9 @@ int batch_upload(sdr_batch* b, hipStream_t s)
     n_chunks += c.n_chunks;
     n_segs += c.segs.size();
   }
-  // FsstState: FSST_STATE_WORDS + n words per column
+  // FsstState: FSST_STATE_WORDS + n words per column, and again
   size_t state_words = 0;
-  for (auto& c : b->cols) state_words += FSST_STATE_WORDS + c.n_chunks;
+  for (auto& c : b->cols) state_words += 2u * (FSST_STATE_WORDS + c.n_chunks);
   size_t off                  = al(sizeof(BatchQueue));
   b->off_items                = off;
   off                         = al(off + n_entries * sizeof(BatchItem));
@@ -414,7 +412,7 @@ int batch_upload(sdr_batch* b, hipStream_t s)
     HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&b->h_stage), upload_bytes + upload_bytes / 4, hipHostMallocDefault));
     b->stage_bytes = upload_bytes + upload_bytes / 4;
   }
-  const size_t readback_bytes = b->cols.size() * sizeof(FsstResult) + b->mask_units.size() * sizeof(uint32_t);
+  const size_t readback_bytes = 2u * b->cols.size() * sizeof(FsstResult) + b->mask_units.size() * sizeof(uint32_t);
   b->n_results = b->cols.size();
   if (readback_bytes > b->readback_cap) {
     if (b->launch_done) HIP_TRY(hipEventSynchronize(b->launch_done));  // its kernels write there
@@ -444,10 +442,7 @@ int batch_upload(sdr_batch* b, hipStream_t s)
   q.fsst_status   = reinterpret_cast<uint64_t*>(d + b->off_state);
   q.n_fsst_segs   = static_cast<uint32_t>(n_segs);
   b->n_fsst_segs  = q.n_fsst_segs;
-  const uint32_t bound = tune(SDR_TUNE_FSST_SPIN_LIMIT);
-  q.ordered       = fsst_unordered(bound) ? 0u : 1u;
-  q.spin_limit    = q.ordered ? bound : bound / FSST_UNORDERED_SHARE;
-  b->spin_limit   = bound;
+  q.spin_limit    = tune(SDR_TUNE_FSST_SPIN_LIMIT);
   q.fsst_segs     = reinterpret_cast<const FsstSeg*>(d + b->off_segs);
   q.fsst_chunks   = reinterpret_cast<FsstChunk*>(d + b->off_chunks);
   q.fsst_info     = reinterpret_cast<FsstChunkInfo*>(d + off_info);
@@ -466,6 +461,7 @@ int batch_upload(sdr_batch* b, hipStream_t s)
     fc.info       = reinterpret_cast<const FsstChunkInfo*>(d + off_info) + ck;
     fc.tabs       = reinterpret_cast<const FsstSymTab*>(d + off_tabs);  // chunk seg indices are batch-wide
     fc.state      = reinterpret_cast<FsstState*>(reinterpret_cast<uint64_t*>(d + b->off_state) + st);
+    fc.again      = reinterpret_cast<FsstState*>(reinterpret_cast<uint64_t*>(fc.state) + FSST_STATE_WORDS + c.n_chunks);
     fc.offsets    = c.offsets;
     fc.chars      = c.chars;
     fc.chars_cap  = c.cap;
@@ -479,7 +475,7 @@ int batch_upload(sdr_batch* b, hipStream_t s)
     }
     ck += c.n_chunks;
     sg += c.segs.size();
-    st += FSST_STATE_WORDS + c.n_chunks;
+    st += 2u * (FSST_STATE_WORDS + c.n_chunks);
   }
   if (!dcols.empty()) std::memcpy(h + b->off_cols, dcols.data(), dcols.size() * sizeof(FsstColumn));
   if (!b->mask_units.empty())
@@ -503,8 +499,7 @@ int batch_upload(sdr_batch* b, hipStream_t s)
       dst.n_units    = std::min(per[g], it.n_units - u);
     }
   }
-  b->upload_bytes = upload_bytes;
-  HIP_TRY(launch_batch_setup(d, h, upload_bytes, q.fsst_status, q.n_fsst_status, q.results, q.n_cols, s));
+  HIP_TRY(launch_batch_setup(d, h, upload_bytes, q.fsst_status, q.n_fsst_status, q.results, 2u * q.n_cols, s));
   if (!b->upload_done) HIP_TRY(hipEventCreateWithFlags(&b->upload_done, hipEventDisableTiming));
   HIP_TRY(hipEventRecord(b->upload_done, s));
   b->upload_pending = true;
@@ -560,7 +555,7 @@ hipError_t launch_fixed_grids(const sdr_batch* b, hipStream_t s, const FixedSeg*
 // The null counts of the mask pieces, behind the columns' results.
 uint32_t* mask_counts(const sdr_batch* b)
 {
-  return reinterpret_cast<uint32_t*>(b->h_readback + b->n_results * sizeof(FsstResult));
+  return reinterpret_cast<uint32_t*>(b->h_readback + 2u * b->n_results * sizeof(FsstResult));
 }
 
 // The validity masks (UNCOMPRESSED overlays) in a launch of their own.
@@ -724,6 +719,7 @@ int batch_launch(sdr_batch* b, hipStream_t s)
   } else {
     HIP_TRY(enqueue_direct(b, q, items, mask, grid, cnt, b->n_fsst_segs, s));
   }
+  if (strings) HIP_TRY(launch_batch_again(q, cnt[BG_FSST], s));
   if (b->use_graph && (mask || !b->fixed.empty())) HIP_TRY(launch_masks(b, s));
   // a column of no rows has no chunk to write its closing offset
   for (const auto& c : b->cols)
@@ -745,46 +741,22 @@ int batch_ready(sdr_batch* b)
   return fail(SDR_E_HIP, "batch launch: %s", hipGetErrorString(e));
 }
 
-// The string columns of the finished launch once more, their chunks by ticket,
-// from the upload as it still is in the staging copy.
-int batch_strings_ordered(sdr_batch* b)
-{
-  hipStream_t s = b->last_stream;
-  auto* hq      = reinterpret_cast<BatchQueue*>(b->h_stage);
-  auto* q       = reinterpret_cast<BatchQueue*>(b->d_arena);
-  hq->ordered    = 1u;
-  hq->spin_limit = b->spin_limit;
-  HIP_TRY(launch_batch_setup(b->d_arena, b->h_stage, b->upload_bytes, hq->fsst_status, hq->n_fsst_status, hq->results,
-                             hq->n_cols, s));
-  HIP_TRY(launch_batch_fsst_prep(q, s));
-  HIP_TRY(launch_batch_group(reinterpret_cast<const BatchItem*>(b->d_arena + b->off_items), q, BG_FSST,
-                             b->entry_count[BG_FSST], s));
-  HIP_TRY(hipStreamSynchronize(s));
-  return SDR_OK;
-}
-
 // After the last launch finished: write string totals and null counts back
 // into the added columns and report look-back failures and overflow.
 int batch_collect(sdr_batch* b)
 {
   if (!b->launched) return SDR_OK;
   b->launched = false;
-  const auto* res = reinterpret_cast<const FsstResult*>(b->h_readback);
-  if (b->n_results && !reinterpret_cast<const BatchQueue*>(b->h_stage)->ordered) {
-    bool again = false;  // chunks were not started in order
-    for (size_t i = 0; i < b->n_results; ++i) again = again || res[i].error;
-    if (again) {
-      const int rc = batch_strings_ordered(b);
-      if (rc) return rc;
-    }
-  }
+  const auto* first = reinterpret_cast<const FsstResult*>(b->h_readback);
   const uint32_t* nulls = mask_counts(b);
-  int rc = SDR_OK;
+  int rc   = SDR_OK;
+  size_t i = 0;
   for (auto& c : b->cols) {
-    if (res == reinterpret_cast<const FsstResult*>(b->h_readback) + b->n_results) break;  // added after the launch
-    const uint64_t err   = res->error;
-    const uint64_t total = res->total;
-    ++res;
+    if (i == b->n_results) break;  // added after the launch
+    const FsstResult& res = first[i].error ? first[b->n_results + i] : first[i];  // of the column's last attempt
+    const uint64_t err    = res.error;
+    const uint64_t total  = res.total;
+    ++i;
     c.user->chars_used = total;
     c.status           = err ? SDR_E_HIP : (total > 0x7FFFFFFFull || total > c.cap) ? SDR_E_OVERFLOW : SDR_OK;
     if (c.status && !rc)

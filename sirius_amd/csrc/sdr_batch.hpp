@@ -29,6 +29,7 @@ struct FsstColumn {
   const FsstChunkInfo* info;  // per chunk, from the segment pre-pass
   const FsstSymTab* tabs;     // per row range of the batch (a chunk's seg indexes it), from the pre-pass
   FsstState* state;
+  FsstState* again;           // of the second attempt
   int32_t* offsets;
   uint8_t* chars;
   uint64_t chars_cap;
@@ -71,22 +72,15 @@ enum BatchGroup : uint32_t {
   BG_COUNT
 };
 
-// A claim counter on a cache line of its own: the group kernels run at once
-// and each claims from its own counter.
-struct alignas(128) BatchCounter {
-  uint32_t v;
-};
-
 // Queue header read by the kernels.
 struct BatchQueue {
-  BatchCounter claimed[BG_COUNT];  // next unclaimed entry of each group (uploaded as 0)
-  uint32_t first[BG_COUNT];        // each group's entries: [first, first + count)
+  uint32_t first[BG_COUNT];  // each group's entries: [first, first + count)
   uint32_t count[BG_COUNT];
   uint32_t n_items;
   uint32_t error;
   uint32_t n_fsst_status;  // words of `fsst_status`, cleared by a launch's first kernel
   uint32_t spin_limit;     // look-back wait bound of the FSST chunks
-  uint32_t ordered;        // their entries by ticket, see FSST_UNORDERED_SHARE
+  uint32_t ticket;         // of the second attempt: its next entry (uploaded as 0)
   uint32_t n_fsst_segs;    // row ranges of all FSST columns, for the pre-pass
   uint32_t bp_chunk_rows[4];  // most rows a bitpacking wavefront stages at once, per width 1/2/4/8
   uint64_t* fsst_status;   // contiguous FsstState storage of all FSST columns
@@ -96,7 +90,8 @@ struct BatchQueue {
   FsstSymTab* fsst_tabs;
   const FsstEntry* fsst_entries;  // the FSST group's entries (first[BG_FSST] is 0)
   const FsstColumn* fsst_cols;    // the string columns they index
-  FsstResult* results;            // what they report, in pinned memory
+  FsstResult* results;            // what they report, in pinned memory: n_cols of the
+                                  // first attempt, n_cols of the second
   uint32_t n_cols;
 };
 
@@ -129,6 +124,9 @@ hipError_t launch_batch_front(BatchQueue* q, uint32_t n_fsst_segs, const FixedGr
                               const FixedSeg* segs, const MaskUnit* units, uint32_t* counts, hipStream_t s, bool* done);
 // FSST segment pre-pass over the queue's segments.
 hipError_t launch_batch_fsst_prep(BatchQueue* q, hipStream_t s);
+// The string columns that the launch's first attempt could not complete, again; see
+// FSST_UNORDERED_SHARE.
+hipError_t launch_batch_again(BatchQueue* q, uint32_t n_entries, hipStream_t s);
 // The persistent kernel of group g over `grid` blocks.
 hipError_t launch_batch_group(const BatchItem* items, BatchQueue* q, uint32_t g, uint32_t grid, hipStream_t s);
 // Kernel, block size and resident blocks per CU of group g (for graph nodes

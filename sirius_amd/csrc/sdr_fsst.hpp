@@ -21,7 +21,9 @@ constexpr uint32_t FSST_SPIN_LIMIT = 1u << 24;     // look-back wait bound (neve
 // workgroups draw as they start, which needs no assumption but costs each of
 // them one of a queue of atomics on one word, 13 ns apart (16 Mi rows 293 us,
 // without 274; 2 M rows of 27 chars 44 us, 35 us; a batch's strings 182 us, 168 us).
-// A bound below 1024 (tests) goes to the tickets at once.
+// A call that waits for its result before it returns looks at it and decodes again
+// (with a bound below 1024, for tests, by ticket at once); behind a batch's chunks, whose
+// outputs are to be complete in stream order, a kernel does (k_batch_again).
 constexpr uint32_t FSST_UNORDERED_SHARE = 1024;
 inline bool fsst_unordered(uint32_t spin_limit) { return spin_limit >= FSST_UNORDERED_SHARE; }
 
