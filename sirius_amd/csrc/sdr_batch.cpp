@@ -345,6 +345,8 @@ int batch_upload(sdr_batch* b, hipStream_t s)
     for (auto& fl : b->fixed)
       for (uint32_t j = 0; j < fl.n; ++j) fl.max_rows = std::max(fl.max_rows, fsegs[fl.base + j].row_count);
   }
+  b->mask_units.clear();
+  b->mask_ends.clear();
   b->fixed_src = sdr_batch::FS_ARENA;
   if (b->fixed_grids && mask == 0 && b->cols.empty() && b->masks.empty() && !b->fixed.empty()) {
     // nothing on the device reads the arena: up to two launches of
@@ -376,8 +378,6 @@ int batch_upload(sdr_batch* b, hipStream_t s)
   off                         = al(off + b->cols.size() * sizeof(FsstColumn));
   b->off_segs                 = off;
   off                         = al(off + n_segs * sizeof(FsstSeg));
-  b->mask_units.clear();
-  b->mask_ends.clear();
   for (const auto& m : b->masks) {
     if (m.fixed) add_mask_units(m.fixed->validity, m.fixed->n_validity, m.fixed->total_rows, m.fixed->d_null_mask, b->mask_units);
     else add_mask_units(m.str->validity, m.str->n_validity, m.str->total_rows, m.str->d_null_mask, b->mask_units);
@@ -765,7 +765,7 @@ int batch_collect(sdr_batch* b)
              : fail(SDR_E_OVERFLOW, "total_chars (%llu) exceeds capacity (%llu) or int32 max",
                     static_cast<unsigned long long>(total), static_cast<unsigned long long>(c.cap));
   }
-  for (size_t i = 0, u = 0; i < b->masks.size(); ++i) {
+  for (size_t i = 0, u = 0; i < b->mask_ends.size(); ++i) {  // of the masks launched; later ones come behind them
     int64_t n = 0;
     for (; u < b->mask_ends[i]; ++u) n += nulls[u];
     if (b->masks[i].fixed) b->masks[i].fixed->null_count = n;
