@@ -405,11 +405,16 @@ int masks_prepare(const std::vector<MaskUnit>& units, MaskLaunch* m, void** toke
 
 namespace {
 
-// The pieces in launches of their own.
-hipError_t launch_masks(const MaskLaunch& m, hipStream_t s)
+// The pieces in launches of their own; with `shared` those of each column in turn.
+hipError_t launch_masks(const MaskLaunch& m, hipStream_t s, bool shared = false)
 {
-  const bool host = m.host && m.n <= MASKS_INLINE;
-  return launch_null_mask(host ? m.host : m.units, m.n, m.counts, nullptr, s, host);
+  const bool host        = m.host && m.n <= MASKS_INLINE;
+  const MaskUnit* pieces = host ? m.host : m.units;
+  if (!shared) return launch_null_mask(pieces, m.n, m.counts, nullptr, s, host);
+  hipError_t e = hipSuccess;
+  for (uint32_t c = 0, at = 0; e == hipSuccess && c < m.n_cols; at = m.ends[c++])
+    e = launch_null_mask(pieces + at, m.ends[c] - at, m.counts + at, nullptr, s, host);
+  return e;
 }
 
 }  // namespace
@@ -518,17 +523,32 @@ int build_batches(const std::vector<RunTarget>& targets, std::vector<Batch>& bat
   return SDR_OK;
 }
 
+// Whether some of the outputs share bytes (taken in the order of the runs, whose
+// segments are neighbours whatever their codecs).
+static bool outputs_share(const std::vector<RunTarget>& targets, const MaskUnit* units, size_t n_units)
+{
+  WrittenBytes w;
+  for (const RunTarget& t : targets)
+    for (uint32_t k = 0; k < t.run->n_segments; ++k) {
+      const sdr_segment& g = t.run->segments[k];
+      w.add(static_cast<uint8_t*>(t.d_out) + uint64_t{g.row_offset} * t.type_size, uint64_t{g.row_count} * t.type_size);
+    }
+  for (size_t i = 0; i < n_units; ++i) w.add(units[i].dst, units[i].bytes);
+  return w.any_twice();
+}
+
 // `d`: the descriptors on the device, or null to carry them in the kernel
-// arguments from `all`.
+// arguments from `all`; `shared`: outputs share bytes, so that each codec and width,
+// and each column's mask, is a launch of its own, in order.
 hipError_t launch_batches(const std::vector<Batch>& batches, const std::vector<FixedSeg>& all, const FixedSeg* d,
-                          uint32_t mode, uint32_t codec_filter, hipStream_t s, const MaskLaunch& masks)
+                          uint32_t mode, uint32_t codec_filter, hipStream_t s, const MaskLaunch& masks, bool shared)
 {
   hipError_t e = hipSuccess;
   const bool host      = d == nullptr;
   const FixedSeg* segs = host ? all.data() : d;
   size_t live = masks.n ? 1 : 0;
   for (const Batch& b : batches) live += b.count != 0;
-  if (live > 1 && mode != SDR_LAUNCH_PER_SEGMENT && !codec_filter) {
+  if (live > 1 && mode != SDR_LAUNCH_PER_SEGMENT && !codec_filter && !shared) {
     std::vector<FixedGroup> groups;
     if (masks.n) groups.push_back({MASK_GROUP, 0, 0, masks.n, 0});
     for (const Batch& b : batches)
@@ -548,7 +568,7 @@ hipError_t launch_batches(const std::vector<Batch>& batches, const std::vector<F
       e = launch_batch(b, segs, b.first, b.count, b.max_rows, s, host);
     }
   }
-  if (e == hipSuccess && masks.n && !codec_filter) e = launch_masks(masks, s);
+  if (e == hipSuccess && masks.n && !codec_filter) e = launch_masks(masks, s, shared);
   return e;
 }
 
@@ -569,8 +589,9 @@ int decode_runs(const std::vector<RunTarget>& targets, hipStream_t s, uint32_t m
   std::vector<FixedSeg> all;
   build_batches(targets, batches, all);
   if (all.empty() && !masks.n) return SDR_OK;
+  const bool shared = batches.size() + masks.n_cols > 1 && outputs_share(targets, masks.host, masks.n);
   if (inline_descriptors(batches, mode)) {
-    const hipError_t e = launch_batches(batches, all, nullptr, mode, 0, s, masks);
+    const hipError_t e = launch_batches(batches, all, nullptr, mode, 0, s, masks, shared);
     if (e != hipSuccess) return fail(SDR_E_HIP, "kernel launch failed: %s", hipGetErrorString(e));
     return SDR_OK;
   }
@@ -578,7 +599,7 @@ int decode_runs(const std::vector<RunTarget>& targets, hipStream_t s, uint32_t m
   void* token = nullptr;
   int rc = desc_pinned(all.data(), all.size() * sizeof(FixedSeg), &d, &token);
   if (rc) return rc;
-  const hipError_t e = launch_batches(batches, all, static_cast<FixedSeg*>(d), mode, 0, s, masks);
+  const hipError_t e = launch_batches(batches, all, static_cast<FixedSeg*>(d), mode, 0, s, masks, shared);
   rc                 = desc_release(token, s);
   if (e != hipSuccess) return fail(SDR_E_HIP, "kernel launch failed: %s", hipGetErrorString(e));
   return rc;
@@ -603,14 +624,16 @@ int decode_table(sdr_column* cols, uint32_t n_cols, hipStream_t s, uint32_t mode
   for (uint32_t c = 0; c < n_cols; ++c)
     if (cols[c].has_nulls && cols[c].n_validity && cols[c].total_rows) masked.push_back(c);
   std::vector<MaskUnit> units;
-  std::vector<size_t> ends;
+  std::vector<uint32_t> ends;
   for (uint32_t c : masked) {
     add_mask_units(cols[c].validity, cols[c].n_validity, cols[c].total_rows, cols[c].d_null_mask, units);
-    ends.push_back(units.size());
+    ends.push_back(static_cast<uint32_t>(units.size()));
   }
   MaskLaunch masks;
   void* token = nullptr;
   if (!masked.empty()) rc = masks_prepare(units, &masks, &token);
+  masks.ends   = ends.data();
+  masks.n_cols = static_cast<uint32_t>(ends.size());
   if (!rc) rc = decode_runs(targets, s, mode, masks);
   if (!masked.empty()) {
     const hipError_t e = rc ? hipErrorUnknown : hipStreamSynchronize(s);
@@ -675,6 +698,7 @@ int plan_create(const sdr_column* cols, uint32_t n_cols, uint32_t mode, hipStrea
     add_mask_units(col.validity, col.n_validity, col.total_rows, col.d_null_mask, units);
     p->mask_ends.push_back(static_cast<uint32_t>(units.size()));
   }
+  p->shared = outputs_share(targets, units.data(), units.size());
   if (e == hipSuccess && !units.empty())
     e = hipMalloc(reinterpret_cast<void**>(&p->d_units), units.size() * sizeof(MaskUnit));
   if (e == hipSuccess && !units.empty())
@@ -697,8 +721,9 @@ int plan_launch(sdr_plan* p, uint32_t codec, hipStream_t s)
   clear_error();
   if (!p) return fail(SDR_E_INVALID_ARG, "plan is NULL");
   MaskLaunch masks;
-  if (!p->masked.empty()) masks = MaskLaunch{nullptr, p->d_units, p->d_counts, p->mask_ends.back()};
-  const hipError_t e = launch_batches(p->batches, p->all, p->d_segs, p->mode, codec, s, masks);
+  if (!p->masked.empty()) masks = MaskLaunch{nullptr, p->d_units, p->d_counts, p->mask_ends.back(), p->mask_ends.data(),
+                                                  static_cast<uint32_t>(p->mask_ends.size())};
+  const hipError_t e = launch_batches(p->batches, p->all, p->d_segs, p->mode, codec, s, masks, p->shared);
   if (e != hipSuccess) return fail(SDR_E_HIP, "kernel launch failed: %s", hipGetErrorString(e));
   return SDR_OK;
 }

@@ -36,6 +36,7 @@ struct sdr_batch {
   std::vector<MaskJob> masks;
   std::vector<sdr::MaskUnit> mask_units;  // the masks' pieces of the last upload
   std::vector<size_t> mask_ends;          // ... and where each mask's end
+  bool shared          = false;           // the last upload's outputs share bytes
   // device arena and pinned staging
   uint8_t* d_arena     = nullptr;
   size_t arena_bytes   = 0;
@@ -69,6 +70,7 @@ struct sdr_batch {
   std::vector<sdr::FixedLaunch> graph_fixed;        // ... that the recorded graph launches
   size_t graph_fsegs   = 0;                         // ... and where their descriptors were
   uint32_t graph_fsst  = 0;                         // ... and its FSST grid (one block per chunk)
+  bool graph_shared    = false;                     // ... and whether its grids are launches of their own
   // where the per-codec grids of the last upload read their descriptors: the
   // arena, or (a batch of fixed-width segments alone, no graph) the kernel
   // arguments or a descriptor slot, as the batched table call passes them
@@ -347,6 +349,15 @@ int batch_upload(sdr_batch* b, hipStream_t s)
   }
   b->mask_units.clear();
   b->mask_ends.clear();
+  for (const auto& m : b->masks) {
+    if (m.fixed) add_mask_units(m.fixed->validity, m.fixed->n_validity, m.fixed->total_rows, m.fixed->d_null_mask, b->mask_units);
+    else add_mask_units(m.str->validity, m.str->n_validity, m.str->total_rows, m.str->d_null_mask, b->mask_units);
+    b->mask_ends.push_back(b->mask_units.size());
+  }
+  WrittenBytes written;
+  for (const BatchItem& it : b->items) written.add(it.out, uint64_t{it.row_count} * it.ts);
+  for (const MaskUnit& u : b->mask_units) written.add(u.dst, u.bytes);
+  b->shared    = written.any_twice();
   b->fixed_src = sdr_batch::FS_ARENA;
   if (b->fixed_grids && mask == 0 && b->cols.empty() && b->masks.empty() && !b->fixed.empty()) {
     // nothing on the device reads the arena: up to two launches of
@@ -378,11 +389,6 @@ int batch_upload(sdr_batch* b, hipStream_t s)
   off                         = al(off + b->cols.size() * sizeof(FsstColumn));
   b->off_segs                 = off;
   off                         = al(off + n_segs * sizeof(FsstSeg));
-  for (const auto& m : b->masks) {
-    if (m.fixed) add_mask_units(m.fixed->validity, m.fixed->n_validity, m.fixed->total_rows, m.fixed->d_null_mask, b->mask_units);
-    else add_mask_units(m.str->validity, m.str->n_validity, m.str->total_rows, m.str->d_null_mask, b->mask_units);
-    b->mask_ends.push_back(b->mask_units.size());
-  }
   b->off_units                = off;
   off                         = al(off + b->mask_units.size() * sizeof(MaskUnit));
   b->off_state                = off;
@@ -524,8 +530,9 @@ std::vector<FixedGroup> fixed_groups(const sdr_batch* b)
   return g;
 }
 
-// The per-codec grids of the batch's fixed-width segments, in one launch or one
-// per codec kind and value width: descriptors in the arena, in the kernel
+// The per-codec grids of the batch's fixed-width segments, in one launch or (where
+// outputs share bytes, or one can not hold them) one per codec kind and value width:
+// descriptors in the arena, in the kernel
 // arguments (FS_INLINE) or at `slot` (FS_SLOT).
 hipError_t launch_fixed_grids(const sdr_batch* b, hipStream_t s, const FixedSeg* slot = nullptr)
 {
@@ -535,8 +542,9 @@ hipError_t launch_fixed_grids(const sdr_batch* b, hipStream_t s, const FixedSeg*
                                                           : reinterpret_cast<const FixedSeg*>(b->d_arena + b->off_fsegs);
   const std::vector<FixedGroup> groups = fixed_groups(b);
   bool done    = false;
-  hipError_t e = launch_groups(groups.data(), static_cast<uint32_t>(groups.size()), segs, nullptr, nullptr, nullptr, s,
-                               host, &done);
+  hipError_t e = hipSuccess;
+  if (!b->shared)
+    e = launch_groups(groups.data(), static_cast<uint32_t>(groups.size()), segs, nullptr, nullptr, nullptr, s, host, &done);
   if (done || e != hipSuccess) return e;
   for (const auto& fl : b->fixed) {
     switch (fl.kind) {
@@ -558,11 +566,18 @@ uint32_t* mask_counts(const sdr_batch* b)
   return reinterpret_cast<uint32_t*>(b->h_readback + 2u * b->n_results * sizeof(FsstResult));
 }
 
-// The validity masks (UNCOMPRESSED overlays) in a launch of their own.
+// The validity masks (UNCOMPRESSED overlays) in a launch of their own, or each in
+// one where outputs share bytes.
 hipError_t launch_masks(const sdr_batch* b, hipStream_t s)
 {
-  return launch_null_mask(reinterpret_cast<const MaskUnit*>(b->d_arena + b->off_units),
-                          static_cast<uint32_t>(b->mask_units.size()), mask_counts(b), nullptr, s, false);
+  const auto* units = reinterpret_cast<const MaskUnit*>(b->d_arena + b->off_units);
+  if (!b->shared)
+    return launch_null_mask(units, static_cast<uint32_t>(b->mask_units.size()), mask_counts(b), nullptr, s, false);
+  hipError_t e = hipSuccess;
+  size_t at    = 0;
+  for (size_t i = 0; e == hipSuccess && i < b->mask_ends.size(); at = b->mask_ends[i++])
+    e = launch_null_mask(units + at, static_cast<uint32_t>(b->mask_ends[i] - at), mask_counts(b) + at, nullptr, s, false);
+  return e;
 }
 
 // Every kernel of a recorded launch in stream order: the FSST pre-pass, the group
@@ -588,10 +603,11 @@ hipError_t enqueue_direct(const sdr_batch* b, BatchQueue* q, const BatchItem* it
   for (const FixedGroup& g : fixed_groups(b)) groups.push_back(g);
   const uint32_t n_segs = mask & (1u << BG_FSST) ? n_fsst_segs : 0u;
   bool done             = false;
-  hipError_t e          = launch_batch_front(q, n_segs, groups.data(), static_cast<uint32_t>(groups.size()),
-                                             reinterpret_cast<const FixedSeg*>(b->d_arena + b->off_fsegs),
-                                             reinterpret_cast<const MaskUnit*>(b->d_arena + b->off_units),
-                                             mask_counts(b), s, &done);
+  hipError_t e          = hipSuccess;
+  if (!b->shared)
+    e = launch_batch_front(q, n_segs, groups.data(), static_cast<uint32_t>(groups.size()),
+                           reinterpret_cast<const FixedSeg*>(b->d_arena + b->off_fsegs),
+                           reinterpret_cast<const MaskUnit*>(b->d_arena + b->off_units), mask_counts(b), s, &done);
   if (e == hipSuccess && !done && n_segs) e = launch_batch_fsst_prep(q, s);
   for (uint32_t g = 0; e == hipSuccess && g < BG_COUNT; ++g)
     if (mask >> g & 1u) e = launch_batch_group(items, q, g, std::min(grid[g], cnt[g]), s);
@@ -644,7 +660,8 @@ int batch_launch(sdr_batch* b, hipStream_t s)
     // with per-codec grids the graph is recorded from the stream order (on
     // the batch's own stream), and recorded again when the grids change
     if (!b->gexec || b->graph_arena != b->d_arena || b->graph_mask != mask || b->graph_gridopt != b->grid ||
-        !(b->graph_fixed == b->fixed) || b->graph_fsegs != b->off_fsegs || b->graph_fsst != cnt[BG_FSST]) {
+        !(b->graph_fixed == b->fixed) || b->graph_fsegs != b->off_fsegs || b->graph_fsst != cnt[BG_FSST] ||
+        b->graph_shared != b->shared) {
       if (b->gexec) HIP_TRY(hipGraphExecDestroy(b->gexec));
       if (b->graph) HIP_TRY(hipGraphDestroy(b->graph));
       b->gexec = nullptr;
@@ -664,6 +681,7 @@ int batch_launch(sdr_batch* b, hipStream_t s)
       b->graph_gridopt = b->grid;
       b->graph_fixed   = b->fixed;
       b->graph_fsegs   = b->off_fsegs;
+      b->graph_shared  = b->shared;
       b->graph_fsst    = cnt[BG_FSST];
     }
     HIP_TRY(hipGraphLaunch(b->gexec, s));

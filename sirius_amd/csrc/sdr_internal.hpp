@@ -6,6 +6,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cstdint>
+#include <utility>
 #include <vector>
 
 namespace sdr {
@@ -58,9 +61,35 @@ struct MaskLaunch {
   const MaskUnit* units = nullptr;
   uint32_t* counts      = nullptr;
   uint32_t n            = 0;
+  const uint32_t* ends  = nullptr;  // a call's: where each of n_cols columns' pieces end
+  uint32_t n_cols       = 0;
 };
 // Pieces and counts in pinned memory, to be launched; `token` as for masks_launch.
 int masks_prepare(const std::vector<MaskUnit>& units, MaskLaunch* m, void** token);
+
+// Bytes that a call's launches write.  Segments may share rows, and columns outputs
+// and masks: the codec or the column that comes later wins, launch after launch.
+// Blocks of one launch have no order, so what shares a byte may not share a launch.
+class WrittenBytes {
+ public:
+  void add(const void* p, uint64_t bytes)
+  {
+    const uintptr_t lo = reinterpret_cast<uintptr_t>(p);
+    if (bytes == 0) return;
+    if (!spans_.empty() && spans_.back().second == lo) spans_.back().second = lo + bytes;
+    else spans_.push_back({lo, lo + bytes});
+  }
+  bool any_twice()
+  {
+    std::sort(spans_.begin(), spans_.end());
+    for (size_t i = 1; i < spans_.size(); ++i)
+      if (spans_[i].first < spans_[i - 1].second) return true;
+    return false;
+  }
+
+ private:
+  std::vector<std::pair<uintptr_t, uintptr_t>> spans_;  // one for a column whose segments come in row order
+};
 
 // One fixed-width run and where its rows go.
 struct RunTarget {
@@ -100,6 +129,7 @@ struct sdr_plan {
   std::vector<sdr::Batch> batches;
   std::vector<sdr::FixedSeg> all;
   sdr::FixedSeg* d_segs = nullptr;
+  bool shared = false;  // outputs share bytes
   std::vector<sdr_column> masked;  // columns with a null mask, in column order
   std::vector<bool> col_masked;
   std::vector<uint32_t> mask_ends;  // per masked column: its pieces end here in the list of all
