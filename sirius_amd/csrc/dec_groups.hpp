@@ -244,6 +244,9 @@ struct Group {
   uint32_t per_seg;        // blocks of a segment
   uint32_t a, b;           // as the codec's own kernel takes them
 };
+// Workgroups along a dimension of a grid: a launch of 2^32 threads or more along one
+// reports no error and starts what is left of that modulo 2^32.
+constexpr uint32_t MAX_BLOCKS = 0xFFFFFFFFu / BLOCK_THREADS;
 constexpr uint32_t GROUPS_MAX = 24;  // 22 pairs of codec and width, and the masks
 struct GroupTable {
   uint32_t n;

@@ -262,9 +262,10 @@ hipError_t launch_batch_front(BatchQueue* q, uint32_t n_fsst_segs, const FixedGr
   GroupTable t{};
   uint32_t blocks = 0;
   *done           = n_groups == 0 || device_groups(groups, n_groups, units, counts, &t, &blocks);
-  if (!*done) return hipSuccess;
   // a multiple of 8 blocks ahead of the groups': a block's XCD stays its own
   const uint32_t prep = (std::min(n_fsst_segs, BATCH_PREP_GRID) + BATCH_XCDS - 1u) / BATCH_XCDS * BATCH_XCDS;
+  *done               = *done && blocks <= MAX_BLOCKS - prep;
+  if (!*done) return hipSuccess;
   if (prep + blocks == 0) return hipSuccess;
   hipLaunchKernelGGL(k_batch_front, dim3(prep + blocks), dim3(BLOCK_THREADS), 0, s, q, prep, DevSegs{segs, 0}, t);
   return hipGetLastError();

@@ -160,8 +160,8 @@ hipError_t launch_rle(const FixedSeg* segs, uint32_t seg_base, uint32_t n, uint3
   if (n == 0 || max_rows == 0) return hipSuccess;
   const uint32_t sr     = rle_slice_rows(n, max_rows, ts);
   const uint32_t slices = (max_rows + sr - 1) / sr;
-  // segments per launch so that the 1-D grid stays below 2^31 blocks
-  const uint32_t per = static_cast<uint32_t>(std::min<uint64_t>(MAX_GRID_Y, (0x7FFFFFF0ull / slices)));
+  // segments per launch so that the 1-D grid is one
+  const uint32_t per = std::min(MAX_GRID_Y, MAX_BLOCKS / slices);
   return for_segs(segs, seg_base, n, host, per, [&](auto src, uint32_t m) {
     using S = decltype(src);
     const dim3 grid(m * slices), block(RLE_THREADS);
@@ -305,7 +305,7 @@ static Group group_of(const FixedGroup& f, uint32_t n)
       g.per_seg = static_cast<uint32_t>((uint64_t{f.max_rows} * f.ts + COPY_UNIT - 1) / COPY_UNIT);
   }
   blocks = uint64_t{n} * g.per_seg;
-  g.blocks = blocks < 0x7FFFFFF0u ? static_cast<uint32_t>(blocks) : 0u;  // 0: too many for a launch
+  g.blocks = blocks <= MAX_BLOCKS ? static_cast<uint32_t>(blocks) : 0u;  // 0: too many for a launch
   return g;
 }
 
@@ -344,7 +344,7 @@ bool device_groups(const FixedGroup* in_groups, uint32_t n_groups, const MaskUni
     if (!groups[i].count) continue;
     if (t->n == GROUPS_MAX) return false;
     Group g = group_of(groups[i], groups[i].count);
-    if (g.blocks == 0 || first + g.blocks > 0x7FFFFFF0u) return false;
+    if (g.blocks == 0 || first + g.blocks > MAX_BLOCKS) return false;
     g.first = static_cast<uint32_t>(first);
     g.seg   = groups[i].codec == MASK_GROUP ? 0u : groups[i].first;
     if (groups[i].codec == MASK_GROUP) g.a = 0;
@@ -397,7 +397,7 @@ hipError_t launch_groups(const FixedGroup* in_groups, uint32_t n_groups, const F
       if (here && held == SEGS_INLINE) flush();
       const uint32_t n = here ? std::min(f.count - b, SEGS_INLINE - held) : f.count;
       Group g          = group_of(f, n);
-      if (g.blocks == 0 || (t.n && blocks + g.blocks + N_XCD > 0x7FFFFFF0ull)) return hipSuccess;
+      if (g.blocks == 0 || blocks + g.blocks > MAX_BLOCKS) return hipSuccess;
       g.first = static_cast<uint32_t>(blocks);
       if (f.codec == MASK_GROUP) g.a = b;
       if (here) {
