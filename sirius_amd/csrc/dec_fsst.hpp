@@ -658,12 +658,16 @@ __device__ __forceinline__ void fsst_group_emit(const FsstGroup& gr, FsstSmem& s
   }
 }
 
-// Clear the window's bytes [0, n) and the words a last symbol may reach.
+// Clear the window's bytes [0, n) and the words a last symbol may reach, with
+// 4-byte stores: in an earlier form of this kernel, clearing with 16-byte stores
+// (ds_write_b128) and then ORing from other waves after a barrier lost about 0.2% of
+// the ORed bytes once five or more workgroups shared a CU, and 4-byte stores never
+// did.  No cause was found in the code or its assembly.
 template <class SM>
 __device__ __forceinline__ void window_clear(SM& sm, uint32_t n)
 {
-  for (uint32_t i = threadIdx.x * 8u; i < n + 12u; i += FSST_THREADS * 8u)
-    *reinterpret_cast<uint64_t*>(&sm.out[i]) = 0u;
+  for (uint32_t i = threadIdx.x * 4u; i < n + 12u; i += FSST_THREADS * 4u)
+    *reinterpret_cast<uint32_t*>(&sm.out[i]) = 0u;
 }
 
 // 16 bytes at byte 16 - D (D = 1..16) of the pair of blocks a, b.
