@@ -412,8 +412,9 @@ typedef enum sdr_tune_key {
                                        predecessors' chars offsets before its
                                        decode reports SDR_E_HIP, 0..2^31
                                        (2^24, never reached); a first attempt
-                                       waits a 1024th of it.  0 reports at
-                                       once without waiting (for tests)      */
+                                       waits a 1024th of it, 1024 sleeps at
+                                       most.  0 reports at once without
+                                       waiting (for tests)                   */
   /* work units per queue entry of a persistent batch, for every batch that
    * does not set SDR_BATCH_UNITS_* itself: 1..2^20 */
   SDR_TUNE_BATCH_UNITS_BITPACKING = 6, /* 2048-row groups (16)               */

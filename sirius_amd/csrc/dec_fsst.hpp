@@ -47,6 +47,7 @@ constexpr uint64_t FSST_CORRUPT   = 32774747032022883ull;  // "corrupt\0"
 constexpr uint32_t SYMTAB_MAX     = 8192;
 constexpr uint64_t ST_AGG         = 1ull << 62;  // aggregate published
 constexpr uint64_t ST_INC         = 2ull << 62;  // inclusive prefix published
+constexpr uint64_t ST_RUN         = 3ull << 62;  // a long chunk, begun: nothing published yet
 constexpr uint64_t ST_VAL         = (1ull << 62) - 1;
 
 // Bytes of a segment read in order through aligned words; bytes at or past
@@ -732,10 +733,12 @@ __device__ __forceinline__ void window_store(const SM& sm, uintptr_t g, uint32_t
 // 0: publish this chunk's aggregate T (fsst_lookback_publish), then sum
 // predecessors 64 at a time back to the nearest published inclusive prefix
 // (fsst_lookback_wait).  Between the two the workgroup may do other work.  A
-// chunk waits at most `spin_limit` sleeps for an unpublished predecessor;
+// chunk waits at most `spin_limit` sleeps for predecessors that show nothing;
 // past that (or at once when spin_limit is 0, which only tests set) it sets
-// the column's error flag and ends, so the host reports the failure and no
-// wave hangs.  A status word carries its flag and value together and is the
+// the column's error flag and ends, so that the decode is repeated or its failure
+// reported and no wave hangs.  Where the only ones missing have said that they
+// have begun (fsst_lookback_begin), which chunks do whose lengths take long, it
+// waits for them FSST_SPIN_LIMIT sleeps, whatever `spin_limit`.  A status word carries its flag and value together and is the
 // only datum exchanged between chunks, so device-scope relaxed atomics
 // (coherent across the XCDs' L2s) suffice; release/acquire orderings would
 // add an L2 write-back / invalidate per access.
@@ -746,6 +749,15 @@ __device__ __forceinline__ void fsst_lookback_publish(uint32_t c, uint64_t T, Fs
     if (c == 0) __hip_atomic_store(&status[0], ST_INC | T, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     else if (spin_limit != 0) __hip_atomic_store(&status[c], ST_AGG | T, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+}
+
+// Chunk c has begun and will publish: for chunks that take long to (the
+// compressed bytes of several runs, or of rows that no run holds, are walked
+// first: a row of 120 KB takes milliseconds).
+__device__ __forceinline__ void fsst_lookback_begin(uint32_t c, FsstState* st, uint32_t spin_limit)
+{
+  if (threadIdx.x == 0 && spin_limit != 0)
+    __hip_atomic_store(&gbl(st->status)[c], ST_RUN, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 __device__ __forceinline__ void fsst_lookback_failed(FsstState* st)
@@ -769,7 +781,7 @@ __device__ __forceinline__ uint64_t fsst_lookback_wait(uint32_t c, uint32_t n_ch
     } else if (spin_limit == 0) {  // no waiting allowed: report the look-back as failed
       if (lane == 0) fsst_lookback_failed(st);
     } else {
-      uint32_t p = c - 1, spins = 0;
+      uint32_t p = c - 1, spins = 0, begun = 0;
       for (;;) {
         const bool valid = lane <= p;
         const uint64_t s =
@@ -778,8 +790,9 @@ __device__ __forceinline__ uint64_t fsst_lookback_wait(uint32_t c, uint32_t n_ch
         const uint64_t incm = ballot(valid && flag == ST_INC);
         const uint32_t stop = incm ? static_cast<uint32_t>(__builtin_ctzll(incm)) : (p < WAVE - 1 ? p : WAVE - 1);
         const uint64_t need = stop == WAVE - 1 ? ~0ull : ((2ull << stop) - 1ull);
-        if (ballot(valid && flag == 0) & need) {  // a predecessor has not published yet
-          if (++spins > spin_limit) {              // never expected: give up rather than hang
+        const uint64_t none = ballot(valid && flag == 0) & need;
+        if (none | (ballot(valid && flag == ST_RUN) & need)) {  // a predecessor has not published yet
+          if (none ? ++spins > spin_limit : ++begun > FSST_SPIN_LIMIT) {  // give up rather than hang
             if (lane == 0) fsst_lookback_failed(st);
             break;
           }
@@ -2082,6 +2095,7 @@ __device__ __attribute__((noinline)) void fsst_chunk_runs(const uint8_t* seg, ui
 {
   FsstSmem& sm         = *(FsstSmem*)smp;
   const uint32_t tid   = threadIdx.x;
+  fsst_lookback_begin(c, st, spin_limit);
   const bool ok        = flags & FI_OK;
   const uint8_t* end   = seg + bytes_size;
   const uint32_t width = flags & FI_WIDTH;

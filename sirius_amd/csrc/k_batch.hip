@@ -118,7 +118,7 @@ __device__ __forceinline__ void fsst_entry(const BatchQueue* __restrict__ q, uin
   const FsstColumn col = sload(q->fsst_cols + e.col);
   fsst_chunk(ch, ci, q->fsst_tabs + (ch.seg == FSST_GAP ? 0u : ch.seg), e.chunk, col.n_chunks,
              again ? col.again : col.state, col.offsets, col.chars, col.chars_cap, col.total_rows,
-             again ? q->spin_limit : q->spin_limit / FSST_UNORDERED_SHARE, sm);
+             again ? q->spin_limit : fsst_unordered_spins(q->spin_limit), sm);
 }
 
 // One block per FSST entry (the grid is the group's entry count), that of its own

@@ -319,7 +319,7 @@ hipError_t launch_fsst(bool ordered, uint32_t chunk_rows, const FsstChunk* d_chu
   if (n == 0) return hipSuccess;
   // Tickets are global chunk numbers: a launch covering [first, first + n)
   // runs after every launch of lower chunks on the same stream.
-  const uint32_t bound = tune(SDR_TUNE_FSST_SPIN_LIMIT), spin = ordered ? bound : bound / FSST_UNORDERED_SHARE;
+  const uint32_t bound = tune(SDR_TUNE_FSST_SPIN_LIMIT), spin = ordered ? bound : fsst_unordered_spins(bound);
   if (chunk_rows) {
     static_assert(FSST_CHUNK_ROWS == 2u * FSST_THREADS && WIDE_CHUNK_ROWS == 8u * FSST_THREADS, "one kernel a size");
     auto* const k = chunk_rows <= FSST_CHUNK_ROWS ? k_plain<2> : chunk_rows < WIDE_CHUNK_ROWS ? k_plain<4> : k_plain<8>;

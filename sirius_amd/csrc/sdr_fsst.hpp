@@ -16,15 +16,25 @@ constexpr uint32_t FSST_GAP        = 0xFFFFFFFFu;  // chunk of rows no segment c
 constexpr uint32_t FSST_SPIN_LIMIT = 1u << 24;     // look-back wait bound (never reached)
 // A chunk waits on the chunks before it, so these must be running or done.  A
 // decode first takes each workgroup's number for its chunk's, the order in which
-// workgroups are in fact started, and waits a 1024th of the bound; if that was not
-// enough the decode is done again with chunks in the order of a ticket that
+// workgroups are in fact started, and waits a 1024th of the bound, 1024 sleeps or
+// about a millisecond at most; if that was not enough the decode is done again with chunks in the order of a ticket that
 // workgroups draw as they start, which needs no assumption but costs each of
 // them one of a queue of atomics on one word, 13 ns apart (16 Mi rows 293 us,
 // without 274; 2 M rows of 27 chars 44 us, 35 us; a batch's strings 182 us, 168 us).
 // A call that waits for its result before it returns looks at it and decodes again
 // (with a bound below 1024, for tests, by ticket at once); behind a batch's chunks, whose
 // outputs are to be complete in stream order, a kernel does (k_batch_again).
+//
+// It is not enough where the XCDs, each of which starts its share of a launch by
+// itself, are full of workgroups that wait: of two string launches on two streams,
+// one that came first on some XCDs and the other on the others, or beside a long
+// kernel that holds some of them.  That costs the wait, and the decode twice.
 constexpr uint32_t FSST_UNORDERED_SHARE = 1024;
+constexpr uint32_t FSST_UNORDERED_MOST  = 1024;
+__host__ __device__ inline uint32_t fsst_unordered_spins(uint32_t bound)
+{
+  return bound / FSST_UNORDERED_SHARE < FSST_UNORDERED_MOST ? bound / FSST_UNORDERED_SHARE : FSST_UNORDERED_MOST;
+}
 inline bool fsst_unordered(uint32_t spin_limit) { return spin_limit >= FSST_UNORDERED_SHARE; }
 
 // A row range of a column: a segment, or (bytes == nullptr) rows no
