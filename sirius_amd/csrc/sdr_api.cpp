@@ -73,7 +73,12 @@ namespace {
 // read them has completed.  At most DESC_SLOTS_PER_DEV are in flight per
 // device; a call beyond that waits for the oldest one (the GPU still has
 // the others queued), so once the slots exist a decode allocates nothing.
-// The depth lets the GPU ride out host stalls of a few milliseconds.
+// The depth lets the GPU ride out host stalls of a few milliseconds.  A call
+// that waits for its own result waits for no other stream's: it takes a slot
+// beyond those, of which there are no more than such calls at once.
+//
+// The device buffers of such calls come from the stream-ordered pool, the larger
+// ones go back to it but for BIG_SLOTS_PER_DEV of them.
 struct DescSlot {
   void* h         = nullptr;
   void* d         = nullptr;
@@ -83,6 +88,7 @@ struct DescSlot {
   hipEvent_t up   = nullptr;  // recorded after the slot's upload on the copy stream
   int dev         = -1;
   bool held       = false;  // acquired and not yet released
+  bool pooled     = false;  // d is the stream-ordered pool's
   uint64_t seq    = 0;      // release order
 };
 std::mutex g_desc_mu;
@@ -90,6 +96,7 @@ std::vector<DescSlot*> g_desc;
 uint64_t g_desc_seq = 0;
 constexpr size_t DESC_SLOTS_PER_DEV = 32;  // about 8 ms of headline steps queued ahead of the host
 constexpr size_t DESC_MIN_BYTES     = 64u << 10;
+constexpr size_t BIG_SLOTS_PER_DEV  = 8;   // with device buffers of more than DESC_MIN_BYTES, of the pool's
 
 // One copy stream per device (default priority, not synchronising with the
 // null stream) carries descriptor uploads while the caller's stream is busy,
@@ -112,8 +119,9 @@ int copy_stream(int dev, hipStream_t* out)
 
 namespace {
 // A held slot of device `dev` with at least `h_bytes` of pinned and `d_bytes`
-// of device memory.
-int slot_hold(int dev, size_t h_bytes, size_t d_bytes, DescSlot** out)
+// of device memory.  `own`: the stream of a call that waits for its result, which
+// alone uses the device memory; null (or no `own`) elsewhere.
+int slot_hold(int dev, size_t h_bytes, size_t d_bytes, const hipStream_t* own, DescSlot** out)
 {
   *out = nullptr;
   DescSlot* pick = nullptr;
@@ -137,7 +145,7 @@ int slot_hold(int dev, size_t h_bytes, size_t d_bytes, DescSlot** out)
         oldest = sl;
       }
     }
-    if (!pick && (n_dev < DESC_SLOTS_PER_DEV || !oldest)) {
+    if (!pick && (n_dev < DESC_SLOTS_PER_DEV || !oldest || own)) {
       pick      = new DescSlot;
       pick->dev = dev;
       g_desc.push_back(pick);
@@ -180,10 +188,13 @@ int slot_hold(int dev, size_t h_bytes, size_t d_bytes, DescSlot** out)
     if (e == hipSuccess) pick->cap_h = grown(h_bytes);
   }
   if (e == hipSuccess && pick->cap_d < d_bytes) {
-    if (pick->d) e = hipFree(pick->d);
-    pick->d     = nullptr;
-    pick->cap_d = 0;
-    if (e == hipSuccess) e = hipMalloc(&pick->d, grown(d_bytes));
+    // (hipFree waits for the whole device)
+    if (pick->d) e = pick->pooled && own ? hipFreeAsync(pick->d, *own) : hipFree(pick->d);
+    pick->d      = nullptr;
+    pick->cap_d  = 0;
+    pick->pooled = own != nullptr;
+    if (own) ensure_pool(dev);
+    if (e == hipSuccess) e = own ? hipMallocAsync(&pick->d, grown(d_bytes), *own) : hipMalloc(&pick->d, grown(d_bytes));
     if (e == hipSuccess) pick->cap_d = grown(d_bytes);
   }
   if (e != hipSuccess) return unhold(fail(SDR_E_HIP, "descriptor slot: %s", hipGetErrorString(e)));
@@ -200,13 +211,13 @@ int slot_unhold(DescSlot* sl, int rc)
 }
 }  // namespace
 
-int slot_acquire(size_t h_bytes, size_t d_bytes, void** h_out, void** d_out, void** token)
+int slot_acquire(size_t h_bytes, size_t d_bytes, hipStream_t s, void** h_out, void** d_out, void** token)
 {
   *h_out = *d_out = *token = nullptr;
   int dev = 0;
   HIP_TRY(hipGetDevice(&dev));
   DescSlot* sl = nullptr;
-  const int rc = slot_hold(dev, h_bytes, d_bytes, &sl);
+  const int rc = slot_hold(dev, h_bytes, d_bytes, &s, &sl);
   if (rc) return rc;
   *h_out = sl->h;
   *d_out = sl->d;
@@ -214,17 +225,36 @@ int slot_acquire(size_t h_bytes, size_t d_bytes, void** h_out, void** d_out, voi
   return SDR_OK;
 }
 
-void slot_release_idle(void* token)
+void slot_release_idle(void* token, hipStream_t s)
 {
-  if (token) (void)slot_unhold(static_cast<DescSlot*>(token), SDR_OK);
+  if (!token) return;
+  auto* sl   = static_cast<DescSlot*>(token);
+  void* over = nullptr;  // given back to the pool
+  {
+    std::lock_guard<std::mutex> lk(g_desc_mu);
+    auto big = [&](const DescSlot* x) { return x->dev == sl->dev && x->pooled && x->cap_d > DESC_MIN_BYTES; };
+    if (big(sl) && static_cast<size_t>(std::count_if(g_desc.begin(), g_desc.end(), big)) > BIG_SLOTS_PER_DEV) {
+      over      = sl->d;
+      sl->d     = nullptr;
+      sl->cap_d = 0;
+    }
+    sl->held = false;
+  }
+  device_free(over, s);
 }
 
-int desc_pinned(const void* h_src, size_t bytes, void** p, void** token)
+int desc_pinned(const void* h_src, size_t bytes, hipStream_t s, bool waits, void** p, void** token)
 {
-  void* d      = nullptr;
-  const int rc = slot_acquire(bytes, 0, p, &d, token);
-  if (!rc) std::memcpy(*p, h_src, bytes);
-  return rc;
+  *p = *token = nullptr;
+  int dev     = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  DescSlot* sl = nullptr;
+  const int rc = slot_hold(dev, bytes, 0, waits ? &s : nullptr, &sl);
+  if (rc) return rc;
+  std::memcpy(sl->h, h_src, bytes);
+  *p     = sl->h;
+  *token = sl;
+  return SDR_OK;
 }
 
 int desc_acquire(const void* h_src, size_t bytes, hipStream_t s, void** d_out, void** token)
@@ -234,7 +264,7 @@ int desc_acquire(const void* h_src, size_t bytes, hipStream_t s, void** d_out, v
   int dev = 0;
   HIP_TRY(hipGetDevice(&dev));
   DescSlot* pick = nullptr;
-  const int hrc  = slot_hold(dev, bytes, bytes, &pick);
+  const int hrc  = slot_hold(dev, bytes, bytes, nullptr, &pick);
   if (hrc) return hrc;
   auto unhold  = [&](int rc) { return slot_unhold(pick, rc); };
   hipError_t e = hipSuccess;
@@ -391,11 +421,11 @@ void add_mask_units(const sdr_run* runs, uint32_t n, uint32_t total_rows, uint8_
 
 // Pieces and their counts in pinned memory: the kernel writes the counts and
 // reads a long list of pieces there, with no copy and no clear on the stream.
-int masks_prepare(const std::vector<MaskUnit>& units, MaskLaunch* m, void** token)
+int masks_prepare(const std::vector<MaskUnit>& units, hipStream_t s, MaskLaunch* m, void** token)
 {
   const size_t n = units.size(), b_counts = (n * sizeof(uint32_t) + 15u) & ~size_t{15};
   void *h = nullptr, *d = nullptr;
-  const int rc = slot_acquire(b_counts + n * sizeof(MaskUnit), 0, &h, &d, token);
+  const int rc = slot_acquire(b_counts + n * sizeof(MaskUnit), 0, s, &h, &d, token);
   if (rc) return rc;
   auto* hu = reinterpret_cast<MaskUnit*>(static_cast<uint8_t*>(h) + b_counts);
   std::memcpy(hu, units.data(), n * sizeof(MaskUnit));
@@ -422,7 +452,7 @@ hipError_t launch_masks(const MaskLaunch& m, hipStream_t s, bool shared = false)
 int masks_launch(const std::vector<MaskUnit>& units, hipStream_t s, const uint32_t** counts, void** token)
 {
   MaskLaunch m;
-  const int rc = masks_prepare(units, &m, token);
+  const int rc = masks_prepare(units, s, &m, token);
   if (rc) return rc;
   const hipError_t e = launch_masks(m, s);
   if (e != hipSuccess) {
@@ -597,7 +627,7 @@ int decode_runs(const std::vector<RunTarget>& targets, hipStream_t s, uint32_t m
   }
   void* d     = nullptr;
   void* token = nullptr;
-  int rc = desc_pinned(all.data(), all.size() * sizeof(FixedSeg), &d, &token);
+  int rc = desc_pinned(all.data(), all.size() * sizeof(FixedSeg), s, masks.n != 0, &d, &token);
   if (rc) return rc;
   const hipError_t e = launch_batches(batches, all, static_cast<FixedSeg*>(d), mode, 0, s, masks, shared);
   rc                 = desc_release(token, s);
@@ -631,7 +661,7 @@ int decode_table(sdr_column* cols, uint32_t n_cols, hipStream_t s, uint32_t mode
   }
   MaskLaunch masks;
   void* token = nullptr;
-  if (!masked.empty()) rc = masks_prepare(units, &masks, &token);
+  if (!masked.empty()) rc = masks_prepare(units, s, &masks, &token);
   masks.ends   = ends.data();
   masks.n_cols = static_cast<uint32_t>(ends.size());
   if (!rc) rc = decode_runs(targets, s, mode, masks);
@@ -643,7 +673,7 @@ int decode_table(sdr_column* cols, uint32_t n_cols, hipStream_t s, uint32_t mode
       (void)desc_release(token, s);
       return rc ? rc : fail(SDR_E_HIP, "null count: %s", hipGetErrorString(e));
     }
-    slot_release_idle(token);
+    slot_release_idle(token, s);
   }
   if (rc) return rc;
   hipError_t e = hipPeekAtLastError();

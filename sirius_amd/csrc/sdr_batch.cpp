@@ -627,7 +627,7 @@ int batch_launch(sdr_batch* b, hipStream_t s)
     void* d     = nullptr;
     void* token = nullptr;
     if (b->fixed_src == sdr_batch::FS_SLOT) {
-      rc = desc_pinned(b->h_fsegs.data(), b->h_fsegs.size() * sizeof(FixedSeg), &d, &token);
+      rc = desc_pinned(b->h_fsegs.data(), b->h_fsegs.size() * sizeof(FixedSeg), s, false, &d, &token);
       if (rc) return rc;
     }
     const hipError_t e = launch_fixed_grids(b, s, static_cast<const FixedSeg*>(d));

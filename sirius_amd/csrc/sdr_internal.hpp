@@ -35,12 +35,14 @@ int desc_release(void* token, hipStream_t s);
 // place.  For descriptors of which a workgroup reads one: its 24 bytes over the
 // bus cost a launch less than the copy before it and the event between them (64
 // Mi rows in 1641 segments 238 -> 234 us, 32 Mi nullable rows in 547 97 -> 93 us).
-int desc_pinned(const void* h_src, size_t bytes, void** p, void** token);
+// `waits`: the call waits for its result.
+int desc_pinned(const void* h_src, size_t bytes, hipStream_t s, bool waits, void** p, void** token);
 // A slot's pinned (device-accessible) and device buffers of at least these
-// sizes, nothing copied; given back with desc_release, or, when no work on
-// them can be pending (the stream was synchronised), slot_release_idle.
-int slot_acquire(size_t h_bytes, size_t d_bytes, void** h_out, void** d_out, void** token);
-void slot_release_idle(void* token);
+// sizes, nothing copied, for a call that waits for its result on `s`; given back
+// with desc_release, or, when no work on them can be pending (the stream was
+// synchronised), slot_release_idle.
+int slot_acquire(size_t h_bytes, size_t d_bytes, hipStream_t s, void** h_out, void** d_out, void** token);
+void slot_release_idle(void* token, hipStream_t s);
 
 bool type_ok_for(uint32_t codec, uint32_t ts);
 bool codec_fixed(uint32_t codec);
@@ -65,7 +67,7 @@ struct MaskLaunch {
   uint32_t n_cols       = 0;
 };
 // Pieces and counts in pinned memory, to be launched; `token` as for masks_launch.
-int masks_prepare(const std::vector<MaskUnit>& units, MaskLaunch* m, void** token);
+int masks_prepare(const std::vector<MaskUnit>& units, hipStream_t s, MaskLaunch* m, void** token);
 
 // Bytes that a call's launches write.  Segments may share rows, and columns outputs
 // and masks: the codec or the column that comes later wins, launch after launch.

@@ -98,7 +98,7 @@ struct CallMemory {
   {
     if (bytes > STRINGS_KEEP_BYTES) return device_alloc(reinterpret_cast<void**>(&p), bytes, s);
     void *h = nullptr, *d = nullptr;
-    const int rc = slot_acquire(0, bytes, &h, &d, &slot);
+    const int rc = slot_acquire(0, bytes, s, &h, &d, &slot);
     p            = static_cast<uint8_t*>(d);
     return rc;
   }
@@ -106,7 +106,7 @@ struct CallMemory {
   void release(hipStream_t s, bool synced)
   {
     if (!slot) device_free(p, s);
-    else if (synced) slot_release_idle(slot);
+    else if (synced) slot_release_idle(slot, s);
     else (void)desc_release(slot, s);
     p    = nullptr;
     slot = nullptr;
@@ -322,10 +322,10 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
   } else {
     const size_t b_pinned =
       sizeof(FsstResult) + hsegs.size() * sizeof(FsstSeg) + (dfsst ? DictFsstCall::pinned_bytes(n_ranges) : 0u);
-    rc = slot_acquire(b_pinned, own ? 0 : total_bytes, &h_slot, &d_slot, &slot);
+    rc = slot_acquire(b_pinned, own ? 0 : total_bytes, s, &h_slot, &d_slot, &slot);
     if (!rc && own) rc = device_alloc(reinterpret_cast<void**>(&d), total_bytes, s);
     if (rc) {
-      slot_release_idle(slot);
+      slot_release_idle(slot, s);
       return rc;
     }
     if (!own) d = static_cast<uint8_t*>(d_slot);
@@ -334,7 +334,7 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
   bool synced  = false;  // nothing enqueued on the slot's memory is pending
   auto release = [&]() {
     if (own) device_free(d, s);
-    if (synced) slot_release_idle(slot);
+    if (synced) slot_release_idle(slot, s);
     else (void)desc_release(slot, s);
   };
   auto* d_segs   = reinterpret_cast<FsstSeg*>(d);
@@ -380,7 +380,7 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
     add_mask_units(col->validity, col->has_nulls ? col->n_validity : 0u, n, col->d_null_mask, units);
   MaskLaunch beside;  // the pieces built beside the pre-pass
   if (!units.empty() && !scratch_mem && !dc.n_d) {
-    rc     = masks_prepare(units, &beside, &counts_token);
+    rc     = masks_prepare(units, s, &beside, &counts_token);
     counts = beside.counts;
     if (rc) {
       release_all();
@@ -444,7 +444,7 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
   }
   for (size_t u = 0; synced && counts && u < units.size(); ++u) h_nulls += counts[u];
   for (uint32_t u = 0; synced && dc.any_inline && u < dfsst_null_counts(n); ++u) h_nulls += dc.counts[u];
-  if (synced) slot_release_idle(counts_token);
+  if (synced) slot_release_idle(counts_token, s);
   else (void)desc_release(counts_token, s);
   release_all();
   if (e != hipSuccess) return fail(SDR_E_HIP, "string decode: %s", hipGetErrorString(e));
