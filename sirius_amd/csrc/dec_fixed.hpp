@@ -157,20 +157,21 @@ __device__ __forceinline__ void bp_group(const uint8_t* seg, uint32_t bytes, uin
     // A lane's VPL rows of the step at s0: read without a branch, which would
     // hold each LDS read back until the one before it is done (a row group of
     // dates, where latency is all: 5.8 -> 5.0 us); rows past the chunk read its
-    // last row again.
+    // last row again and count as zero, so that a next chunk's carry is right.
     auto step = [&](uint32_t s0, auto full) {
       const uint32_t r = s0 + lane_id() * VPL;
       T v[VPL];
 #pragma unroll
       for (uint32_t i = 0; i < VPL; ++i) {
-        const uint32_t row = decltype(full)::value || r + i < rows ? r + i : rows - 1u;
+        const bool in      = decltype(full)::value || r + i < rows;
+        const uint32_t row = in ? r + i : rows - 1u;
         const uint32_t bp  = head + row * width;
         T u;
         if constexpr (TS == 8) u = static_cast<T>(lds_bits64(lds, bp, width));
         else u = static_cast<T>(lds_bits32(lds, bp, width));
-        v[i] = static_cast<T>(static_cast<A>(tframe) + static_cast<A>(u));
+        v[i] = in ? static_cast<T>(static_cast<A>(tframe) + static_cast<A>(u)) : T(0);
       }
-      if (mode == BP_DELTA_FOR) {  // rows past the chunk come last: nothing that is stored adds them
+      if (mode == BP_DELTA_FOR) {
         A loc[VPL];
         loc[0] = v[0];
 #pragma unroll
