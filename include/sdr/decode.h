@@ -400,8 +400,10 @@ int sdr_server_destroy(sdr_server* server);
  * table that sdr_tune_load applies. */
 typedef enum sdr_tune_key {
   SDR_TUNE_RLE_SLICE_ROWS      = 1, /* rows one 256-thread block expands:
-                                       1024..1048576, multiple of 64 (16384:
-                                       each launch chooses by its size)      */
+                                       1024..1048576, multiple of 64; 0, or
+                                       until it is set: by each launch's size
+                                       (reads as 16384, the value that queue
+                                       entries of a batch then take)         */
   SDR_TUNE_BP_GROUPS_PER_WAVE  = 2, /* 2048-row groups one wavefront decodes
                                        in turn, 1..16 (1)                    */
   SDR_TUNE_BP_CHUNK_ROWS       = 3, /* most rows a wavefront stages per LDS

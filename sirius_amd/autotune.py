@@ -7,10 +7,11 @@ under each candidate value: the per-codec kernels (HIP events around
 repeated launches of a prepared plan) for the launch-shape knobs, and the
 persistent batch with its fixed-width segments in the group kernels
 (replayed launches of one batch, SDR_BATCH_FIXED_KERNELS = 1) for the
-units-per-entry knobs, which shape only those kernels.  The fastest value of each (knob, width) is kept before the next one
-is tried, and the result is written as a table that ``sdr_tune_load``
-applies: ``name@width value`` lines, timings as comments.  Knobs change
-launch shapes only, never results.
+units-per-entry knobs, which shape only those kernels.  The fastest value of each
+(knob, width) is kept before the next one is tried (the RLE slices stay chosen by
+each launch's size unless a value is much faster), and the result is written as a
+table that ``sdr_tune_load`` applies: ``name@width value`` lines, timings as
+comments.  Knobs change launch shapes only, never results.
 
     python -m sirius_amd.autotune [--out PATH] [--rows N] [--reps R]
 """
@@ -32,7 +33,7 @@ DEFAULT_TABLE = Path(__file__).resolve().parent / "tuning" / "gfx950.txt"
 
 # knob -> (candidate values, the codecs whose kernels it shapes, timed path)
 CANDIDATES = {
-    A.TUNE_RLE_SLICE_ROWS: ([4096, 8192, 12288, 16384, 24576, 32768, 61440], [A.RLE], "plan"),
+    A.TUNE_RLE_SLICE_ROWS: ([0, 4096, 8192, 12288, 16384, 24576, 32768, 61440], [A.RLE], "plan"),
     A.TUNE_BP_CHUNK_ROWS: ([1024, 2048], [A.BITPACKING], "plan"),
     A.TUNE_BP_GROUPS_PER_WAVE: ([1, 2, 4], [A.BITPACKING], "plan"),
     A.TUNE_ALP_VECTORS_PER_WAVE: ([1, 2, 4], [A.ALP, A.ALPRD], "plan"),
@@ -156,6 +157,11 @@ def main(argv=None) -> int:
                 results.append((ms, v))
                 log(f"[autotune] {name}@{w}={v}: {ms * 1e3:.1f} us")
             best_ms, best = min(results)
+            # 0 chooses by the launch's size, which is timed at one large size here: a value that is
+            # a little better there loses more in small launches (ten row groups of int32 in runs of
+            # 200: 6.5 us by size, 8.4 us in slices of 8192 rows)
+            if values[0] == 0 and results[0][0] < 1.25 * best_ms:
+                best = 0
             L.check(lib.sdr_tune_set_width(knob, w, best))
             lines.append(f"# {name}@{w} ({path}): " + ", ".join(f"{v}={ms * 1e3:.1f}us" for ms, v in results))
             lines.append(f"{name}@{w} {best}")

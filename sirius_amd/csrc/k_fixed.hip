@@ -147,8 +147,7 @@ hipError_t launch_bitpacking(const FixedSeg* segs, uint32_t seg_base, uint32_t n
 // ten segments in slices of 8192 or 2048 rows are 150 or 600 blocks: 8.4 us, 6.5 us.
 static uint32_t rle_slice_rows(uint32_t n_segs, uint32_t max_rows, uint32_t ts)
 {
-  const uint32_t set = tune(SDR_TUNE_RLE_SLICE_ROWS, ts);
-  if (set != RLE_SLICE_ROWS) return set;
+  if (!tune_rle_by_size(ts)) return tune(SDR_TUNE_RLE_SLICE_ROWS, ts);
   uint32_t sr = 8192;
   while (sr > 2048u && uint64_t{n_segs} * ((max_rows + sr - 1u) / sr) < 512u) sr /= 2u;
   return sr;

@@ -16,8 +16,8 @@ struct FixedSeg {
 };
 static_assert(sizeof(FixedSeg) == 24, "FixedSeg layout");
 
-// Rows of one RLE slice (one 256-thread block decodes a slice): the knob's
-// default, at which a launch chooses by its size.
+// Rows of one RLE slice (one 256-thread block decodes a slice) where nothing else
+// is said: in a batch's queue entries.  Launches of their own choose by size.
 constexpr uint32_t RLE_SLICE_ROWS = 16384;
 
 // Descriptors a launch can carry in its kernel arguments.

@@ -17,6 +17,12 @@ struct Knob {
   const char* name;
   uint64_t lo, hi, def;
   std::atomic<uint64_t> value[4];
+  std::atomic<bool> set[4] = {};
+  void put(int w, uint64_t v)
+  {
+    value[w].store(v, std::memory_order_relaxed);
+    set[w].store(true, std::memory_order_relaxed);
+  }
 };
 
 #define SDR_KNOB(name, lo, hi, def) {name, lo, hi, def, {{def}, {def}, {def}, {def}}}
@@ -38,6 +44,7 @@ constexpr uint32_t N_KNOBS = sizeof(g_knobs) / sizeof(g_knobs[0]);
 bool valid(uint32_t key, uint64_t v)
 {
   const Knob& k = g_knobs[key - 1];
+  if (key == SDR_TUNE_RLE_SLICE_ROWS && v == 0) return true;  // by the launch's size
   if (v < k.lo || v > k.hi) return false;
   if (key == SDR_TUNE_RLE_SLICE_ROWS && v % 64u) return false;
   if (key == SDR_TUNE_BP_CHUNK_ROWS && v != 512 && v != 1024 && v != 2048) return false;
@@ -60,8 +67,16 @@ int width_index(uint32_t ts)
 
 uint32_t tune(uint32_t key, uint32_t ts)
 {
-  const int w = width_index(ts);
-  return static_cast<uint32_t>(g_knobs[key - 1].value[w < 0 ? 2 : w].load(std::memory_order_relaxed));
+  const int w      = width_index(ts);
+  const uint64_t v = g_knobs[key - 1].value[w < 0 ? 2 : w].load(std::memory_order_relaxed);
+  return key == SDR_TUNE_RLE_SLICE_ROWS && v == 0 ? RLE_SLICE_ROWS : static_cast<uint32_t>(v);
+}
+
+bool tune_rle_by_size(uint32_t ts)
+{
+  const Knob& k = g_knobs[SDR_TUNE_RLE_SLICE_ROWS - 1];
+  const int w   = width_index(ts);
+  return !k.set[w].load(std::memory_order_relaxed) || k.value[w].load(std::memory_order_relaxed) == 0;
 }
 
 }  // namespace sdr
@@ -77,7 +92,7 @@ int sdr_tune_set(uint32_t key, uint64_t value)
   if (!valid(key, value))
     return fail(SDR_E_INVALID_ARG, "%s = %llu out of range", g_knobs[key - 1].name,
                 static_cast<unsigned long long>(value));
-  for (auto& v : g_knobs[key - 1].value) v.store(value, std::memory_order_relaxed);
+  for (int w = 0; w < 4; ++w) g_knobs[key - 1].put(w, value);
   return SDR_OK;
 }
 
@@ -90,7 +105,7 @@ int sdr_tune_set_width(uint32_t key, uint32_t type_size, uint64_t value)
   if (!valid(key, value))
     return fail(SDR_E_INVALID_ARG, "%s = %llu out of range", g_knobs[key - 1].name,
                 static_cast<unsigned long long>(value));
-  g_knobs[key - 1].value[w].store(value, std::memory_order_relaxed);
+  g_knobs[key - 1].put(w, value);
   return SDR_OK;
 }
 
