@@ -305,7 +305,7 @@ __device__ __forceinline__ uint32_t fsst_row_len(const uint8_t* p, uint32_t n, c
 // reading the compressed bytes from global memory.  Rows whose compressed
 // range leaves [0, dict_end) decode to nothing.
 template <class SM>
-__device__ __attribute__((noinline)) uint32_t fsst_lengths_rows(SM& sm, bool ok, const uint8_t* seg,
+__device__ __attribute__((noinline)) uint32_t fsst_lengths_rows(SM& sm, const uint8_t* seg,
                                                                 uint32_t dict_end, uint32_t rows)
 {
   uint32_t T = 0;
@@ -313,7 +313,7 @@ __device__ __attribute__((noinline)) uint32_t fsst_lengths_rows(SM& sm, bool ok,
   for (uint32_t k = 0; k < ROWS_PER_THR; ++k) {
     const uint32_t r = k * FSST_THREADS + threadIdx.x;
     uint32_t d       = 0;
-    if (ok && r < rows) {
+    if (r < rows) {
       const uint32_t cum = sm.comp[r + 1], prev = sm.comp[r];
       if (cum <= dict_end && prev <= cum && cum != prev) d = fsst_row_len(seg + dict_end - cum, cum - prev, sm);
     }
@@ -2012,12 +2012,12 @@ __device__ __forceinline__ void fsst_fields2(const uint32_t* lw, uint32_t bit0, 
 
 // The segment's symbol table and the chunk's length fields on their way to
 // LDS (LDS-direct loads); returns bit0 of fsst_fields2.
-__device__ __forceinline__ uint32_t fsst_issue_front(FsstSmem& sm, bool ok, const FsstSymTab* tab, bool lfast,
+__device__ __forceinline__ uint32_t fsst_issue_front(FsstSmem& sm, const FsstSymTab* tab, bool lfast,
                                                      const uint8_t* seg, uint32_t row_begin, uint32_t rows,
                                                      uint32_t width)
 {
-  if (ok) block_issue<FSST_THREADS>(reinterpret_cast<uint32_t*>(sm.sym), reinterpret_cast<const uint8_t*>(tab),
-                                    sizeof(FsstSymTab));
+  block_issue<FSST_THREADS>(reinterpret_cast<uint32_t*>(sm.sym), reinterpret_cast<const uint8_t*>(tab),
+                            sizeof(FsstSymTab));
   if (!lfast) return 0;
   const uint64_t b0 = (uint64_t{row_begin} * width) >> 3;
   const uint64_t b1 = (uint64_t{row_begin + rows} * width + 7u) >> 3;
@@ -2096,11 +2096,10 @@ __device__ __attribute__((noinline)) void fsst_chunk_runs(const uint8_t* seg, ui
   FsstSmem& sm         = *(FsstSmem*)smp;
   const uint32_t tid   = threadIdx.x;
   fsst_lookback_begin(c, st, spin_limit);
-  const bool ok        = flags & FI_OK;
   const uint8_t* end   = seg + bytes_size;
   const uint32_t width = flags & FI_WIDTH;
-  const bool lfast     = ok && width && (flags & FI_LFAST);
-  const uint32_t bit0  = fsst_issue_front(sm, ok, tab, lfast, seg, row_begin, rows, width);
+  const bool lfast     = width && (flags & FI_LFAST);
+  const uint32_t bit0  = fsst_issue_front(sm, tab, lfast, seg, row_begin, rows, width);
   __builtin_amdgcn_s_waitcnt(WAITCNT_VMEM_DONE);
   __syncthreads();
   const uint32_t* lw = reinterpret_cast<const uint32_t*>(sm.out);
@@ -2115,12 +2114,12 @@ __device__ __attribute__((noinline)) void fsst_chunk_runs(const uint8_t* seg, ui
   const uint32_t x1 = x0 + cl0, x2 = x1 + cl1;
   // Rows shorter than 1 MiB keep the prefix sums from wrapping, so they rise
   // from c_lo to c_hi.
-  if (!ok || (flags & FI_HUGE) || c_hi < c_lo || c_hi > dict_end || n_all >> 16) {
+  if ((flags & FI_HUGE) || c_hi < c_lo || c_hi > dict_end || n_all >> 16) {
     if (tid == 0) sm.comp[0] = c_lo;
     if (r0 < rows) sm.comp[r0 + 1u] = c_lo + x1;
     if (r1 < rows) sm.comp[r1 + 1u] = c_lo + x2;
     __syncthreads();
-    const uint32_t T    = fsst_lengths_rows(sm, ok, seg, dict_end, rows);
+    const uint32_t T    = fsst_lengths_rows(sm, seg, dict_end, rows);
     const uint64_t base = fsst_lookback(c, n_chunks, T, st, spin_limit, sm);
     fsst_offsets(FsstChunk{0u, row_begin, rows, col_row}, c, n_chunks, rows, T, base, offsets, total_rows, sm);
     if (T == 0 || base >= chars_cap) return;
@@ -2228,16 +2227,26 @@ __device__ __forceinline__ void fsst_chunk(const FsstChunk ch, const FsstChunkIn
     plain_chunk<ROWS_PER_THR>(args, sm);
     return;
   }
+  // No row has bytes: none of a segment's, or of one with a bad header, or none that
+  // is not empty or NULL.  (Rows shorter than 1 MiB do not wrap their sum.)  1 M such
+  // rows took 69 us, and 86 us in a batch, as a run of no bytes, which is called; so
+  // 29 us and 39 us.
+  if (!ok || (!(ci.flags & FI_HUGE) && ci.c_hi == ci.c_lo)) {
+    const uint64_t base = fsst_lookback(c, n_chunks, 0u, st, spin_limit, sm);
+    for (uint32_t r = tid; r < rows; r += FSST_THREADS)
+      gbl(offsets)[ch.col_row + r] = static_cast<int32_t>(static_cast<uint32_t>(base));
+    if (c == n_chunks - 1u && tid == 0) gbl(offsets)[total_rows] = static_cast<int32_t>(static_cast<uint32_t>(base));
+    return;
+  }
   // Rows are stored back to front ending at dict_end: the chunk's bytes are
   // [dict_end - c_hi, dict_end - c_lo).  One run holds them nearly always.
   const uint8_t* seg = ci.bytes;
   const uint32_t C   = ci.c_hi - ci.c_lo;
   const uintptr_t ca = reinterpret_cast<uintptr_t>(seg + ci.dict_end - ci.c_hi);
   const uint32_t c_h = static_cast<uint32_t>(ca & 15u);
-  if (!ok || !rows || (ci.flags & FI_HUGE) || ci.c_hi <= ci.c_lo || ci.c_hi > ci.dict_end || C > FSST_CSTAGE - c_h) {
-    fsst_chunk_runs(ok ? seg : nullptr, ok ? ci.bytes_size : 0u, ok ? ci.dict_end : 0u, ok ? ci.flags : 0u,
-                    ok ? ci.c_lo : 0u, ok ? ci.c_hi : 0u, ch.row_begin, rows, ch.col_row, tab, c, n_chunks, st,
-                    offsets, chars, chars_cap, total_rows, spin_limit, (LdsPtr<FsstSmem>)(&sm));
+  if ((ci.flags & FI_HUGE) || ci.c_hi < ci.c_lo || ci.c_hi > ci.dict_end || C > FSST_CSTAGE - c_h) {
+    fsst_chunk_runs(seg, ci.bytes_size, ci.dict_end, ci.flags, ci.c_lo, ci.c_hi, ch.row_begin, rows, ch.col_row, tab, c,
+                    n_chunks, st, offsets, chars, chars_cap, total_rows, spin_limit, (LdsPtr<FsstSmem>)(&sm));
     return;
   }
   const uint8_t* end   = seg + ci.bytes_size;
@@ -2245,7 +2254,7 @@ __device__ __forceinline__ void fsst_chunk(const FsstChunk ch, const FsstChunkIn
   const bool lfast     = width && (ci.flags & FI_LFAST);
   const uint32_t y_hi  = c_h + C;
   const uint8_t* stage = reinterpret_cast<const uint8_t*>(ca - c_h);
-  const uint32_t bit0  = fsst_issue_front(sm, true, tab, lfast, seg, ch.row_begin, rows, width);
+  const uint32_t bit0  = fsst_issue_front(sm, tab, lfast, seg, ch.row_begin, rows, width);
   // The groups' loads go out last and unconditionally, so the wait below
   // leaves exactly these 2 * GROUPS_PER_THR loads in flight: the compressed
   // prefix runs while they arrive.
