@@ -737,7 +737,9 @@ int batch_launch(sdr_batch* b, hipStream_t s)
   } else {
     HIP_TRY(enqueue_direct(b, q, items, mask, grid, cnt, b->n_fsst_segs, s));
   }
-  if (strings) HIP_TRY(launch_batch_again(q, cnt[BG_FSST], s));
+  // (a column of one chunk waits for none: nothing to try again)
+  if (std::any_of(b->cols.begin(), b->cols.end(), [](const sdr_batch::Col& c) { return c.n_chunks > 1u; }))
+    HIP_TRY(launch_batch_again(q, cnt[BG_FSST], s));
   if (b->use_graph && (mask || !b->fixed.empty())) HIP_TRY(launch_masks(b, s));
   // a column of no rows has no chunk to write its closing offset
   for (const auto& c : b->cols)
