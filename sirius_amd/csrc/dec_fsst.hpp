@@ -764,6 +764,7 @@ __device__ __forceinline__ void fsst_lookback_failed(FsstState* st)
 {
   __hip_atomic_fetch_or(gbl(&st->error), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (FsstResult* const r = *gbl(&st->result)) *gbl(&r->error) = 1u;
+  if (uint32_t* const f = *gbl(&st->failed)) *gbl(f) = 1u;
 }
 
 // The wait half: synchronises the workgroup and returns the exclusive prefix

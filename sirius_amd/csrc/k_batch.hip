@@ -144,10 +144,7 @@ __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6)
 {
   __shared__ FsstSmem sm;
   __shared__ uint32_t s_next;
-  bool failed = false;
-  for (uint32_t i = threadIdx.x; i < q->n_cols; i += FSST_THREADS)
-    failed = failed || *gbl(&gload(q->fsst_cols + i).state->error) != 0u;
-  if (!__syncthreads_or(failed)) return;
+  if (q->failed == 0u) return;
   for (;;) {
     if (threadIdx.x == 0) s_next = atomicAdd(&q->ticket, 1u);
     __syncthreads();
@@ -162,13 +159,14 @@ __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6)
 // The FSST segment pre-pass over the queue's segments with `blocks` workgroups, of
 // which this is the `block`-th; the first tells each column where its result goes.
 template <uint32_t NT>
-__device__ __forceinline__ void batch_prep(const BatchQueue* __restrict__ q, uint32_t block, uint32_t blocks,
+__device__ __forceinline__ void batch_prep(BatchQueue* __restrict__ q, uint32_t block, uint32_t blocks,
                                            FsstPrepSmem<NT>& sm)
 {
   if (block == 0)
     for (uint32_t i = threadIdx.x; i < q->n_cols; i += NT) {
       const FsstColumn col      = gload(q->fsst_cols + i);
       gbl(col.state)->result = q->results + i;
+      gbl(col.state)->failed = &q->failed;
       gbl(col.again)->result = q->results + q->n_cols + i;
     }
   const uint32_t n = q->n_fsst_segs;
@@ -176,7 +174,7 @@ __device__ __forceinline__ void batch_prep(const BatchQueue* __restrict__ q, uin
     fsst_prep_segment(gload(q->fsst_segs + i), i, q->fsst_chunks, q->fsst_info, q->fsst_tabs + i, sm);
 }
 
-__global__ __launch_bounds__(BATCH_PREP_THREADS) void k_batch_fsst_prep(const BatchQueue* __restrict__ q)
+__global__ __launch_bounds__(BATCH_PREP_THREADS) void k_batch_fsst_prep(BatchQueue* __restrict__ q)
 {
   __shared__ FsstPrepSmem<BATCH_PREP_THREADS> sm;
   batch_prep(q, blockIdx.x, gridDim.x, sm);
@@ -199,7 +197,7 @@ __global__ __launch_bounds__(256) void k_batch_setup(u32x4* __restrict__ dst, co
 // the null masks: the pre-pass waits on memory for most of its time and fills
 // half the chip, so the others run beside it.
 __global__ __launch_bounds__(BLOCK_THREADS) __attribute__((amdgpu_waves_per_eu(8))) void k_batch_front(
-  const BatchQueue* __restrict__ q, uint32_t prep, DevSegs src, GroupTable t)
+  BatchQueue* __restrict__ q, uint32_t prep, DevSegs src, GroupTable t)
 {
   __shared__ union Smem {
     FsstPrepSmem<BLOCK_THREADS> prep;

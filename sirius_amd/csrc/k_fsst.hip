@@ -100,6 +100,7 @@ __device__ __forceinline__ void fsst_prep_block(const Src& src, uint32_t n_segs,
     st->error  = 0;
     st->total  = 0;
     st->result = result;
+    st->failed = nullptr;
   }
   for (uint32_t i = block; i < n_segs; i += blocks) {
     const FsstSeg sg = src.at(i);

@@ -80,6 +80,7 @@ struct BatchQueue {
   uint32_t error;
   uint32_t n_fsst_status;  // words of `fsst_status`, cleared by a launch's first kernel
   uint32_t spin_limit;     // look-back wait bound of the FSST chunks
+  uint32_t failed;         // some column's first attempt was given up (uploaded as 0)
   uint32_t ticket;         // of the second attempt: its next entry (uploaded as 0)
   uint32_t n_fsst_segs;    // row ranges of all FSST columns, for the pre-pass
   uint32_t bp_chunk_rows[4];  // most rows a bitpacking wavefront stages at once, per width 1/2/4/8

@@ -179,9 +179,10 @@ struct FsstState {
   uint32_t error;
   uint64_t total;
   FsstResult* result;
+  uint32_t* failed;    // a batch's: where a failure is told as well (may be null)
   uint64_t status[1];  // n_chunks entries
 };
-constexpr uint32_t FSST_STATE_WORDS = 3;  // 8-byte words before status
+constexpr uint32_t FSST_STATE_WORDS = 4;  // 8-byte words before status
 
 // Segment pre-pass over n_segs ranges: writes the chunk list, the chunks'
 // FsstChunkInfo and the segments' symbol tables, and sets up the state (its

@@ -20,7 +20,7 @@
 // (sdr_decode_strings_column_noalloc): a fixed array in the code object, one
 // copy per GPU, held until the process ends.  Host code never uses its name
 // as an address: the per-device address comes from hipGetSymbolAddress.
-static __device__ __align__(256) uint8_t scratch[SDR_NOALLOC_SCRATCH_BYTES + 256];  // and FsstState::result
+static __device__ __align__(256) uint8_t scratch[SDR_NOALLOC_SCRATCH_BYTES + 256];  // and FsstState's pointers
 
 namespace sdr {
 
@@ -313,9 +313,9 @@ int decode_strings(sdr_string_column* col, hipStream_t s, uint32_t mode, uint8_t
   const bool own = !scratch_mem && total_bytes > STRINGS_KEEP_BYTES;
   if (scratch_mem) {
     // The limit is on columns, not on how they are cut: it counts chunks of
-    // FSST_CHUNK_ROWS rows, and not FsstState::result, unused here.
+    // FSST_CHUNK_ROWS rows, and not FsstState's pointers, unused here.
     const size_t counted = seg_bytes + al(n_narrow * sizeof(FsstChunk)) + al(n_narrow * sizeof(FsstChunkInfo)) + tab_bytes +
-                           al(sizeof(FsstState) - sizeof(FsstResult*) + sizeof(uint64_t) * n_narrow) + sizeof(unsigned long long);
+                           al(sizeof(FsstState) - 2u * sizeof(void*) + sizeof(uint64_t) * n_narrow) + sizeof(unsigned long long);
     if (counted > SDR_NOALLOC_SCRATCH_BYTES)
       return fail(SDR_E_CAPACITY, "string decode needs %llu bytes of descriptors; the no-allocation scratch holds %u",
                   static_cast<unsigned long long>(counted), SDR_NOALLOC_SCRATCH_BYTES);
