@@ -144,7 +144,8 @@ typedef struct sdr_string_column {
 
 /* Launch strategies for the fixed-width and string paths. */
 typedef enum sdr_launch_mode {
-  SDR_LAUNCH_BATCHED     = 0, /* one launch per codec and type size (default)  */
+  SDR_LAUNCH_BATCHED     = 0, /* one launch for all, or one per codec and type
+                                 size where that is not possible (default)     */
   SDR_LAUNCH_PER_SEGMENT = 1, /* one launch per segment (the plain baseline)   */
   SDR_LAUNCH_PERSISTENT  = 2  /* one persistent mixed-codec launch (sdr_batch) */
 } sdr_launch_mode;
@@ -205,9 +206,9 @@ int sdr_plan_create(const sdr_column* cols, uint32_t n_cols, uint32_t launch_mod
 int sdr_plan_launch(sdr_plan* plan, sdr_stream_t stream);
 /* Launch only the kernels of one codec (codec 0 = all). */
 int sdr_plan_launch_codec(sdr_plan* plan, uint32_t codec, sdr_stream_t stream);
-/* Number of decode launches of a plan, one for each codec and width (in the
- * plain mode for each segment); sdr_plan_launch enqueues those of a batched
- * plan as one kernel where it can. */
+/* Number of a plan's codecs and widths, in the plain mode of its segments: the
+ * decode launches that it makes at most. sdr_plan_launch enqueues the codecs of
+ * a batched plan as one kernel where it can. */
 int sdr_plan_num_launches(const sdr_plan* plan);
 int sdr_plan_null_counts(sdr_plan* plan, int64_t* counts, uint32_t n_cols, sdr_stream_t stream);
 int sdr_plan_destroy(sdr_plan* plan);

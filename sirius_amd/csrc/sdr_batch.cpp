@@ -2,8 +2,9 @@
 // device work queue (one arena: header, entries grouped by decoder and
 // width, FSST columns, chunks, segments, look-back state) in pinned memory, and
 // launches a kernel that copies it to the device, one for the string pre-pass,
-// the fixed-width segments and the null masks, and one for the string chunks;
-// optionally all but the first as a replayed hipGraph.
+// the fixed-width segments and the null masks, one for the string chunks and one
+// for columns that must be tried again; optionally the middle two as a replayed
+// hipGraph.
 #include "sdr_batch.hpp"
 #include "sdr_internal.hpp"
 #include "sdr_kernels.hpp"

@@ -277,8 +277,8 @@ int collect(sdr_server* sv)
   for (auto& sl : sv->slots) {
     if (!sl.busy) continue;
     int rc = SDR_OK;
-    // the end event is the slot's last work (after a batch's read-back), so
-    // once it has passed the launch is done and its times are readable
+    // the end event is the slot's last work, so once it has passed the launch
+    // is done and its times are readable
     const hipError_t e = hipEventQuery(sl.ev_end);
     if (e == hipErrorNotReady) continue;
     if (e != hipSuccess) return fail(SDR_E_HIP, "server launch: %s", hipGetErrorString(e));
