@@ -10,8 +10,8 @@
 // A fixed-width group kernel's grid is its resident capacity.  Fixed-width
 // entries are independent, so block b takes entries b, b + grid, ... with no
 // claim at all; its four wavefronts decode an entry's units (an RLE slice is
-// decoded by the whole block).  The FSST kernel runs one block per chunk; a
-// chunk waits on its predecessors' offsets.  By
+// decoded by the whole block).  The FSST kernel runs one block per chunk, which
+// waits for the offsets of the chunks before it in its column.  By
 // default fixed-width segments are not queued: the front kernel decodes them
 // beside the FSST pre-pass.
 #include "dec_fsst.hpp"
@@ -138,9 +138,10 @@ __global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6)
 // workgroups that run, in whatever order those are started.  Right behind it on the
 // stream: what follows a launch finds its columns complete.  Nearly always there are
 // none (a served batch of 128 requests 334 us without this kernel, 333 us with it, 355 us
-// with a ticket for each chunk at once).
-// (Its occupancy is that of k_bgroup_fsst, with which it shares a called function.)
-__global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_batch_again(BatchQueue* __restrict__ q, uint32_t n)
+// with a ticket for each chunk at once).  Its occupancy is that of k_bgroup_fsst, with
+// which it shares a called function.
+__global__ __launch_bounds__(FSST_THREADS) __attribute__((amdgpu_waves_per_eu(6))) void k_batch_again(
+  BatchQueue* __restrict__ q, uint32_t n)
 {
   __shared__ FsstSmem sm;
   __shared__ uint32_t s_next;
